@@ -140,6 +140,7 @@ constexpr Launcher kLaunchers[] = {rt::launch_gemv,          // streaming kernel
                                    rt::launch_gemm_stream,   // f16 / Q8_0H weights against a few dozen activation rows: one pass over the weight
                                    rt::launch_gemm_nt,       // K-contiguous f16 / Q8_0H problems: the large-tile kernel
                                    rt::launch_gemm_nn_smalln, // f16 products with an untransposed narrow rhs (attention P.V)
+                                   rt::launch_gemm_limb,     // f32 activations against f32 operands or Q8_0F weights: bf16 matrix cores, exact limbs
                                    rt::launch_gemm_f32,      // f32 products whose operands each have a contiguous axis
                                    rt::launch_gemm_q4k,      // Q4_K weights against many activation rows
                                    rt::launch_gemm};         // anything
@@ -383,8 +384,9 @@ rt_status rt_matmul_workspace_bytes(rt_ctx *ctx, const rt_matmul_desc *desc, uin
     std::string why;
     rt_status st = rt::make_spec(*desc, spec, p, &why);
     if (st != RT_OK) return fail(ctx, st, why);
-    // only the large-tile GEMM shares a problem among workgroups; the streaming kernels take M <= 16
+    // only the tiled kernels share a problem among workgroups; the streaming kernels take M <= 16
     if (p.kernel == RT_KERNEL_GEMM_F16) *bytes = rt::gemm_nt_workspace_bytes(p, ctx->dev);
+    if (p.kernel == RT_KERNEL_GEMM_F32) *bytes = rt::gemm_limb_workspace_bytes(p, ctx->dev);
     return RT_OK;
     RT_GUARD_END(ctx)
 }

@@ -486,11 +486,12 @@ RT_TUNABLE(g_gemm_tile, 0);
 hipError_t launch_gemm(const Problem &p, const void *A, const void *B, const void *bias, void *out,
                        hipStream_t stream, const DeviceInfo &dev) {
     if (p.stacks > 65535) return hipErrorNotSupported;
-    // 128 x 128 tiles unless they would leave the chip under two workgroups per compute unit
-    int ts = 128;
+    // f16: 128 x 128 tiles unless they would leave the chip under two workgroups per compute unit.  Only small f32 products
+    // come here (gemm_limb_kernel takes the rest): 64 x 64.
+    int ts = p.act_dt == RT_F16 ? 128 : 64;
     const int64_t big = ((p.M + 127) / 128) * ((p.N + 127) / 128) * p.stacks;
     if (big < 2 * (int64_t)dev.num_cus) ts = 64;
-    if (g_gemm_tile == 64 || g_gemm_tile == 128) ts = g_gemm_tile;
+    if (p.act_dt == RT_F16 && (g_gemm_tile == 64 || g_gemm_tile == 128)) ts = g_gemm_tile;
     const int64_t gy = (p.M + ts - 1) / ts, gx = (p.N + ts - 1) / ts;
     if (gy > 65535) return hipErrorNotSupported;
     GemmArgs g{};
@@ -521,8 +522,7 @@ hipError_t launch_gemm(const Problem &p, const void *A, const void *B, const voi
         if (ts == 64) launch_a<half_t, 64>(amode, bmode, grid, stream, g);
         else launch_a<half_t, 128>(amode, bmode, grid, stream, g);
     } else {
-        if (ts == 64) launch_a<float, 64>(amode, bmode, grid, stream, g);
-        else launch_a<float, 128>(amode, bmode, grid, stream, g);
+        launch_a<float, 64>(amode, bmode, grid, stream, g);
     }
     return hipGetLastError();
 }

@@ -1,18 +1,18 @@
-// f32 GEMM on the matrix cores for operands with a contiguous axis:
+// Small f32 products on the f32 matrix cores:
 //   C[s, i, j] = sum_k A[s, i, k] * B[s, k, j] (+ bias),  f32 in, f32 accumulate, f32 out,
-// A K-contiguous; B either N-contiguous (`lhs.matmul(rhs)`, the Whisper encoder's
-// [1500 x 384] . [384 x 1536]) or K-contiguous (Linear's W.gemm(x, b, false, true, true) with f32
-// weights).  v_mfma_f32_16x16x4_f32 takes one f32 per lane and operand, so neither tile needs a
-// transpose: A sits in LDS as [row][k] and B as it lies in memory, [k][col] or [col][k].
+// A K-contiguous; B either N-contiguous (`lhs.matmul(rhs)`) or K-contiguous (Linear's W.gemm(x, b, false, true, true) with
+// f32 weights).  gemm_limb_kernel takes every f32 product that is worth splitting into bf16 limbs (it is declined only
+// when K is at most two of its stages and its tiles do not fill the compute units, see launch_gemm_limb); what is left
+// here is bound by launch, first loads and stores, and the f32 MFMA's operands need no splitting: 8 heads x
+// [232 x 64] . [64 x 232] 4.6 us here, 5.2 there.
+// v_mfma_f32_16x16x4_f32 takes one f32 per lane and operand, so neither tile needs a transpose: A sits in LDS as [row][k]
+// and B as it lies in memory, [k][col] or [col][k].
 //
-// 128 x 128, 96 x 96 or 32 x 96 outputs per 256-thread workgroup (2 x 2 wavefronts of 4 x 4, 3 x 3 or
-// 1 x 3 MFMA tiles).  An f32 MFMA is slow (32 cycles for 2048 flop), so LDS and memory traffic are light and
-// the launcher picks the tile by how much the fixed costs weigh (see launch_gemm_f32).  K tile 32,
-// two LDS stages, one bare barrier per tile; tile t+1 waits in registers while tile t is multiplied
-// and tile t+2 is in flight.  With K a whole number of tiles the loop has no bound to check; other K
-// (a multiple of 4: attention scores over a head dimension of 80) run the KTAIL variant, whose loads
-// clamp their K offset and whose LDS stores write zeros past K -- selects, not branches, so the loop
-// stays straight-line code either way.
+// 32 x 96 or 32 x 64 outputs per 256-thread workgroup (2 x 2 wavefronts of 1 x 3 or 1 x 2 MFMA tiles), so that about three
+// workgroups share a compute unit and their fixed parts overlap.  K tile 32, two LDS stages, one bare barrier per tile; tile
+// t+1 waits in registers while tile t is multiplied and tile t+2 is in flight.  With K a whole number of tiles the loop has
+// no bound to check; other K (a multiple of 4) run the KTAIL variant, whose loads clamp their K offset and whose LDS stores
+// write zeros past K -- selects, not branches, so the loop stays straight-line code either way.
 //
 // LDS rows are padded so that every fragment read is conflict-free on 64 banks:
 //   [row][k] tiles, stride 36: lane (r = l % 16, q = l / 16) reads word 36 r + 4 kk + q; 36 r mod 64
@@ -20,8 +20,7 @@
 //   [k][col] tile, stride BN + 16 (= 48 mod 64): word (4 kk + q) (BN + 16) + c, the four q rows
 //     start 16 banks apart.
 //
-// Roles in the reference: ops/gemm.rs:305-657 with f32 operands (test_sgemm, ops/matmul.rs:757-829;
-// the Whisper encoder's MLP and attention projections, whisper/mlp.rs:18-22).
+// Roles in the reference: ops/gemm.rs:305-657 with f32 operands (test_sgemm, ops/matmul.rs:757-829).
 #include "device_common.h"
 
 namespace rt {
@@ -276,7 +275,6 @@ static hipError_t launch_f32(const GemmF32Args &g, int64_t stacks, hipStream_t s
     return g.K % F32_BK == 0 ? launch_f32_kt<BM, BN, B_KCONT, false>(g, stacks, st) : launch_f32_kt<BM, BN, B_KCONT, true>(g, stacks, st);
 }
 
-RT_TUNABLE(g_gemm_f32_bm, 0);      // 32 or 96 forces that tile height (0 = by shape)
 RT_TUNABLE(g_gemm_f32_disable, 0); // non-zero sends f32 problems to the generic kernel (for comparisons)
 
 // f32 x f32 with A K-contiguous and B contiguous along K or along its columns, 16-byte aligned
@@ -300,22 +298,9 @@ hipError_t launch_gemm_f32(const Problem &p, const void *A, const void *B, const
     g.o_bs = p.o_bs, g.o_is = p.o_is, g.o_js = p.o_js;
     g.has_bias = p.has_bias, g.bias_on_rows = p.bias_on_rows, g.act = p.act;
     g.nt_out = p.o_js == 1 && (p.o_is * 4) % 128 == 0 && (p.o_bs * 4) % 128 == 0 && ((uintptr_t)out & 127u) == 0;
-    // 32-row tiles put about three workgroups on a compute unit, whose prologues and epilogues then
-    // overlap with each other's MFMAs: better while the fixed costs weigh (26.3 against 28.2 us at
-    // K = 384); 96-row tiles read less LDS per MFMA and win from K of about 1000 on (78 against 81 us at 1536).
-    const int64_t tiles96 = ((p.M + 95) / 96) * ((p.N + 95) / 96) * p.stacks;
-    int bm = (p.K <= 768 || tiles96 < dev.num_cus) ? 32 : 96;
-    // Short contractions (attention scores spelled [.., M, K] . [.., K, N], K = 80): nearly all the time goes
-    // into fetching operands and writing the output, so the largest tile wins while it still gives every
-    // compute unit two workgroups (25.4 against 30.6 us at 32 x [512 x 80] . [80 x 512]).
-    const int64_t tiles128 = ((p.M + 127) / 128) * ((p.N + 127) / 128) * p.stacks;
-    if (p.K <= 128 && tiles128 >= 2 * (int64_t)dev.num_cus) bm = 128;
-    if (g_gemm_f32_bm == 32 || g_gemm_f32_bm == 96 || g_gemm_f32_bm == 128) bm = g_gemm_f32_bm;
-    if (bm == 128) return b_kcont ? launch_f32<128, 128, true>(g, p.stacks, stream) : launch_f32<128, 128, false>(g, p.stacks, stream);
     // up to 64 columns (P . V over a head dimension of 64): 64-column tiles, not two thirds of 96
-    if (bm == 32 && p.N <= 64) return b_kcont ? launch_f32<32, 64, true>(g, p.stacks, stream) : launch_f32<32, 64, false>(g, p.stacks, stream);
-    if (bm == 32) return b_kcont ? launch_f32<32, 96, true>(g, p.stacks, stream) : launch_f32<32, 96, false>(g, p.stacks, stream);
-    return b_kcont ? launch_f32<96, 96, true>(g, p.stacks, stream) : launch_f32<96, 96, false>(g, p.stacks, stream);
+    if (p.N <= 64) return b_kcont ? launch_f32<32, 64, true>(g, p.stacks, stream) : launch_f32<32, 64, false>(g, p.stacks, stream);
+    return b_kcont ? launch_f32<32, 96, true>(g, p.stacks, stream) : launch_f32<32, 96, false>(g, p.stacks, stream);
 }
 
 } // namespace rt

@@ -1,0 +1,90 @@
+"""f32 products on the bf16 matrix cores (kernels_gemm_limb.hip) at the sizes and values where they can go wrong, against
+float64.
+
+The tolerance is the rounding of the accumulation: a sum of K products takes at most six MFMAs per 16 k, each of which rounds
+the accumulator once, plus the fold of a block, the sum over the shares of K and the bias, every rounding at most 2^-24 of
+the magnitudes summed."""
+import numpy as np
+import pytest
+import torch
+
+from ratchet_amd import DType, Device, Tensor, Quantization, Quantizer, dequantize
+
+pytestmark = pytest.mark.gpu
+
+
+def bound(x, y, bias):
+    k = x.shape[-1]
+    mag = np.abs(x).astype(np.float64) @ np.abs(y).astype(np.float64)
+    return 2.0**-24 * (6 * (k / 16 + 1) + 4) * (mag + (0 if bias is None else np.abs(bias)))
+
+
+def run(device, a, b, bias, tl, tr, to):
+    t = lambda v: None if v is None else Tensor.from_data(v).to(device)
+    return t(a).gemm(t(b), t(bias), tl, tr, to).resolve().to(Device.CPU).storage
+
+
+@pytest.mark.parametrize("tl,tr,to", [(False, False, False), (True, False, False), (False, True, False), (True, False, True), (False, True, True)])
+@pytest.mark.parametrize("stacks,m,k,n", [
+    (1, 65, 65, 129), (1, 97, 1500, 64), (3, 130, 99, 70), (1, 1500, 68, 33), (1, 16, 2049, 300), (1, 40, 3001, 40), (7, 300, 65, 301),
+    (1, 9, 66, 20001), (40, 129, 64, 130), (1, 2000, 96, 1999)])
+def test_layouts_and_edges(device, stacks, m, k, n, tl, tr, to):
+    rng = np.random.default_rng(m * 7 + k)
+    x, y = rng.standard_normal((stacks, m, k)).astype(np.float32), rng.standard_normal((stacks, k, n)).astype(np.float32)
+    bias = rng.standard_normal(m if to else n).astype(np.float32) if stacks == 1 else None
+    got = run(device, np.swapaxes(x, 1, 2) if tl else x, np.swapaxes(y, 1, 2) if tr else y, bias, tl, tr, to)
+    b = 0 if bias is None else bias[:, None] if to else bias
+    want = x.astype(np.float64) @ y.astype(np.float64) + b
+    err = np.abs((np.swapaxes(got, 1, 2) if to else got) - want)
+    assert (err <= bound(x, y, None if bias is None else b)).all(), (err / bound(x, y, None if bias is None else b)).max()
+
+
+@pytest.mark.parametrize("rows,n,k", [(9, 33, 64), (17, 127, 96), (65, 129, 32), (129, 257, 320), (200, 2560, 10240), (300, 100, 4096), (13, 20000, 288)])
+@pytest.mark.parametrize("swap", [False, True])
+def test_codes_with_f32_scales(device, rows, n, k, swap):
+    rng = np.random.default_rng(rows + k)
+    w = Quantizer(Quantization.SInt8).quantize(Tensor.from_data(rng.standard_normal((n, k)).astype(np.float32)).to(device))
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    wf = dequantize(w).to(Device.CPU).storage
+    bias = rng.standard_normal(n if not swap else n).astype(np.float32)
+    xt, bt = Tensor.from_data(x).to(device), Tensor.from_data(bias).to(device)
+    if swap:  # out [n, rows], whose contiguous axis is the activations': no bias there
+        got = w.gemm(xt, None, False, True, False).resolve().to(Device.CPU).storage.T
+        bias = np.zeros_like(bias)
+    else:
+        got = w.gemm(xt, bt, False, True, True).resolve().to(Device.CPU).storage
+    want = x.astype(np.float64) @ wf.astype(np.float64).T + bias
+    assert (np.abs(got - want) <= bound(x, wf.T, bias)).all()
+
+
+@pytest.mark.parametrize("scale_x,scale_y", [(1e-36, 1e3), (1e18, 1e18), (1e-20, 1e-15), (1e30, 1e-30)])
+def test_magnitudes(device, scale_x, scale_y):
+    """Limbs of small numbers reach into bf16's subnormals; results leave the range of f32 at either end."""
+    rng = np.random.default_rng(3)
+    x, y = (rng.standard_normal((70, 200)) * scale_x).astype(np.float32), (rng.standard_normal((200, 90)) * scale_y).astype(np.float32)
+    got = run(device, x, y, None, False, False, False)
+    want = x.astype(np.float64) @ y.astype(np.float64)
+    with np.errstate(over="ignore"):
+        inside = np.abs(want) < 3e38
+    # the last limb is a multiple of bf16's smallest subnormal number, 2^-133: half of that of the other operand per product;
+    # and the results' own subnormals
+    tiny = 2.0**-134 * (np.abs(y).sum(0)[None, :] + np.abs(x).sum(1)[:, None]) + 200 * 2.0**-149
+    assert (np.abs(got - want) <= bound(x, y, None) + tiny)[inside].all()
+    assert np.isinf(got[np.abs(want) > 4e38]).all()
+
+
+def test_values_that_are_not_finite(device):
+    """What the f32 arithmetic gives: infinities of either sign, NaN from inf - inf, inf * 0 and NaN operands, numbers that
+    round past the largest bf16."""
+    rng = np.random.default_rng(4)
+    x, y = rng.standard_normal((130, 160)).astype(np.float32), rng.standard_normal((160, 140)).astype(np.float32)
+    x[3, 5], x[7, 0], x[9, 9], x[9, 10] = np.inf, -np.inf, np.inf, -np.inf
+    x[20, 159], x[64, 31], y[8, 60], y[5, 100] = np.nan, 3.4e38, np.inf, 0.0
+    y[31, 2] = 0.25
+    for trans in (False, True):
+        got = run(device, x, y.T.copy() if trans else y, None, False, trans, False)
+        with np.errstate(invalid="ignore", over="ignore"):
+            want = (x.astype(np.float64) @ y.astype(np.float64)).astype(np.float32)
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+        fine = np.isfinite(want)
+        assert np.isfinite(got[fine]).all() and np.allclose(got[fine], want[fine], rtol=1e-4, atol=1e-4)
