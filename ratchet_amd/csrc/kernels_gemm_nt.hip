@@ -1,7 +1,9 @@
 // MFMA GEMMs for the Linear / QK^T form, where both operands are K-contiguous:
 //   C[s, i, j] = sum_k A[s, i, k] * B[s, j, k] (+ bias),  f16 in, f32 accumulate, f16 out.
-// A is f16 or a Q8_0H weight; B is f16.  Four kernels, chosen by launch_gemm_nt:
+// A is f16 or a Q8_0H weight; B is f16.  Five kernels, chosen by launch_gemm_nt:
 //
+//   gemm_nt_wide_kernel    f16 x f16, K % 64 == 0, many activation rows: 320 x 256 tiles, eight wavefronts that
+//                          both load and multiply (half the operand bytes per product of the 160 x 128 tiles)
 //   gemm_nt_dl_kernel      f16 x f16, K % 64 == 0: 160 x 128 tiles, tiles loaded global -> LDS
 //                          directly into a ring of stages by two wavefronts that do nothing else,
 //                          issue order pinned (the fast path for the Phi-2 prefill shape:
@@ -14,11 +16,11 @@
 //   gemm_nt_kernel         everything else this file takes (ragged K, Q8_0H with K % 256 != 0,
 //                          short K without a contiguous output axis): register-staged, two LDS stages
 //
-// Common to all: 2 x 2 multiplying wavefronts, v_mfma_f32_16x16x32_f16 with A rows on the MFMA's
+// Common to all: 2 x 2 multiplying wavefronts (the wide kernel: 2 x 4), v_mfma_f32_16x16x32_f16 with A rows on the MFMA's
 // lane index, XOR-swizzled or odd-stride LDS rows so that fragment reads are conflict-free, an
 // epilogue that transposes through LDS and stores 128 bits along the contiguous output axis, and
-// (large tiles) workgroup ids remapped so that the 8 XCDs each take a contiguous range of A row
-// blocks: all column blocks of one A row block share one L2 copy of its tiles.
+// workgroup ids remapped so that each of the 8 XCDs takes a block of neighbouring tiles, whose
+// operands its L2 holds once (nt_tile_of).
 //
 // gemm_nt_kernel's pipeline per K tile of 64: global loads of tile t+2 into registers, MFMAs on LDS
 // stage t, then the registers of tile t+1 -> the other LDS stage, one barrier.  For Q8_0H it widens
@@ -29,6 +31,7 @@
 // W.gemm(x, b, false, true, true) (crates/ratchet-nn/src/linear.rs:17-24) and attention's
 // Q.matmul(K, false, true) (phi3/attn.rs:142-158) as the callers.
 #include "device_common.h"
+#include <algorithm>
 #include <utility>
 
 namespace rt {
@@ -46,6 +49,7 @@ struct GemmNtArgs {
     int64_t o_bs, o_is, o_js;
     int has_bias, bias_on_rows, act;
     int tiles_i, tiles_j;
+    int xi, pj; // XCD-aware order of the tiles (nt_tile_of)
     int vec_epilogue; // o_is == 1 and rows of the output 16-byte aligned: LDS-staged 128-bit stores
     // split K (direct-to-LDS kernels): blockIdx.z owns K range [z * k_len, (z + 1) * k_len) and writes its
     // f32 sums to partial [stack][split][N][M]; a second kernel adds them up, then bias, activation, rounding
@@ -54,27 +58,24 @@ struct GemmNtArgs {
     float *partial;
 };
 
-// Which output tile a workgroup takes.  Workgroup ids go round the 8 XCDs, each with an L2 of its own:
-// XCD x takes the contiguous range x * ntiles / 8 .. of the tiles in row-major order (A row block major),
-// so all column blocks of one A row block share one L2 copy of it.  When that range is whole A row
-// blocks and there are more than four column blocks, the range is walked in panels of four column
-// blocks (all of the XCD's row blocks against four column blocks, then the next four): the 32
-// workgroups an XCD runs at a time then share 8 + 4 operand blocks instead of 1 + 32, which at
-// [4096 x 2560] . [10240 x 2560]^T cut what the L2s fetch from 1.39 GB per launch (19 x the operands).
-__device__ __forceinline__ void nt_tile_of(int64_t wg, int tiles_i, int tiles_j, int64_t &ti, int64_t &tj) {
-    constexpr int PJ = 4;
-    const int64_t ntiles = (int64_t)tiles_i * tiles_j;
-    if (ntiles % 8 == 0) wg = (wg & 7) * (ntiles >> 3) + (wg >> 3);
-    if (tiles_i % 8 == 0 && tiles_j > PJ) {
-        const int64_t rows = tiles_i >> 3, chunk = rows * tiles_j; // per XCD
-        const int64_t x = wg / chunk, r = wg - x * chunk;
-        const int64_t panels = (tiles_j + PJ - 1) / PJ;
-        const int64_t p = min(r / (rows * PJ), panels - 1), q = r - p * rows * PJ;
-        const int64_t w = min<int64_t>(PJ, tiles_j - p * PJ); // the last panel may be narrower
-        ti = x * rows + q / w, tj = p * PJ + q % w;
+// Which output tile a workgroup takes.  Workgroup ids go round the 8 XCDs, each with an L2 of its own.
+// g.xi > 0: the grid of tiles is cut into xi x (8 / xi) equal blocks, one per XCD, and a block is walked in panels
+// of g.pj columns, so that the 32 workgroups an XCD runs at a time share the fewest operand rows
+// (nt_set_tiles chooses both).  Otherwise XCD x takes the contiguous range x * ntiles / 8 .. of the tiles in row-major
+// order when that comes out even, and the plain order when not.
+__device__ __forceinline__ void nt_tile_of(const GemmNtArgs &g, int64_t wg, int64_t &ti, int64_t &tj) {
+    const int64_t ntiles = (int64_t)g.tiles_i * g.tiles_j;
+    if (g.xi > 0) {
+        const int64_t x = wg & 7, r = wg >> 3;
+        const int64_t rows = g.tiles_i / g.xi, xj = 8 / g.xi, cols = g.tiles_j / xj; // an XCD's block
+        const int64_t panels = (cols + g.pj - 1) / g.pj;
+        const int64_t p = min(r / (rows * g.pj), panels - 1), q = r - p * rows * g.pj;
+        const int64_t w = min<int64_t>(g.pj, cols - p * g.pj); // the last panel may be narrower
+        ti = (x / xj) * rows + q / w, tj = (x % xj) * cols + p * g.pj + q % w;
         return;
     }
-    ti = wg / tiles_j, tj = wg - ti * tiles_j;
+    if (ntiles % 8 == 0) wg = (wg & 7) * (ntiles >> 3) + (wg >> 3);
+    ti = wg / g.tiles_j, tj = wg - ti * g.tiles_j;
 }
 
 // Timing-only variants of gemm_nt_dl_kernel for the measurement probes (a bit mask: 1 no tile loads, 2 no MFMAs,
@@ -107,7 +108,8 @@ __device__ __forceinline__ void nt_cvt_i8x4(uint32_t v, half2_t &lo, half2_t &hi
 // axis is contiguous in the output (o_is == 1): the wavefront's sub-tile is transposed through
 // LDS (free once the main loop's last barrier has passed) so that every lane stores 8
 // consecutive outputs (128 bits); otherwise bounds-checked scalar stores.
-template <int TM, int TN, int WM, int WN>
+// PARTS: the transposition takes the B rows in that many parts, one after the other through the same LDS.
+template <int TM, int TN, int WM, int WN, int PARTS = 1>
 __device__ __forceinline__ void nt_epilogue(const GemmNtArgs &g, float4_t (&acc)[TM][TN], uint8_t *smem, int64_t s,
                                             int64_t i0, int64_t j0, int wi, int wj, int wave, int lane) {
     const int fr = lane & 15, fg = lane >> 4;
@@ -130,38 +132,48 @@ __device__ __forceinline__ void nt_epilogue(const GemmNtArgs &g, float4_t (&acc)
     half_t *out = g.out + s * g.o_bs;
     if (g.vec_epilogue) {
         constexpr int EROW = WM + 8;                       // halfs per staged B-row (+16 B pad)
-        half_t *es = (half_t *)smem + wave * (WN * EROW);
-        rt_with_act(g.act, [&](auto has_act) {
+        constexpr int TP = TN / PARTS, WP = WN / PARTS;    // MFMA tiles and B rows of a part
+        static_assert(TN % PARTS == 0, "parts are whole MFMA tiles");
+        half_t *es = (half_t *)smem + wave * (WP * EROW);
+        float bi[TM]; // the bias of this lane's A rows, asked for once
 #pragma unroll
-            for (int a = 0; a < TM; a++) {
-                const int64_t i = i0 + wi * WM + a * 16 + fr;
-                float bi = 0.f;
-                if (g.has_bias && g.bias_on_rows && i < g.M) bi = (float)g.bias[i];
+        for (int a = 0; a < TM; a++) {
+            const int64_t i = i0 + wi * WM + a * 16 + fr;
+            bi[a] = g.has_bias && g.bias_on_rows && i < g.M ? (float)g.bias[i] : 0.f;
+        }
 #pragma unroll
-                for (int b = 0; b < TN; b++)
+        for (int h = 0; h < PARTS; h++) {
+            const int64_t jh = j0 + wj * WN + h * WP;
+            rt_with_act(g.act, [&](auto has_act) {
 #pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        const int jl = b * 16 + 4 * fg + r;
-                        float v = acc[a][b][r] + bi;
-                        if (g.has_bias && !g.bias_on_rows) v += (float)g.bias[min(j0 + wj * WN + jl, g.N - 1)];
-                        v = rt_act_k<decltype(has_act)::value>(v);
-                        es[jl * EROW + a * 16 + fr] = (half_t)v;
+                for (int a = 0; a < TM; a++) {
+#pragma unroll
+                    for (int b = 0; b < TP; b++)
+#pragma unroll
+                        for (int r = 0; r < 4; r++) {
+                            const int jl = b * 16 + 4 * fg + r;
+                            float v = acc[a][h * TP + b][r] + bi[a];
+                            if (g.has_bias && !g.bias_on_rows) v += (float)g.bias[min(jh + jl, g.N - 1)];
+                            v = rt_act_k<decltype(has_act)::value>(v);
+                            es[jl * EROW + a * 16 + fr] = (half_t)v;
+                        }
+                }
+            });
+            asm volatile("" ::: "memory"); // same wavefront reads back below; DS operations complete in order
+            constexpr int VPR = WM / 8;    // 128-bit vectors per staged row
+            for (int v = lane; v < WP * VPR; v += 64) {
+                const int jl = v / VPR, c = v - jl * VPR;
+                const int64_t j = jh + jl, i = i0 + wi * WM + 8 * c;
+                if (j < g.N) {
+                    if (i + 8 <= g.M) {
+                        __builtin_nontemporal_store(*(const uint4_t *)(es + jl * EROW + 8 * c), (uint4_t *)(out + j * g.o_js + i)); // written once, not read back here
+                    } else {
+                        for (int e = 0; e < 8; e++)
+                            if (i + e < g.M) out[j * g.o_js + i + e] = es[jl * EROW + 8 * c + e];
                     }
-            }
-        });
-        asm volatile("" ::: "memory"); // same wavefront reads back below; DS operations complete in order
-        constexpr int VPR = WM / 8;    // 128-bit vectors per staged row
-        for (int v = lane; v < WN * VPR; v += 64) {
-            const int jl = v / VPR, c = v - jl * VPR;
-            const int64_t j = j0 + wj * WN + jl, i = i0 + wi * WM + 8 * c;
-            if (j < g.N) {
-                if (i + 8 <= g.M) {
-                    __builtin_nontemporal_store(*(const uint4_t *)(es + jl * EROW + 8 * c), (uint4_t *)(out + j * g.o_js + i)); // written once, not read back here
-                } else {
-                    for (int e = 0; e < 8; e++)
-                        if (i + e < g.M) out[j * g.o_js + i + e] = es[jl * EROW + 8 * c + e];
                 }
             }
+            asm volatile("" ::: "memory");
         }
         return;
     }
@@ -209,7 +221,7 @@ __global__ __launch_bounds__(NT_THREADS, (BM * BN <= 128 * 64 ? 3 : 1)) void gem
     const int fr = lane & 15, fg = lane >> 4;            // fragment row / K group
 
     int64_t ti, tj;
-    nt_tile_of(blockIdx.x, g.tiles_i, g.tiles_j, ti, tj); // XCD-aware tile order (see the file comment)
+    nt_tile_of(g, blockIdx.x, ti, tj); // XCD-aware tile order (see the file comment)
     const int64_t i0 = ti * BM, j0 = tj * BN;
     const int64_t s = blockIdx.y;
     const int64_t a_el = (g.a_stack == 1 ? 0 : s) * g.a_bs, b_el = (g.b_stack == 1 ? 0 : s) * g.b_bs;
@@ -413,7 +425,7 @@ __global__ __launch_bounds__(NT_THREADS + 64 * LW) void gemm_nt_dl_kernel(GemmNt
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
 
     int64_t ti, tj;
-    nt_tile_of(blockIdx.x, g.tiles_i, g.tiles_j, ti, tj); // XCD-aware tile order (see the file comment)
+    nt_tile_of(g, blockIdx.x, ti, tj); // XCD-aware tile order (see the file comment)
     const int64_t i0 = ti * BM, j0 = tj * BN;
     const int64_t s = blockIdx.y;
     const int64_t kbase = (int64_t)blockIdx.z * g.k_len;
@@ -544,6 +556,121 @@ __global__ __launch_bounds__(NT_THREADS + 64 * LW) void gemm_nt_dl_kernel(GemmNt
 }
 
 // ---------------------------------------------------------------------------
+// f16 x f16 with many activation rows: 320 x 256 outputs per workgroup, one workgroup per compute unit.
+// A K step of 64 is 2560 cycles of MFMAs per SIMD against 74 KB of tiles to fetch (29 bytes per cycle;
+// the 160 x 128 tile needs 58, more than the L2s deliver to all compute units at once) and 1792 of
+// LDS fragment reads.  Eight wavefronts of 160 x 64 outputs, two per SIMD: 160 accumulator registers leave no
+// room for a second fragment set of everything, so an A fragment is read for the next half step into the registers
+// its last MFMA has just left, and only the B fragments and the last two A fragments are held twice.  Every
+// wavefront loads an eighth of each tile (LDS-DMA, between its MFMAs): wavefronts that only load would halve the
+// registers of the ones that multiply.
+//
+// Two LDS stages.  Per tile: half step 0 on the fragments in registers, reading half step 1's; then, all of the stage read
+// and the next tile landed (its loads have had a whole tile's time), one barrier; half step 1, reading the next
+// tile's first fragments and issuing the loads of the tile after it into the stage just left.
+// 10240 x 2560 weights against 2048 / 4096 activation rows: 89.7 / 177.0 us (1.20 / 1.21 PFLOP/s) where the 160 x 128 tiles take
+// 110.7 / 218.5; 12288 x 3072 against 1300 rows 102 for 148.
+// ---------------------------------------------------------------------------
+template <int BM, int BN, int WI, int WJ>
+__global__ __launch_bounds__(64 * WI * WJ) void gemm_nt_wide_kernel(GemmNtArgs g) {
+    constexpr int WAVES = WI * WJ, WM = BM / WI, WN = BN / WJ, TM = WM / 16, TN = WN / 16;
+    constexpr int TD = 2, TS = TM - TD; // A fragments held twice (the last TD) and once
+    constexpr int ACH = BM / 8 / WAVES, BCH = BN / 8 / WAVES; // 8-row chunks of a tile per wavefront
+    constexpr int STAGE_BYTES = (BM + BN) * NT_LDK * 2;
+    static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0 && TS >= TD + TN && ACH + BCH <= TM, "chunks must deal out evenly");
+
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    int64_t ti, tj;
+    nt_tile_of(g, blockIdx.x, ti, tj); // XCD-aware tile order (see the file comment)
+    const int64_t i0 = ti * BM, j0 = tj * BN;
+    const int64_t s = blockIdx.y;
+    const half_t *A = (const half_t *)g.A + (g.a_stack == 1 ? 0 : s) * g.a_bs + i0 * g.a_rs;
+    const half_t *B = g.B + (g.b_stack == 1 ? 0 : s) * g.b_bs + j0 * g.b_js;
+    const int nk = (int)(g.K / NT_BK);
+    const int a_last = (int)min<int64_t>(BM, g.M - i0) - 1, b_last = (int)min<int64_t>(BN, g.N - j0) - 1; // rows past them repeat the last
+
+    // Chunk c of this wavefront: LDS rows 8 (wave + WAVES c) .. + 7 of the A rows, then of the B rows; lane l fills row l / 8,
+    // slot l % 8, which holds K-vector (l % 8) ^ ((row >> 1) & 7).  Row offsets are computed at each use: the vector ALU has
+    // time for it, the register file has no room to keep them.
+    auto issue_chunk = [&](int c, uint32_t stage, int64_t k0) __attribute__((always_inline)) {
+        const bool is_a = c < ACH;
+        const int cc = is_a ? c : c - ACH;
+        int l = lane;
+        asm volatile("" : "+v"(l));
+        const int row = (wave + WAVES * cc) * 8 + (l >> 3);
+        const uint32_t kv = (uint32_t)((l & 7) ^ ((row >> 1) & 7));
+        const uint32_t off = (uint32_t)min(row, is_a ? a_last : b_last) * (uint32_t)(2 * (is_a ? g.a_rs : g.b_js)) + 16u * kv; // < 2^32: launcher
+        const uint8_t *base = (const uint8_t *)((is_a ? A : B) + k0); // wave-uniform
+        const uint32_t dst = stage + (uint32_t)((is_a ? 0 : BM) + (wave + WAVES * cc) * 8) * (NT_LDK * 2);
+        // as asm: behind the builtin the compiler waits for every load in flight before the next fragment read, which it
+        // cannot tell from a read of what the load writes; no register is written, and the barrier's wait covers it
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off), "s"(base) : "memory");
+    };
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)smem;
+
+    const int wi = wave / WJ, wj = wave % WJ;
+    const int fr = lane & 15, fg = lane >> 4;
+    // byte addresses of this lane's first A and B fragments of half step 0 in stage 0 (half step 1: the slot's bit 2 flipped)
+    const uint32_t slot = (uint32_t)((fg ^ ((fr >> 1) & 7)) << 4);
+    const uint32_t ra0 = (uint32_t)(wi * WM + fr) * (NT_LDK * 2) + slot, rb0 = (uint32_t)(BM + wj * WN + fr) * (NT_LDK * 2) + slot;
+
+    float4_t acc[TM][TN];
+#pragma unroll
+    for (int a = 0; a < TM; a++)
+#pragma unroll
+        for (int b = 0; b < TN; b++) acc[a][b] = float4_t{0.f, 0.f, 0.f, 0.f};
+    half8_t fs[TS], fd0[TD], fd1[TD], fb0[TN], fb1[TN];
+
+    // One half step: the MFMAs of the fragments in hand, the next half step's read behind them from `ra`, `rb`.
+    auto half_step = [&](half8_t (&fd)[TD], half8_t (&fb)[TN], half8_t (&fdn)[TD], half8_t (&fbn)[TN], uint32_t ra, uint32_t rb, auto Lc, uint32_t stage,
+                         int64_t k0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int a = 0; a < TM; a++) {
+#pragma unroll
+            for (int b = 0; b < TN; b++) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb[b], a < TS ? fs[a < TS ? a : 0] : fd[a < TS ? 0 : a - TS], acc[a][b], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            if (a < TS) fs[a < TS ? a : 0] = __builtin_bit_cast(half8_t, *(const uint4_t *)(smem + ra + a * 16 * NT_LDK * 2));
+            if (a < TN) fbn[a < TN ? a : 0] = __builtin_bit_cast(half8_t, *(const uint4_t *)(smem + rb + a * 16 * NT_LDK * 2));
+            if (a >= TN && a < TN + TD) fdn[a >= TN && a < TN + TD ? a - TN : 0] = __builtin_bit_cast(half8_t, *(const uint4_t *)(smem + ra + (TS + a - TN) * 16 * NT_LDK * 2));
+            if (decltype(Lc)::value && a < ACH + BCH) issue_chunk(a, stage, k0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto meet = [&]() __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); // this wavefront's loads landed, its fragment reads done
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    const std::integral_constant<bool, true> with_loads;
+    const std::integral_constant<bool, false> no_loads;
+
+#pragma unroll
+    for (int c = 0; c < ACH + BCH; c++) issue_chunk(c, lds0, 0);
+    meet(); // tile 0
+#pragma unroll
+    for (int c = 0; c < ACH + BCH; c++) issue_chunk(c, lds0 + STAGE_BYTES, (int64_t)min(1, nk - 1) * NT_BK);
+#pragma unroll
+    for (int a = 0; a < TS; a++) fs[a] = __builtin_bit_cast(half8_t, *(const uint4_t *)(smem + ra0 + a * 16 * NT_LDK * 2));
+#pragma unroll
+    for (int a = 0; a < TD; a++) fd0[a] = __builtin_bit_cast(half8_t, *(const uint4_t *)(smem + ra0 + (TS + a) * 16 * NT_LDK * 2));
+#pragma unroll
+    for (int b = 0; b < TN; b++) fb0[b] = __builtin_bit_cast(half8_t, *(const uint4_t *)(smem + rb0 + b * 16 * NT_LDK * 2));
+    uint32_t cur = 0; // stage of tile kt, in bytes
+    for (int kt = 0; kt < nk; kt++) {
+        half_step(fd0, fb0, fd1, fb1, (ra0 ^ 64u) + cur, (rb0 ^ 64u) + cur, no_loads, 0, 0);
+        meet(); // tile kt + 1 is whole, stage `cur` is free
+        const uint32_t nxt = STAGE_BYTES - cur;
+        // past the last tile: the last one again, into a stage nobody reads from before the loop has ended
+        half_step(fd1, fb1, fd0, fb0, ra0 + nxt, rb0 + nxt, with_loads, lds0 + cur, (int64_t)min(kt + 2, nk - 1) * NT_BK);
+        cur = nxt;
+    }
+    meet(); // nothing may land once the epilogue reuses the stages
+    nt_epilogue<TM, TN, WM, WN, 2>(g, acc, smem, s, i0, j0, wi, wj, wave, lane);
+}
+
+// ---------------------------------------------------------------------------
 // Q8_0H x f16.  Four loading wavefronts, one per SIMD, fetch the int8 tile into registers (a lane: 16 codes of
 // one row), widen it to f16 (exact) and store f16 code tiles into the ring in the f16 kernel's swizzled layout;
 // the activation tile goes global -> LDS directly.  The four multiplying wavefronts run the f16 kernel's
@@ -582,7 +709,7 @@ __global__ __launch_bounds__(NT_THREADS + 64 * LW) void gemm_nt_q8w_kernel(GemmN
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
 
     int64_t ti, tj;
-    nt_tile_of(blockIdx.x, g.tiles_i, g.tiles_j, ti, tj); // XCD-aware tile order (see the file comment)
+    nt_tile_of(g, blockIdx.x, ti, tj); // XCD-aware tile order (see the file comment)
     const int64_t i0 = ti * BM, j0 = tj * BN;
     const int64_t s = blockIdx.y;
     const int64_t kbase = (int64_t)blockIdx.z * g.k_len; // this workgroup's share of K (all of it without a split)
@@ -949,10 +1076,20 @@ static hipError_t launch_nt_dl(const GemmNtArgs &g, int64_t stacks, hipStream_t 
     return g.ksplit > 1 ? launch_splitk_reduce(g, stacks, st) : hipSuccess;
 }
 
+static hipError_t launch_nt_wide(const GemmNtArgs &g, int64_t stacks, hipStream_t st) {
+    constexpr int BM = 320, BN = 256;
+    const size_t lds = (size_t)2 * (BM + BN) * NT_LDK * 2;
+    if (const hipError_t e = ensure_lds_limit<&gemm_nt_wide_kernel<BM, BN, 2, 4>>(); e != hipSuccess) return e;
+    dim3 grid((unsigned)((int64_t)g.tiles_i * g.tiles_j), (unsigned)stacks);
+    hipLaunchKernelGGL((gemm_nt_wide_kernel<BM, BN, 2, 4>), grid, dim3(512), lds, st, g);
+    return hipGetLastError();
+}
+
 // Tunables: non-zero keeps f16 problems on the register-staged kernel; LDS ring depth
 // (3 or 4, 0 = 3) of the direct-to-LDS kernel (for comparisons).
 RT_TUNABLE(g_gemm_nt_no_direct, 0);
 RT_TUNABLE(g_gemm_nt_stages, 0);
+RT_TUNABLE(g_gemm_nt_wide, 0); // 1 / 2: never / always the 320 x 256 tiles (for comparisons)
 RT_TUNABLE(g_gemm_nt_narrow, 0); // 1: never the 64- and 96-row tiles for few activation rows (for comparisons)
 RT_TUNABLE(g_gemm_nt_shortk_parts, 0); // workgroups per strip of the short-K kernel (0 = automatic)
 
@@ -963,6 +1100,29 @@ static hipError_t launch_nt(const GemmNtArgs &g, int64_t stacks, hipStream_t st)
     dim3 grid((unsigned)((int64_t)g.tiles_i * g.tiles_j), (unsigned)stacks);
     hipLaunchKernelGGL((gemm_nt_kernel<BM, BN, Q8, KFULL>), grid, dim3(NT_THREADS), lds, st, g);
     return hipGetLastError();
+}
+
+// The grid of bm x bn tiles and the order its workgroups take them in.  An XCD's share of the tiles is a block of
+// (tiles_i / xi) x (tiles_j xi / 8) where the grid can be cut that way; of the possible cuts, the one whose 32
+// resident workgroups load the fewest bytes of operands per K step that their L2 does not hold already: for
+// [2048 x 10240] . [2560 x 10240]^T (16 x 16 tiles) four row blocks and eight column blocks per XCD
+// instead of two and sixteen.  a_bytes: of an element of A (the codes' one for Q8_0H).
+static bool nt_set_tiles(GemmNtArgs &g, int bm, int bn, int a_bytes) {
+    const int64_t ti = (g.M + bm - 1) / bm, tj = (g.N + bn - 1) / bn;
+    if (ti * tj > 0x7fffffff) return false;
+    g.tiles_i = (int)ti, g.tiles_j = (int)tj;
+    g.xi = 0, g.pj = 1;
+    int64_t least = 0;
+    for (int xi = 8; xi >= 1; xi /= 2) {
+        const int xj = 8 / xi;
+        if (ti % xi || tj % xj) continue;
+        const int64_t rows = ti / xi, cols = tj / xj;
+        // panels of four columns, wider when the block has too few rows to give 32 workgroups eight of them
+        const int64_t pj = std::min(cols, std::max<int64_t>(4, 32 / rows));
+        const int64_t cost = std::min<int64_t>(rows, (31 + pj) / pj) * bm * a_bytes + pj * bn * 2;
+        if (!g.xi || cost < least) g.xi = xi, g.pj = (int)pj, least = cost;
+    }
+    return true;
 }
 
 // Tunable: 0 = automatic, 1 = never take this kernel (for comparisons).
@@ -1057,16 +1217,14 @@ hipError_t launch_gemm_nt(const Problem &p0, const void *A, const void *B, const
         // the K loop.  128 x 64 tiles need a third of the registers and LDS, so several
         // workgroups share a compute unit and one's epilogue overlaps another's loads.
         constexpr int SBM = 128, SBN = 64; // 128 outputs along the contiguous axis: whole cache lines per wavefront row
-        const int64_t ti = (p.M + SBM - 1) / SBM, tj = (p.N + SBN - 1) / SBN;
-        if (ti * tj > 0x7fffffff) return hipErrorNotSupported;
-        g.tiles_i = (int)ti, g.tiles_j = (int)tj;
+        if (!nt_set_tiles(g, SBM, SBN, 2)) return hipErrorNotSupported;
         return kfull ? launch_nt<SBM, SBN, false, true>(g, p.stacks, stream)
                      : launch_nt<SBM, SBN, false, false>(g, p.stacks, stream);
     }
     constexpr int BM = 160, BN = 128;
-    const int64_t ti = (p.M + BM - 1) / BM, tj = (p.N + BN - 1) / BN;
-    if (ti * tj > 0x7fffffff) return hipErrorNotSupported;
-    g.tiles_i = (int)ti, g.tiles_j = (int)tj;
+    const int a_bytes = q8 ? 1 : 2;
+    if (!nt_set_tiles(g, BM, BN, a_bytes)) return hipErrorNotSupported;
+    const int64_t ti = g.tiles_i, tj = g.tiles_j;
     // few activation rows: 160-row tiles leave most compute units idle and a workgroup takes as long for one
     // column of tiles as for four; 64-row tiles, while all of them still run at once, put 2.5 times the workgroups to work
     // (10240 x 2560 f16 weights: 65..128 rows 24.6-25.4 -> 17.2-18.1 us); 96-row tiles where those no longer fit.
@@ -1082,23 +1240,30 @@ hipError_t launch_gemm_nt(const Problem &p0, const void *A, const void *B, const
             g.ksplit = ks, g.k_len = p.K / ks, g.partial = (float *)p.workspace;
     }
     if ((dl_f16 || dl_q8) && bm != BM && g.ksplit == 1) {
-        g.tiles_i = (int)(bm == 64 ? ti64 : ti96);
+        // (up to 64 activation rows: one column of tiles either way)
+        if (!nt_set_tiles(g, bm, BN, a_bytes)) return hipErrorNotSupported;
         // the narrow tiles take as deep a ring as the LDS holds: a stage has only 8 or 12 KB of weights, and what a compute
         // unit has in flight is what it can pull (10240 x 2560 f16 weights, 40 / 64 activation rows, three stages -> six:
         // 22.7 / 23.6 -> 20.0 / 22.1 us with the weights in HBM, 16.3 / 16.8 -> 14.8 / 15.7 from the Infinity Cache)
         if (dl_f16 && bm == 64 && p.N <= 64) {
             // up to 64 activation rows: half the activation tile, a stage of 16 KB and nine of them (40 / 64 rows:
             // 20.0 / 22.1 -> 18.3 / 20.5 us with the weights in HBM, 14.8 / 15.7 -> 12.6 / 13.6 from the Infinity Cache)
-            g.tiles_j = 1;
             return launch_nt_dl<64, 64, 9, 2>(g, p.stacks, stream);
         }
         if (dl_f16) return bm == 64 ? launch_nt_dl<64, BN, 6, 2>(g, p.stacks, stream) : launch_nt_dl<96, BN, 5, 2>(g, p.stacks, stream);
         if (bm == 64 && p.N <= 64) {
             // up to 64 activation rows: half the activation tile is half the MFMAs and folds of a workgroup
-            g.tiles_j = 1;
             return launch_nt_q8w<64, 64, 4>(g, p.stacks, stream);
         }
         return bm == 64 ? launch_nt_q8w<64, BN, 4>(g, p.stacks, stream) : launch_nt_q8w<96, BN, 4>(g, p.stacks, stream);
+    }
+    if (dl_f16 && g.ksplit == 1 && g_gemm_nt_wide != 1 && p.a_rs >= 0 && p.b_js >= 0 && 2 * 320 * std::max(p.a_rs, p.b_js) < (int64_t(1) << 32)) {
+        const int64_t wide = ((p.M + 319) / 320) * ((p.N + 255) / 256) * p.stacks;
+        const int64_t rounds = (ti * tj * p.stacks + dev.num_cus - 1) / dev.num_cus, rounds_wide = (wide + dev.num_cus - 1) / dev.num_cus;
+        // A round of 320 x 256 tiles on all compute units takes 2.5 rounds of 160 x 128 ones (10240 x 2560 weights: 89.7 us at 2048
+        // activation rows, one round, against 110.7 for four; 7680 x 2560, one against three, 76.5 for 82.9).  Two against
+        // five (11008 x 4096 at 2048 rows) and everything with fewer rounds stays on the small tiles.
+        if ((g_gemm_nt_wide == 2 || 5 * rounds_wide < 2 * rounds) && nt_set_tiles(g, 320, 256, 2)) return launch_nt_wide(g, p.stacks, stream);
     }
     if (dl_f16) {
         // two loading wavefronts: one and four measured the same within run-to-run spread
