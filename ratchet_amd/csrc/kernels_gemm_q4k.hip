@@ -23,9 +23,13 @@
 // output tile, run under super-block sb + 1.
 //
 // A workgroup owns 128 weight rows x 64 activation rows: four multiplying wavefronts (32 weight rows
-// x 64 activation rows each: 64 MFMAs per super-block, 8 for the min term) and four that only issue
-// the activation tiles' LDS-DMA loads (one per SIMD, so that no multiplying wavefront shares its SIMD
-// with all of them), one super-block ahead in a ring of two stages.  A staged row is 32 K-vectors
+// x 64 activation rows each: 64 MFMAs per super-block, 8 for the min term).  The activation tiles come by
+// LDS-DMA one super-block ahead in a ring of two stages.  With at most one workgroup per compute unit four more
+// wavefronts issue those loads and nothing else (one per SIMD).  With more the multiplying wavefronts issue
+// them: at 250 registers a SIMD holds two wavefronts, and a second workgroup's multiplying one is worth more there
+// than a loading one, since the parts of a wavefront's step add up (below) and another's run beside them
+// (8192 x 3072 at 300 / 512 / 1000 / 2048 activation rows 42.2 / 42.9 / 85.7 / 177.6 -> 37.9 / 40.3 / 78.3 / 161.5 us;
+// 3072 x 8192 at 1000 rows 99.8 -> 91.9).  A staged row is 32 K-vectors
 // and one of padding: the 16 rows of a fragment read start 4 banks apart and a read address is a
 // base + 16 * step, an immediate.  One barrier per super-block.  The output tile leaves through LDS
 // as 16-byte stores when the output is contiguous along the weight rows.
@@ -67,12 +71,12 @@ constexpr int QR_XSB = QR_BN * QR_ROWB; // bytes per stage = 33 LDS-DMA instruct
 // tiles in flight) measured the same to 1 % at every grid size tried (alternating runs on one device), so the smaller
 // footprint stays: two workgroups fit a compute unit's LDS.
 constexpr int QR_XST = 2;
-constexpr int QR_LW = 4;               // wavefronts that only issue the LDS-DMA, one per SIMD
 constexpr size_t QR_LDS = (size_t)QR_XST * QR_XSB + 2 * QR_BN * 4 * 8;
 
-// TA: MFMA tiles of weight rows per wavefront; MW: multiplying wavefronts (4: each sums the activation fragment of its number)
-template <int TA, int MW>
-__global__ __launch_bounds__(64 * (MW + QR_LW)) void gemm_q4k_kernel(GemmQ4kArgs g) {
+// TA: MFMA tiles of weight rows per wavefront; MW: multiplying wavefronts (4: each sums the activation fragment of its number);
+// LW: wavefronts that only issue the LDS-DMA (4, one per SIMD, or none: the multiplying ones issue it)
+template <int TA, int MW, int LW>
+__global__ __launch_bounds__(64 * (MW + LW), 2) void gemm_q4k_kernel(GemmQ4kArgs g) {
     constexpr int TB = 4;             // MFMA tiles per wavefront: TA of weight rows (second operand), TB of activation rows (first)
     constexpr int BM = 16 * TA * MW;  // weight rows per workgroup
     static_assert(MW == 4, "wavefront w sums the x of activation fragment w: four fragments, four wavefronts");
@@ -95,7 +99,7 @@ __global__ __launch_bounds__(64 * (MW + QR_LW)) void gemm_q4k_kernel(GemmQ4kArgs
     const int64_t last = g.nsb - 1;
     const bool vec_out = g.vec_out && i0 + BM <= g.M; // a whole tile of weight rows, stored 16 bytes at a time
 
-    if (wave >= MW) {
+    if (LW > 0 && wave >= MW) {
         // ---- loading wavefront lw: LDS-DMA instruction i of a stage (i = lw, lw + 4, ...; 33 in all) fills the 1 KB
         // run of slots 64 i .. + 63; slot p is K-vector p % 33 of row p / 33 (the 33rd is padding and repeats the 32nd).
         // Each of the four issues nine: the ninth of wavefronts 1..3 repeats instruction 32.
@@ -203,9 +207,32 @@ __global__ __launch_bounds__(64 * (MW + QR_LW)) void gemm_q4k_kernel(GemmQ4kArgs
     // wavefront's sums of the super-block before are visible.
     auto tile_ready = [&]() {
         asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0)
+        __builtin_amdgcn_s_waitcnt(LW == 0 ? 0x0070 : 0xC07F); // lgkmcnt(0); and, without loading wavefronts, vmcnt(0)
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
+    };
+
+    // LW == 0: this wavefront's share of the activation tile's LDS-DMA, the loading wavefronts' instructions.  As asm: behind the
+    // builtin the compiler makes every fragment read wait for all loads in flight; no register is written by it, and
+    // tile_ready waits for it.
+    constexpr int NX = LW == 0 ? 9 : 1;
+    uint32_t xoff[NX];
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)smem;
+    if constexpr (LW == 0) {
+#pragma unroll
+        for (int n = 0; n < NX; n++) {
+            const uint32_t p = 64u * (uint32_t)min(4 * n + wave, 32) + (uint32_t)lane, row = p / 33u, v = min(p - 33u * row, 31u);
+            xoff[n] = 2u * ((uint32_t)min(j0 + (int64_t)row, g.N - 1) * (uint32_t)g.b_js + 8u * v);
+        }
+    }
+    auto issue_x = [&](int stage, int64_t sb) __attribute__((always_inline)) {
+        if constexpr (LW == 0) {
+            const half_t *xk = X + sb * 256;
+#pragma unroll
+            for (int n = 0; n < NX; n++)
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds0 + (uint32_t)(stage * QR_XSB + min(4 * n + wave, 32) * 1024)),
+                             "v"(xoff[n]), "s"(xk) : "memory");
+        }
     };
 
     float4_t acc[TA][TB], P[2][TA][TB];
@@ -250,6 +277,7 @@ __global__ __launch_bounds__(64 * (MW + QR_LW)) void gemm_q4k_kernel(GemmQ4kArgs
     auto step = [&](auto Pc, int64_t sb, const Raw (&cur)[TA], Raw (&nxt)[TA]) {
         constexpr int PP = decltype(Pc)::value;
         tile_ready();
+        issue_x(xcur ^ 1, min(sb + 1, last)); // past the end: the last one again, into a stage nobody reads
         load_raw(min(sb + 1, last), nxt);
         uint2_t hl[TB];
         read_sums(PP ^ 1, hl);
@@ -305,6 +333,7 @@ __global__ __launch_bounds__(64 * (MW + QR_LW)) void gemm_q4k_kernel(GemmQ4kArgs
     };
 
     Raw r0[TA], r1[TA];
+    issue_x(0, 0);
     load_raw(0, r0);
     // two super-blocks per trip, one straight run of instructions (a branch inside it makes the compiler wait
     // for every load in flight)
@@ -401,21 +430,23 @@ hipError_t launch_gemm_q4k(const Problem &p, const void *A, const void *B, const
     const int64_t tiles_j = (p.N + QR_BN - 1) / QR_BN;
     g.tiles_j = (int)tiles_j;
     g.vec_out = p.o_is == 1 && p.o_js % 8 == 0 && p.o_bs % 8 == 0 && ((uintptr_t)out & 15u) == 0;
-    auto go = [&](auto kernel, int bm) -> hipError_t {
+    auto go = [&](auto kernel, int bm, int lw) -> hipError_t {
         const int64_t tiles_i = (p.M + bm - 1) / bm;
         if (tiles_i * tiles_j > 0x7fffffff) return hipErrorNotSupported;
         g.remap = (tiles_i * tiles_j) % 8 == 0;
         if (const hipError_t e = ensure_lds_limit<decltype(kernel)::value>(); e != hipSuccess) return e;
-        hipLaunchKernelGGL(decltype(kernel)::value, dim3((unsigned)(tiles_i * tiles_j), (unsigned)p.stacks), dim3(64 * (4 + QR_LW)), QR_LDS, stream, g);
+        hipLaunchKernelGGL(decltype(kernel)::value, dim3((unsigned)(tiles_i * tiles_j), (unsigned)p.stacks), dim3(64 * (4 + lw)), QR_LDS, stream, g);
         return hipGetLastError();
     };
     // Four multiplying wavefronts of 32 weight rows x 64 activation rows each; when the grid of 16-row wavefronts
     // (64 weight rows per workgroup) still fits the compute units in one round, those: half the work per wavefront
     // (8192 x 3072 at 64 / 128 rows: 15.7 / 16.8 us against 22.6 / 23.6; 3072 x 8192 at 256 rows: 35 against 52 us).
-    const int64_t wgs_small = ((p.M + 63) / 64) * tiles_j;
+    const int64_t wgs_small = ((p.M + 63) / 64) * tiles_j, wgs = ((p.M + 127) / 128) * tiles_j * p.stacks;
     const bool small = g_gemm_q4k_cfg == 14 || (g_gemm_q4k_cfg == 0 && wgs_small <= dev.num_cus);
-    if (small) return go(std::integral_constant<void (*)(GemmQ4kArgs), &gemm_q4k_kernel<1, 4>>{}, 64);
-    return go(std::integral_constant<void (*)(GemmQ4kArgs), &gemm_q4k_kernel<2, 4>>{}, 128);
+    if (small) return go(std::integral_constant<void (*)(GemmQ4kArgs), &gemm_q4k_kernel<1, 4, 4>>{}, 64, 4);
+    // more than one workgroup per compute unit: no loading wavefronts (see the file comment); their offsets are in bytes
+    if (wgs > dev.num_cus && p.N * p.b_js < (int64_t(1) << 31)) return go(std::integral_constant<void (*)(GemmQ4kArgs), &gemm_q4k_kernel<2, 4, 0>>{}, 128, 0);
+    return go(std::integral_constant<void (*)(GemmQ4kArgs), &gemm_q4k_kernel<2, 4, 4>>{}, 128, 4);
 }
 
 } // namespace rt
