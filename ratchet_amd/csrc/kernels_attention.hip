@@ -550,6 +550,251 @@ __global__ __launch_bounds__(256 * NKQ) void attention_kernel(AttnArgs g) {
     }
 }
 
+// Many query rows, no mask tensor: a workgroup of four wavefronts owns 128 query rows of one head, a wavefront 32 of them
+// (two MFMA tiles) against all 64 keys of every block.  What bounds the kernel above is instructions: its wavefronts
+// own 16 rows x 32 keys a step, and a step's key and value fragment reads, its cross-lane maxima, its
+// bookkeeping and its barrier are as many for 16 rows as for 32, for 32 keys as for 64.  Here a fragment read from LDS
+// serves two MFMAs, there are two cross-lane maxima per 64 keys and row tile instead of four, and nothing is merged at the
+// end.  Two workgroups share a compute unit (two stages of the ring at head_dim 128, three below), so that one's
+// softmax runs beside the other's MFMAs.  The LDS-DMA is issued from assembly: behind the builtin the compiler makes
+// every transposing read wait for all loads into LDS; no register is written by it, and publish() waits for it.
+// DC: head_dim (64, 80, 96 or 128).
+constexpr int AL_BQ = 128, AL_BK = 64;
+constexpr int AL_MIN_WGS = 448; // workgroups from which it is the faster one (launch_attention)
+constexpr int al_stages(int dc) { return dc > 96 ? 2 : 3; }
+typedef __fp16 fp16x4_t __attribute__((ext_vector_type(4)));
+
+template <int DC>
+__global__ __launch_bounds__(256, 2) void attention_long_kernel(AttnArgs g) {
+    constexpr int KK = (DC + 31) / 32, DT = (DC + 15) / 16, DV = DC / 8; // MFMA steps over head_dim, output tiles, 16-byte chunks per row
+    constexpr int STAGES = al_stages(DC);
+    constexpr int BLK = AL_BK * DC;             // halfs of one packed block of keys (or values)
+    constexpr int NI = (2 * DV + 3) / 4;        // load instructions per wavefront and block (64 chunks each: DV for the keys, DV for the values)
+    constexpr bool SWZ = DC == 64 || DC == 128; // rows whose chunks are XOR-swizzled (at_chunk_pos)
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const half_t *ring = (const half_t *)smem;  // [STAGES][keys | values][64 rows][DC]
+
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int fr = lane & 15, fg = lane >> 4;
+    // XCD x takes the x-th eighth of the (head, query block) items: all query blocks of a head share an L2.  Within it, where
+    // it is whole heads and the flag is set, the long query blocks (late rows) come first; when every workgroup is
+    // resident at once (two per compute unit) the second half comes in the opposite order, so that a compute unit's two add up
+    // to about the same everywhere.
+    const uint32_t nqb = gridDim.x, total = gridDim.x * gridDim.y;
+    uint32_t lin = blockIdx.x + gridDim.x * blockIdx.y;
+    uint32_t bhi = blockIdx.y, qbi = blockIdx.x;
+    if ((total & 7u) == 0) {
+        const uint32_t chunk = total >> 3, r = lin >> 3, x = lin & 7u;
+        if (g.causal && chunk % nqb == 0) {
+            const uint32_t hx = chunk / nqb, q = r / hx;
+            bhi = x * hx + (r - q * hx);
+            qbi = total <= 512 && nqb % 2 == 0 && 2 * q >= nqb ? q - nqb / 2 : nqb - 1 - q;
+        } else {
+            lin = x * chunk + r;
+            bhi = lin / nqb, qbi = lin - bhi * nqb;
+        }
+    }
+    const int q0 = (int)qbi * AL_BQ, qw = q0 + 32 * wave; // first query row of the workgroup, of the wavefront
+    const int bh = (int)bhi, b = bh / g.heads, h = bh - b * g.heads;
+    const half_t *Q = g.Q + b * g.q_bs + h * g.q_hs;
+    const half_t *K = g.K + b * g.k_bs + h * g.k_hs;
+    const half_t *V = g.V + b * g.v_bs + h * g.v_hs;
+    half_t *O = g.O + b * g.o_bs + h * g.o_hs;
+    const int off = g.kv_len - g.q_len; // causal: query i sees keys <= i + off
+
+    // Q fragments: row qw + 16 u + fr, head_dim 32 kk + 8 fg .. + 7 (zero past head_dim)
+    half8_t fq[2][KK];
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const half_t *qp = Q + (int64_t)min(qw + 16 * u + fr, g.q_len - 1) * g.q_rs;
+#pragma unroll
+        for (int kk = 0; kk < KK; kk++) {
+            const int d = 32 * kk + 8 * fg;
+            fq[u][kk] = d < DC ? __builtin_bit_cast(half8_t, *(const uint4_t *)(qp + d)) : half8_t{};
+        }
+    }
+    // awaited here: a first use inside the loop would put the wait for these loads, and with them for every LDS-DMA in
+    // flight, into every step
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+        for (int kk = 0; kk < KK; kk++) asm volatile("" : "+v"(fq[u][kk]));
+    // this wavefront's load instructions, as in the kernel above: instruction j fills chunks 64 j' .. of the keys or the values
+    int lrow[NI];
+    uint32_t lcol[NI];
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+        const int j = min(wave + 4 * i, 2 * DV - 1), jj = j >= DV ? j - DV : j;
+        const int q = 64 * jj + lane;
+        lrow[i] = q / DV;
+        lcol[i] = 16u * (uint32_t)(at_chunk_pos(lrow[i], q - lrow[i] * DV, DV) - lrow[i] * DV);
+    }
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)smem;
+    // block kb into stage `stage`; rows past the last key re-read it: finite data, and their scores are masked
+    auto issue_loads = [&](int stage, int kb) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NI; i++) {
+            const int j = min(wave + 4 * i, 2 * DV - 1); // wave-uniform, as all but `o`
+            const bool val = j >= DV;
+            const uint32_t rs = 2u * (uint32_t)(val ? g.v_rs : g.k_rs);
+            const uint32_t o = (uint32_t)min(kb * AL_BK + lrow[i], g.kv_len - 1) * rs + lcol[i]; // < 2^32: launcher
+            const uint32_t dst = lds0 + (uint32_t)(2 * (stage * 2 * BLK + (val ? BLK : 0)) + 1024 * (val ? j - DV : j));
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(o), "s"(val ? V : K) : "memory");
+        }
+    };
+    // all but the newest `keep` blocks' loads of this wavefront have landed, all LDS reads have returned; then everybody's have
+    auto publish = [&](auto keep) __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(at_waitcnt(decltype(keep)::value * NI));
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    float4_t acc[2][DT];
+    float m_run[2], l_run[2]; // of row fr of tile u: the running maximum in base-2 units, this lane's share of the sum
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        m_run[u] = -INFINITY, l_run[u] = 0.f;
+#pragma unroll
+        for (int d = 0; d < DT; d++) acc[u][d] = float4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    // causal: blocks wholly above the diagonal are not visited by the workgroup, nor multiplied by a wavefront
+    auto blocks_to = [&](int rows_end) { return ((g.causal ? max(0, min(g.kv_len, rows_end + off)) : g.kv_len) + AL_BK - 1) / AL_BK; };
+    const int nkb = blocks_to(min(q0 + AL_BQ, g.q_len)), nkb_w = min(nkb, blocks_to(qw + 32)), last = max(nkb - 1, 0);
+
+    // fragment offsets inside a stage (halfs); tiles of sixteen rows are 16 DC apart (the swizzle repeats)
+    int koff[KK];
+#pragma unroll
+    for (int kk = 0; kk < KK; kk++) koff[kk] = 8 * at_chunk_pos(fr, min(4 * kk + fg, DV - 1), DV);
+    constexpr int VN = SWZ ? DT : 1; // without a swizzle the tiles' fragments are 16 halfs apart
+    int voff[VN];
+#pragma unroll
+    for (int d = 0; d < VN; d++) voff[d] = BLK + 8 * at_chunk_pos(4 * fg + (fr >> 2), 2 * d + ((fr & 3) >> 1), DV) + 4 * (fr & 1);
+
+    auto step = [&](int stage, int kb, auto lean_c) __attribute__((always_inline)) {
+        constexpr bool LEAN = decltype(lean_c)::value;
+        const half_t *st = ring + stage * 2 * BLK;
+        float4_t S[2][4];
+#pragma unroll
+        for (int bt = 0; bt < 4; bt++) {
+            half8_t fk[KK];
+#pragma unroll
+            for (int kk = 0; kk < KK; kk++) fk[kk] = __builtin_bit_cast(half8_t, *(const uint4_t *)(st + koff[kk] + bt * 16 * DC));
+#pragma unroll
+            for (int u = 0; u < 2; u++) S[u][bt] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int kk = 0; kk < KK; kk++)
+#pragma unroll
+                for (int u = 0; u < 2; u++) S[u][bt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fk[kk], fq[u][kk], S[u][bt], 0, 0, 0);
+        }
+        half8_t fp[2][2];
+        float alpha[2];
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            float bmax = -INFINITY;
+            if constexpr (LEAN) { // scale > 0: the maximum of the raw scores, the scale folded into the exponent's argument
+#pragma unroll
+                for (int e = 0; e < 16; e++) bmax = fmaxf(bmax, S[u][e >> 2][e & 3]);
+                bmax *= g.scale_log2e;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 16; e++) {
+                    const int key = kb * AL_BK + 16 * (e >> 2) + 4 * fg + (e & 3);
+                    float s = S[u][e >> 2][e & 3] * g.scale_log2e;
+                    if (key >= g.kv_len || (g.causal && key > qw + 16 * u + fr + off)) s = -INFINITY;
+                    S[u][e >> 2][e & 3] = s;
+                    bmax = fmaxf(bmax, s);
+                }
+            }
+            bmax = at_groups_max(bmax);
+            const float m_new = fmaxf(m_run[u], bmax);
+            const float m_use = m_new == -INFINITY ? 0.f : m_new; // a row without a finite score yet: exp2(-inf - 0) = 0
+            alpha[u] = __builtin_amdgcn_exp2f(m_run[u] - m_use);
+            m_run[u] = m_new;
+            const float sc = LEAN ? g.scale_log2e : 1.f;
+            float psum = 0.f;
+#pragma unroll
+            for (int e = 0; e < 16; e++) {
+                const float p = __builtin_amdgcn_exp2f(fmaf(S[u][e >> 2][e & 3], sc, -m_use));
+                psum += p;
+                fp[u][e >> 3][e & 7] = (half_t)p;
+            }
+            l_run[u] = l_run[u] * alpha[u] + psum;
+        }
+        // the running maxima rarely move after the first blocks: rescale only if some row's did
+        if (__builtin_amdgcn_ballot_w64(alpha[0] != 1.f || alpha[1] != 1.f) != 0) {
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                float al = alpha[u];
+                asm volatile("" : "+v"(al)); // keeps the products inside the branch: the compiler would form them on every step and select
+#pragma unroll
+                for (int d = 0; d < DT; d++) acc[u][d] *= al;
+            }
+        }
+        // O += P V: within 32 keys the lane's eight probabilities are, as they lie, one operand; the other comes
+        // transposed out of LDS, four keys of one column per lane and read (see the file comment)
+#pragma unroll
+        for (int hh = 0; hh < 2; hh++)
+#pragma unroll
+            for (int d = 0; d < DT; d++) {
+                typedef uint64_t u64x2_t __attribute__((ext_vector_type(2)));
+                const half_t *vp = st + voff[SWZ ? d : 0] + (SWZ ? 0 : 16 * d) + hh * 32 * DC;
+                typedef __attribute__((address_space(3))) fp16x4_t *lds4;
+                const uint64_t v0 = __builtin_bit_cast(uint64_t, __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds4)vp));
+                const uint64_t v1 = __builtin_bit_cast(uint64_t, __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds4)(vp + 16 * DC)));
+                const half8_t fv = __builtin_bit_cast(half8_t, u64x2_t{v0, v1});
+#pragma unroll
+                for (int u = 0; u < 2; u++) acc[u][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fv, fp[u][hh], acc[u][d], 0, 0, 0);
+            }
+    };
+    // blocks that cross neither the end of the keys nor this wavefront's diagonal need no test per element
+    int n_lean = 0;
+    if (g.scale_log2e > 0.f) {
+        n_lean = g.kv_len / AL_BK;
+        if (g.causal) n_lean = min(n_lean, qw + off + 1 < 0 ? 0 : (qw + off + 1) / AL_BK);
+        n_lean = min(n_lean, nkb_w);
+    }
+    if (nkb > 0) {
+#pragma unroll
+        for (int sidx = 0; sidx < STAGES - 1; sidx++) issue_loads(sidx, min(sidx, last));
+        publish(std::integral_constant<int, STAGES - 2>{});
+        int cur = 0, fill = STAGES - 1, kb = 0;
+        // three loops, so that each keeps the accumulators in registers of its own
+        auto turn = [&](auto body) __attribute__((always_inline)) {
+            issue_loads(fill, min(kb + STAGES - 1, last)); // past the end: the last block again, into a stage nobody reads
+            body();
+            publish(std::integral_constant<int, STAGES - 2>{});
+            cur = cur + 1 == STAGES ? 0 : cur + 1, fill = fill + 1 == STAGES ? 0 : fill + 1;
+        };
+        for (; kb < n_lean; kb++) turn([&]() { step(cur, kb, std::true_type{}); });
+        for (; kb < nkb_w; kb++) turn([&]() { step(cur, kb, std::false_type{}); });
+        for (; kb < nkb; kb++) turn([]() {}); // blocks only other wavefronts need
+    }
+    __builtin_amdgcn_s_waitcnt(at_waitcnt(0)); // nothing lands after the workgroup has ended
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const int row = qw + 16 * u + fr;
+        const float inv = 1.f / at_groups_sum(l_run[u]); // no visible key: 0 / 0 = NaN, what the unfused sequence yields
+        if (row >= g.q_len) continue;
+        half_t *op = O + (int64_t)row * g.o_rs;
+#pragma unroll
+        for (int d = 0; d < DT; d++) {
+            const half_t o4[4] = {(half_t)(acc[u][d][0] * inv), (half_t)(acc[u][d][1] * inv), (half_t)(acc[u][d][2] * inv), (half_t)(acc[u][d][3] * inv)};
+            *(uint64_t *)(op + 16 * d + 4 * fg) = *(const uint64_t *)o4;
+        }
+    }
+}
+
+template <int DC> static hipError_t launch_attention_long(const AttnArgs &g, int stacks, hipStream_t st) {
+    if (const hipError_t e = ensure_lds_limit<&attention_long_kernel<DC>>(); e != hipSuccess) return e;
+    hipLaunchKernelGGL((attention_long_kernel<DC>), dim3((unsigned)((g.q_len + AL_BQ - 1) / AL_BQ), (unsigned)stacks), dim3(256),
+                       (size_t)al_stages(DC) * 2 * AL_BK * DC * sizeof(half_t), st, g);
+    return hipGetLastError();
+}
+
 // Second pass of a split launch: per row, the partial (maximum, sum, output) triples of the splits are
 // combined exactly as the two key halves are inside the kernel, then normalised and rounded once.
 // One workgroup per (stack, query block); a thread owns four columns of one row and reads every split's
@@ -843,6 +1088,15 @@ hipError_t launch_attention(const rt_attention_desc &d, const void *q, const voi
         if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
         hipLaunchKernelGGL(attention_decode_merge_kernel, dim3((unsigned)stacks), dim3(128), 0, stream, g);
         return hipGetLastError();
+    }
+    if (!mask && g.splits == 1 && ((int64_t)d.q_len + AL_BQ - 1) / AL_BQ * stacks >= AL_MIN_WGS) {
+        switch (d.head_dim) {
+        case 64: return launch_attention_long<64>(g, (int)stacks, stream);
+        case 80: return launch_attention_long<80>(g, (int)stacks, stream);
+        case 96: return launch_attention_long<96>(g, (int)stacks, stream);
+        case 128: return launch_attention_long<128>(g, (int)stacks, stream);
+        default: break;
+        }
     }
     if (d.head_dim <= 64) return launch_attention_dp<64, 64>(g, (int)stacks, stream);
     if (d.head_dim == 80) return launch_attention_dp<96, 80>(g, (int)stacks, stream);

@@ -1,0 +1,58 @@
+"""The attention kernel for many query rows (attention_long_kernel: 128 rows of one head per workgroup, a grid of at least 448 of
+them, no mask tensor) at the sizes where it can go wrong, against float64.
+
+The tolerance: a probability is rounded to f16 (2^-11 of itself, 2^-25 absolute below f16's normal numbers) after scores with the
+rounding of an f32 sum of head_dim products, the output once more."""
+import math
+
+import pytest
+import torch
+
+from ratchet_amd import DType, Tensor
+
+pytestmark = pytest.mark.gpu
+
+
+def tensor(device, t):
+    return Tensor(tuple(t.shape), DType.F16, device, t.contiguous().view(torch.uint8).reshape(-1))
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("heads,head_dim,rows,keys,scale", [
+    (128, 64, 512, 512, None),     # every workgroup resident, paired
+    (112, 80, 500, 500, None),     # the last query block and the last key block ragged
+    (56, 96, 1025, 1100, None),    # a query block of one row, an odd number of query blocks
+    (448, 128, 65, 1, None),       # one key
+    (448, 96, 3, 63, None), (460, 80, 128, 65, None), (257, 64, 129, 128, None),
+    (256, 128, 256, 191, None),    # causal: the first rows see no key
+    (64, 64, 900, 1283, -0.2), (112, 96, 512, 320, 0.0),
+    (9, 80, 6600, 192, None),      # few heads: not whole ones per XCD
+])
+def test_against_float64(device, heads, head_dim, rows, keys, scale, causal):
+    gen = torch.Generator("cuda:0").manual_seed(heads + head_dim + rows + keys)
+    cap = keys + 3  # a cache with room: rows past `keys` are never read
+    q = torch.randn((1, heads, rows, head_dim), generator=gen, device="cuda:0").half()
+    k, v = (torch.randn((1, heads, cap, head_dim), generator=gen, device="cuda:0").half() for _ in range(2))
+    q[0, 0, rows // 2] *= 30  # a row whose maximum moves far
+    k[:, :, keys:], v[:, :, keys:] = math.nan, math.nan
+    node = tensor(device, q).attention(tensor(device, k), tensor(device, v), causal=causal, kv_len=keys, scale=scale)
+    node.op.use_workspace = False
+    got = node.resolve().storage.view(torch.float16)[: q.numel()].view(q.shape).double()
+    s = 1 / math.sqrt(head_dim) if scale is None else scale
+    for h in range(0, heads, 16):
+        sl = slice(h, min(h + 16, heads))
+        qd, kd, vd = q[0, sl].double(), k[0, sl, :keys].double(), v[0, sl, :keys].double()
+        scores = torch.matmul(qd, kd.transpose(1, 2).contiguous()) * s
+        mag = torch.matmul(qd.abs(), kd.abs().transpose(1, 2).contiguous()) * abs(s)
+        if causal:
+            hidden = torch.arange(keys, device="cuda:0")[None, :] > torch.arange(rows, device="cuda:0")[:, None] + (keys - rows)
+            scores = scores.masked_fill(hidden, -math.inf)
+        p = torch.softmax(scores, -1)
+        want = torch.matmul(p, vd)
+        # a probability's relative error: f16's, and that of its score and of the row's maximum
+        e = 2.0**-11 + 2.0**-24 * ((head_dim / 32 + 4) * mag + 8)
+        bound = torch.matmul(2 * e.amax(-1, keepdim=True) * p + 2.0**-25, vd.abs()) + 2.0**-11 * want.abs() + 2.0**-25
+        g = got[0, sl]
+        assert torch.equal(torch.isnan(g), torch.isnan(want))
+        ok = ((g - want).abs() <= bound) | torch.isnan(want)
+        assert ok.all(), float(((g - want).abs() / bound)[~torch.isnan(want)].max())
