@@ -24,6 +24,8 @@
 // generators).
 #include "device_common.h"
 
+#include <algorithm>
+
 namespace rt {
 
 constexpr int BK = 32;
@@ -43,6 +45,7 @@ struct GemmArgs {
     int64_t b_bs, b_ks, b_js;
     int64_t o_bs, o_is, o_js;
     int has_bias, bias_on_rows, act;
+    int64_t i_first; // first output row of the launch
 };
 
 template <typename T> struct Tile;
@@ -253,7 +256,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(GemmArgs g) {
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int wi = wave >> 1, wj = wave & 1; // wave position in the 2 x 2 grid
     const int64_t s = blockIdx.z;
-    const int64_t i0 = (int64_t)blockIdx.y * BM, j0 = (int64_t)blockIdx.x * BN;
+    const int64_t i0 = g.i_first + (int64_t)blockIdx.y * BM, j0 = (int64_t)blockIdx.x * BN;
     // an operand's stack is either the full stack or 1 (broadcast)
     const int64_t a_el = (g.a_stack == 1 ? 0 : s) * g.a_bs, b_el = (g.b_stack == 1 ? 0 : s) * g.b_bs;
 
@@ -487,13 +490,14 @@ hipError_t launch_gemm(const Problem &p, const void *A, const void *B, const voi
                        hipStream_t stream, const DeviceInfo &dev) {
     if (p.stacks > 65535) return hipErrorNotSupported;
     // f16: 128 x 128 tiles unless they would leave the chip under two workgroups per compute unit.  Only small f32 products
-    // come here (gemm_limb_kernel takes the rest): 64 x 64.
+    // and those whose strides are too large for gemm_limb_kernel's offsets come here: 64 x 64, in two launches where the rows
+    // are more than a grid's 65535 tiles.
     int ts = p.act_dt == RT_F16 ? 128 : 64;
     const int64_t big = ((p.M + 127) / 128) * ((p.N + 127) / 128) * p.stacks;
     if (big < 2 * (int64_t)dev.num_cus) ts = 64;
     if (p.act_dt == RT_F16 && (g_gemm_tile == 64 || g_gemm_tile == 128)) ts = g_gemm_tile;
     const int64_t gy = (p.M + ts - 1) / ts, gx = (p.N + ts - 1) / ts;
-    if (gy > 65535) return hipErrorNotSupported;
+    if (gy > (p.act_dt == RT_F16 ? 65535 : 2 * 65535)) return hipErrorNotSupported;
     GemmArgs g{};
     g.A = A, g.B = B, g.bias = bias, g.out = out;
     g.M = p.M, g.N = p.N, g.K = p.K;
@@ -517,12 +521,15 @@ hipError_t launch_gemm(const Problem &p, const void *A, const void *B, const voi
     }
     const int bmode = float_mode(B, esz, p.N, p.K, p.b_js, p.b_ks, p.b_bs);
 
-    dim3 grid((unsigned)gx, (unsigned)gy, (unsigned)p.stacks);
-    if (p.act_dt == RT_F16) {
-        if (ts == 64) launch_a<half_t, 64>(amode, bmode, grid, stream, g);
-        else launch_a<half_t, 128>(amode, bmode, grid, stream, g);
-    } else {
-        launch_a<float, 64>(amode, bmode, grid, stream, g);
+    for (int64_t first = 0; first < gy; first += 65535) {
+        g.i_first = first * ts;
+        const dim3 grid((unsigned)gx, (unsigned)std::min<int64_t>(gy - first, 65535), (unsigned)p.stacks);
+        if (p.act_dt == RT_F16) {
+            if (ts == 64) launch_a<half_t, 64>(amode, bmode, grid, stream, g);
+            else launch_a<half_t, 128>(amode, bmode, grid, stream, g);
+        } else {
+            launch_a<float, 64>(amode, bmode, grid, stream, g);
+        }
     }
     return hipGetLastError();
 }

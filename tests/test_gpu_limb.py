@@ -88,3 +88,16 @@ def test_values_that_are_not_finite(device):
         assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
         fine = np.isfinite(want)
         assert np.isfinite(got[fine]).all() and np.allclose(got[fine], want[fine], rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("m", [65535 * 64, 65535 * 64 + 1, 65536 * 64 + 65])
+def test_rows_beyond_one_grid(device, m):
+    """Strides of millions of values are the generic kernel's, whose 65535 tiles along a grid's second axis hold 4.2 million rows."""
+    gen = torch.Generator("cuda:0").manual_seed(m)
+    x, y = torch.randn((3, m), generator=gen, device="cuda:0"), torch.randn((3, 20), generator=gen, device="cuda:0")
+    t = lambda v: Tensor(tuple(v.shape), DType.F32, device, v.view(torch.uint8).reshape(-1))
+    got = t(x).gemm(t(y), None, True, False, False).resolve().storage.view(torch.float32)[: 20 * m].view(m, 20)
+    for lo in range(0, m, 1 << 20):  # three products, at most three roundings
+        xd = x[:, lo : lo + (1 << 20)].double().T.contiguous()
+        err = (got[lo : lo + (1 << 20)].double() - xd @ y.double()).abs()
+        assert (err <= 2.0**-24 * 4 * (xd.abs() @ y.double().abs()) + 2.0**-149).all()
