@@ -362,8 +362,10 @@ __global__ __launch_bounds__(256 + 64 * PW) void gemm_limb_kernel(GemmLimbArgs g
         float odd = 0.f; // NaN once an output of this lane is not finite
         // offsets inside the tile are 32-bit (the launcher checks)
         const uint32_t ois = (uint32_t)o_is, ojs = (uint32_t)o_js;
-        if (ojs == 1 && !row_bias) {
-            // Bounds are the buffer's: it ends with the tile's last element, and columns outside get an offset past any end.
+        if (ojs == 1 && !row_bias && (int)ois >= jl) {
+            // Bounds are the buffer's: it ends with the tile's last element, and columns outside get an offset past any end.  Rows
+            // outside lie past the end only where a row of the output is as long as the tile's part of it: an output of one
+            // row may have any stride, a transposed one (one column of [N, 1]) has 1.
             const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(out, 0, il > 0 && jl > 0 ? (int)(4 * (((uint32_t)il - 1) * ois + (uint32_t)jl)) : 0, 0x00027000);
             rt_with_act(act, [&](auto has_act) {
 #pragma unroll

@@ -101,3 +101,31 @@ def test_rows_beyond_one_grid(device, m):
         xd = x[:, lo : lo + (1 << 20)].double().T.contiguous()
         err = (got[lo : lo + (1 << 20)].double() - xd @ y.double()).abs()
         assert (err <= 2.0**-24 * 4 * (xd.abs() @ y.double().abs()) + 2.0**-149).all()
+
+
+@pytest.mark.parametrize("tl", [False, True])
+@pytest.mark.parametrize("k,n", [(65, 9), (96, 63), (96, 64), (200, 65), (300, 127), (511, 128), (65, 129), (600, 300), (3001, 131), (70, 20001)])
+def test_one_row_written_as_a_column(device, monkeypatch, k, n, tl):
+    """[1, K] . [K, N] with the output transposed: both strides of the output are 1, and rows past the only one must not be
+    stored.  With and without K shared."""
+    rng = np.random.default_rng(k + n)
+    x, y = rng.standard_normal((1, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    want, b = x.astype(np.float64) @ y.astype(np.float64), bound(x, y, None)
+    for share in (True, False):
+        monkeypatch.setattr("ratchet_amd.tensor.SPLIT_K", share)
+        got = run(device, x.T.copy() if tl else x, y, None, tl, False, True)
+        assert got.shape == (n, 1) and (np.abs(got.T - want) <= b).all(), (share, (np.abs(got.T - want) / b).max())
+
+
+@pytest.mark.parametrize("n,k", [(33, 64), (300, 96), (1000, 4096)])
+def test_codes_against_one_misaligned_row(device, n, k):
+    """One activation row that the streaming kernels do not take (4 bytes past a 16-byte boundary), the output [N, 1]."""
+    rng = np.random.default_rng(n + k)
+    w = Quantizer(Quantization.SInt8).quantize(Tensor.from_data(rng.standard_normal((n, k)).astype(np.float32)).to(device))
+    x = rng.standard_normal((k, 1)).astype(np.float32)
+    room = torch.zeros(4 * k + 16, dtype=torch.uint8, device="cuda:0")
+    room[4 : 4 + 4 * k] = torch.from_numpy(x.view(np.uint8).reshape(-1)).to("cuda:0")
+    xt = Tensor((k, 1), DType.F32, device, room[4 : 4 + 4 * k])
+    wf = dequantize(w).to(Device.CPU).storage
+    got = w.gemm(xt, None, False, False, False).resolve().to(Device.CPU).storage
+    assert got.shape == (n, 1) and (np.abs(got - wf.astype(np.float64) @ x.astype(np.float64)) <= bound(x.T, wf.T, None).T).all()
