@@ -62,7 +62,7 @@ struct GemmNtArgs {
 // Which output tile a workgroup takes.  Workgroup ids go round the 8 XCDs, each with an L2 of its own.
 // g.xi > 0: the grid of tiles is cut into xi x (8 / xi) equal blocks, one per XCD, and a block is walked in panels
 // of g.pj columns, so that the 32 workgroups an XCD runs at a time share the fewest operand rows
-// (nt_set_tiles chooses both).  Otherwise XCD x takes the contiguous range x * ntiles / 8 .. of the tiles in row-major
+// (nt_set_tiles chooses).  Otherwise XCD x takes the contiguous range x * ntiles / 8 .. of the tiles in row-major
 // order when that comes out even, and the plain order when not.  In 32 bits and with the block's sides from the host: every
 // workgroup waits for this before its first load, and six 64-bit divisions were 0.3 us a launch (a 512-row prompt through
 // a layer with Q8_0H weights, four products: 178.8 -> 176.6 us).
@@ -1104,25 +1104,30 @@ static hipError_t launch_nt(const GemmNtArgs &g, int64_t stacks, hipStream_t st)
     return hipGetLastError();
 }
 
-// The grid of bm x bn tiles and the order its workgroups take them in.  An XCD's share of the tiles is a block of
-// (tiles_i / xi) x (tiles_j xi / 8) where the grid can be cut that way; of the possible cuts, the one whose 32
-// resident workgroups load the fewest bytes of operands per K step that their L2 does not hold already: for
-// [2048 x 10240] . [2560 x 10240]^T (16 x 16 tiles) four row blocks and eight column blocks per XCD
-// instead of two and sixteen.  a_bytes: of an element of A (the codes' one for Q8_0H).
+// The grid of bm x bn tiles and the order its workgroups take them in.  An XCD's share of the tiles is either a block of
+// (tiles_i / xi) x (tiles_j xi / 8) where the grid can be cut that way, or the x-th eighth of them in row-major order;
+// of the possible ones, the one whose resident workgroups (up to 32) load the fewest bytes of operands per K step that
+// their L2 does not hold already: for [2048 x 10240] . [2560 x 10240]^T (16 x 16 tiles) four row blocks and eight column
+// blocks per XCD instead of two and sixteen; for 11008 x 4096 weights against 1000 rows (69 x 8 tiles) the
+// plain eighths, nine row blocks by eight columns, where the only cut has 69 row blocks of one column (115.9 and
+// 107.8 us; 8192 x 3072 against 200 rows, 52 x 2 tiles, K shared: 27.7 and 23.9).  a_bytes: of an element of A (the
+// codes' one for Q8_0H).
 static bool nt_set_tiles(GemmNtArgs &g, int bm, int bn, int a_bytes) {
     const int64_t ti = (g.M + bm - 1) / bm, tj = (g.N + bn - 1) / bn;
     if (ti * tj > 0x7fffffff) return false;
     g.tiles_i = (int)ti, g.tiles_j = (int)tj;
     g.xi = 0, g.pj = 1;
-    int64_t least = 0;
+    const int64_t res = std::min<int64_t>(32, (ti * tj + 7) / 8); // workgroups resident on an XCD
+    // the plain order: a share that is not whole rows of tiles begins in the middle of one
+    int64_t least = ((res + tj - 1) / tj + ((ti * tj / 8) % tj ? 1 : 0)) * bm * a_bytes + std::min(tj, res) * bn * 2;
     for (int xi = 8; xi >= 1; xi /= 2) {
         const int xj = 8 / xi;
         if (ti % xi || tj % xj) continue;
         const int64_t rows = ti / xi, cols = tj / xj;
         // panels of four columns, wider when the block has too few rows to give 32 workgroups eight of them
         const int64_t pj = std::min(cols, std::max<int64_t>(4, 32 / rows));
-        const int64_t cost = std::min<int64_t>(rows, (31 + pj) / pj) * bm * a_bytes + pj * bn * 2;
-        if (!g.xi || cost < least) g.xi = xi, g.pj = (int)pj, least = cost;
+        const int64_t cost = std::min<int64_t>(rows, (res + pj - 1) / pj) * bm * a_bytes + pj * bn * 2;
+        if (cost < least) g.xi = xi, g.pj = (int)pj, least = cost;
     }
     if (g.xi) {
         g.xj_log2 = g.xi == 8 ? 0 : g.xi == 4 ? 1 : g.xi == 2 ? 2 : 3;

@@ -53,3 +53,13 @@ def test_edges(device, m, k, n, weight_first):
 ])
 def test_tile_orders(device, m, k, n):
     check(device, m, k, n, True)
+
+
+@pytest.mark.parametrize("m,k,n", [
+    (8192, 3072, 200),    # 52 x 2, K shared: no cut fetches less than the plain eighths
+    (4160, 320, 1000),    # 26 x 8
+    (11008, 320, 1000),   # 69 x 8, a share ends inside a row of tiles
+    (4096, 1024, 400),    # 64 x 4 tiles of 64 rows
+])
+def test_tiles_in_row_order(device, m, k, n):
+    check(device, m, k, n, True)
