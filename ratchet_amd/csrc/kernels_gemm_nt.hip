@@ -1271,10 +1271,14 @@ hipError_t launch_gemm_nt(const Problem &p0, const void *A, const void *B, const
     if (dl_f16 && g.ksplit == 1 && g_gemm_nt_wide != 1 && p.a_rs >= 0 && p.b_js >= 0 && 2 * 320 * std::max(p.a_rs, p.b_js) < (int64_t(1) << 32)) {
         const int64_t wide = ((p.M + 319) / 320) * ((p.N + 255) / 256) * p.stacks;
         const int64_t rounds = (ti * tj * p.stacks + dev.num_cus - 1) / dev.num_cus, rounds_wide = (wide + dev.num_cus - 1) / dev.num_cus;
-        // A round of 320 x 256 tiles on all compute units takes 2.5 rounds of 160 x 128 ones (10240 x 2560 weights: 89.7 us at 2048
-        // activation rows, one round, against 110.7 for four; 7680 x 2560, one against three, 76.5 for 82.9).  Two against
-        // five (11008 x 4096 at 2048 rows) and everything with fewer rounds stays on the small tiles.
-        if ((g_gemm_nt_wide == 2 || 5 * rounds_wide < 2 * rounds) && nt_set_tiles(g, 320, 256, 2)) return launch_nt_wide(g, p.stacks, stream);
+        // A round of 320 x 256 tiles takes 12 + 0.030 K us on all compute units, one of 160 x 128 tiles 6.4 + 0.0080 K: four small
+        // rounds are always longer (10240 x 2560 weights, 2048 activation rows: 108.5 us against 89.7), two never.  Three are
+        // longer for a short K (1500 rows, K = 1024: 43.9 against 39.3), the same at K = 2560 and shorter beyond (1000 rows
+        // x 11008 x 4096: 107.0 against 118.9; two wide rounds against six small ones alike) -- unless the small tiles do not deal out
+        // evenly to the XCDs, whose L2s then share little (1300 rows x 8192 x 4096, 572 tiles: 133.5 against 114.2).
+        const bool even = ti * tj % 8 == 0;
+        const bool longer = 5 * rounds_wide < 2 * rounds && (3 * rounds_wide < rounds || !even || p.K <= 2048);
+        if ((g_gemm_nt_wide == 2 || longer) && nt_set_tiles(g, 320, 256, 2)) return launch_nt_wide(g, p.stacks, stream);
     }
     if (dl_f16) {
         // two loading wavefronts: one and four measured the same within run-to-run spread
