@@ -140,6 +140,7 @@ constexpr Launcher kLaunchers[] = {rt::launch_gemv,          // streaming kernel
                                    rt::launch_gemm_stream,   // f16 / Q8_0H weights against a few dozen activation rows: one pass over the weight
                                    rt::launch_gemm_nt,       // K-contiguous f16 / Q8_0H problems: the large-tile kernel
                                    rt::launch_gemm_nn_smalln, // f16 products with an untransposed narrow rhs (attention P.V)
+                                   rt::launch_gemm_f32_small, // f32 products too small to split into limbs
                                    rt::launch_gemm_limb,     // f32 activations against f32 operands or Q8_0F weights: bf16 matrix cores, exact limbs
                                    rt::launch_gemm_f32,      // f32 products whose operands each have a contiguous axis
                                    rt::launch_gemm_q4k,      // Q4_K weights against many activation rows

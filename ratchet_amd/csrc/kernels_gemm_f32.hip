@@ -1,15 +1,14 @@
-// Small f32 products on the f32 matrix cores:
+// f32 products on the f32 matrix cores:
 //   C[s, i, j] = sum_k A[s, i, k] * B[s, k, j] (+ bias),  f32 in, f32 accumulate, f32 out,
 // A K-contiguous; B either N-contiguous (`lhs.matmul(rhs)`) or K-contiguous (Linear's W.gemm(x, b, false, true, true) with
-// f32 weights).  gemm_limb_kernel takes every f32 product that is worth splitting into bf16 limbs (it is declined only
-// when K is at most two of its stages and its tiles do not fill the compute units, see launch_gemm_limb); what is left
-// here is bound by launch, first loads and stores, and the f32 MFMA's operands need no splitting: 8 heads x
-// [232 x 64] . [64 x 232] 4.6 us here, 5.2 there.
+// f32 weights).  gemm_limb_kernel takes the f32 products whose MFMAs weigh; here are the ones bound by launch, first
+// loads and stores, whose operands need no splitting (launch_gemm_f32_small says which), and those whose strides are
+// too large for its offsets.
 // v_mfma_f32_16x16x4_f32 takes one f32 per lane and operand, so neither tile needs a transpose: A sits in LDS as [row][k]
 // and B as it lies in memory, [k][col] or [col][k].
 //
 // 32 x 96 or 32 x 64 outputs per 256-thread workgroup (2 x 2 wavefronts of 1 x 3 or 1 x 2 MFMA tiles), so that about three
-// workgroups share a compute unit and their fixed parts overlap.  K tile 32, two LDS stages, one bare barrier per tile; tile
+// workgroups share a compute unit and their fixed parts overlap; 128 x 128 (4 x 4) for large outputs.  K tile 32, two LDS stages, one bare barrier per tile; tile
 // t+1 waits in registers while tile t is multiplied and tile t+2 is in flight.  With K a whole number of tiles the loop has
 // no bound to check; other K (a multiple of 4) run the KTAIL variant, whose loads clamp their K offset and whose LDS stores
 // write zeros past K -- selects, not branches, so the loop stays straight-line code either way.
@@ -298,9 +297,29 @@ hipError_t launch_gemm_f32(const Problem &p, const void *A, const void *B, const
     g.o_bs = p.o_bs, g.o_is = p.o_is, g.o_js = p.o_js;
     g.has_bias = p.has_bias, g.bias_on_rows = p.bias_on_rows, g.act = p.act;
     g.nt_out = p.o_js == 1 && (p.o_is * 4) % 128 == 0 && (p.o_bs * 4) % 128 == 0 && ((uintptr_t)out & 127u) == 0;
+    // A K of one tile and two large tiles for every compute unit: nearly all the time goes into the operands and the output, of which
+    // the largest tile reads least (32 x [512 x 16] . [16 x 512]: 11.2 us; 32-row tiles 12.5).
+    const int64_t tiles128 = ((p.M + 127) / 128) * ((p.N + 127) / 128) * p.stacks;
+    if (p.K <= F32_BK && tiles128 >= 2 * (int64_t)dev.num_cus)
+        return b_kcont ? launch_f32<128, 128, true>(g, p.stacks, stream) : launch_f32<128, 128, false>(g, p.stacks, stream);
     // up to 64 columns (P . V over a head dimension of 64): 64-column tiles, not two thirds of 96
     if (p.N <= 64) return b_kcont ? launch_f32<32, 64, true>(g, p.stacks, stream) : launch_f32<32, 64, false>(g, p.stacks, stream);
     return b_kcont ? launch_f32<32, 96, true>(g, p.stacks, stream) : launch_f32<32, 96, false>(g, p.stacks, stream);
+}
+
+// The f32 products that are faster here than on gemm_limb_kernel, which is asked next: there splitting lies between the
+// first load and the first MFMA, and a tile is at least 64 x 64.
+//   K <= 32                     one stage, nothing to pipeline (32 x [512 x 4 / 16 / 32] . [.. x 512] 10.0 / 11.2 / 12.5 us here,
+//                               13.6 / 13.5 / 13.1 there; 20 x [300 x 16] . [16 x 300] 6.5 / 7.8)
+//   K <= 128, few tiles         at most a 64 x 64 tile per compute unit (scores of 32 heads x 56 positions, head_dim 96: 3.8 / 5.2 us;
+//                               8 heads x 128 x 128: 4.7 / 5.2; P . V of 128 keys into 64 columns 4.2 / 5.6; of 232 keys 7.6 / 7.6)
+//   K < 512, few tiles, B K-contiguous with 48 to 64 columns   Linear over a few dozen positions (48 rows x 1536 x 384:
+//                               8.4 / 8.8 us); from 512 on the other kernel shares K among workgroups.
+hipError_t launch_gemm_f32_small(const Problem &p, const void *A, const void *B, const void *bias, void *out, hipStream_t stream,
+                                 const DeviceInfo &dev) {
+    const bool few = ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.stacks <= dev.num_cus;
+    const bool takes = p.K <= F32_BK || (few && (p.K <= 128 || (p.K < 512 && p.b_ks == 1 && p.N <= 64)));
+    return takes ? launch_gemm_f32(p, A, B, bias, out, stream, dev) : hipErrorNotSupported;
 }
 
 } // namespace rt

@@ -623,10 +623,9 @@ bool limb_orient(Problem &p) {
     return true;
 }
 
-// Everything with f32 activations but the smallest f32 products: with at most two stages and less than a tile of 64 x 64 per
-// compute unit there is nothing to pipeline, and splitting lies between the first load and the first MFMA (attention over
-// 56 positions, 32 heads: 12.6 us for its three operators here, 10.2 on the f32 matrix cores; 8 heads x 22 positions 12.8
-// and 12.0; from 300 positions on the limbs win: 16 heads 32.8 there, 24.8 here).
+// Everything with f32 activations but small f32 products.  Those launch_gemm_f32_small has taken before; of what it
+// cannot (operands not aligned to 16 bytes, few rows), with at most two stages and less than a tile of 64 x 64 per compute
+// unit there is nothing to pipeline (8 heads x 22 positions, the attention's three operators: 12.8 us here, 12.0 on the generic kernel).
 bool limb_takes(const Problem &p, const DeviceInfo &dev) {
     if (p.act_dt != RT_F32 || (p.a_dt != RT_F32 && p.a_dt != RT_Q8_0F) || p.M <= 0 || p.N <= 0 || p.K <= 0 || p.stacks <= 0) return false;
     return p.a_dt == RT_Q8_0F || p.K > 64 || ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.stacks > dev.num_cus;

@@ -129,3 +129,19 @@ def test_codes_against_one_misaligned_row(device, n, k):
     wf = dequantize(w).to(Device.CPU).storage
     got = w.gemm(xt, None, False, False, False).resolve().to(Device.CPU).storage
     assert got.shape == (n, 1) and (np.abs(got - wf.astype(np.float64) @ x.astype(np.float64)) <= bound(x.T, wf.T, None).T).all()
+
+
+@pytest.mark.parametrize("tr", [False, True])
+@pytest.mark.parametrize("stacks,m,k,n", [
+    (32, 512, 4, 512), (3, 2041, 32, 2044), (20, 300, 28, 300),  # one K tile: 128 x 128 tiles, ragged ones, the small tiles
+    (1, 520, 32, 48), (8, 128, 128, 128), (1, 96, 132, 96),      # few tiles: up to K = 128 and past it
+    (16, 100, 100, 64), (1, 1536, 508, 52), (1, 1536, 512, 52), (1, 300, 384, 64)])
+def test_small_products_on_either_side_of_the_rules(device, stacks, m, k, n, tr):
+    """Products that stay on the f32 matrix cores (launch_gemm_f32_small) and the first ones past them."""
+    rng = np.random.default_rng(m + k + n)
+    x, y = rng.standard_normal((stacks, m, k)).astype(np.float32), rng.standard_normal((stacks, k, n)).astype(np.float32)
+    bias = rng.standard_normal(n).astype(np.float32)
+    got = run(device, x, np.swapaxes(y, 1, 2) if tr else y, bias, False, tr, False)
+    want = x.astype(np.float64) @ y.astype(np.float64) + bias
+    # the f32 matrix cores round after each product
+    assert (np.abs(got - want) <= 2.0**-24 * (k + 2) * (np.abs(x).astype(np.float64) @ np.abs(y).astype(np.float64) + np.abs(bias))).all()
