@@ -145,3 +145,18 @@ def test_small_products_on_either_side_of_the_rules(device, stacks, m, k, n, tr)
     want = x.astype(np.float64) @ y.astype(np.float64) + bias
     # the f32 matrix cores round after each product
     assert (np.abs(got - want) <= 2.0**-24 * (k + 2) * (np.abs(x).astype(np.float64) @ np.abs(y).astype(np.float64) + np.abs(bias))).all()
+
+
+@pytest.mark.parametrize("tl,tr", [(False, False), (False, True), (True, False)])
+@pytest.mark.parametrize("stacks,m,n", [(1, 1100, 1029), (32, 512, 512), (1, 70, 90)])
+def test_outer_products_are_rounded_once(device, stacks, m, n, tl, tr):
+    """K = 1: every output is the correctly rounded product.  K = 2: the sum of two products is rounded twice."""
+    rng = np.random.default_rng(m + n)
+    for k in (1, 2):
+        x, y = rng.standard_normal((stacks, m, k)).astype(np.float32), rng.standard_normal((stacks, k, n)).astype(np.float32)
+        got = run(device, np.swapaxes(x, 1, 2) if tl else x, np.swapaxes(y, 1, 2) if tr else y, None, tl, tr, False)
+        want = x.astype(np.float64) @ y.astype(np.float64)
+        if k == 1:
+            assert np.array_equal(got, want.astype(np.float32))
+        else:
+            assert (np.abs(got - want) <= 2.0**-24 * (np.abs(x[..., :1].astype(np.float64) * y[:, :1]) + np.abs(got)) * (1 + 2.0**-20)).all()
