@@ -13,8 +13,8 @@
 // The sum of the limbs is exact down to 2^-133, bf16's smallest subnormal number (the matrix cores take subnormal operands):
 // a value below 2^-109 = 1.5e-33 is represented to 2^-134 instead of to 24 bits.
 // An operand whose limbs are not finite (infinities, NaNs, magnitudes that round past the largest bf16) makes its outputs
-// NaN: every output that is not finite is computed once more as a plain f32 dot product, so what the f32 arithmetic gives
-// for such inputs is what is stored.
+// NaN: a 32 x 32 tile with an output that is not finite is computed once more on the f32 matrix cores, so what the f32
+// arithmetic gives for such inputs is what is stored.
 //
 // Wavefronts 4 and up load (global -> registers two stages ahead), split into limbs and store the limb planes to LDS;
 // wavefronts 0..3 read fragments and multiply.  The split is five and a half vector instructions per value.  Beside a
@@ -351,6 +351,7 @@ __global__ __launch_bounds__(256 + 64 * PW) void gemm_limb_kernel(GemmLimbArgs g
             bj[b] = g.has_bias && !g.bias_on_i && g.ksplit == 1 ? g.bias[min(j, g.N - 1)] : 0.f;
         }
     };
+    uint64_t again = 0; // not zero once an output of this wavefront is not finite
     auto finish = [&](const Item &it) {
         const bool share = g.ksplit > 1;
         const int64_t iw = it.i0 + wi * (BI / WI), jw = it.j0 + wj * (BJ / WJ);
@@ -405,29 +406,7 @@ __global__ __launch_bounds__(256 + 64 * PW) void gemm_limb_kernel(GemmLimbArgs g
                     }
                 }
         }
-        if (__any(odd != odd)) {
-            // the plain f32 dot product for every output of this wavefront that is not finite (each lane its own outputs)
-            const float *X = g.X + (g.x_stack == 1 ? 0 : it.s) * g.x_bs;
-            const int64_t y_el = (g.y_stack == 1 ? 0 : it.s) * g.y_bs;
-            const int64_t kend = min(g.K, it.k0 + (int64_t)g.nk * 32);
-#pragma unroll 1
-            for (int e = 0; e < TM * TN * 16; e++) {
-                const int r = e & 15, ab = e >> 4, a = ab / TN, b = ab - a * TN;
-                const int i = 32 * a + 4 * fh + 8 * (r >> 2) + (r & 3), j = 32 * b + fr;
-                if (i >= il || j >= jl) continue;
-                float *o = out + (uint32_t)i * ois + (uint32_t)j * ojs;
-                if (__builtin_fabsf(*o) <= 3.4028234e38f) continue;
-                const int64_t gi = iw + i, gj = jw + j;
-                float v = 0.f;
-                for (int64_t k = it.k0; k < kend; k++) {
-                    const float y = Q8 ? (float)((const int8_t *)g.Y)[y_el + gj * g.y_js + k] * g.scales[(y_el + gj * g.y_js + k) >> 5]
-                                       : ((const float *)g.Y)[y_el + gj * g.y_js + k * g.y_ks];
-                    v = fmaf(X[gi * g.x_is + k * g.x_ks], y, v);
-                }
-                if (g.has_bias && !share) v += g.bias[g.bias_on_i ? gi : gj];
-                *o = rt_act(v, act);
-            }
-        }
+        again |= __builtin_amdgcn_ballot_w64(odd != odd);
     };
 
     // Steps of a stage: f32, half h of the 32 k and row tile a, with X's fragments of the step and Y's of the half in two
@@ -536,6 +515,82 @@ __global__ __launch_bounds__(256 + 64 * PW) void gemm_limb_kernel(GemmLimbArgs g
             kt = 0, n++; // with several items per workgroup every item has the same number of stages
             if (n < count) fetch_bias(item(n));
             clear();
+        }
+    }
+    if (__builtin_expect_with_probability(again == 0, 1, 1.0)) return; // or the registers go to the loops below
+    // The tiles with outputs that are not finite once more on the f32 matrix cores (see the file comment), after everything else: beside
+    // the main loop's registers there is no room for it.  The arguments are read again through a pointer the compiler cannot
+    // see through, or they would be kept, in spilled registers, from the kernel's start on.
+    auto *ka = (const __attribute__((address_space(4))) GemmLimbArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(ka));
+    const int64_t x_ks = XKC ? 1 : ka->x_ks, y_ks = YKC ? 1 : ka->y_ks;
+    const bool share = ka->ksplit > 1, row_bias = ka->has_bias && ka->bias_on_i && !share;
+    const int act = share ? RT_ACT_NONE : ka->act;
+    const uint32_t ois = (uint32_t)(share ? ka->N : ka->o_is), ojs = share ? 1u : (uint32_t)ka->o_js;
+#pragma unroll 1
+    for (n = 0; n < count; n++) {
+        const Item it = item(n);
+        const int64_t iw = it.i0 + wi * (BI / WI), jw = it.j0 + wj * (BJ / WJ);
+        float *out = (share ? ka->partial + (it.s * ka->ksplit + it.z) * ka->M * ka->N : ka->out + it.s * ka->o_bs) + iw * ois + jw * ojs;
+        const int il = ka->M - iw < BI ? (int)(ka->M - iw) : BI, jl = ka->N - jw < BJ ? (int)(ka->N - jw) : BJ;
+        const int64_t kend = min(ka->K, it.k0 + (int64_t)ka->nk * 32);
+        const float *X = ka->X + (ka->x_stack == 1 ? 0 : it.s) * ka->x_bs;
+        const int64_t y_el = (ka->y_stack == 1 ? 0 : it.s) * ka->y_bs;
+#pragma unroll 1
+        for (int ab = 0; ab < TM * TN; ab++) {
+            const int a = ab / TN, b = ab - a * TN, ir = 32 * a + 4 * fh, j = 32 * b + fr; // this lane's outputs: rows ir + 8 (r / 4) + r % 4
+            const uint32_t at0 = (uint32_t)ir * ois + (uint32_t)j * ojs;
+            uint32_t bad = 0, at = at0; // bit r: output r
+#pragma unroll 1
+            for (int r = 0; r < 16; r++) {
+                if (ir + 8 * (r >> 2) + (r & 3) < il && j < jl && !(__builtin_fabsf(out[at]) <= 3.4028234e38f)) bad |= 1u << r;
+                at += (r & 3) == 3 ? 5 * ois : ois;
+            }
+            if (!__any(bad != 0)) continue;
+            // lane half h supplies k + 4 h .. + 3 of eight, one of them to each MFMA
+            const float *xp = X + min(iw + 32 * a + fr, ka->M - 1) * ka->x_is + (it.k0 + 4 * fh) * x_ks;
+            const int64_t ye = y_el + min(jw + j, ka->N - 1) * ka->y_js + (it.k0 + 4 * fh) * y_ks;
+            const float *yp = (const float *)ka->Y + ye;           // f32
+            const int8_t *cp = (const int8_t *)ka->Y + ye;         // Q8_0F
+            const float *sp = ka->scales + (ye >> 5);
+            float16_t P = zero;
+            auto four = [&](auto last, int64_t n) __attribute__((always_inline)) { // n: of this lane's four, inside K
+                constexpr bool LAST = decltype(last)::value;
+                float xv[4], yv[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) xv[e] = !LAST || e < n ? *xp : 0.f, xp += x_ks;
+                if constexpr (Q8) { // K is whole blocks of 32
+                    const uint32_t c = *(const uint32_t *)cp;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) yv[e] = (float)(int8_t)(c >> (8 * e)) * *sp;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) yv[e] = !LAST || e < n ? *yp : 0.f, yp += y_ks;
+                }
+                xp += 4 * x_ks, yp += 4 * y_ks, cp += 8;
+#pragma unroll
+                for (int e = 0; e < 4; e++) P = __builtin_amdgcn_mfma_f32_32x32x2f32(xv[e], yv[e], P, 0, 0, 0);
+            };
+            int64_t left = kend - it.k0;
+            // eights at a time: more only where a load's address costs no registers of its own
+            constexpr int CH = XKC && (Q8 || YKC) ? 4 : 1;
+#pragma unroll 1
+            for (; left >= 8 * CH; left -= 8 * CH) {
+#pragma unroll
+                for (int u = 0; u < CH; u++) four(std::false_type{}, 4);
+                if constexpr (Q8) sp += CH == 4 || (left & 31) == 8; // at the end of a block
+            }
+            if constexpr (!Q8) {
+#pragma unroll 1
+                for (; left > 0; left -= 8) four(std::true_type{}, left - 4 * fh);
+            }
+            const float bias_j = ka->has_bias && !ka->bias_on_i && !share ? ka->bias[min(jw + j, ka->N - 1)] : 0.f;
+            at = at0;
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                if (bad >> r & 1) out[at] = rt_act(P[r] + (row_bias ? ka->bias[iw + ir + 8 * (r >> 2) + (r & 3)] : bias_j), act);
+                at += (r & 3) == 3 ? 5 * ois : ois;
+            }
         }
     }
 }

@@ -4,6 +4,8 @@ float64.
 The tolerance is the rounding of the accumulation: a sum of K products takes at most six MFMAs per 16 k, each of which rounds
 the accumulator once, plus the fold of a block, the sum over the shares of K and the bias, every rounding at most 2^-24 of
 the magnitudes summed."""
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -160,3 +162,53 @@ def test_outer_products_are_rounded_once(device, stacks, m, n, tl, tr):
             assert np.array_equal(got, want.astype(np.float32))
         else:
             assert (np.abs(got - want) <= 2.0**-24 * (np.abs(x[..., :1].astype(np.float64) * y[:, :1]) + np.abs(got)) * (1 + 2.0**-20)).all()
+
+
+def close_or_alike(got, want, b):
+    """Within the bound where the result is finite; the same infinities and NaNs where it is not."""
+    fine = np.isfinite(want)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    assert (np.abs(got[fine].astype(np.float64) - want[fine]) <= b[fine] + 2.0**-24 * np.abs(want[fine])).all()
+
+
+@pytest.mark.parametrize("tl,tr,to", [(False, False, False), (True, False, False), (False, True, False), (True, True, False), (False, True, True), (True, False, True)])
+@pytest.mark.parametrize("m,k,n", [(130, 68, 70), (200, 99, 260), (64, 1055, 96), (70, 2049, 90), (1, 150, 90), (1500, 96, 1500)])
+def test_products_computed_once_more(device, m, k, n, tl, tr, to):
+    """Rows and columns that are not finite and numbers past the largest bf16, in every layout, K shared and not, with ragged K: a
+    tile that holds one is computed again and its finite outputs stay what they are."""
+    rng = np.random.default_rng(m + k + n)
+    x, y = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    bias = rng.standard_normal(m if to else n).astype(np.float32)
+    x[m // 2], x[m - 1, k - 1], y[k - 1, n // 3] = np.nan, np.inf, -np.inf
+    x[0, 0], y[0] = 3.4e38, rng.choice([-0.25, 0.0, 0.5], n).astype(np.float32)  # the limbs of the first are not finite, the product is
+    got = run(device, x.T.copy() if tl else x, y.T.copy() if tr else y, bias, tl, tr, to)
+    with np.errstate(invalid="ignore", over="ignore"):
+        b = bias[:, None] if to else bias
+        want = (x.astype(np.float64) @ y.astype(np.float64) + b).astype(np.float32)
+        # computed again: rounded after each product
+        limit = 2.0**-24 * (k + 6) * (np.abs(x).astype(np.float64) @ np.abs(y).astype(np.float64) + np.abs(b))
+    close_or_alike(got.T if to else got, want, limit)
+
+
+@pytest.mark.parametrize("to", [True, False])
+@pytest.mark.parametrize("rows,n,k", [(33, 100, 64), (200, 257, 96), (200, 2560, 2560), (20, 40, 4096)])
+def test_codes_computed_once_more(device, rows, n, k, to):
+    """The same against Q8_0F weights with a scale that is infinite, in both orders of the output, with a bias on either axis."""
+    rng = np.random.default_rng(rows + k)
+    w = Quantizer(Quantization.SInt8).quantize(Tensor.from_data(rng.standard_normal((n, k)).astype(np.float32)).to(device))
+    scales = w.storage[(n * k + 255) // 256 * 256 :].view(torch.float32)
+    scales[(n // 2) * (k // 32) + k // 32 - 1] = math.inf
+    codes = w.storage[: n * k].view(torch.int8).cpu().numpy().reshape(n, k)
+    with np.errstate(invalid="ignore"):
+        wf = codes * np.repeat(scales[: n * k // 32].cpu().numpy().reshape(n, -1), 32, axis=1)
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    x[rows // 2], x[rows - 1, 0] = np.nan, 3.4e38
+    wf[:, 0] = np.where(codes[:, 0] == 0, 0.0, wf[:, 0])
+    bias = rng.standard_normal(n if to else rows).astype(np.float32)
+    t = lambda v: Tensor.from_data(v).to(device)
+    got = w.gemm(t(x), t(bias), False, True, to).resolve().to(Device.CPU).storage
+    with np.errstate(invalid="ignore", over="ignore"):
+        b = bias if to else bias[:, None]
+        want = (x.astype(np.float64) @ wf.astype(np.float64).T + b).astype(np.float32)
+        limit = 2.0**-24 * (2 * k + 6) * (np.abs(x).astype(np.float64) @ np.abs(wf).astype(np.float64).T + np.abs(b))
+    close_or_alike(got if to else got.T, want, limit)
