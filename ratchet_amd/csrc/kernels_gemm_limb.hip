@@ -10,14 +10,15 @@
 //   f32 x Q8_0F  a code is an integer of at most eight bits, one exact limb: three MFMAs per tile and 16 k, from a zero
 //                accumulator per block of 32, whose sums are folded into the accumulators with the block's scale in f32,
 //                so no weight is rounded.
-// The sum of the limbs is exact down to 2^-133, bf16's smallest subnormal number (the matrix cores take subnormal operands):
-// a value below 2^-109 = 1.5e-33 is represented to 2^-134 instead of to 24 bits.
-// An operand whose limbs are not finite (infinities, NaNs, magnitudes that round past the largest bf16) makes its outputs
-// NaN: a 32 x 32 tile with an output that is not finite is computed once more on the f32 matrix cores, so what the f32
+// bf16's smallest subnormal number is 2^-133 (the matrix cores take subnormal operands), f32's 2^-149: f32 operands are
+// multiplied by 2^16 before they are split, so the sum of the limbs is exact for every f32 number, and the accumulator by
+// 2^-32 (2^-16 against codes) as the bias is added.
+// An operand whose limbs are not finite (infinities, NaNs, magnitudes from 2^112 on) makes its outputs NaN, a sum past 2^96
+// (2^112) is infinite: a 32 x 32 tile with an output that is not finite is computed once more on the f32 matrix cores, so what the f32
 // arithmetic gives for such inputs is what is stored.
 //
 // Wavefronts 4 and up load (global -> registers two stages ahead), split into limbs and store the limb planes to LDS;
-// wavefronts 0..3 read fragments and multiply.  The split is five and a half vector instructions per value.  Beside a
+// wavefronts 0..3 read fragments and multiply.  The split is six and a half vector instructions per value.  Beside a
 // wavefront that issues 32x32x16 MFMAs back to back a SIMD still issues a vector instruction of its other wavefronts every
 // 5.6 cycles (measured; 6.4 beside 16x16x32, whose MFMAs take 19 cycles for 16), so the splitting hides behind the MFMAs
 // of a large tile, and two loading wavefronts per SIMD use those slots better than one.  Three LDS stages of 32 k: while
@@ -81,6 +82,8 @@ __device__ __forceinline__ int limb_swz(int r) { // 0, 2, 3, 1 for r / 4 mod 4 =
     const int i = (r >> 2) & 3;
     return (((i ^ (i >> 1)) & 1) << 1) | (i >> 1);
 }
+
+constexpr float kLimbScale = 65536.f;
 
 // two f32 -> two bf16 in one register, and what is left of each
 __device__ __forceinline__ uint32_t limb_take(float &x0, float &x1) {
@@ -172,7 +175,7 @@ template <int R, bool KC, int PT> struct LimbFloat {
             uint8_t *d = st + rw * 64 + (((q & 3) ^ limb_swz(rw)) << 4) + ((q >> 2) << 3);
             float x[W];
 #pragma unroll
-            for (int e = 0; e < W; e++) x[e] = r[set][u * W + e];
+            for (int e = 0; e < W; e++) x[e] = r[set][u * W + e] * kLimbScale;
 #pragma unroll
             for (int l = 0; l < 3; l++) {
                 uint32_t h[W / 2];
@@ -359,6 +362,7 @@ __global__ __launch_bounds__(256 + 64 * PW) void gemm_limb_kernel(GemmLimbArgs g
         float *out = (share ? g.partial + (it.s * g.ksplit + it.z) * g.M * g.N : g.out + it.s * g.o_bs) + iw * o_is + jw * o_js;
         const bool row_bias = g.has_bias && g.bias_on_i && !share;
         const int act = share ? RT_ACT_NONE : g.act;
+        constexpr float unscale = Q8 ? 1.f / kLimbScale : 1.f / (kLimbScale * kLimbScale);
         const int il = g.M - iw < BI ? (int)(g.M - iw) : BI, jl = g.N - jw < BJ ? (int)(g.N - jw) : BJ; // rows and columns inside
         float odd = 0.f; // NaN once an output of this lane is not finite
         // offsets inside the tile are 32-bit (the launcher checks)
@@ -379,7 +383,7 @@ __global__ __launch_bounds__(256 + 64 * PW) void gemm_limb_kernel(GemmLimbArgs g
                         for (int r = 0; r < 16; r++) {
                             float v = acc[a][b][r];
                             odd = fmaf(v, 0.f, odd);
-                            v = rt_act_k<decltype(has_act)::value>(v + bj[b]);
+                            v = rt_act_k<decltype(has_act)::value>(fmaf(v, unscale, bj[b]));
                             __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rsrc, off, 0, 0);
                             off += (r & 3) == 3 ? 20u * ois : 4u * ois;
                             if ((r & 7) == 7) __builtin_amdgcn_sched_barrier(0); // eight at a time: their chains of operations overlap
@@ -397,7 +401,7 @@ __global__ __launch_bounds__(256 + 64 * PW) void gemm_limb_kernel(GemmLimbArgs g
                     for (int r = 0; r < 16; r++) {
                         float v = acc[a][b][r];
                         odd = fmaf(v, 0.f, odd);
-                        v += bj[b];
+                        v = fmaf(v, unscale, bj[b]);
                         if (row_bias) v += g.bias[min(iw + i, g.M - 1)];
                         v = rt_act(v, act);
                         if (i < il && j < jl) out[(uint32_t)i * ois + (uint32_t)j * ojs] = v;

@@ -212,3 +212,54 @@ def test_codes_computed_once_more(device, rows, n, k, to):
         want = (x.astype(np.float64) @ wf.astype(np.float64).T + b).astype(np.float32)
         limit = 2.0**-24 * (2 * k + 6) * (np.abs(x).astype(np.float64) @ np.abs(wf).astype(np.float64).T + np.abs(b))
     close_or_alike(got if to else got.T, want, limit)
+
+
+@pytest.mark.parametrize("tr", [False, True])
+@pytest.mark.parametrize("scale_x,scale_y", [(1e-34, 1e3), (1e-36, 1e3), (1e-38, 1e5), (1e-40, 1e10), (1e-43, 1e20), (1e-36, 1e36), (1e-20, 1e-15), (1e34, 1e-38)])
+def test_small_numbers_keep_their_digits(device, scale_x, scale_y, tr):
+    """Every f32 number is the exact sum of its limbs, down to f32's subnormal ones; what is left is the rounding of the sums and
+    of results that are subnormal."""
+    rng = np.random.default_rng(5)
+    x, y = (rng.standard_normal((150, 200)) * scale_x).astype(np.float32), (rng.standard_normal((200, 290)) * scale_y).astype(np.float32)
+    got = run(device, x, y.T.copy() if tr else y, None, False, tr, False)
+    want = x.astype(np.float64) @ y.astype(np.float64)
+    assert (np.abs(got - want) <= bound(x, y, None) + 2.0**-149).all()
+
+
+def test_small_activations_against_codes_keep_their_digits(device):
+    rng = np.random.default_rng(6)
+    for scale_x, scale_w in ((1e-36, 1.0), (1e-41, 1e6), (1e-3, 1e-37), (1e20, 1e-37)):
+        w = Quantizer(Quantization.SInt8).quantize(Tensor.from_data((rng.standard_normal((140, 96)) * scale_w).astype(np.float32)).to(device))
+        wf = w.storage[: 140 * 96].view(torch.int8).double().view(-1, 32) * w.storage[(140 * 96 + 255) // 256 * 256 :].view(torch.float32)[: 140 * 3].double()[:, None]
+        wf = wf.view(140, 96).cpu().numpy()
+        x = (rng.standard_normal((40, 96)) * scale_x).astype(np.float32)
+        got = w.gemm(Tensor.from_data(x).to(device), None, False, True, True).resolve().to(Device.CPU).storage
+        assert (np.abs(got - x.astype(np.float64) @ wf.T) <= bound(x, wf.T, None) + 4 * 2.0**-149).all()
+
+
+@pytest.mark.parametrize("tl,tr", [(False, False), (False, True), (True, False)])
+def test_every_limb_counts(device, tl, tr):
+    """One product per output: six MFMAs make it, the last one's sum is cut at 2^-23 of it, and what the sums before it and the products
+    left out (2^-26) miss is less than that.  Without any one limb product 2^-18 of it would be missing."""
+    rng = np.random.default_rng(7)
+    for m, k, n in ((300, 96, 300), (130, 2048, 70), (1500, 68, 1500)):
+        x, y = np.zeros((m, k), np.float32), rng.standard_normal((k, n)).astype(np.float32)
+        at = rng.integers(0, k, m)
+        x[np.arange(m), at] = rng.standard_normal(m)
+        got = run(device, x.T.copy() if tl else x, y.T.copy() if tr else y, None, tl, tr, False)
+        want = x[np.arange(m), at].astype(np.float64)[:, None] * y[at]
+        assert (np.abs(got - want) <= 4 * 2.0**-24 * np.abs(want)).all(), (np.abs(got - want) / np.abs(want)).max() * 2**24
+
+
+def test_every_limb_counts_against_codes(device):
+    """Three MFMAs make a product of an activation and a code, and the fold with the scale rounds once more."""
+    rng = np.random.default_rng(8)
+    n, k, rows = 300, 96, 200
+    w = Quantizer(Quantization.SInt8).quantize(Tensor.from_data(rng.standard_normal((n, k)).astype(np.float32)).to(device))
+    wf = (w.storage[: n * k].view(torch.int8).double().view(-1, 32) * w.storage[(n * k + 255) // 256 * 256 :].view(torch.float32)[: n * k // 32].double()[:, None])
+    wf = wf.view(n, k).cpu().numpy()
+    x, at = np.zeros((rows, k), np.float32), rng.integers(0, k, rows)
+    x[np.arange(rows), at] = rng.standard_normal(rows)
+    got = w.gemm(Tensor.from_data(x).to(device), None, False, True, True).resolve().to(Device.CPU).storage
+    want = x[np.arange(rows), at].astype(np.float64)[:, None] * wf[:, at].T
+    assert (np.abs(got - want) <= 4 * 2.0**-24 * np.abs(want)).all()
