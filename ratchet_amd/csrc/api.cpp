@@ -437,7 +437,9 @@ rt_status rt_matmul_enqueue_static(rt_ctx *ctx, const rt_matmul_desc *desc, cons
     uint64_t need = 0;
     const rt_status st = rt_matmul_workspace_bytes(ctx, desc, &need);
     if (st != RT_OK) return st;
-    if (need == 0) // this product is not split: no scratch is touched
+    // Not split, or f32 activations: no scratch is touched.  f32 products never used the buffer, and a program may have them in
+    // flight on several streams at once.
+    if (need == 0 || (desc->lhs_dt != RT_F16 && desc->rhs_dt != RT_F16))
         return rt_matmul_enqueue_ws(ctx, desc, lhs, rhs, bias, out, activation, nullptr, 0, stream);
     if (need > kStaticScratchBytes)
         return fail(ctx, RT_ERR_UNSUPPORTED,

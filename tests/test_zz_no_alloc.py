@@ -133,3 +133,34 @@ def test_static_scratch_allocates_nothing_and_passes_checked_mode(device, oracle
         assert np.array_equal(out.cpu().numpy(), first)
     finally:
         L.rt_ctx_destroy(ctx)
+
+
+@pytest.mark.parametrize("wt", ["f32", "q8_0f"])
+def test_products_with_f32_activations_never_touch_the_static_scratch(device, oracle, wt):
+    """Such calls may overlap on different streams: each runs in one pass, with the bits of rt_matmul_enqueue_fused, also where
+    rt_matmul_enqueue_ws would share K."""
+    rng = np.random.default_rng(5)
+    N, M, K = 384, 200, 4096
+    w = (rng.standard_normal((N, K)) * 0.05).astype(np.float32)
+    dt = _ffi.RT_F32 if wt == "f32" else _ffi.RT_Q8_0F
+    dw = _dev(w if wt == "f32" else oracle.q8_0_quantize_f32(w))
+    xs = [_dev(rng.standard_normal((1, M, K)).astype(np.float32)) for _ in range(2)]
+    desc = _ffi.make_desc(dt, (N, K), _ffi.RT_F32, (1, M, K), False, True, True)
+    L, need = _ffi.lib(), ctypes.c_uint64()
+    assert L.rt_matmul_workspace_bytes(device.ctx, ctypes.byref(desc), ctypes.byref(need)) == _ffi.RT_OK and need.value > 0
+    streams = [torch.cuda.Stream() for _ in xs]
+
+    def run(fn, x, out, stream):
+        assert fn(device.ctx, ctypes.byref(desc), dw.data_ptr(), x.data_ptr(), None, ctypes.c_void_p(out.data_ptr()), _ffi.RT_ACT_NONE,
+                  ctypes.c_void_p(stream.cuda_stream)) == _ffi.RT_OK
+
+    one, both = ([torch.full((M * N,), float("nan"), device="cuda") for _ in xs] for _ in range(2))
+    torch.cuda.synchronize()
+    for x, out in zip(xs, one):
+        run(L.rt_matmul_enqueue_fused, x, out, streams[0])
+    torch.cuda.synchronize()
+    for _ in range(5):
+        for x, out, stream in zip(xs, both, streams):
+            run(L.rt_matmul_enqueue_static, x, out, stream)
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(one, both))
