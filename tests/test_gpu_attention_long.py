@@ -56,3 +56,10 @@ def test_against_float64(device, heads, head_dim, rows, keys, scale, causal):
         assert torch.equal(torch.isnan(g), torch.isnan(want))
         ok = ((g - want).abs() <= bound) | torch.isnan(want)
         assert ok.all(), float(((g - want).abs() / bound)[~torch.isnan(want)].max())
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("heads,head_dim,rows,keys", [(448, 64, 64, 300), (512, 96, 16, 130), (512, 128, 1, 90), (448, 80, 65, 300)])
+def test_few_rows_of_many_heads(device, heads, head_dim, rows, keys, causal):
+    """Both sides of the number of rows from which the kernel for many rows takes over."""
+    test_against_float64(device, heads, head_dim, rows, keys, None, causal)
