@@ -63,3 +63,31 @@ def test_against_float64(device, heads, head_dim, rows, keys, scale, causal):
 def test_few_rows_of_many_heads(device, heads, head_dim, rows, keys, causal):
     """Both sides of the number of rows from which the kernel for many rows takes over."""
     test_against_float64(device, heads, head_dim, rows, keys, None, causal)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("heads,head_dim,rows,keys", [(112, 64, 512, 512), (64, 80, 900, 960), (150, 96, 300, 320), (56, 128, 1000, 1024)])
+def test_the_largest_probability_of_a_block_is_exact(device, heads, head_dim, rows, keys, causal):
+    """One key of every block of 64 has the weight, their scores within a factor of 2^8 of each other and in any order, and the values
+    nearly cancel: a probability relative to its own block's maximum is exactly 1, so what is left is the f32 arithmetic and
+    the output's rounding.  Relative to the row's maximum each would be off by up to 2^-11 of itself."""
+    gen = torch.Generator("cuda:0").manual_seed(heads + rows)
+    q, k = (torch.zeros((1, heads, n, head_dim), dtype=torch.float16, device="cuda:0") for n in (rows, keys))
+    v = torch.randn((1, heads, keys, head_dim), generator=gen, device="cuda:0").half()
+    q[..., 0] = 1
+    k[..., 0] = -300
+    at = torch.arange(0, keys, 64, device="cuda:0") + torch.randint(0, 64, (keys // 64,), generator=gen, device="cuda:0")
+    k[0, :, at, 0] = torch.rand((heads, len(at)), generator=gen, device="cuda:0").mul(5).sub(2.5).half()
+    node = tensor(device, q).attention(tensor(device, k), tensor(device, v), causal=causal, kv_len=keys, scale=1.0)
+    node.op.use_workspace = False
+    got = node.resolve().storage.view(torch.float16)[: q.numel()].view(q.shape).double()[0]
+    s = k[0, :, None, :, 0].double().expand(heads, rows, keys)
+    if causal:
+        s = s.masked_fill(torch.arange(keys, device="cuda:0")[None, :] > torch.arange(rows, device="cuda:0")[:, None] + (keys - rows), -math.inf)
+    p = torch.softmax(s, -1)
+    want, mag = torch.matmul(p, v[0].double()), torch.matmul(p, v[0].double().abs())
+    # exp2 of a difference of scores of up to 2^3: 2^-21 of itself; a sum over the blocks
+    hot = p.amax(-1, keepdim=True) > 1e-3 * (p.sum(-1, keepdim=True))
+    seen = (s > -100).any(-1, keepdim=True) & hot
+    ok = ((got - want).abs() <= 2.0**-11 * want.abs() + 2.0**-25 + 2.0**-18 * mag) | ~seen
+    assert ok.all(), float(((got - want).abs() / mag)[seen.expand_as(want)].max())
