@@ -38,7 +38,9 @@ FLAGS = [
     # rotates the loop-carried accumulators of the tiled GEMMs through dozens of
     # v_accvgpr_mov per iteration.
     "-mllvm", "-amdgpu-mfma-vgpr-form=1",
-    "-Wall", "-Wno-unused-function", "-x", "hip",
+    # the LDS-DMA issued from assembly names m0 as clobbered, which the compiler remarks on because it never
+    # allocates that register; it does merge its own writes of m0, and must not across those statements
+    "-Wall", "-Wno-unused-function", "-Wno-inline-asm", "-x", "hip",
 ]
 
 

@@ -640,7 +640,7 @@ __global__ __launch_bounds__(256, 2) void attention_long_kernel(AttnArgs g) {
             const uint32_t rs = 2u * (uint32_t)(val ? g.v_rs : g.k_rs);
             const uint32_t o = (uint32_t)min(kb * AL_BK + lrow[i], g.kv_len - 1) * rs + lcol[i]; // < 2^32: launcher
             const uint32_t dst = lds0 + (uint32_t)(2 * (stage * 2 * BLK + (val ? BLK : 0)) + 1024 * (val ? j - DV : j));
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(o), "s"(val ? V : K) : "memory");
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(o), "s"(val ? V : K) : "m0", "memory");
         }
     };
     // all but the newest `keep` blocks' loads of this wavefront have landed, all LDS reads have returned; then everybody's have

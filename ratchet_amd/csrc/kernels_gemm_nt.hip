@@ -608,7 +608,7 @@ __global__ __launch_bounds__(64 * WI * WJ) void gemm_nt_wide_kernel(GemmNtArgs g
         const uint32_t dst = stage + (uint32_t)((is_a ? 0 : BM) + (wave + WAVES * cc) * 8) * (NT_LDK * 2);
         // as asm: behind the builtin the compiler waits for every load in flight before the next fragment read, which it
         // cannot tell from a read of what the load writes; no register is written, and the barrier's wait covers it
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off), "s"(base) : "memory");
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off), "s"(base) : "m0", "memory");
     };
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)smem;
 

@@ -231,7 +231,7 @@ __global__ __launch_bounds__(64 * (MW + LW), 2) void gemm_q4k_kernel(GemmQ4kArgs
 #pragma unroll
             for (int n = 0; n < NX; n++)
                 asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds0 + (uint32_t)(stage * QR_XSB + min(4 * n + wave, 32) * 1024)),
-                             "v"(xoff[n]), "s"(xk) : "memory");
+                             "v"(xoff[n]), "s"(xk) : "m0", "memory");
         }
     };
 
