@@ -26,7 +26,7 @@
 // x 64 activation rows each: 64 MFMAs per super-block, 8 for the min term).  The activation tiles come by
 // LDS-DMA one super-block ahead in a ring of two stages.  With at most one workgroup per compute unit four more
 // wavefronts issue those loads and nothing else (one per SIMD).  With more the multiplying wavefronts issue
-// them: at 250 registers a SIMD holds two wavefronts, and a second workgroup's multiplying one is worth more there
+// them: at 256 registers a SIMD holds two wavefronts, and a second workgroup's multiplying one is worth more there
 // than a loading one, since the parts of a wavefront's step add up (below) and another's run beside them
 // (8192 x 3072 at 300 / 512 / 1000 / 2048 activation rows 42.2 / 42.9 / 85.7 / 177.6 -> 37.9 / 40.3 / 78.3 / 161.5 us;
 // 3072 x 8192 at 1000 rows 99.8 -> 91.9).  A staged row is 32 K-vectors
@@ -92,7 +92,8 @@ __global__ __launch_bounds__(64 * (MW + LW), 2) void gemm_q4k_kernel(GemmQ4kArgs
     // holds that block's raw weights for all of them
     uint32_t b = blockIdx.x;
     if (g.remap) b = (b & 7) * (gridDim.x >> 3) + (b >> 3);
-    const uint32_t ti = b / (uint32_t)g.tiles_j, tj = b - ti * (uint32_t)g.tiles_j;
+    // (a division runs on the vector units: its result back into a scalar register, where it costs the main loop none of its own)
+    const uint32_t ti = __builtin_amdgcn_readfirstlane(b / (uint32_t)g.tiles_j), tj = b - ti * (uint32_t)g.tiles_j;
     const int64_t i0 = (int64_t)ti * BM, j0 = (int64_t)tj * QR_BN;
     const uint8_t *blocks = g.blocks + (g.a_stack == 1 ? 0 : s) * g.M * g.nsb * 144;
     const half_t *X = g.X + (g.b_stack == 1 ? 0 : s) * g.b_bs;
