@@ -589,7 +589,7 @@ rt_status rt_attention_enqueue(rt_ctx *ctx, const rt_attention_desc *desc, const
     if ((int64_t)desc->batch * desc->heads > 65535) return fail(ctx, RT_ERR_UNSUPPORTED, "attention: batch * heads above 65535");
     DeviceGuard dg(ctx->dev.ordinal);
     if (!dg.ok) return fail(ctx, RT_ERR_NO_DEVICE, "hipSetDevice failed");
-    hipError_t e = rt::launch_attention(*desc, q, k, v, mask, out, workspace, workspace_bytes, (hipStream_t)stream);
+    hipError_t e = rt::launch_attention(*desc, q, k, v, mask, out, workspace, workspace_bytes, (hipStream_t)stream, ctx->dev);
     if (e == hipErrorNotSupported) return fail(ctx, RT_ERR_UNSUPPORTED, "attention: a head's keys or values span 2^31 elements or more");
     if (e != hipSuccess) return hip_fail(ctx, "attention launch", e);
     return RT_OK;

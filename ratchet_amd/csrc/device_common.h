@@ -185,7 +185,7 @@ hipError_t launch_cache_write(void *cache, const void *src, void *cache2, const 
                               int len, int64_t row_bytes, hipStream_t stream);
 hipError_t launch_softmax(int dtype, void *x, int64_t rows, int64_t n, hipStream_t stream);
 hipError_t launch_attention(const rt_attention_desc &d, const void *q, const void *k, const void *v, const void *mask,
-                            void *out, void *workspace, uint64_t workspace_bytes, hipStream_t stream);
+                            void *out, void *workspace, uint64_t workspace_bytes, hipStream_t stream, const DeviceInfo &dev);
 uint64_t attention_workspace_bytes(const rt_attention_desc &d);
 hipError_t launch_quantize_q8_0(const float *src, uint64_t numel, void *dst, hipStream_t stream);
 hipError_t launch_dequantize(int dtype, const void *src, uint64_t numel, float *dst, hipStream_t stream);

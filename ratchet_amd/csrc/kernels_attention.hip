@@ -51,6 +51,7 @@ struct AttnArgs {
     float scale_log2e;  // scale * log2(e): the exponentials are base 2
     int splits;         // workgroups sharing the keys of one query block (blockIdx.z); > 1 needs `partial`
     float *partial;     // [stack][query block][split][64 rows][4 + DP]: running maximum, sum, two unused, unnormalised output
+    int resident;       // attention_long_kernel: workgroups resident at once
 };
 
 constexpr int AT_BQ = 64, AT_BK = 64; // query rows of a workgroup; keys of a block of the eight-wavefront kernel (the unit the split heuristic counts in)
@@ -560,7 +561,6 @@ __global__ __launch_bounds__(256 * NKQ) void attention_kernel(AttnArgs g) {
 // every transposing read wait for all loads into LDS; no register is written by it, and publish() waits for it.
 // DC: head_dim (64, 80, 96 or 128).
 constexpr int AL_BQ = 128, AL_BK = 64;
-constexpr int AL_MIN_WGS = 448; // workgroups from which it is the faster one (launch_attention)
 constexpr int al_stages(int dc) { return dc > 96 ? 2 : 3; }
 typedef __fp16 fp16x4_t __attribute__((ext_vector_type(4)));
 
@@ -589,7 +589,7 @@ __global__ __launch_bounds__(256, 2) void attention_long_kernel(AttnArgs g) {
         if (g.causal && chunk % nqb == 0) {
             const uint32_t hx = chunk / nqb, q = r / hx;
             bhi = x * hx + (r - q * hx);
-            qbi = total <= 512 && nqb % 2 == 0 && 2 * q >= nqb ? q - nqb / 2 : nqb - 1 - q;
+            qbi = total <= (uint32_t)g.resident && nqb % 2 == 0 && 2 * q >= nqb ? q - nqb / 2 : nqb - 1 - q;
         } else {
             lin = x * chunk + r;
             bhi = lin / nqb, qbi = lin - bhi * nqb;
@@ -1062,8 +1062,9 @@ uint64_t attention_workspace_bytes(const rt_attention_desc &d) {
 // f16 tensors, head_dim a multiple of 8 up to 128, rows 16-byte aligned.  `workspace` may be null
 // (or too small): the launch then runs in one pass.
 hipError_t launch_attention(const rt_attention_desc &d, const void *q, const void *k, const void *v, const void *mask,
-                            void *out, void *workspace, uint64_t workspace_bytes, hipStream_t stream) {
+                            void *out, void *workspace, uint64_t workspace_bytes, hipStream_t stream, const DeviceInfo &dev) {
     AttnArgs g{};
+    g.resident = 2 * dev.num_cus;
     g.Q = (const half_t *)q, g.K = (const half_t *)k, g.V = (const half_t *)v, g.mask = mask, g.O = (half_t *)out;
     g.heads = d.heads, g.q_len = d.q_len, g.kv_len = d.kv_len, g.D = d.head_dim;
     g.q_bs = d.q_strides[0], g.q_hs = d.q_strides[1], g.q_rs = d.q_strides[2];
@@ -1090,11 +1091,13 @@ hipError_t launch_attention(const rt_attention_desc &d, const void *q, const voi
         hipLaunchKernelGGL(attention_decode_merge_kernel, dim3((unsigned)stacks), dim3(128), 0, stream, g);
         return hipGetLastError();
     }
+    // The kernel for many query rows, from seven eighths of the workgroups on that are resident at once: fewer leave more of the
+    // chip idle than a step of theirs saves.
     // A block of keys has one exact probability (see the kernel), and the other kernel a running maximum for each 32 of 64 or 128 keys:
     // below four blocks the error there is the smaller one (1.02 times as large here at 64 keys, 1.01 at 130, 1.00 at 256).
     // Up to 64 rows the kernel with 64 of them per workgroup: half of the long one's wavefronts would have none (512 heads x 16
     // rows x 2048 keys x head_dim 64: 44.9 and 55.4 us; 65 rows 74 and 53).
-    if (!mask && g.splits == 1 && d.q_len > AT_BQ && d.kv_len >= 4 * AL_BK && ((int64_t)d.q_len + AL_BQ - 1) / AL_BQ * stacks >= AL_MIN_WGS) {
+    if (!mask && g.splits == 1 && d.q_len > AT_BQ && d.kv_len >= 4 * AL_BK && 8 * (((int64_t)d.q_len + AL_BQ - 1) / AL_BQ * stacks) >= 7 * (int64_t)g.resident) {
         switch (d.head_dim) {
         case 64: return launch_attention_long<64>(g, (int)stacks, stream);
         case 80: return launch_attention_long<80>(g, (int)stacks, stream);

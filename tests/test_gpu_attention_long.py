@@ -1,5 +1,5 @@
 """The attention kernel for many query rows (attention_long_kernel: 128 rows of one head per workgroup, a grid of at least 448 of
-them, no mask tensor) at the sizes where it can go wrong, against float64.
+them, more than 64 rows and from 256 keys on, no mask tensor) and its neighbours on the other side of those rules, at the sizes where it can go wrong, against float64.
 
 The tolerance: a probability is rounded to f16 (2^-11 of itself, 2^-25 absolute below f16's normal numbers) after scores with the
 rounding of an f32 sum of head_dim products, the output once more."""
@@ -91,3 +91,13 @@ def test_the_largest_probability_of_a_block_is_exact(device, heads, head_dim, ro
     seen = (s > -100).any(-1, keepdim=True) & hot
     ok = ((got - want).abs() <= 2.0**-11 * want.abs() + 2.0**-25 + 2.0**-18 * mag) | ~seen
     assert ok.all(), float(((got - want).abs() / mag)[seen.expand_as(want)].max())
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("heads,head_dim,rows,keys,scale", [
+    (448, 128, 65, 256, None), (460, 80, 128, 257, None), (257, 64, 129, 319, None),
+    (150, 128, 350, 256, None),   # causal: the first rows see no key
+    (9, 80, 6600, 300, None),     # few heads: not whole ones per XCD
+    (448, 96, 66, 1030, -0.2), (230, 64, 200, 700, 0.0), (448, 80, 100, 255, None)])
+def test_edges_from_four_key_blocks_on(device, heads, head_dim, rows, keys, scale, causal):
+    test_against_float64(device, heads, head_dim, rows, keys, scale, causal)
