@@ -54,8 +54,9 @@ typedef enum rt_status {
     RT_ERR_DTYPE_MISMATCH = 3, /* (lhs, rhs) pair not allowed, or bias dtype != activation dtype */
     RT_ERR_UNSUPPORTED = 4,    /* transposed quantized operand, K not a multiple of the block;   */
                                /* at enqueue: a shape no kernel takes (more than 65535 stacks or */
-                               /* 65535 x 64 rows on the generic kernel's path, or a quantized   */
-                               /* operand that is not 16-byte aligned)                           */
+                               /* 65535 x 64 rows, 131070 x 64 with f32 activations, on the      */
+                               /* generic kernel's path, or a quantized operand that is not      */
+                               /* 16-byte aligned)                                               */
     RT_ERR_NO_DEVICE = 5,      /* no HIP device / ordinal out of range                           */
     RT_ERR_HIP = 6,            /* a HIP runtime call failed; see rt_last_hip_error               */
     RT_ERR_OOM = 7             /* hipMalloc failed                                               */

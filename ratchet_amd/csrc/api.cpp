@@ -186,7 +186,7 @@ rt_status run_matmul(rt_ctx *ctx, const Lowered &low, const void *lhs, const voi
     // no kernel takes the shape (more than 65535 stacks or row tiles of the generic kernel, a misaligned
     // quantized operand): a limit of this library, not a failure of the runtime
     if (e == hipErrorNotSupported)
-        return fail(ctx, RT_ERR_UNSUPPORTED, "matmul: no kernel takes this shape (over 65535 stacks or 65535 row tiles, or a "
+        return fail(ctx, RT_ERR_UNSUPPORTED, "matmul: no kernel takes this shape (over 65535 stacks, over 65535 row tiles (f16) or 131070 (f32), or a "
                                              "quantized operand that is not 16-byte aligned)");
     if (e != hipSuccess) return hip_fail(ctx, "matmul launch", e);
     return RT_OK;

@@ -489,13 +489,15 @@ RT_TUNABLE(g_gemm_tile, 0);
 hipError_t launch_gemm(const Problem &p, const void *A, const void *B, const void *bias, void *out,
                        hipStream_t stream, const DeviceInfo &dev) {
     if (p.stacks > 65535) return hipErrorNotSupported;
-    // f16: 128 x 128 tiles unless they would leave the chip under two workgroups per compute unit.  Only small f32 products
-    // and those whose strides are too large for gemm_limb_kernel's offsets come here: 64 x 64, in two launches where the rows
-    // are more than a grid's 65535 tiles.
-    int ts = p.act_dt == RT_F16 ? 128 : 64;
-    const int64_t big = ((p.M + 127) / 128) * ((p.N + 127) / 128) * p.stacks;
-    if (big < 2 * (int64_t)dev.num_cus) ts = 64;
-    if (p.act_dt == RT_F16 && (g_gemm_tile == 64 || g_gemm_tile == 128)) ts = g_gemm_tile;
+    // f16: 128 x 128 tiles unless they would leave the chip under two workgroups per compute unit.  Of the f32 products only those
+    // with a K of one or two, small ones in layouts the f32 kernel does not take, and those whose strides are too large
+    // for gemm_limb_kernel's offsets come here: 64 x 64, in two launches where the rows are more than a grid's 65535 tiles.
+    int ts = 64;
+    if (p.act_dt == RT_F16) {
+        const int64_t big = ((p.M + 127) / 128) * ((p.N + 127) / 128) * p.stacks;
+        if (big >= 2 * (int64_t)dev.num_cus) ts = 128;
+        if (g_gemm_tile == 64 || g_gemm_tile == 128) ts = g_gemm_tile;
+    }
     const int64_t gy = (p.M + ts - 1) / ts, gx = (p.N + ts - 1) / ts;
     if (gy > (p.act_dt == RT_F16 ? 65535 : 2 * 65535)) return hipErrorNotSupported;
     GemmArgs g{};

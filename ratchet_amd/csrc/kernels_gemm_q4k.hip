@@ -419,7 +419,7 @@ hipError_t launch_gemm_q4k(const Problem &p, const void *A, const void *B, const
     if (g_gemm_q4k_disable || p.a_dt != RT_Q4_K || p.act_dt != RT_F16) return hipErrorNotSupported;
     if (p.K % 256 != 0 || p.K < 256 || p.b_ks != 1 || p.M < 64 || p.N < 17 || p.stacks > 65535) return hipErrorNotSupported;
     if (((uintptr_t)A & 15u) || ((uintptr_t)B & 15u) || (p.b_js * 2) % 16 || (p.b_bs * 2) % 16) return hipErrorNotSupported;
-    // 32-bit offsets within a stack
+    // 32-bit offsets within a stack, in bytes
     if (p.M * (p.K / 256) * 144 >= (int64_t(1) << 32) || p.N * p.b_js >= (int64_t(1) << 31)) return hipErrorNotSupported;
     GemmQ4kArgs g{};
     g.blocks = (const uint8_t *)A, g.X = (const half_t *)B, g.bias = (const half_t *)bias, g.out = (half_t *)out;
@@ -445,8 +445,8 @@ hipError_t launch_gemm_q4k(const Problem &p, const void *A, const void *B, const
     const int64_t wgs_small = ((p.M + 63) / 64) * tiles_j, wgs = ((p.M + 127) / 128) * tiles_j * p.stacks;
     const bool small = g_gemm_q4k_cfg == 14 || (g_gemm_q4k_cfg == 0 && wgs_small <= dev.num_cus);
     if (small) return go(std::integral_constant<void (*)(GemmQ4kArgs), &gemm_q4k_kernel<1, 4, 4>>{}, 64, 4);
-    // more than one workgroup per compute unit: no loading wavefronts (see the file comment); their offsets are in bytes
-    if (wgs > dev.num_cus && p.N * p.b_js < (int64_t(1) << 31)) return go(std::integral_constant<void (*)(GemmQ4kArgs), &gemm_q4k_kernel<2, 4, 0>>{}, 128, 0);
+    // more than one workgroup per compute unit: no loading wavefronts (see the file comment)
+    if (wgs > dev.num_cus) return go(std::integral_constant<void (*)(GemmQ4kArgs), &gemm_q4k_kernel<2, 4, 0>>{}, 128, 0);
     return go(std::integral_constant<void (*)(GemmQ4kArgs), &gemm_q4k_kernel<2, 4, 4>>{}, 128, 4);
 }
 

@@ -263,3 +263,43 @@ def test_every_limb_counts_against_codes(device):
     got = w.gemm(Tensor.from_data(x).to(device), None, False, True, True).resolve().to(Device.CPU).storage
     want = x[np.arange(rows), at].astype(np.float64)[:, None] * wf[:, at].T
     assert (np.abs(got - want) <= 4 * 2.0**-24 * np.abs(want)).all()
+
+
+@pytest.mark.parametrize("wt", ["f32", "q8_0f"])
+def test_rows_of_four_million(device, wt):
+    """Row strides that the limb kernel's 32-bit offsets do not reach: f32 on the f32 kernel, Q8_0F weights on the generic one."""
+    n, rows, k = 50, 49, 4_000_000
+    gen = torch.Generator("cuda:0").manual_seed(1)
+    x = torch.randn((rows, k), generator=gen, device="cuda:0")
+    t = lambda v: Tensor(tuple(v.shape), DType.F32, device, v.view(torch.uint8).reshape(-1))
+    w = t(torch.randn((n, k), generator=gen, device="cuda:0"))
+    if wt == "q8_0f":
+        w = Quantizer(Quantization.SInt8).quantize(w)
+        codes, scales = w.storage[: n * k].view(torch.int8).view(-1, 32), w.storage[(n * k + 255) // 256 * 256 :].view(torch.float32)[: n * k // 32]
+        wf = (codes.float() * scales[:, None]).view(n, k)
+    else:
+        wf = w.storage.view(torch.float32).view(n, k)
+    got = w.gemm(t(x), None, False, True, True).resolve().storage.view(torch.float32)[: rows * n].view(rows, n).double()
+    want = torch.zeros((rows, n), dtype=torch.float64, device="cuda:0")
+    for lo in range(0, k, 1 << 19):
+        want += x[:, lo : lo + (1 << 19)].double() @ wf[:, lo : lo + (1 << 19)].double().T
+    # k roundings, each at most 2^-24 of a partial sum of about sqrt(k), of either sign: eight times their root mean square
+    assert ((got - want).abs() <= 8 * 2.0**-24 * k).all()
+
+
+@pytest.mark.parametrize("rows,n,k", [(17, 127, 96), (200, 2560, 10240), (300, 100, 4096), (64, 500, 64)])
+def test_codes_with_a_bias_on_the_weight_rows_of_a_row_major_output(device, rows, n, k):
+    """W.gemm(x, bias, False, True, False): out [n, rows] with a bias per column, the kernel's row axis, also where K is shared, and with
+    an activation behind it."""
+    rng = np.random.default_rng(rows + n)
+    w = Quantizer(Quantization.SInt8).quantize(Tensor.from_data((rng.standard_normal((n, k)) / math.sqrt(k)).astype(np.float32)).to(device))
+    x, bias = rng.standard_normal((rows, k)).astype(np.float32), rng.standard_normal(rows).astype(np.float32)
+    wf = dequantize(w).to(Device.CPU).storage
+    t = lambda v: Tensor.from_data(v).to(device)
+    want = wf.astype(np.float64) @ x.astype(np.float64).T + bias
+    limit = bound(wf, x.T, bias)
+    got = w.gemm(t(x), t(bias), False, True, False).resolve().to(Device.CPU).storage
+    assert (np.abs(got - want) <= limit).all()
+    got = w.gemm(t(x), t(bias), False, True, False).silu().resolve().to(Device.CPU).storage
+    # silu's slope is at most 1.1; the hardware's exponential and reciprocal are within 2^-22 of their values for these arguments
+    assert (np.abs(got - want / (1 + np.exp(-want))) <= 1.1 * limit + 2.0**-20 * np.abs(want)).all()
