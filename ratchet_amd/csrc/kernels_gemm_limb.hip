@@ -4,9 +4,12 @@
 // exact sum of three bf16 ones ("limbs"): l0 = rn(x), l1 = rn(x - l0), l2 = x - l0 - l1, eight significant bits each and
 // every difference exact.
 //   f32 x f32    six MFMAs per tile and 16 k: l0.l0, l0.l1, l1.l0, l1.l1, l0.l2, l2.l0.  The three products left out are at
-//                most 2^-26 of |x.y| together, a quarter of the rounding of a single f32 product.  The matrix cores
-//                add 16 products per rounding of the accumulator where the f32 MFMA adds four, so the result is nearer
-//                to the exact sum than the f32 form's (against float64: 3.3e-7 for 4.0e-7 at K = 384, 4.4e-7 for 8.1e-7 at 1536).
+//                most 2^-26 of |x.y| together, a quarter of the rounding of a single f32 product.  The f32 MFMA rounds after every
+//                product (K = 2 and 4: 0.77 and 0.62 of its results are correctly rounded, as of a chain of fused
+//                multiply-adds); here sixteen products are added before the accumulator is rounded, six times per 16 k.
+//                Relative errors against float64 at K = 3 / 64 / 384 / 2560 / 10240: 3.3e-8 / 1.1e-7 / 2.9e-7 / 2.8e-7 /
+//                4.1e-7 (the last two with K shared), f32 MFMA 3.5e-8 / 1.4e-7 / 3.5e-7 / 9.1e-7 / 1.8e-6.  The sums are cut off, not
+//                rounded to nearest: -1e-8 to -4e-7 on positive data for K = 100 to 10240, within the errors above.
 //   f32 x Q8_0F  a code is an integer of at most eight bits, one exact limb: three MFMAs per tile and 16 k, from a zero
 //                accumulator per block of 32, whose sums are folded into the accumulators with the block's scale in f32,
 //                so no weight is rounded.
@@ -35,7 +38,7 @@
 // Whisper attention's [6 x 1500 x 64] . [6 x 64 x 1500] 31.5 -> 23.6, P . V 47.2 -> 22.0; Q8_0F weights against 200 rows,
 // 10240 x 2560 163 -> 62 us, 2560 x 10240 (K shared) 299 -> 56.  What bounds it: the splitting and code conversion beside the
 // MFMAs (a stage of 96 x 128 f32 takes 1650 cycles for 1190 of MFMAs), 2.7 us from launch to the first MFMA, and 1.7 us of
-// output behind the last.
+// output behind the last.  The f32 forms keep 20 to 50 scalar registers in lanes of vector registers; nothing goes to scratch.
 #include "device_common.h"
 
 #include <algorithm>
