@@ -686,14 +686,15 @@ bool limb_orient(Problem &p) {
 }
 
 // Everything with f32 activations but small f32 products.  Those launch_gemm_f32_small has taken before; of what it
-// cannot (operands not aligned to 16 bytes, few rows), with at most two stages and less than a tile of 64 x 64 per compute
-// unit there is nothing to pipeline (8 heads x 22 positions, the attention's three operators: 12.8 us here, 12.0 on the generic kernel).
+// cannot (operands not aligned to 16 bytes, few rows), with two stages and less than a tile of 64 x 64 per compute unit, or
+// one stage and less than two, there is nothing to pipeline (8 heads x 22 positions, the attention's three operators: 12.8 us here,
+// 12.0 on the generic kernel; 20 x [300 x 31] . [31 x 300] 7.7 and 6.7, 32 x [512 x 31] . [31 x 512] 13.5 and 17.0).
 // K of 1 and 2 go to the generic kernel: the f32 MFMA rounds once per product, so it gives an outer product correctly rounded,
 // and the limbs cannot (relative error against float64 2.5e-8 and 3.1e-8 there, 3.5e-8 and 3.3e-8 here; from K = 3 on it is smaller
 // here, 3.3e-8 to 3.5e-8).
 bool limb_takes(const Problem &p, const DeviceInfo &dev) {
     if (p.act_dt != RT_F32 || (p.a_dt != RT_F32 && p.a_dt != RT_Q8_0F) || p.M <= 0 || p.N <= 0 || p.K <= 0 || p.stacks <= 0) return false;
-    return p.a_dt == RT_Q8_0F || p.K > 64 || (p.K > 2 && ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.stacks > dev.num_cus);
+    return p.a_dt == RT_Q8_0F || p.K > 64 || (p.K > 2 && ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.stacks > (p.K <= 32 ? 2 : 1) * (int64_t)dev.num_cus);
 }
 
 template <int BI, int BJ, int WI, int PW, bool Q8, bool XKC, bool YKC> hipError_t launch_limb_k(const GemmLimbArgs &g, unsigned grid, hipStream_t st) {
