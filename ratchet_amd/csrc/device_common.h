@@ -164,6 +164,7 @@ hipError_t launch_gemm_q4k(const Problem &p, const void *A, const void *B, const
                            const DeviceInfo &dev);
 hipError_t launch_gemm_f32(const Problem &p, const void *A, const void *B, const void *bias, void *out, hipStream_t stream,
                            const DeviceInfo &dev);
+bool gemm_f32_few_tiles(const Problem &p, const DeviceInfo &dev);
 hipError_t launch_gemm_f32_small(const Problem &p, const void *A, const void *B, const void *bias, void *out, hipStream_t stream,
                                  const DeviceInfo &dev);
 uint64_t gemm_limb_workspace_bytes(const Problem &p, const DeviceInfo &dev);

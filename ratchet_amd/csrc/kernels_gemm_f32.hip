@@ -307,6 +307,11 @@ hipError_t launch_gemm_f32(const Problem &p, const void *A, const void *B, const
     return b_kcont ? launch_f32<32, 96, true>(g, p.stacks, stream) : launch_f32<32, 96, false>(g, p.stacks, stream);
 }
 
+// at most one of this kernel's tiles per compute unit
+bool gemm_f32_few_tiles(const Problem &p, const DeviceInfo &dev) {
+    return ((p.M + 31) / 32) * (p.N <= 64 ? 1 : (p.N + 95) / 96) * p.stacks <= dev.num_cus;
+}
+
 // The f32 products that are faster here than on gemm_limb_kernel, which is asked next: there splitting lies between the
 // first load and the first MFMA, and a tile is at least 64 x 64.
 //   K <= 32                     one stage, nothing to pipeline (32 x [512 x 4 / 16 / 32] . [.. x 512] 10.0 / 11.2 / 12.5 us here,
@@ -314,13 +319,11 @@ hipError_t launch_gemm_f32(const Problem &p, const void *A, const void *B, const
 //   K <= 128, few tiles         at most one of the tiles here per compute unit (scores of 32 heads x 56 positions, head_dim 96: 3.8 /
 //                               5.2 us; 8 heads x 232 x 232 4.9 / 5.4, 300 x 300 6.2 / 5.6; P . V of 128 keys into 64 columns 4.2 / 5.6;
 //                               of 232 keys 7.6 / 7.6)
-//   48 to 64 columns, few tiles, B K-contiguous   Linear over a few dozen positions (48 rows x 1536 x 384: 8.4 / 8.8 us; x 384 x 1536
-//                               23.4 / 25.2).  From K = 512 on the other kernel shares K among workgroups when it has a workspace.
+//   K < 512, few tiles, 48 to 64 columns, B K-contiguous   Linear over a few dozen positions (48 rows x 1536 x 384: 8.4 /
+//                               8.8 us); from 512 on the other kernel shares K among workgroups, or comes back here when it cannot.
 hipError_t launch_gemm_f32_small(const Problem &p, const void *A, const void *B, const void *bias, void *out, hipStream_t stream,
                                  const DeviceInfo &dev) {
-    const bool narrow = p.N <= 64;
-    const bool few = ((p.M + 31) / 32) * (narrow ? 1 : (p.N + 95) / 96) * p.stacks <= dev.num_cus;
-    const bool takes = p.K <= F32_BK || (few && (p.K <= 128 || (narrow && p.b_ks == 1 && (p.K < 512 || !p.workspace))));
+    const bool takes = p.K <= F32_BK || (gemm_f32_few_tiles(p, dev) && (p.K <= 128 || (p.K < 512 && p.N <= 64 && p.b_ks == 1)));
     return takes ? launch_gemm_f32(p, A, B, bias, out, stream, dev) : hipErrorNotSupported;
 }
 

@@ -725,15 +725,22 @@ uint64_t gemm_limb_workspace_bytes(const Problem &p0, const DeviceInfo &dev) {
 }
 
 // Any strides; quantized rows 16-byte aligned.  hipErrorNotSupported: another kernel must take the problem.
-hipError_t launch_gemm_limb(const Problem &p0, const void *A, const void *B, const void *bias, void *out, hipStream_t stream,
+hipError_t launch_gemm_limb(const Problem &p0, const void *A0, const void *B0, const void *bias, void *out, hipStream_t stream,
                             const DeviceInfo &dev) {
     Problem p = p0;
+    const void *A = A0, *B = B0;
     if (limb_orient(p)) std::swap(A, B);
     if (!limb_takes(p, dev)) return hipErrorNotSupported;
     const bool q8 = p.a_dt == RT_Q8_0F;
     if (q8 && ((uintptr_t)A & 15u)) return hipErrorNotSupported;
     LimbPlan pl = limb_plan(p, dev, p.workspace != nullptr && !((uintptr_t)p.workspace & 15u));
     if (pl.ksplit > 1 && p.workspace_bytes < (uint64_t)p.stacks * pl.ksplit * p.M * p.N * sizeof(float)) pl = limb_plan(p, dev, false);
+    // A long K that is not shared, in few tiles: a workgroup's own chain of stages is all there is, and with 48 to 64 columns, both
+    // operands K-contiguous, the f32 kernel's is the shorter (48 rows x 384 x 1536: 23.4 us, 25.2 here; x 2560 x 2560 37.2, 40.1).
+    // From here, not as a family of its own: a plan keeps the family, and the workspace may come and go.
+    if (!q8 && pl.ksplit == 1 && p0.N <= 64 && p0.b_ks == 1 && gemm_f32_few_tiles(p0, dev)) {
+        if (const hipError_t e = launch_gemm_f32(p0, A0, B0, bias, out, stream, dev); e != hipErrorNotSupported) return e;
+    }
     GemmLimbArgs g{};
     g.bias = (const float *)bias, g.out = (float *)out;
     g.K = p.K, g.o_bs = p.o_bs, g.has_bias = p.has_bias, g.act = p.act;

@@ -303,3 +303,33 @@ def test_codes_with_a_bias_on_the_weight_rows_of_a_row_major_output(device, rows
     got = w.gemm(t(x), t(bias), False, True, False).silu().resolve().to(Device.CPU).storage
     # silu's slope is at most 1.1; the hardware's exponential and reciprocal are within 2^-22 of their values for these arguments
     assert (np.abs(got - want / (1 + np.exp(-want))) <= 1.1 * limit + 2.0**-20 * np.abs(want)).all()
+
+
+def test_a_plan_gives_the_same_bits_whatever_workspace_came_before(device):
+    """A plan offers its product first to the family that took it last; a workspace given on one call and not on the next must lead
+    where rt_matmul_enqueue_ws leads without a plan."""
+    import ctypes
+
+    from ratchet_amd import _ffi
+
+    rng = np.random.default_rng(9)
+    L = _ffi.lib()
+    dev = lambda v: torch.from_numpy(v).to("cuda:0")
+    for n, k, rows in ((384, 1536, 48), (300, 2048, 64), (384, 1536, 200), (384, 384, 48)):
+        w, x, bias = (dev(rng.standard_normal(s).astype(np.float32)) for s in ((n, k), (rows, k), (n,)))
+        desc = _ffi.make_desc(_ffi.RT_F32, (n, k), _ffi.RT_F32, (rows, k), False, True, True, _ffi.RT_F32, (n,))
+        need, plan = ctypes.c_uint64(), ctypes.c_void_p()
+        assert L.rt_matmul_workspace_bytes(device.ctx, ctypes.byref(desc), ctypes.byref(need)) == _ffi.RT_OK
+        ws = torch.empty(max(need.value, 16), dtype=torch.uint8, device="cuda:0")
+        assert L.rt_matmul_plan_create(device.ctx, ctypes.byref(desc), _ffi.RT_ACT_NONE, ctypes.byref(plan)) == _ffi.RT_OK
+        stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        ptrs = (w.data_ptr(), x.data_ptr(), bias.data_ptr())
+        try:
+            for size in (need.value, 0, 0, need.value, need.value, 0):
+                a, b = (torch.full((rows, n), float("nan"), device="cuda:0") for _ in range(2))
+                args = (ctypes.c_void_p(ws.data_ptr()) if size else None, size, stream)
+                assert L.rt_matmul_plan_enqueue(plan, *ptrs, ctypes.c_void_p(a.data_ptr()), *args) == _ffi.RT_OK
+                assert L.rt_matmul_enqueue_ws(device.ctx, ctypes.byref(desc), *ptrs, ctypes.c_void_p(b.data_ptr()), _ffi.RT_ACT_NONE, *args) == _ffi.RT_OK
+                assert torch.equal(a, b), (n, k, rows, size)
+        finally:
+            L.rt_matmul_plan_destroy(plan)
