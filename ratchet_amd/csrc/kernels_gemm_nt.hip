@@ -1,20 +1,21 @@
 // MFMA GEMMs for the Linear / QK^T form, where both operands are K-contiguous:
 //   C[s, i, j] = sum_k A[s, i, k] * B[s, j, k] (+ bias),  f16 in, f32 accumulate, f16 out.
-// A is f16 or a Q8_0H weight; B is f16.  Five kernels, chosen by launch_gemm_nt:
+// A is f16 or a Q8_0H weight; B is f16.  Six kernels, chosen by launch_gemm_nt:
 //
 //   gemm_nt_wide_kernel    f16 x f16, K % 64 == 0, many activation rows: 320 x 256 tiles, eight wavefronts that
 //                          both load and multiply (half the operand bytes per product of the 160 x 128 tiles)
-//   gemm_nt_dl_kernel      f16 x f16, K % 64 == 0: 160 x 128 tiles, tiles loaded global -> LDS
+//   gemm_nt_dl_kernel      f16 x f16, K % 32 == 0: tiles of 64 x 64 to 160 x 128 (nt_choose), loaded global -> LDS
 //                          directly into a ring of stages by two wavefronts that do nothing else,
 //                          issue order pinned (the fast path for the Phi-2 prefill shape:
 //                          10240 x 512 outputs = 256 workgroups, one per CU)
 //   gemm_nt_q8w_kernel     Q8_0H x f16, K % 256 == 0: the same pipeline; four loading wavefronts widen the int8
 //                          tile to f16 codes on its way into LDS, each block of 32 is multiplied from zero and
 //                          its partial sums are folded into the accumulators with the block's scale in f32
+//   gemm_nt_q8r_kernel     Q8_0H x f16, any other K
 //   gemm_nt_shortk_kernel  f16 x f16, K <= 128 (attention scores): a resident strip of B rows,
 //                          A tiles prefetched through registers, output written as it is produced
-//   gemm_nt_kernel         everything else this file takes (ragged K, Q8_0H with K % 256 != 0,
-//                          short K without a contiguous output axis): register-staged, two LDS stages
+//   gemm_nt_kernel         f16 x f16 with a K that is no multiple of 32, or short and without a contiguous
+//                          output axis: register-staged, two LDS stages
 //
 // Common to all: 2 x 2 multiplying wavefronts (the wide kernel: 2 x 4), v_mfma_f32_16x16x32_f16 with A rows on the MFMA's
 // lane index, XOR-swizzled or odd-stride LDS rows so that fragment reads are conflict-free, an
@@ -23,9 +24,7 @@
 // operands its L2 holds once (nt_tile_of).
 //
 // gemm_nt_kernel's pipeline per K tile of 64: global loads of tile t+2 into registers, MFMAs on LDS
-// stage t, then the registers of tile t+1 -> the other LDS stage, one barrier.  For Q8_0H it widens
-// the int8 codes to f16 on the way into LDS (exact), accumulates each block of 32 separately and
-// folds it in with its scale in f32, so no weight is ever rounded.
+// stage t, then the registers of tile t+1 -> the other LDS stage, one barrier.
 //
 // Roles in the reference: ops/gemm.rs:305-657 (GEMM generators), with Linear's
 // W.gemm(x, b, false, true, true) (crates/ratchet-nn/src/linear.rs:17-24) and attention's
@@ -36,9 +35,12 @@
 
 namespace rt {
 
+typedef uint32_t uint4_d __attribute__((ext_vector_type(4), aligned(4)));
+
 struct GemmNtArgs {
     const void *A;       // f16 [.., M, K] or Q8_0H codes
-    const half_t *scales; // Q8_0H scale stream of A
+    const half_t *scales; // Q8_0H scale stream of A, dwords in it (whole 256 bytes)
+    int64_t scale_dwords;
     const half_t *B;     // f16 [.., N, K]
     const half_t *bias;
     half_t *out;
@@ -201,14 +203,82 @@ __device__ __forceinline__ void nt_epilogue(const GemmNtArgs &g, float4_t (&acc)
     });
 }
 
+// The same for accumulators of 32 x 32 MFMA tiles: lane l holds A row l % 32 and B rows 8 * (r / 4) + 4 * (l / 32) + r % 4.
+template <int TM, int TN, int WM, int WN>
+__device__ __forceinline__ void nt_epilogue32(const GemmNtArgs &g, float16_t (&acc)[TM][TN], uint8_t *smem, int64_t s, int64_t i0, int64_t j0, int wi, int wj,
+                                              int wave, int lane) {
+    const int fr = lane & 31, fh = lane >> 5;
+    const int64_t iw = i0 + wi * WM, jw = j0 + wj * WN;
+    if (g.ksplit > 1) { // this workgroup's share of K: the sums as they are, [j][i] with i contiguous
+        float *pt = g.partial + ((s * g.ksplit + blockIdx.z) * g.N) * g.M;
+#pragma unroll
+        for (int a = 0; a < TM; a++) {
+            const int64_t i = iw + a * 32 + fr;
+#pragma unroll
+            for (int b = 0; b < TN; b++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int64_t j = jw + b * 32 + 8 * (r >> 2) + 4 * fh + (r & 3);
+                    if (i < g.M && j < g.N) pt[j * g.M + i] = acc[a][b][r];
+                }
+        }
+        return;
+    }
+    half_t *out = g.out + s * g.o_bs;
+    constexpr int EROW = WM + 8; // halfs per staged B row (+16 B pad)
+    half_t *es = (half_t *)smem + wave * (WN * EROW);
+    float bi[TM]; // the bias of this lane's A rows, asked for once
+#pragma unroll
+    for (int a = 0; a < TM; a++) {
+        const int64_t i = iw + a * 32 + fr;
+        bi[a] = g.has_bias && g.bias_on_rows && i < g.M ? (float)g.bias[i] : 0.f;
+    }
+    rt_with_act(g.act, [&](auto has_act) {
+#pragma unroll
+        for (int a = 0; a < TM; a++)
+#pragma unroll
+            for (int b = 0; b < TN; b++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int jl = b * 32 + 8 * (r >> 2) + 4 * fh + (r & 3);
+                    float v = acc[a][b][r] + bi[a];
+                    if (g.has_bias && !g.bias_on_rows) v += (float)g.bias[min(jw + jl, g.N - 1)];
+                    v = rt_act_k<decltype(has_act)::value>(v);
+                    es[jl * EROW + a * 32 + fr] = (half_t)v;
+                }
+    });
+    asm volatile("" ::: "memory"); // same wavefront reads back below; DS operations complete in order
+    if (g.vec_epilogue) {
+        constexpr int VPR = WM / 8; // 128-bit vectors per staged row
+        for (int v = lane; v < WN * VPR; v += 64) {
+            const int jl = v / VPR, c = v - jl * VPR;
+            const int64_t j = jw + jl, i = iw + 8 * c;
+            if (j < g.N) {
+                if (i + 8 <= g.M) {
+                    __builtin_nontemporal_store(*(const uint4_t *)(es + jl * EROW + 8 * c), (uint4_t *)(out + j * g.o_js + i)); // written once, not read back here
+                } else {
+                    for (int e = 0; e < 8; e++)
+                        if (i + e < g.M) out[j * g.o_js + i + e] = es[jl * EROW + 8 * c + e];
+                }
+            }
+        }
+    } else { // rows that do not start on 16 bytes, or another axis contiguous: value by value, along i
+        for (int v = lane; v < WN * WM; v += 64) {
+            const int jl = v / WM, il = v - jl * WM;
+            const int64_t j = jw + jl, i = iw + il;
+            if (j < g.N && i < g.M) out[i * g.o_is + j * g.o_js] = es[jl * EROW + il];
+        }
+    }
+}
+
 // KFULL: K is a multiple of the K step, so no load or store needs a bound.
-template <int BM, int BN, bool Q8, bool KFULL>
+template <int BM, int BN, bool KFULL>
 __global__ __launch_bounds__(NT_THREADS, (BM * BN <= 128 * 64 ? 3 : 1)) void gemm_nt_kernel(GemmNtArgs g) {
     constexpr int WM = BM / 2, WN = BN / 2;      // wavefront sub-tile
     constexpr int TM = WM / 16, TN = WN / 16;    // MFMA tiles per wavefront
     static_assert(WM % 16 == 0 && WN % 16 == 0, "tile must split into 16x16 MFMA tiles");
     // 16-byte vectors per K tile row, and per thread
-    constexpr int A_VPR = Q8 ? NT_BK / 16 : NT_BK / 8;
+    constexpr int A_VPR = NT_BK / 8;
     constexpr int A_VEC = (BM * A_VPR + NT_THREADS - 1) / NT_THREADS;
     constexpr int B_VPR = NT_BK / 8;
     constexpr int B_VEC = (BN * B_VPR + NT_THREADS - 1) / NT_THREADS;
@@ -216,7 +286,6 @@ __global__ __launch_bounds__(NT_THREADS, (BM * BN <= 128 * 64 ? 3 : 1)) void gem
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     half_t *As = (half_t *)smem;                         // [2][BM][NT_LDK]
     half_t *Bs = As + 2 * BM * NT_LDK;                   // [2][BN][NT_LDK]
-    float *Sd = (float *)(Bs + 2 * BN * NT_LDK);         // [2 stages][2 blocks][BM]   (Q8 only)
 
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int wi = wave >> 1, wj = wave & 1;
@@ -230,30 +299,18 @@ __global__ __launch_bounds__(NT_THREADS, (BM * BN <= 128 * 64 ? 3 : 1)) void gem
 
     // two register sets: the loads of tile t+2 are in flight while tile t is multiplied
     uint4_t ra0[A_VEC], rb0[B_VEC], ra1[A_VEC], rb1[B_VEC];
-    half_t rsc0[2], rsc1[2]; // Q8: this thread's scales for the tile's two blocks (threads < BM)
 
     // Loads are unconditional (addresses past K are clamped to a valid one) so that no branch
     // separates them from the LDS store that consumes them and the hardware counters can let
     // the other register set's loads stay in flight; store_tiles zeroes what lies past K.
-    auto load_tiles = [&](int64_t k0, uint4_t (&ra)[A_VEC], uint4_t (&rb)[B_VEC], half_t (&rsc)[2]) {
+    auto load_tiles = [&](int64_t k0, uint4_t (&ra)[A_VEC], uint4_t (&rb)[B_VEC]) {
 #pragma unroll
         for (int e = 0; e < A_VEC; e++) {
             const int v = min(e * NT_THREADS + t, BM * A_VPR - 1);
             const int r = v / A_VPR, c = v - r * A_VPR;
             const int64_t gr = min(i0 + r, g.M - 1); // rows past the end duplicate the last one; never stored
-            if constexpr (Q8) {
-                const int64_t gk = KFULL ? k0 + 16 * c : min(k0 + 16 * c, g.K - 16);
-                ra[e] = *(const uint4_t *)((const uint8_t *)g.A + a_el + gr * g.a_rs + gk);
-            } else {
-                const int64_t gk = KFULL ? k0 + 8 * c : min(k0 + 8 * c, g.K - 8);
-                ra[e] = *(const uint4_t *)((const half_t *)g.A + a_el + gr * g.a_rs + gk);
-            }
-        }
-        if constexpr (Q8) {
-            const int64_t gr = min(i0 + min(t, BM - 1), g.M - 1);
-            const int64_t row_blk = (a_el + gr * g.a_rs) >> 5, kb = k0 >> 5, last = (g.K >> 5) - 1;
-            rsc[0] = g.scales[row_blk + (KFULL ? kb : min(kb, last))];
-            rsc[1] = g.scales[row_blk + (KFULL ? kb + 1 : min(kb + 1, last))];
+            const int64_t gk = KFULL ? k0 + 8 * c : min(k0 + 8 * c, g.K - 8);
+            ra[e] = *(const uint4_t *)((const half_t *)g.A + a_el + gr * g.a_rs + gk);
         }
 #pragma unroll
         for (int e = 0; e < B_VEC; e++) {
@@ -265,8 +322,7 @@ __global__ __launch_bounds__(NT_THREADS, (BM * BN <= 128 * 64 ? 3 : 1)) void gem
         }
     };
 
-    auto store_tiles = [&](int stage, int64_t k0, const uint4_t (&ra)[A_VEC], const uint4_t (&rb)[B_VEC],
-                           const half_t (&rsc)[2]) {
+    auto store_tiles = [&](int stage, int64_t k0, const uint4_t (&ra)[A_VEC], const uint4_t (&rb)[B_VEC]) {
         half_t *as = As + stage * BM * NT_LDK, *bs = Bs + stage * BN * NT_LDK;
         const uint4_t zero4 = {0, 0, 0, 0};
 #pragma unroll
@@ -274,26 +330,7 @@ __global__ __launch_bounds__(NT_THREADS, (BM * BN <= 128 * 64 ? 3 : 1)) void gem
             const int v = e * NT_THREADS + t;
             if (v < BM * A_VPR) {
                 const int r = v / A_VPR, c = v - r * A_VPR;
-                if constexpr (Q8) {
-                    const uint4_t raw = (KFULL || k0 + 16 * c < g.K) ? ra[e] : zero4;
-                    half2_t h[8];
-#pragma unroll
-                    for (int d = 0; d < 4; d++) nt_cvt_i8x4(raw[d], h[2 * d], h[2 * d + 1]);
-                    uint4_t lo = {__builtin_bit_cast(uint32_t, h[0]), __builtin_bit_cast(uint32_t, h[1]),
-                                  __builtin_bit_cast(uint32_t, h[2]), __builtin_bit_cast(uint32_t, h[3])};
-                    uint4_t hi = {__builtin_bit_cast(uint32_t, h[4]), __builtin_bit_cast(uint32_t, h[5]),
-                                  __builtin_bit_cast(uint32_t, h[6]), __builtin_bit_cast(uint32_t, h[7])};
-                    *(uint4_t *)(as + nt_slot(r, 2 * c)) = lo;
-                    *(uint4_t *)(as + nt_slot(r, 2 * c + 1)) = hi;
-                } else {
-                    *(uint4_t *)(as + nt_slot(r, c)) = (KFULL || k0 + 8 * c < g.K) ? ra[e] : zero4;
-                }
-            }
-        }
-        if constexpr (Q8) {
-            if (t < BM) {
-                Sd[(stage * 2 + 0) * BM + t] = (KFULL || k0 < g.K) ? (float)rsc[0] : 0.f;
-                Sd[(stage * 2 + 1) * BM + t] = (KFULL || k0 + 32 < g.K) ? (float)rsc[1] : 0.f;
+                *(uint4_t *)(as + nt_slot(r, c)) = (KFULL || k0 + 8 * c < g.K) ? ra[e] : zero4;
             }
         }
 #pragma unroll
@@ -317,7 +354,6 @@ __global__ __launch_bounds__(NT_THREADS, (BM * BN <= 128 * 64 ? 3 : 1)) void gem
     const int swz = (fr >> 1) & 7;
     struct Frags {
         half8_t fa[TM], fb[TN];
-        float d[Q8 ? TM : 1]; // Q8: scale of this lane's A row, per tile, for the block this K step covers
     };
     auto read_frags = [&](int stage, int kk, Frags &f) {
         const half_t *as = As + stage * BM * NT_LDK + (wi * WM + fr) * NT_LDK + (((kk * 4 + fg) ^ swz) << 3);
@@ -326,30 +362,13 @@ __global__ __launch_bounds__(NT_THREADS, (BM * BN <= 128 * 64 ? 3 : 1)) void gem
         for (int a = 0; a < TM; a++) f.fa[a] = __builtin_bit_cast(half8_t, *(const uint4_t *)(as + a * 16 * NT_LDK));
 #pragma unroll
         for (int b = 0; b < TN; b++) f.fb[b] = __builtin_bit_cast(half8_t, *(const uint4_t *)(bs + b * 16 * NT_LDK));
-        if constexpr (Q8) {
-#pragma unroll
-            for (int a = 0; a < TM; a++) f.d[a] = Sd[(stage * 2 + kk) * BM + wi * WM + a * 16 + fr];
-        }
     };
     auto mma_step = [&](const Frags &f) {
-        if constexpr (Q8) {
-            // one Q8_0 block: fresh partial sums, then acc += scale * partial (scale per lane = per A row)
 #pragma unroll
-            for (int a = 0; a < TM; a++)
+        for (int a = 0; a < TM; a++)
 #pragma unroll
-                for (int b = 0; b < TN; b++) {
-                    const float4_t zero = {0.f, 0.f, 0.f, 0.f};
-                    const float4_t p = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.fb[b], f.fa[a], zero, 0, 0, 0);
-#pragma unroll
-                    for (int r = 0; r < 4; r++) acc[a][b][r] = fmaf(f.d[a], p[r], acc[a][b][r]);
-                }
-        } else {
-#pragma unroll
-            for (int a = 0; a < TM; a++)
-#pragma unroll
-                for (int b = 0; b < TN; b++)
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.fb[b], f.fa[a], acc[a][b], 0, 0, 0);
-        }
+            for (int b = 0; b < TN; b++)
+                acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.fb[b], f.fa[a], acc[a][b], 0, 0, 0);
     };
 
     // Software pipeline: tile t is multiplied from LDS stage t % 2 while tile t+1 sits in one
@@ -367,22 +386,22 @@ __global__ __launch_bounds__(NT_THREADS, (BM * BN <= 128 * 64 ? 3 : 1)) void gem
         mma_step(f1);
     };
     if (nk > 0) {
-        load_tiles(0, ra0, rb0, rsc0);
-        load_tiles(kclamp(1), ra1, rb1, rsc1);
-        store_tiles(0, 0, ra0, rb0, rsc0);
+        load_tiles(0, ra0, rb0);
+        load_tiles(kclamp(1), ra1, rb1);
+        store_tiles(0, 0, ra0, rb0);
     }
     __syncthreads();
     for (int64_t kt = 0; kt < nk; kt += 2) {
         // even tile: set 1 holds tile kt+1, set 0 is free for tile kt+2
-        load_tiles(kclamp(kt + 2), ra0, rb0, rsc0);
+        load_tiles(kclamp(kt + 2), ra0, rb0);
         compute(0);
-        store_tiles(1, (kt + 1) * NT_BK, ra1, rb1, rsc1);
+        store_tiles(1, (kt + 1) * NT_BK, ra1, rb1);
         __syncthreads();
         if (kt + 1 >= nk) break;
         // odd tile: set 0 holds tile kt+2, set 1 is free for tile kt+3
-        load_tiles(kclamp(kt + 3), ra1, rb1, rsc1);
+        load_tiles(kclamp(kt + 3), ra1, rb1);
         compute(1);
-        store_tiles(0, (kt + 2) * NT_BK, ra0, rb0, rsc0);
+        store_tiles(0, (kt + 2) * NT_BK, ra0, rb0);
         __syncthreads();
     }
     __syncthreads(); // every wavefront is done with the tile stages: the epilogue reuses them
@@ -396,7 +415,7 @@ __global__ __launch_bounds__(NT_THREADS, (BM * BN <= 128 * 64 ? 3 : 1)) void gem
 // registers.  A wavefront's load instruction writes 1 KiB of LDS contiguously
 // (lane l at base + 16 l), i.e. 8 whole rows of the swizzled tile; the swizzle is
 // applied on the global side by choosing which K-vector each lane fetches.
-// Requires K % 64 == 0; full tiles are not required (rows are clamped).
+// Requires K % 32 == 0; full tiles are not required (rows are clamped, and a last tile of 32 is multiplied as half a one).
 //
 // The loads are issued by wavefronts of their own.  A wavefront issues in order, one per SIMD
 // here: when the memory pipeline pushes back on a load, the MFMAs behind it wait too, and with
@@ -424,7 +443,7 @@ __global__ __launch_bounds__(NT_THREADS + 64 * LW) void gemm_nt_dl_kernel(GemmNt
     half_t *ring = (half_t *)smem; // [STAGES][BM + BN][64]
 
     const int t = threadIdx.x, lane = t & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6); if (wave < 4) __builtin_amdgcn_s_setprio(3);
 
     int64_t ti, tj;
     nt_tile_of(g, blockIdx.x, ti, tj); // XCD-aware tile order (see the file comment)
@@ -432,7 +451,8 @@ __global__ __launch_bounds__(NT_THREADS + 64 * LW) void gemm_nt_dl_kernel(GemmNt
     const int64_t s = blockIdx.y;
     const int64_t kbase = (int64_t)blockIdx.z * g.k_len;
     const int64_t a_el = (g.a_stack == 1 ? 0 : s) * g.a_bs + kbase, b_el = (g.b_stack == 1 ? 0 : s) * g.b_bs + kbase;
-    const int64_t nk = g.k_len / NT_BK; // nk >= 1
+    const int kn = (int)min(g.k_len, g.K - kbase); // this workgroup's share of K: > 0, a multiple of 32 (launcher)
+    const int nk = (kn + NT_BK - 1) / NT_BK;
 
     if (wave >= 4) {
         // ---- loading wavefront: lane l fills LDS row chunk * 8 + l / 8, slot l % 8, which must
@@ -443,16 +463,17 @@ __global__ __launch_bounds__(NT_THREADS + 64 * LW) void gemm_nt_dl_kernel(GemmNt
 #pragma unroll
         for (int c = 0; c < LCH; c++) {
             const int row = (lw + c * LW) * 8 + (lane >> 3);
-            const int kv = (lane & 7) ^ ((row >> 1) & 7);
-            gp[c] = row < BM ? (const half_t *)g.A + a_el + min(i0 + row, g.M - 1) * g.a_rs + 8 * kv
-                             : g.B + b_el + min(j0 + (row - BM), g.N - 1) * g.b_js + 8 * kv;
+            gp[c] = row < BM ? (const half_t *)g.A + a_el + min(i0 + row, g.M - 1) * g.a_rs : g.B + b_el + min(j0 + (row - BM), g.N - 1) * g.b_js;
         }
-        auto issue_tile = [&](int stage, int64_t k0) {
+        static_assert(LW % 2 == 0, "one K-vector per lane for all chunks");
+        const int kv = 8 * ((lane & 7) ^ ((lw * 4 + (lane >> 4)) & 7)); // (lane % 8) ^ (row / 2 % 8)
+        auto issue_tile = [&](int stage, int tile) {
+            const int k = min(min(tile, nk - 1) * NT_BK + kv, kn - 8); // past the last tile that one again, past the end of K its last vector: never used
             half_t *st = ring + stage * STAGE_HALFS;
             if (RT_NT_ABLATION & 1) return; // timing only: no tile loads
 #pragma unroll
             for (int c = 0; c < LCH; c++)
-                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(gp[c] + k0),
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(gp[c] + k),
                                                  (__attribute__((address_space(3))) void *)(st + (lw + c * LW) * 8 * NT_LDK),
                                                  16, 0, 0);
         };
@@ -466,12 +487,12 @@ __global__ __launch_bounds__(NT_THREADS + 64 * LW) void gemm_nt_dl_kernel(GemmNt
             asm volatile("" ::: "memory");
         };
 #pragma unroll
-        for (int st = 0; st < STAGES - 1; st++) issue_tile(st, min<int64_t>(st, nk - 1) * NT_BK);
+        for (int st = 0; st < STAGES - 1; st++) issue_tile(st, st);
         publish(); // tile 0
         int wr = STAGES - 1;
-        for (int64_t kt = 0; kt < nk; kt++) {
+        for (int kt = 0; kt < nk; kt++) {
             // stage wr was read for the last time before the barrier that ended iteration kt - 1
-            issue_tile(wr, min(kt + STAGES - 1, nk - 1) * NT_BK);
+            issue_tile(wr, kt + STAGES - 1);
             publish(); // tile kt + 1
             wr = wr + 1 == STAGES ? 0 : wr + 1;
         }
@@ -521,7 +542,7 @@ __global__ __launch_bounds__(NT_THREADS + 64 * LW) void gemm_nt_dl_kernel(GemmNt
     // a fragment read behind every second MFMA, or behind every one where the tile has too few of them
     constexpr int RS = TM * TN / 2 >= TM + TN ? 2 : 1;
     static_assert(TM * TN / RS >= TM + TN, "not enough MFMAs to spread the reads over");
-    for (int64_t kt = 0; kt < nk; kt++) {
+    for (int kt = 0; kt < nk; kt++) {
 #pragma unroll
         for (int m = 0; m < TM * TN; m++) {
             if (!(RT_NT_ABLATION & 2)) acc[m / TN][m % TN] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f0.fb[m % TN], f0.fa[m / TN], acc[m / TN][m % TN], 0, 0, 0);
@@ -531,6 +552,7 @@ __global__ __launch_bounds__(NT_THREADS + 64 * LW) void gemm_nt_dl_kernel(GemmNt
             }
         }
         meet(); // tile kt + 1 visible
+        if (kt + 1 == nk && kn % NT_BK) break; // K ends with the first half of this tile
 #pragma unroll
         for (int m = 0; m < TM * TN; m++) {
             if (!(RT_NT_ABLATION & 2)) acc[m / TN][m % TN] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f1.fb[m % TN], f1.fa[m / TN], acc[m / TN][m % TN], 0, 0, 0);
@@ -583,7 +605,7 @@ __global__ __launch_bounds__(64 * WI * WJ) void gemm_nt_wide_kernel(GemmNtArgs g
 
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int t = threadIdx.x, lane = t & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6); if (wave < 4) __builtin_amdgcn_s_setprio(3);
     int64_t ti, tj;
     nt_tile_of(g, blockIdx.x, ti, tj); // XCD-aware tile order (see the file comment)
     const int64_t i0 = ti * BM, j0 = tj * BN;
@@ -716,7 +738,7 @@ __global__ __launch_bounds__(NT_THREADS + 64 * LW) void gemm_nt_q8w_kernel(GemmN
     const int64_t s = blockIdx.y;
     const int64_t kbase = (int64_t)blockIdx.z * g.k_len; // this workgroup's share of K (all of it without a split)
     const int64_t a_el = (g.a_stack == 1 ? 0 : s) * g.a_bs + kbase, b_el = (g.b_stack == 1 ? 0 : s) * g.b_bs + kbase;
-    const int64_t nk = g.k_len / NT_BK; // a multiple of 4
+    const int64_t nk = min(g.k_len, g.K - kbase) / NT_BK; // a multiple of 4
 
     if (wave >= 4) {
         const int lw = wave - 4;
@@ -902,6 +924,238 @@ __global__ __launch_bounds__(NT_THREADS + 64 * LW) void gemm_nt_q8w_kernel(GemmN
     nt_epilogue<TM, TN, WM, WN>(g, acc, smem, s, i0, j0, wi, wj, wave, lane);
 }
 
+// ---------------------------------------------------------------------------
+// Q8_0H x f16 for a K that is not a multiple of 256 (any whole number of blocks): the same division of work, with
+//  - the scales of four tiles of K, whose 16 bytes then start at any multiple of two, loaded by the loading wavefronts (a dword-aligned
+//    16-byte load, the dword behind it and a shift) and handed over through LDS;
+//  - a K that ends in the middle of a tile of 64: loads repeat valid addresses past its end, and the multiplying wavefronts leave
+//    the tile's second block out;
+//  - 32 x 32 x 16 MFMAs, two chained from zero per block and tile, sixteen sums per lane folded while the next tile's run.
+// The register-staged kernel that took these shapes had one tile size and one load in flight: 1373 rows x 1152 x 288 56.9 -> 19.5 us with the
+// product behind it, 118 x 3488 x 2592 81.6 -> 20.0, 9 x 5000 x 1504 49.0 -> 10.7, 1633 x 10304 x 1568 with GELU 217 -> 123.
+// For K % 256 == 0 the kernel above stays: one 16-byte load per row and four tiles goes straight to the wavefronts that use it
+// ([512 x 2560] . [10240 x 2560]^T 46.2 us there, 47.0 with this kernel's form; 300 x 1024 x 1024 9.3 and 10.4).
+// What bounds it is what bounds the kernel above: the fold beside the MFMAs, the fill and the LDS traffic add up.
+//
+// Ring of four stages.  Loading wavefront, iteration j: request tile j + 3 (codes and scales into registers, activation rows by
+// LDS-DMA into stage (j + 3) % 4, last read before the barrier that ended iteration j - 1); wait for tile j + 1, requested two
+// iterations ago; widen and store its codes into stage (j + 1) % 4; barrier.
+// ---------------------------------------------------------------------------
+template <int BM, int BN, int WI>
+__global__ __launch_bounds__(2 * NT_THREADS) void gemm_nt_q8r_kernel(GemmNtArgs g) {
+    constexpr int LW = 4, STAGES = 4, AHEAD = 2;
+    constexpr int WJ = 4 / WI, WM = BM / WI, WN = BN / WJ, TM = WM / 32, TN = WN / 32, TILES = TM * TN;
+    constexpr int ROW = NT_LDK * 2;                            // bytes of a staged row
+    constexpr int STAGE = (BM + BN) * ROW;                     // codes, activations
+    constexpr int SCALES = STAGES * STAGE;                     // behind the ring, twice: 16 bytes per row, the eight blocks' scales of four tiles
+    static_assert(TM * 32 * WI == BM && TN * 32 * WJ == BN && BN % (8 * LW) == 0 && BM <= 64 * LW, "tile must split into 32 x 32 MFMA tiles and whole chunks");
+
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[]; // [STAGES][STAGE], [2][64 * LW][16]
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6); if (wave < 4) __builtin_amdgcn_s_setprio(3);
+
+    int64_t ti, tj;
+    nt_tile_of(g, blockIdx.x, ti, tj); // XCD-aware tile order (see the file comment)
+    const int64_t i0 = ti * BM, j0 = tj * BN;
+    const int64_t s = blockIdx.y;
+    const int64_t kbase = (int64_t)blockIdx.z * g.k_len; // this workgroup's share of K (all of it without a split)
+    const int64_t a_el = (g.a_stack == 1 ? 0 : s) * g.a_bs + kbase, b_el = (g.b_stack == 1 ? 0 : s) * g.b_bs + kbase;
+    const int kn = (int)min(g.k_len, g.K - kbase);        // > 0, a multiple of 32: launcher
+    const int nk = (kn + NT_BK - 1) / NT_BK;
+
+    if (wave >= 4) {
+        const int lw = wave - 4;
+        constexpr int ACH = BM / 16;            // 16-row pieces of the code tile (one load instruction each)
+        constexpr int NA = (ACH + LW - 1) / LW; // per loading wavefront
+        constexpr int LCHB = BN / 8 / LW;       // 8-row chunks of the activation tile per loading wavefront
+        constexpr int NL = LCHB + NA;           // load instructions of a request, without the scales' two
+        static_assert(AHEAD * NL + 2 < 64, "the wait counter has six bits");
+        const uint8_t *ga[NA];
+        int adst[NA]; // this lane's row within the code tile
+        bool alive[NA];
+        const int piece = lane & 3;
+#pragma unroll
+        for (int c = 0; c < NA; c++) {
+            const int ch = lw + c * LW;
+            alive[c] = ch < ACH; // wave-uniform
+            const int row = min(ch, ACH - 1) * 16 + (lane >> 2);
+            ga[c] = (const uint8_t *)g.A + a_el + min(i0 + row, g.M - 1) * g.a_rs;
+            adst[c] = row;
+        }
+        const half_t *gb[LCHB];
+        const int kv = (lane & 7) ^ ((lw * 4 + (lane >> 4)) & 7); // of row (lw + c LW) 8 + lane / 8: the same for every c
+#pragma unroll
+        for (int c = 0; c < LCHB; c++) gb[c] = g.B + b_el + min(j0 + (lw + c * LW) * 8 + (lane >> 3), g.N - 1) * g.b_js;
+        const int srow = lw * 64 + lane; // this lane's row of the scales
+        // The scales of four tiles are 16 bytes that start at any multiple of two: a dword-aligned 16-byte load, the dword behind it,
+        // and a shift by `off` values.  A row near the end of the stream (padded to 256 bytes) loads the last 16 bytes.
+        const int64_t s0 = (a_el + min(i0 + min(srow, BM - 1), g.M - 1) * g.a_rs) >> 5;
+        const int64_t s_last = g.scale_dwords - 4;
+        uint4_t ra[STAGES][NA];
+        uint4_t rs;
+        uint32_t rs4;
+        int off = 0;
+        auto request = [&](int slot, int tile, bool scales) __attribute__((always_inline)) {
+            const int k0 = min(tile, nk - 1) * NT_BK; // past the last tile: re-read it, never used ...
+            const int to = tile < nk + 3 ? slot : nk & 3; // ... and not stored where the last one is read
+            uint8_t *st = smem + to * STAGE + BM * ROW;
+            const int kb = min(k0 + 8 * kv, kn - 8), ka = min(k0 + 16 * piece, kn - 16);
+#pragma unroll
+            for (int c = 0; c < LCHB; c++)
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(gb[c] + kb),
+                                                 (__attribute__((address_space(3))) void *)(st + (lw + c * LW) * 8 * ROW), 16, 0, 0);
+            __builtin_amdgcn_sched_barrier(0); // the wait in widen_store counts whole requests
+#pragma unroll
+            for (int c = 0; c < NA; c++) ra[slot][c] = *(const uint4_t *)(ga[c] + ka);
+            if (scales) { // tile is a multiple of four
+                const int64_t at = s0 + (k0 >> 5), dw = min(at >> 1, s_last);
+                off = (int)(at - 2 * dw); // 0 .. 7
+                rs = *(const uint4_d *)((const uint32_t *)g.scales + dw);
+                rs4 = ((const uint32_t *)g.scales)[min(dw + 4, s_last + 3)];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto widen_store = [&](int slot, auto NEWER, bool scales, int group) __attribute__((always_inline)) { // NEWER: of the two requests behind this tile's, those with scales
+            asm volatile("" ::: "memory");
+            constexpr int left = AHEAD * NL + 2 * decltype(NEWER)::value;
+            __builtin_amdgcn_s_waitcnt(0x0F70 | (left & 0xF) | (((left >> 4) & 0x3) << 14));
+            uint8_t *st = smem + slot * STAGE;
+#pragma unroll
+            for (int c = 0; c < NA; c++) {
+                if (alive[c]) {
+                    half2_t h[8];
+#pragma unroll
+                    for (int d = 0; d < 4; d++) nt_cvt_i8x4(ra[slot][c][d], h[2 * d], h[2 * d + 1]);
+                    const uint4_t lo = {__builtin_bit_cast(uint32_t, h[0]), __builtin_bit_cast(uint32_t, h[1]),
+                                        __builtin_bit_cast(uint32_t, h[2]), __builtin_bit_cast(uint32_t, h[3])};
+                    const uint4_t hi = {__builtin_bit_cast(uint32_t, h[4]), __builtin_bit_cast(uint32_t, h[5]),
+                                        __builtin_bit_cast(uint32_t, h[6]), __builtin_bit_cast(uint32_t, h[7])};
+                    // the four lanes of a row store four of its eight slots, and two neighbouring rows have the same
+                    // swizzle: odd rows store their odd slots first, so that eight consecutive lanes cover eight
+                    // different 16-byte bank groups
+                    const int flip = adst[c] & 1;
+                    *(uint4_t *)((half_t *)st + nt_slot(adst[c], 2 * piece + flip)) = flip ? hi : lo;
+                    *(uint4_t *)((half_t *)st + nt_slot(adst[c], 2 * piece + 1 - flip)) = flip ? lo : hi;
+                }
+            }
+            if (scales) {
+                uint4_t v = rs;
+                uint32_t w = rs4;
+                if (off & 4) v = uint4_t{v[2], v[3], w, w}, w = 0;
+                if (off & 2) v = uint4_t{v[1], v[2], v[3], w}, w = 0;
+                const uint32_t sh = (uint32_t)(off & 1) << 4;
+                v = uint4_t{__builtin_amdgcn_alignbit(v[1], v[0], sh), __builtin_amdgcn_alignbit(v[2], v[1], sh), __builtin_amdgcn_alignbit(v[3], v[2], sh),
+                            __builtin_amdgcn_alignbit(w, v[3], sh)};
+                *(uint4_t *)(smem + SCALES + (group & 1) * (64 * LW * 16) + 16 * srow) = v;
+            }
+        };
+        auto publish = [&](bool meet) __attribute__((always_inline)) {
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0): the widened tile is in LDS
+            if (meet) __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        };
+        request(0, 0, true);
+        request(1, 1, false);
+        request(2, 2, false);
+        widen_store(0, std::integral_constant<int, 0>{}, true, 0);
+        publish(true); // tile 0
+        auto iteration = [&](auto U, int j) __attribute__((always_inline)) { // U: j % 4
+            constexpr int u = decltype(U)::value;
+            request((u + 3) & 3, j + 3, u == 1); // into the stage that was read for the last time before the barrier of iteration j - 1
+            widen_store((u + 1) & 3, std::integral_constant<int, u == 1 || u == 2>{}, u == 3, (j + 1) >> 2); // tile j + 1
+            publish(j + 1 < nk);
+        };
+        const std::integral_constant<int, 0> u0;
+        const std::integral_constant<int, 1> u1;
+        const std::integral_constant<int, 2> u2;
+        const std::integral_constant<int, 3> u3;
+        // nk - 1 iterations, and up to three more without a barrier that nobody waits for but the end: whole turns of the ring without
+        // a way out or around in between, with which the compiler drains every load
+        for (int j = 0; j + 1 < nk; j += 4) iteration(u0, j), iteration(u1, j + 1), iteration(u2, j + 2), iteration(u3, j + 3);
+        __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0): nothing may land once the epilogue reuses the ring
+        __syncthreads();
+        return;
+    }
+
+    // ---- multiplying wavefronts
+    const int wi = wave / WJ, wj = wave % WJ;
+    const int fr = lane & 31, fh = lane >> 5;
+    // 16 k of a row (half m of block kk) are K-vectors 4 kk + 2 m, + 1: this lane's is 4 kk + 2 m + fh.  Byte addresses of this lane's
+    // first fragments in stage 0 for m = kk = 0; m flips bit 5 of them, kk bit 6.
+    const uint32_t slot = (uint32_t)((fh ^ ((fr >> 1) & 7)) << 4);
+    const uint32_t ra0 = (uint32_t)(wi * WM + fr) * ROW + slot, rb0 = (uint32_t)(BM + wj * WN + fr) * ROW + slot;
+    const uint32_t rs0 = (uint32_t)(SCALES + (wi * WM + fr) * 16);
+    auto frag = [&](uint32_t at) __attribute__((always_inline)) { return __builtin_bit_cast(half8_t, *(const uint4_t *)(smem + at)); };
+    auto next_tile = [&]() __attribute__((always_inline)) {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0): this tile's fragment reads have returned
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    const float16_t zero = {};
+    float16_t acc[TM][TN], P[2];
+#pragma unroll
+    for (int a = 0; a < TM; a++)
+#pragma unroll
+        for (int b = 0; b < TN; b++) acc[a][b] = zero;
+    half8_t fa[TM][2], fb[2][TN][2];
+    half2_t sc[TM], last = {(half_t)0.f, (half_t)0.f}; // scales of this tile's two blocks; of the tile before, its last rows'
+    P[0] = P[1] = zero;
+    next_tile(); // tile 0
+#pragma unroll
+    for (int a = 0; a < TM; a++) {
+        fa[a][0] = frag(ra0 + a * 32 * ROW), fa[a][1] = frag((ra0 ^ 32u) + a * 32 * ROW);
+        sc[a] = *(const half2_t *)(smem + rs0 + a * 512);
+    }
+#pragma unroll
+    for (int b = 0; b < TN; b++) fb[0][b][0] = frag(rb0 + b * 32 * ROW), fb[0][b][1] = frag((rb0 ^ 32u) + b * 32 * ROW);
+
+    // One block of 32: per MFMA tile two MFMAs, then the fold of the tile before.  The next block's fragments are read from `ra`, `rb`
+    // behind their registers' last use (the activations', which all tiles of a column share, into a second set).
+    auto block = [&](auto KK, uint32_t ra, uint32_t rb, uint32_t rs) __attribute__((always_inline)) {
+        constexpr int kk = decltype(KK)::value;
+#pragma unroll
+        for (int idx = 0; idx < TILES; idx++) {
+            const int a = idx / TN, b = idx % TN, p = (kk * TILES + idx) & 1;
+            const int pa = idx ? (idx - 1) / TN : TM - 1, pb = idx ? (idx - 1) % TN : TN - 1;
+            P[p] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb[kk][b][0], fa[a][0], zero, 0, 0, 0);
+            P[p] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb[kk][b][1], fa[a][1], P[p], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            if (b == TN - 1) fa[a][0] = frag(ra + a * 32 * ROW), fa[a][1] = frag((ra ^ 32u) + a * 32 * ROW);
+            if (idx < TN) fb[kk ^ 1][idx][0] = frag(rb + idx * 32 * ROW), fb[kk ^ 1][idx][1] = frag((rb ^ 32u) + idx * 32 * ROW);
+            const float d = (float)(idx == 0 ? (kk ? sc[pa][0] : last[1]) : sc[pa][kk]);
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[pa][pb][r] = fmaf(d, P[p ^ 1][r], acc[pa][pb][r]);
+            if (kk && idx && pb == TN - 1) sc[pa] = *(const half2_t *)(smem + rs + pa * 512);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (kk) last = sc[TM - 1], sc[TM - 1] = *(const half2_t *)(smem + rs + (TM - 1) * 512);
+    };
+    const std::integral_constant<int, 0> first_block;
+    const std::integral_constant<int, 1> second_block;
+    uint32_t cur = 0; // stage of tile kt, in bytes
+    const bool half = kn % NT_BK != 0;
+    for (int kt = 0; kt + 1 < nk; kt++) {
+        block(first_block, (ra0 ^ 64u) + cur, (rb0 ^ 64u) + cur, 0);
+        next_tile(); // tile kt + 1 is whole, stage `cur` is free
+        cur = cur == (STAGES - 1) * STAGE ? 0 : cur + STAGE;
+        block(second_block, ra0 + cur, rb0 + cur, rs0 + ((kt + 1) & 3) * 4 + ((kt + 1) >> 2 & 1) * (64 * LW * 16));
+    }
+    block(first_block, (ra0 ^ 64u) + cur, (rb0 ^ 64u) + cur, 0);
+    if (!half) block(second_block, ra0 + cur, rb0 + cur, rs0); // (what it reads ahead is not used)
+    {
+        // the last tile's sums: of the second block, or of the first where K ends with it
+        const float d = (float)(half ? sc[TM - 1][0] : last[1]);
+        constexpr int p0 = (TILES - 1) & 1, p1 = (2 * TILES - 1) & 1;
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[TM - 1][TN - 1][r] = fmaf(d, half ? P[p0][r] : P[p1][r], acc[TM - 1][TN - 1][r]);
+    }
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __syncthreads();
+    nt_epilogue32<TM, TN, WM, WN>(g, acc, smem, s, i0, j0, wi, wj, wave, lane);
+}
+
 // Second pass of a split-K launch: out = round(act(sum over the splits + bias)).  One thread per four
 // consecutive i (the partial sums' contiguous axis); M need not be a multiple of four.
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(GemmNtArgs g) {
@@ -952,6 +1206,16 @@ static hipError_t launch_nt_q8w(const GemmNtArgs &g, int64_t stacks, hipStream_t
     if (const hipError_t e = ensure_lds_limit<&gemm_nt_q8w_kernel<BM, BN, LW>>(); e != hipSuccess) return e;
     dim3 grid((unsigned)((int64_t)g.tiles_i * g.tiles_j), (unsigned)stacks, (unsigned)g.ksplit);
     hipLaunchKernelGGL((gemm_nt_q8w_kernel<BM, BN, LW>), grid, dim3(NT_THREADS + 64 * LW), lds, st, g);
+    if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    return g.ksplit > 1 ? launch_splitk_reduce(g, stacks, st) : hipSuccess;
+}
+
+template <int BM, int BN, int WI>
+static hipError_t launch_nt_q8r(const GemmNtArgs &g, int64_t stacks, hipStream_t st) {
+    const size_t lds = (size_t)4 * (BM + BN) * NT_LDK * 2 + 2 * 256 * 16;
+    if (const hipError_t e = ensure_lds_limit<&gemm_nt_q8r_kernel<BM, BN, WI>>(); e != hipSuccess) return e;
+    dim3 grid((unsigned)((int64_t)g.tiles_i * g.tiles_j), (unsigned)stacks, (unsigned)g.ksplit);
+    hipLaunchKernelGGL((gemm_nt_q8r_kernel<BM, BN, WI>), grid, dim3(2 * NT_THREADS), lds, st, g);
     if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     return g.ksplit > 1 ? launch_splitk_reduce(g, stacks, st) : hipSuccess;
 }
@@ -1087,20 +1351,17 @@ static hipError_t launch_nt_wide(const GemmNtArgs &g, int64_t stacks, hipStream_
     return hipGetLastError();
 }
 
-// Tunables: non-zero keeps f16 problems on the register-staged kernel; LDS ring depth
-// (3 or 4, 0 = 3) of the direct-to-LDS kernel (for comparisons).
+// Tunable: non-zero keeps f16 problems on the register-staged kernel (for comparisons).
 RT_TUNABLE(g_gemm_nt_no_direct, 0);
-RT_TUNABLE(g_gemm_nt_stages, 0);
 RT_TUNABLE(g_gemm_nt_wide, 0); // 1 / 2: never / always the 320 x 256 tiles (for comparisons)
-RT_TUNABLE(g_gemm_nt_narrow, 0); // 1: never the 64- and 96-row tiles for few activation rows (for comparisons)
 RT_TUNABLE(g_gemm_nt_shortk_parts, 0); // workgroups per strip of the short-K kernel (0 = automatic)
 
-template <int BM, int BN, bool Q8, bool KFULL>
+template <int BM, int BN, bool KFULL>
 static hipError_t launch_nt(const GemmNtArgs &g, int64_t stacks, hipStream_t st) {
-    const size_t lds = (size_t)2 * (BM + BN) * NT_LDK * 2 + (Q8 ? (size_t)4 * BM * 4 : 0);
-    if (const hipError_t e = ensure_lds_limit<&gemm_nt_kernel<BM, BN, Q8, KFULL>>(); e != hipSuccess) return e;
+    const size_t lds = (size_t)2 * (BM + BN) * NT_LDK * 2;
+    if (const hipError_t e = ensure_lds_limit<&gemm_nt_kernel<BM, BN, KFULL>>(); e != hipSuccess) return e;
     dim3 grid((unsigned)((int64_t)g.tiles_i * g.tiles_j), (unsigned)stacks);
-    hipLaunchKernelGGL((gemm_nt_kernel<BM, BN, Q8, KFULL>), grid, dim3(NT_THREADS), lds, st, g);
+    hipLaunchKernelGGL((gemm_nt_kernel<BM, BN, KFULL>), grid, dim3(NT_THREADS), lds, st, g);
     return hipGetLastError();
 }
 
@@ -1139,20 +1400,54 @@ static bool nt_set_tiles(GemmNtArgs &g, int bm, int bn, int a_bytes) {
 // Tunable: 0 = automatic, 1 = never take this kernel (for comparisons).
 RT_TUNABLE(g_gemm_nt_disable, 0);
 
-// f16 or Q8_0H A with K-contiguous rows, f16 B with K-contiguous rows.
-// hipErrorNotSupported: the problem does not fit; the generic tiled GEMM runs instead.
-// Workgroups that share one output tile's K.  A product with few output tiles and a long K (the
-// Phi-2 down-projection: 64 tiles of 160 x 128, K = 10240) leaves most compute units idle; with a
-// workspace its K is cut into equal shares of a whole number of 256-wide units, at least 1024 each.
-// Applies to the shapes the direct-to-LDS kernels take (after the operand exchange for row-major outputs).
-static int gemm_nt_ksplit(const Problem &p, const DeviceInfo &dev) {
-    if (p.act_dt != RT_F16 || (p.a_dt != RT_F16 && p.a_dt != RT_Q8_0H) || p.K % 256 != 0 || p.K <= 256) return 1;
-    const int64_t tiles = ((p.M + 159) / 160) * ((p.N + 127) / 128) * p.stacks;
-    if (tiles <= 0 || tiles * 2 > dev.num_cus) return 1;
-    const int64_t units = p.K / 256;
-    int best = 1;
-    for (int ks = 2; ks <= 8 && tiles * ks <= dev.num_cus; ks++)
-        if (units % ks == 0 && units / ks >= 4) best = ks;
+// The tiles of the kernels that load global -> LDS and how K is shared among workgroups: the cheapest by an estimate in microseconds,
+//   3 + rounds * (fixed - 3 + step * (1 + crowd * busy) * tiles of 64 k in a share) + the second kernel's time,
+// busy the share of the compute units that has a workgroup.  The constants are a fit to every tile and split of 14 f16 and 18
+// Q8_0H products on the device (worst case 7 % above the best choice, most within 1 %).  The largest tile alone, cut along K where
+// it left half of the compute units idle, was the rule before: [512 x 2560] . [2560 x 2560]^T Q8_0H 30.2 -> 17.7 us (64 x 128 tiles,
+// K whole), [512 x 2560] . [7680 x 2560]^T 43 -> 34.7 (128 x 128), 128 rows x 2560 x 2560 25.1 -> 12.7 (64 x 64, K in three),
+// 1000 x 4096 x 4096 65.6 -> 52.8; f16 30 -> 15.9 of the first kind, [700 x 1280] . [5120 x 1280]^T 17.3 -> 14.9.
+struct NtTile {
+    int bm, bn;
+    float fixed, step;
+};
+constexpr int kNtTiles = 5;
+constexpr NtTile kTilesF16[kNtTiles] = {{160, 128, 8.6f, 0.333f}, {128, 128, 8.1f, 0.27f}, {96, 128, 7.2f, 0.285f}, {64, 128, 6.6f, 0.182f}, {64, 64, 6.0f, 0.13f}};
+constexpr NtTile kTilesQ8w[kNtTiles] = {{160, 128, 8.6f, 0.70f}, {128, 128, 8.0f, 0.51f}, {96, 128, 7.5f, 0.42f}, {64, 128, 6.7f, 0.26f}, {64, 64, 6.2f, 0.17f}};
+constexpr NtTile kTilesQ8r[kNtTiles] = {{160, 128, 8.2f, 0.70f}, {128, 128, 8.8f, 0.48f}, {96, 128, 7.7f, 0.42f}, {64, 128, 7.2f, 0.295f}, {64, 64, 6.7f, 0.21f}};
+struct NtChoice {
+    int bm = 160, bn = 128;
+    int ks = 1;        // workgroups that share one tile's K
+    int64_t k_len = 0; // of a share; the last may be shorter
+};
+// gemm_nt_q8w_kernel's shapes among those with Q8_0H weights
+static bool nt_q8_whole(const Problem &p) { return p.K % 256 == 0 && p.a_bs % 512 == 0; }
+static NtChoice nt_choose(const Problem &p, const DeviceInfo &dev, bool may_split) {
+    const bool q8 = p.a_dt == RT_Q8_0H;
+    const NtTile *tiles = !q8 ? kTilesF16 : nt_q8_whole(p) ? kTilesQ8w : kTilesQ8r;
+    const float crowd = q8 ? 0.23f : 0.37f;
+    const int64_t nk = (p.K + NT_BK - 1) / NT_BK;
+    NtChoice best;
+    best.k_len = p.K;
+    float least = 3.4e38f;
+    for (int i = 0; i < kNtTiles; i++) {
+        const NtTile &t = tiles[i];
+        const int64_t n = ((p.M + t.bm - 1) / t.bm) * ((p.N + t.bn - 1) / t.bn) * p.stacks;
+        if (t.bm < 128 && n > dev.num_cus) continue; // narrow tiles only where they all run at once
+        for (int ks = 1; ks <= (may_split ? 16 : 1); ks++) {
+            if (ks > 1 && n * ks > dev.num_cus) break; // the partial sums stay within 256 of the largest tiles on 256 compute units
+            // where K is whole units of 256 (which gemm_nt_q8w_kernel's shares are too) equal shares, of whole 512s or of at least 1024; else
+            // shares of at least 512, the last one shorter
+            const int64_t share = (nk + ks - 1) / ks;
+            const bool equal = p.K % (512 * ks) == 0 || (p.K % (256 * ks) == 0 && p.K / ks >= 1024);
+            if (ks > 1 && (p.K % 256 == 0 ? !equal : share < 8 || (ks - 1) * share >= nk)) continue;
+            const int64_t rounds = (n * ks + dev.num_cus - 1) / dev.num_cus;
+            const float busy = std::min(1.f, (float)(n * ks) / dev.num_cus);
+            const float second = ks == 1 ? 0.f : 1.9f + 0.1f * ks + (float)(p.stacks * ks * p.M * p.N) * (4.f / 4.5e6f);
+            const float us = 3.f + rounds * (t.fixed - 3.f + t.step * (1.f + crowd * busy) * share) + second;
+            if (us < least) least = us, best.bm = t.bm, best.bn = t.bn, best.ks = ks, best.k_len = ks == 1 ? p.K : share * NT_BK;
+        }
+    }
     return best;
 }
 
@@ -1176,7 +1471,8 @@ uint64_t gemm_nt_workspace_bytes(const Problem &p0, const DeviceInfo &dev) {
     Problem p = p0;
     nt_orient(p);
     if (p.a_ks != 1 || p.b_ks != 1 || p.M < 160 || p.N < 5) return 0;
-    const int ks = gemm_nt_ksplit(p, dev);
+    if ((p.a_dt != RT_F16 && p.a_dt != RT_Q8_0H) || p.K % 32 != 0 || p.K <= 256) return 0;
+    const int ks = nt_choose(p, dev, true).ks;
     return ks > 1 ? (uint64_t)p.stacks * ks * p.M * p.N * sizeof(float) : 0;
 }
 
@@ -1200,7 +1496,11 @@ hipError_t launch_gemm_nt(const Problem &p0, const void *A, const void *B, const
 
     GemmNtArgs g{};
     g.A = A, g.B = (const half_t *)B, g.bias = (const half_t *)bias, g.out = (half_t *)out;
-    if (q8) g.scales = (const half_t *)((const uint8_t *)A + rt_q8_0_scale_offset((uint64_t)p.a_stack * p.M * p.K));
+    if (q8) {
+        const uint64_t n = (uint64_t)p.a_stack * p.M * p.K;
+        g.scales = (const half_t *)((const uint8_t *)A + rt_q8_0_scale_offset(n));
+        g.scale_dwords = (int64_t)((n / 32 * 2 + 255) / 256 * 64);
+    }
     g.M = p.M, g.N = p.N, g.K = p.K;
     g.a_stack = p.a_stack, g.b_stack = p.b_stack;
     g.a_bs = p.a_bs, g.a_rs = p.a_rs;
@@ -1229,66 +1529,52 @@ hipError_t launch_gemm_nt(const Problem &p0, const void *A, const void *B, const
         // workgroups share a compute unit and one's epilogue overlaps another's loads.
         constexpr int SBM = 128, SBN = 64; // 128 outputs along the contiguous axis: whole cache lines per wavefront row
         if (!nt_set_tiles(g, SBM, SBN, 2)) return hipErrorNotSupported;
-        return kfull ? launch_nt<SBM, SBN, false, true>(g, p.stacks, stream)
-                     : launch_nt<SBM, SBN, false, false>(g, p.stacks, stream);
+        return kfull ? launch_nt<SBM, SBN, true>(g, p.stacks, stream)
+                     : launch_nt<SBM, SBN, false>(g, p.stacks, stream);
     }
-    constexpr int BM = 160, BN = 128;
-    const int a_bytes = q8 ? 1 : 2;
-    if (!nt_set_tiles(g, BM, BN, a_bytes)) return hipErrorNotSupported;
-    const int64_t ti = g.tiles_i, tj = g.tiles_j;
-    // few activation rows: 160-row tiles leave most compute units idle and a workgroup takes as long for one
-    // column of tiles as for four; 64-row tiles, while all of them still run at once, put 2.5 times the workgroups to work
-    // (10240 x 2560 f16 weights: 65..128 rows 24.6-25.4 -> 17.2-18.1 us); 96-row tiles where those no longer fit.
-    const int64_t ti64 = (p.M + 63) / 64, ti96 = (p.M + 95) / 96;
-    const bool few = g_gemm_nt_narrow != 1 && ti * tj * p.stacks * 2 <= dev.num_cus;
-    const int bm = few && ti64 * tj * p.stacks <= dev.num_cus ? 64 : few && ti96 * tj * p.stacks <= dev.num_cus ? 96 : BM;
-    const bool dl_f16 = !q8 && kfull && !g_gemm_nt_no_direct;
-    const bool dl_q8 = q8 && p.K % 256 == 0 && !g_gemm_nt_no_direct && ((uintptr_t)g.scales & 15u) == 0 && (p.a_bs % 512) == 0;
-    if (dl_f16 || dl_q8) {
-        const int ks = gemm_nt_ksplit(p, dev);
-        if (ks > 1 && p.workspace && !((uintptr_t)p.workspace & 15u) &&
-            p.workspace_bytes >= (uint64_t)p.stacks * ks * p.M * p.N * sizeof(float))
-            g.ksplit = ks, g.k_len = p.K / ks, g.partial = (float *)p.workspace;
+    if (!q8 && (p.K % 32 != 0 || g_gemm_nt_no_direct)) {
+        if (!nt_set_tiles(g, 160, 128, 2)) return hipErrorNotSupported;
+        return kfull ? launch_nt<160, 128, true>(g, p.stacks, stream) : launch_nt<160, 128, false>(g, p.stacks, stream);
     }
-    if ((dl_f16 || dl_q8) && bm != BM && g.ksplit == 1) {
-        // (up to 64 activation rows: one column of tiles either way)
-        if (!nt_set_tiles(g, bm, BN, a_bytes)) return hipErrorNotSupported;
-        // the narrow tiles take as deep a ring as the LDS holds: a stage has only 8 or 12 KB of weights, and what a compute
-        // unit has in flight is what it can pull (10240 x 2560 f16 weights, 40 / 64 activation rows, three stages -> six:
-        // 22.7 / 23.6 -> 20.0 / 22.1 us with the weights in HBM, 16.3 / 16.8 -> 14.8 / 15.7 from the Infinity Cache)
-        if (dl_f16 && bm == 64 && p.N <= 64) {
-            // up to 64 activation rows: half the activation tile, a stage of 16 KB and nine of them (40 / 64 rows:
-            // 20.0 / 22.1 -> 18.3 / 20.5 us with the weights in HBM, 14.8 / 15.7 -> 12.6 / 13.6 from the Infinity Cache)
-            return launch_nt_dl<64, 64, 9, 2>(g, p.stacks, stream);
-        }
-        if (dl_f16) return bm == 64 ? launch_nt_dl<64, BN, 6, 2>(g, p.stacks, stream) : launch_nt_dl<96, BN, 5, 2>(g, p.stacks, stream);
-        if (bm == 64 && p.N <= 64) {
-            // up to 64 activation rows: half the activation tile is half the MFMAs and folds of a workgroup
-            return launch_nt_q8w<64, 64, 4>(g, p.stacks, stream);
-        }
-        return bm == 64 ? launch_nt_q8w<64, BN, 4>(g, p.stacks, stream) : launch_nt_q8w<96, BN, 4>(g, p.stacks, stream);
-    }
-    if (dl_f16 && g.ksplit == 1 && g_gemm_nt_wide != 1 && p.a_rs >= 0 && p.b_js >= 0 && 2 * 320 * std::max(p.a_rs, p.b_js) < (int64_t(1) << 32)) {
-        const int64_t wide = ((p.M + 319) / 320) * ((p.N + 255) / 256) * p.stacks;
-        const int64_t rounds = (ti * tj * p.stacks + dev.num_cus - 1) / dev.num_cus, rounds_wide = (wide + dev.num_cus - 1) / dev.num_cus;
+    NtChoice c = nt_choose(p, dev, p.K > 256 && p.workspace && !((uintptr_t)p.workspace & 15u));
+    if (c.ks > 1 && p.workspace_bytes < (uint64_t)p.stacks * c.ks * p.M * p.N * sizeof(float)) c = nt_choose(p, dev, false);
+    if (c.ks > 1) g.ksplit = c.ks, g.k_len = c.k_len, g.partial = (float *)p.workspace;
+    if (!q8 && kfull && c.ks == 1 && g_gemm_nt_wide != 1 && p.a_rs >= 0 && p.b_js >= 0 && 2 * 320 * std::max(p.a_rs, p.b_js) < (int64_t(1) << 32)) {
+        const int64_t tiles = ((p.M + 159) / 160) * ((p.N + 127) / 128), wide = ((p.M + 319) / 320) * ((p.N + 255) / 256) * p.stacks;
+        const int64_t rounds = (tiles * p.stacks + dev.num_cus - 1) / dev.num_cus, rounds_wide = (wide + dev.num_cus - 1) / dev.num_cus;
         // A round of 320 x 256 tiles takes 12 + 0.030 K us on all compute units, one of 160 x 128 tiles 6.4 + 0.0080 K: four small
         // rounds are always longer (10240 x 2560 weights, 2048 activation rows: 108.5 us against 89.7), two never.  Three are
         // longer for a short K (1500 rows, K = 1024: 43.9 against 39.3), the same at K = 2560 and shorter beyond (1000 rows
         // x 11008 x 4096: 107.0 against 118.9; two wide rounds against six small ones alike) -- unless the small tiles do not deal out
         // evenly to the XCDs, whose L2s then share little (1300 rows x 8192 x 4096, 572 tiles: 133.5 against 114.2).
-        const bool even = ti * tj % 8 == 0;
+        const bool even = tiles % 8 == 0;
         const bool longer = 5 * rounds_wide < 2 * rounds && (3 * rounds_wide < rounds || !even || p.K <= 2048);
         if ((g_gemm_nt_wide == 2 || longer) && nt_set_tiles(g, 320, 256, 2)) return launch_nt_wide(g, p.stacks, stream);
     }
-    if (dl_f16) {
-        // two loading wavefronts: one and four measured the same within run-to-run spread
-        return g_gemm_nt_stages == 4 ? launch_nt_dl<BM, BN, 4, 2>(g, p.stacks, stream)
-                                     : launch_nt_dl<BM, BN, 3, 2>(g, p.stacks, stream);
+    if (!nt_set_tiles(g, c.bm, c.bn, q8 ? 1 : 2)) return hipErrorNotSupported;
+    if (!q8) {
+        // two loading wavefronts: one and four measured the same within run-to-run spread.  The narrow tiles take as deep a ring as the
+        // LDS holds: what a compute unit has in flight is what it can pull (10240 x 2560 f16 weights, 40 / 64 activation rows,
+        // three stages of 64 x 128 -> six: 22.7 / 23.6 -> 20.0 / 22.1 us with the weights in HBM, 16.3 / 16.8 -> 14.8 / 15.7 from
+        // the Infinity Cache; nine of 64 x 64: 18.3 / 20.5 and 12.6 / 13.6)
+        if (c.bn == 64) return launch_nt_dl<64, 64, 9, 2>(g, p.stacks, stream);
+        if (c.bm == 64) return launch_nt_dl<64, 128, 6, 2>(g, p.stacks, stream);
+        if (c.bm == 96) return launch_nt_dl<96, 128, 5, 2>(g, p.stacks, stream);
+        if (c.bm == 128) return launch_nt_dl<128, 128, 4, 2>(g, p.stacks, stream);
+        return launch_nt_dl<160, 128, 3, 2>(g, p.stacks, stream);
     }
-    if (dl_q8)
-        return launch_nt_q8w<BM, BN, 4>(g, p.stacks, stream);
-    if (q8) return kfull ? launch_nt<BM, BN, true, true>(g, p.stacks, stream) : launch_nt<BM, BN, true, false>(g, p.stacks, stream);
-    return kfull ? launch_nt<BM, BN, false, true>(g, p.stacks, stream) : launch_nt<BM, BN, false, false>(g, p.stacks, stream);
+    if (nt_q8_whole(p)) {
+        if (c.bn == 64) return launch_nt_q8w<64, 64, 4>(g, p.stacks, stream);
+        if (c.bm == 64) return launch_nt_q8w<64, 128, 4>(g, p.stacks, stream);
+        if (c.bm == 96) return launch_nt_q8w<96, 128, 4>(g, p.stacks, stream);
+        if (c.bm == 128) return launch_nt_q8w<128, 128, 4>(g, p.stacks, stream);
+        return launch_nt_q8w<160, 128, 4>(g, p.stacks, stream);
+    }
+    if (c.bn == 64) return launch_nt_q8r<64, 64, 2>(g, p.stacks, stream);
+    if (c.bm == 64) return launch_nt_q8r<64, 128, 1>(g, p.stacks, stream);
+    if (c.bm == 96) return launch_nt_q8r<96, 128, 1>(g, p.stacks, stream);
+    if (c.bm == 128) return launch_nt_q8r<128, 128, 2>(g, p.stacks, stream);
+    return launch_nt_q8r<160, 128, 1>(g, p.stacks, stream);
 }
 
 } // namespace rt

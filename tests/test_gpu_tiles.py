@@ -1,0 +1,93 @@
+"""The tiled f16 and Q8_0H products (launch_gemm_nt): every tile and split its estimate chooses, at the edges of the tiles and for a K that
+ends inside a tile of 64 or is no multiple of 256, against float64.
+
+The tolerance: products of f16 numbers (and of codes) are exact in the MFMA, whose f32 accumulator rounds at most twice per 32 k, and a
+Q8_0H block's sum is scaled and added with one more rounding, each by at most 2^-24 of the magnitudes summed; a shared K adds
+its shares in at most 16 more; then the bias and the result's rounding to f16 (2^-11)."""
+import numpy as np
+import pytest
+import torch
+
+from ratchet_amd import DType, Tensor
+
+pytestmark = pytest.mark.gpu
+
+
+def tensor(device, t):
+    return Tensor(tuple(t.shape), DType.F16, device, t.contiguous().view(torch.uint8).reshape(-1))
+
+
+def weights(device, gen, dt, stack, m, k):
+    if dt == DType.F16:
+        w = torch.randn((*stack, m, k), generator=gen, device="cuda:0").half()
+        return tensor(device, w), w.double()
+    n = m * k * (stack[0] if stack else 1)
+    codes = torch.randint(-127, 128, (n,), generator=gen, device="cuda:0", dtype=torch.int8)
+    scales = (torch.rand((n // 32,), generator=gen, device="cuda:0") * 0.02 + 1e-3).half()
+    pad = lambda t: torch.nn.functional.pad(t.view(torch.uint8), (0, -t.view(torch.uint8).numel() % 256))
+    w = Tensor((*stack, m, k), dt, device, torch.cat([pad(codes), pad(scales)]))
+    return w, (codes.view(-1, 32).double() * scales.double()[:, None]).view(*stack, m, k)
+
+
+def check(device, dt, m, n, k, trans_out=True, stack=()):
+    gen = torch.Generator("cuda:0").manual_seed(m + n + k)
+    w, wd = weights(device, gen, dt, stack, m, k)
+    x, bias = (torch.randn(s, generator=gen, device="cuda:0").half() for s in ((*stack, n, k), (m,)))
+    out = w.gemm(tensor(device, x), tensor(device, bias) if trans_out else None, False, True, trans_out).resolve()
+    got = out.storage.view(torch.float16)[: out.numel()].view(out.shape).double()
+    if not trans_out:
+        got = got.transpose(-1, -2)
+    b = bias.double() if trans_out else 0.0
+    for lo in range(0, n, 512):
+        xs = x[..., lo : lo + 512, :].double()
+        wt = wd.transpose(-1, -2).contiguous()
+        want, mag = xs @ wt + b, xs.abs() @ wt.abs() + (b.abs() if trans_out else 0.0)
+        err = (got[..., lo : lo + 512, :] - want).abs()
+        assert (err <= 2.0**-11 * want.abs() + 2.0**-24 * (3 * k / 32 + 20) * mag + 2.0**-25).all(), float((err / mag).max())
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (333, 64, 288), (161, 7, 32), (200, 5, 96), (300, 65, 64), (4100, 130, 1056),                     # 64 x 64 tiles; one, two and more tiles of K
+    (2051, 64, 4000), (1024, 33, 4128), (700, 300, 4064), (200, 9, 2080), (1000, 64, 8224),           # ... K shared, the last share shorter
+    (5000, 300, 544), (2592, 512, 2592),                                                              # 64 x 128
+    (9000, 200, 416), (20000, 100, 352),                                                              # 96 x 128
+    (4090, 1001, 1440), (12800, 256, 320), (10241, 500, 288), (2560, 520, 10272),                     # 128 x 128, more than one round, K shared
+    (10240, 512, 352), (20479, 511, 416), (10240, 512, 2592),                                         # 160 x 128
+])
+@pytest.mark.parametrize("dt", [DType.Q8_0H, DType.F16])
+def test_k_of_whole_blocks(device, dt, m, n, k):
+    check(device, dt, m, n, k)
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (300, 300, 1024), (1024, 64, 4096), (200, 9, 8192), (2560, 512, 2304), (9000, 200, 512), (7681, 511, 512), (2560, 520, 10240), (10240, 512, 768),
+])
+@pytest.mark.parametrize("dt", [DType.Q8_0H, DType.F16])
+def test_k_of_whole_units(device, dt, m, n, k):
+    check(device, dt, m, n, k)
+
+
+@pytest.mark.parametrize("m,n,k", [(333, 70, 288), (1001, 300, 800), (2600, 130, 4000)])
+@pytest.mark.parametrize("dt", [DType.Q8_0H, DType.F16])
+def test_other_axis_contiguous(device, dt, m, n, k):
+    check(device, dt, m, n, k, trans_out=False)
+
+
+@pytest.mark.parametrize("stacks,m,n,k", [(3, 200, 33, 288), (2, 700, 130, 2080), (5, 161, 9, 1056), (2, 300, 70, 512)])
+@pytest.mark.parametrize("dt", [DType.Q8_0H, DType.F16])
+def test_stacks(device, dt, stacks, m, n, k):
+    check(device, dt, m, n, k, trans_out=False, stack=(stacks,))
+
+
+def test_scales_at_the_end_of_the_stream(device):
+    """Rows whose last scales are the stream's last bytes: 8 blocks too many are asked for at every offset from its end."""
+    for m in range(160, 168):
+        for k in (32, 64, 96, 288, 352):
+            check(device, DType.Q8_0H, m, 9, k)
+
+
+@pytest.mark.parametrize("dt,m,n,k", [(DType.Q8_0H, 700, 300, 4064), (DType.F16, 2051, 64, 4000), (DType.Q8_0H, 2560, 520, 10240)])
+def test_without_a_workspace(device, monkeypatch, dt, m, n, k):
+    import ratchet_amd.tensor as mirror
+    monkeypatch.setattr(mirror, "SPLIT_K", False)
+    check(device, dt, m, n, k)
