@@ -34,6 +34,8 @@
 // with register-staged blocks every step waited out a full trip to memory).
 #include "device_common.h"
 
+#include <algorithm>
+
 namespace rt {
 
 struct AttnArgs {
@@ -798,44 +800,45 @@ template <int DC> static hipError_t launch_attention_long(const AttnArgs &g, int
 
 // Second pass of a split launch: per row, the partial (maximum, sum, output) triples of the splits are
 // combined exactly as the two key halves are inside the kernel, then normalised and rounded once.
-// One workgroup per (stack, query block); a thread owns four columns of one row and reads every split's
-// share of them with all loads issued up front (the loops are unrolled over the most splits there can be).
+// A thread owns four columns of one row and reads every split's share of them with all loads issued up front (the loops are
+// unrolled over MS splits: 4, 8 or 16).  blockIdx.x is (query block, 256 of its items): every item has a thread of its own, where one
+// workgroup per query block walked its 1280 (head_dim 80) five deep and read sixteen splits however few there were
+// (8 heads x 400 x 80, three splits: 8.2 -> 2.5 us, the two launches 15.0 -> 10.0).
 constexpr int AT_MAX_SPLITS = 16;
-template <int DP>
-__global__ __launch_bounds__(256) void attention_merge_kernel(AttnArgs g) {
+template <int DP, int MS>
+__global__ __launch_bounds__(256) void attention_merge_kernel(AttnArgs g, int chunks) {
     const int cg = g.D >> 2;                                   // groups of four columns per row
-    const int rows = min(AT_BQ, g.q_len - (int)blockIdx.x * AT_BQ);
+    const int qb = (int)blockIdx.x / chunks, item = ((int)blockIdx.x - qb * chunks) * 256 + (int)threadIdx.x;
+    const int rows = min(AT_BQ, g.q_len - qb * AT_BQ);
+    if (item >= rows * cg) return;
     const int bh = blockIdx.y, b = bh / g.heads, h = bh - b * g.heads;
-    const float *base = g.partial + (((size_t)blockIdx.y * gridDim.x + blockIdx.x) * g.splits) * AT_BQ * (4 + DP);
     const size_t sstride = (size_t)AT_BQ * (4 + DP);
-    for (int item = threadIdx.x; item < rows * cg; item += blockDim.x) {
-        const int row = item / cg, c = 4 * (item - row * cg);
-        const float *pr = base + (size_t)row * (4 + DP);
-        float ms[AT_MAX_SPLITS], ls[AT_MAX_SPLITS];
-        float4_t vs[AT_MAX_SPLITS];
+    const int row = item / cg, c = 4 * (item - row * cg);
+    const float *pr = g.partial + ((size_t)blockIdx.y * ((g.q_len + AT_BQ - 1) / AT_BQ) + qb) * g.splits * sstride + (size_t)row * (4 + DP);
+    float ms[MS], ls[MS];
+    float4_t vs[MS];
 #pragma unroll
-        for (int s = 0; s < AT_MAX_SPLITS; s++) {
-            const int sc = min(s, g.splits - 1);               // past the last split: re-read it, weight zero below
-            ms[s] = pr[sc * sstride], ls[s] = pr[sc * sstride + 1];
-            vs[s] = *(const float4_t *)(pr + sc * sstride + 4 + c);
-        }
-        float m = -INFINITY;
-#pragma unroll
-        for (int s = 0; s < AT_MAX_SPLITS; s++) m = fmaxf(m, ms[s]);
-        const float m_use = m == -INFINITY ? 0.f : m;
-        float l = 0.f;
-        float4_t o = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s = 0; s < AT_MAX_SPLITS; s++) {
-            const float w = s < g.splits ? __builtin_amdgcn_exp2f(ms[s] - m_use) : 0.f;
-            l += ls[s] * w;
-            o += vs[s] * w;
-        }
-        const float inv = 1.f / l; // no visible key anywhere: 0 / 0 = NaN, as in the single pass
-        half_t *op = g.O + b * g.o_bs + h * g.o_hs + (int64_t)(blockIdx.x * AT_BQ + row) * g.o_rs;
-        const half_t o4[4] = {(half_t)(o[0] * inv), (half_t)(o[1] * inv), (half_t)(o[2] * inv), (half_t)(o[3] * inv)};
-        *(uint64_t *)(op + c) = *(const uint64_t *)o4;
+    for (int s = 0; s < MS; s++) {
+        const int sc = min(s, g.splits - 1);                   // past the last split: re-read it, weight zero below
+        ms[s] = pr[sc * sstride], ls[s] = pr[sc * sstride + 1];
+        vs[s] = *(const float4_t *)(pr + sc * sstride + 4 + c);
     }
+    float m = -INFINITY;
+#pragma unroll
+    for (int s = 0; s < MS; s++) m = fmaxf(m, ms[s]);
+    const float m_use = m == -INFINITY ? 0.f : m;
+    float l = 0.f;
+    float4_t o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < MS; s++) {
+        const float w = s < g.splits ? __builtin_amdgcn_exp2f(ms[s] - m_use) : 0.f;
+        l += ls[s] * w;
+        o += vs[s] * w;
+    }
+    const float inv = 1.f / l; // no visible key anywhere: 0 / 0 = NaN, as in the single pass
+    half_t *op = g.O + b * g.o_bs + h * g.o_hs + (int64_t)(qb * AT_BQ + row) * g.o_rs;
+    const half_t o4[4] = {(half_t)(o[0] * inv), (half_t)(o[1] * inv), (half_t)(o[2] * inv), (half_t)(o[3] * inv)};
+    *(uint64_t *)(op + c) = *(const uint64_t *)o4;
 }
 
 
@@ -866,7 +869,14 @@ __device__ __forceinline__ float ad_row_sum(float v) {
     return v;
 }
 
-__global__ __launch_bounds__(AD_THREADS) void attention_decode_kernel(AttnArgs g) {
+// the mask value of a key in base-2 units (one query row: the mask's first)
+template <int MK> __device__ __forceinline__ float ad_mask(const void *mask, uint32_t key) {
+    if constexpr (MK == 0) return 0.f;
+    else return kLog2e * (MK == 1 ? ((const float *)mask)[key] : (float)((const half_t *)mask)[key]);
+}
+
+// MK: no mask tensor, an f32 one, an f16 one
+template <int MK> __global__ __launch_bounds__(AD_THREADS) void attention_decode_kernel(AttnArgs g) {
     __shared__ float sm[4], sl[4];
     __shared__ __attribute__((aligned(16))) float so[16][16][8]; // [key slot][seg][8 dimensions]
     const int t = threadIdx.x, lane = t & 63;
@@ -892,6 +902,9 @@ __global__ __launch_bounds__(AD_THREADS) void attention_decode_kernel(AttnArgs g
         const uint32_t kc = (uint32_t)min(key0 + 16 * i, g.kv_len - 1);
         vr[i] = __builtin_nontemporal_load((const uint4_t *)(V + (kc * (uint32_t)g.v_rs + 8u * segc)));
     }
+    float mk[AD_L];
+#pragma unroll
+    for (int i = 0; i < AD_L; i++) mk[i] = ad_mask<MK>(g.mask, (uint32_t)min(key0 + 16 * i, g.kv_len - 1));
     uint4_t qv = *(const uint4_t *)(Q + 8 * segc);
     if (seg >= ns) qv = zero4;
 
@@ -906,7 +919,7 @@ __global__ __launch_bounds__(AD_THREADS) void attention_decode_kernel(AttnArgs g
             p = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, qa), __builtin_bit_cast(half2_t, ka), p, false);
         }
         p = ad_row_sum(p);
-        sc[i] = key0 + 16 * i < g.kv_len ? p * g.scale_log2e : -INFINITY;
+        sc[i] = key0 + 16 * i < g.kv_len ? (MK ? fmaf(p, g.scale_log2e, mk[i]) : p * g.scale_log2e) : -INFINITY;
         m = fmaxf(m, sc[i]);
     }
     m = wave_max(m);
@@ -945,6 +958,100 @@ __global__ __launch_bounds__(AD_THREADS) void attention_decode_kernel(AttnArgs g
     }
 }
 
+// The same in one launch, for caches that one workgroup per head streams faster than two launches follow each other: a
+// thread count for up to 128, 256 and 512 keys, all of which are requested at once.  A group of 16 lanes keeps the maximum, sum and
+// output of its own keys, so no wavefront waits for another before the end; there the groups meet in LDS.  (Rounds of 512 keys
+// are right for any number of them, and slower than two launches: 32 heads x 80, 700 / 1024 / 2048 keys 7.4 / 8.0 / 15.1 us for
+// 6.0 / 5.8 / 7.0.)
+constexpr int AO_L = 8;
+template <int MK, int THREADS> __global__ __launch_bounds__(THREADS) void attention_decode_one_kernel(AttnArgs g) {
+    constexpr int GROUPS = THREADS / 16, KEYS = GROUPS * AO_L, PARTS = THREADS / 128; // PARTS of GROUPS / PARTS = 8 groups each
+    __shared__ float sm[GROUPS], sl[GROUPS];
+    __shared__ __attribute__((aligned(16))) float so[GROUPS][16][8]; // [group][seg][8 dimensions]; afterwards [PARTS][128] partial sums
+    const int t = threadIdx.x, seg = t & 15, grp = t >> 4;
+    const int ns = g.D >> 3, segc = min(seg, ns - 1); // idle lanes repeat the last live lane's addresses and contribute zeros
+    const int bh = blockIdx.x, b = bh / g.heads, h = bh - b * g.heads;
+    const half_t *K = g.K + b * g.k_bs + h * g.k_hs;
+    const half_t *V = g.V + b * g.v_bs + h * g.v_hs;
+    const uint4_t zero4 = {0u, 0u, 0u, 0u};
+    uint4_t qv = *(const uint4_t *)(g.Q + b * g.q_bs + h * g.q_hs + 8 * segc);
+    uint4_t kr[AO_L], vr[AO_L];
+    auto load = [&](uint4_t (&r)[AO_L], const half_t *p, uint32_t rs, int key0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < AO_L; i++) {
+            const uint32_t kc = (uint32_t)min(key0 + GROUPS * i, g.kv_len - 1); // past the last key: a valid one, masked below
+            r[i] = __builtin_nontemporal_load((const uint4_t *)(p + (kc * rs + 8u * segc)));
+        }
+    };
+    load(kr, K, (uint32_t)g.k_rs, grp);
+    if (seg >= ns) qv = zero4;
+    float m = -INFINITY, l = 0.f, acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int key0 = grp; key0 - grp < g.kv_len; key0 += KEYS) {
+        load(vr, V, (uint32_t)g.v_rs, key0);
+        float sc[AO_L], m_new = m;
+#pragma unroll
+        for (int i = 0; i < AO_L; i++) {
+            const int key = key0 + GROUPS * i;
+            float p = 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const uint32_t qa = qv[e], ka = kr[i][e];
+                p = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, qa), __builtin_bit_cast(half2_t, ka), p, false);
+            }
+            p = ad_row_sum(p) * g.scale_log2e;
+            if (MK) p += ad_mask<MK>(g.mask, (uint32_t)min(key, g.kv_len - 1));
+            sc[i] = key < g.kv_len ? p : -INFINITY;
+            m_new = fmaxf(m_new, sc[i]);
+        }
+        if (key0 - grp + KEYS < g.kv_len) load(kr, K, (uint32_t)g.k_rs, key0 + KEYS);
+        const float m_use = m_new == -INFINITY ? 0.f : m_new; // no visible key yet: every weight is exp2(-inf) = 0
+        const float a = __builtin_amdgcn_exp2f(m - m_use);
+        l *= a;
+#pragma unroll
+        for (int e = 0; e < 8; e++) acc[e] *= a;
+#pragma unroll
+        for (int i = 0; i < AO_L; i++) {
+            const float p = __builtin_amdgcn_exp2f(sc[i] - m_use);
+            l += p;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const uint32_t va = vr[i][e];
+                const half2_t v2 = __builtin_bit_cast(half2_t, va);
+                acc[2 * e] = fmaf(p, (float)v2[0], acc[2 * e]);
+                acc[2 * e + 1] = fmaf(p, (float)v2[1], acc[2 * e + 1]);
+            }
+        }
+        m = m_new;
+    }
+    if (seg == 0) sm[grp] = m, sl[grp] = l;
+    *(float4_t *)&so[grp][seg][0] = float4_t{acc[0], acc[1], acc[2], acc[3]};
+    *(float4_t *)&so[grp][seg][4] = float4_t{acc[4], acc[5], acc[6], acc[7]};
+    __syncthreads();
+    // every wavefront: lane = group (of GROUPS); its weight against the maximum of all
+    const int lane = t & 63;
+    const float mg = lane < GROUPS ? sm[lane] : -INFINITY, mx = wave_max(mg), m_all = mx == -INFINITY ? 0.f : mx;
+    const float w = __builtin_amdgcn_exp2f(mg - m_all);
+    const float l_all = wave_sum(lane < GROUPS ? sl[lane] * w : 0.f);
+    // dimension d of eight groups, then of the eight partial sums
+    const int d = t & 127, part = t >> 7;
+    float o = 0.f;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const float wk = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), __builtin_amdgcn_readfirstlane(part) * 8 + k));
+        o = fmaf(so[part * 8 + k][d >> 3][d & 7], wk, o);
+    }
+    __syncthreads();
+    float *red = &so[0][0][0];
+    red[part * 128 + d] = o;
+    __syncthreads();
+    if (t < g.D) {
+        o = 0.f;
+#pragma unroll
+        for (int k = 0; k < PARTS; k++) o += red[k * 128 + t];
+        g.O[b * g.o_bs + h * g.o_hs + t] = (half_t)(o / l_all); // no visible key anywhere: 0 / 0 = NaN, as in the tiled kernel
+    }
+}
+
 // One workgroup per head: thread d combines dimension d of the head's splits.
 __global__ __launch_bounds__(128) void attention_decode_merge_kernel(AttnArgs g) {
     const int bh = blockIdx.x, b = bh / g.heads, h = bh - b * g.heads, d = threadIdx.x;
@@ -979,8 +1086,17 @@ __global__ __launch_bounds__(128) void attention_decode_merge_kernel(AttnArgs g)
     if (d < g.D) g.O[b * g.o_bs + h * g.o_hs + d] = (half_t)(o / l); // no visible key anywhere: 0 / 0 = NaN, as in the single pass
 }
 
-// splits of the decode kernel for this problem, or 0 when it does not apply: one query row (the causal rule
-// then hides nothing), a cache long enough to be worth two kernels; a launch with a mask tensor stays tiled
+// Keys up to which a decode step runs in one launch.  32 heads x 80, one launch against two (up to 255 keys, against the tiled
+// kernel): 64 keys 3.6 and 4.3 us, 128 3.6 / 4.8, 255 4.0 / 7.9, 300 5.1 / 5.6, 400 5.7 / 5.9, 512 6.0 / 5.8 (16 heads x 128: 6.6 / 5.6).  A mask
+// tensor, which the two-launch kernel did not take before, adds 0.1 to 0.4 us (300 keys: 11.8 -> 5.7).
+constexpr int kDecodeOneKeys = 448;
+template <int MK> static void launch_decode_one(const AttnArgs &g, unsigned stacks, hipStream_t st) {
+    if (g.kv_len <= 128) hipLaunchKernelGGL((attention_decode_one_kernel<MK, 256>), dim3(stacks), dim3(256), 0, st, g);
+    else if (g.kv_len <= 256) hipLaunchKernelGGL((attention_decode_one_kernel<MK, 512>), dim3(stacks), dim3(512), 0, st, g);
+    else hipLaunchKernelGGL((attention_decode_one_kernel<MK, 1024>), dim3(stacks), dim3(1024), 0, st, g);
+}
+// splits of the two-launch decode kernel for this problem, or 0 when it does not apply: one query row (the causal rule
+// then hides nothing), a cache long enough to be worth two kernels
 static int attention_decode_splits(const rt_attention_desc &d) {
     if (d.q_len != 1 || d.kv_len < 256 || d.head_dim % 8 != 0 || d.head_dim > 128) return 0;
     return (d.kv_len + AD_KEYS - 1) / AD_KEYS;
@@ -1004,7 +1120,11 @@ template <int DP, int MK, int DC, int NKQ> static hipError_t launch_attention_k(
     hipLaunchKernelGGL((attention_kernel<DP, MK, DC, NKQ>), dim3(qb, (unsigned)stacks, (unsigned)g.splits), dim3(256 * NKQ), lds, st, g);
     if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     if (g.splits > 1) {
-        hipLaunchKernelGGL((attention_merge_kernel<DP>), dim3(qb, (unsigned)stacks), dim3(256), 0, st, g);
+        const int chunks = (std::min(AT_BQ, g.q_len) * (g.D >> 2) + 255) / 256; // of the items of a query block
+        const dim3 grid(qb * (unsigned)chunks, (unsigned)stacks);
+        if (g.splits <= 4) hipLaunchKernelGGL((attention_merge_kernel<DP, 4>), grid, dim3(256), 0, st, g, chunks);
+        else if (g.splits <= 8) hipLaunchKernelGGL((attention_merge_kernel<DP, 8>), grid, dim3(256), 0, st, g, chunks);
+        else hipLaunchKernelGGL((attention_merge_kernel<DP, AT_MAX_SPLITS>), grid, dim3(256), 0, st, g, chunks);
         return hipGetLastError();
     }
     return hipSuccess;
@@ -1075,6 +1195,8 @@ hipError_t launch_attention(const rt_attention_desc &d, const void *q, const voi
     g.causal = d.causal != 0;
     g.scale_log2e = d.scale * kLog2e;
     g.splits = 1, g.partial = nullptr;
+    // (Below eight key blocks one pass is faster still -- 8 heads x 400 x 400 x 80 8.8 us, three splits 10.0 -- and rounds more: 2.66e-4
+    // against 2.58e-4 from the exact result, because each split rounds its probabilities against a maximum of its own.)
     if (const uint64_t need = attention_workspace_bytes(d); need > 0 && workspace && workspace_bytes >= need && !((uintptr_t)workspace & 15u))
         g.splits = attention_splits(d), g.partial = (float *)workspace;
     const int64_t stacks = (int64_t)d.batch * d.heads;
@@ -1082,14 +1204,27 @@ hipError_t launch_attention(const rt_attention_desc &d, const void *q, const voi
     // 32-bit element offsets inside one head's keys and values
     if ((int64_t)d.kv_len * g.k_rs >= (int64_t(1) << 31) || (int64_t)d.kv_len * g.v_rs >= (int64_t(1) << 31))
         return hipErrorNotSupported;
-    // one query against a long cache: the streaming kernel, when the caller gave the workspace for it
-    if (const int ds = attention_decode_splits(d); ds > 0 && ds <= 65535 && !mask && workspace && !((uintptr_t)workspace & 15u) &&
-                                                   workspace_bytes >= attention_decode_workspace_bytes(d)) {
-        g.splits = ds, g.partial = (float *)workspace;
-        hipLaunchKernelGGL(attention_decode_kernel, dim3((unsigned)ds, (unsigned)stacks), dim3(AD_THREADS), 0, stream, g);
-        if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-        hipLaunchKernelGGL(attention_decode_merge_kernel, dim3((unsigned)stacks), dim3(128), 0, stream, g);
-        return hipGetLastError();
+    // one query row: a stream over the keys and values, in one launch or, against a long cache and with the workspace for
+    // it, split over workgroups
+    if (d.q_len == 1 && d.kv_len > 0 && d.head_dim % 8 == 0 && d.head_dim <= 128) {
+        const int mk = !mask ? 0 : g.mask_f32 ? 1 : 2, ds = attention_decode_splits(d);
+        const bool can_split = ds > 0 && ds <= 65535 && workspace && !((uintptr_t)workspace & 15u) && workspace_bytes >= attention_decode_workspace_bytes(d);
+        if (d.kv_len <= kDecodeOneKeys) {
+            if (mk == 0) launch_decode_one<0>(g, (unsigned)stacks, stream);
+            else if (mk == 1) launch_decode_one<1>(g, (unsigned)stacks, stream);
+            else launch_decode_one<2>(g, (unsigned)stacks, stream);
+            return hipGetLastError();
+        }
+        if (can_split) {
+            g.splits = ds, g.partial = (float *)workspace;
+            const dim3 grid((unsigned)ds, (unsigned)stacks), block(AD_THREADS);
+            if (mk == 0) hipLaunchKernelGGL((attention_decode_kernel<0>), grid, block, 0, stream, g);
+            else if (mk == 1) hipLaunchKernelGGL((attention_decode_kernel<1>), grid, block, 0, stream, g);
+            else hipLaunchKernelGGL((attention_decode_kernel<2>), grid, block, 0, stream, g);
+            if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+            hipLaunchKernelGGL(attention_decode_merge_kernel, dim3((unsigned)stacks), dim3(128), 0, stream, g);
+            return hipGetLastError();
+        }
     }
     // The kernel for many query rows, from seven eighths of the workgroups on that are resident at once: fewer leave more of the
     // chip idle than a step of theirs saves.
