@@ -271,6 +271,51 @@ __device__ __forceinline__ void nt_epilogue32(const GemmNtArgs &g, float16_t (&a
     }
 }
 
+// The output stage for rows that start on 4 bytes only (o_is == 1, o_js even): staged as nt_epilogue does, stored as pairs, consecutive ones by
+// consecutive lanes, a lane's all read back before they are stored.
+template <int TM, int TN, int WM, int WN>
+__device__ __forceinline__ void nt_epilogue_pairs(const GemmNtArgs &g, float4_t (&acc)[TM][TN], uint8_t *smem, int64_t s, int64_t i0, int64_t j0, int wi,
+                                                  int wj, int wave, int lane) {
+    constexpr int EROW = WM + 8, NPAIR = WN * (WM / 2) / 64;
+    static_assert(WN * (WM / 2) % 64 == 0, "whole instructions");
+    const int fr = lane & 15, fg = lane >> 4;
+    const int64_t iw = i0 + wi * WM, jw = j0 + wj * WN;
+    half_t *es = (half_t *)smem + wave * (WN * EROW);
+    rt_with_act(g.act, [&](auto has_act) {
+#pragma unroll
+        for (int a = 0; a < TM; a++) {
+            const float bi = g.has_bias && g.bias_on_rows ? (float)g.bias[min(iw + a * 16 + fr, g.M - 1)] : 0.f;
+#pragma unroll
+            for (int b = 0; b < TN; b++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int jl = b * 16 + 4 * fg + r;
+                    float v = acc[a][b][r] + bi;
+                    if (g.has_bias && !g.bias_on_rows) v += (float)g.bias[min(jw + jl, g.N - 1)];
+                    es[jl * EROW + a * 16 + fr] = (half_t)rt_act_k<decltype(has_act)::value>(v);
+                }
+        }
+    });
+    asm volatile("" ::: "memory"); // same wavefront reads back below; DS operations complete in order
+    const int jn = (int)min<int64_t>(WN, g.N - jw), in = (int)min<int64_t>(WM, g.M - iw); // rows and values inside
+    half_t *o = g.out + s * g.o_bs + jw * g.o_js + iw;
+    uint32_t x[NPAIR];
+#pragma unroll
+    for (int u = 0; u < NPAIR; u++) {
+        const int v = u * 64 + lane, jl = v / (WM / 2), c = 2 * (v - jl * (WM / 2));
+        x[u] = *(const uint32_t *)(es + jl * EROW + c);
+    }
+#pragma unroll
+    for (int u = 0; u < NPAIR; u++) {
+        const int v = u * 64 + lane, jl = v / (WM / 2), c = 2 * (v - jl * (WM / 2));
+        if (jl >= jn || c >= in) continue;
+        half_t *d = o + jl * g.o_js + c;
+        if (c + 2 <= in) __builtin_nontemporal_store(x[u], (uint32_t *)d);
+        else *d = __builtin_bit_cast(half2_t, x[u])[0];
+    }
+    asm volatile("" ::: "memory");
+}
+
 // KFULL: K is a multiple of the K step, so no load or store needs a bound.
 template <int BM, int BN, bool KFULL>
 __global__ __launch_bounds__(NT_THREADS, (BM * BN <= 128 * 64 ? 3 : 1)) void gemm_nt_kernel(GemmNtArgs g) {
@@ -1227,8 +1272,12 @@ static hipError_t launch_nt_q8r(const GemmNtArgs &g, int64_t stacks, hipStream_t
 // t+1 is prefetched into registers while step t is multiplied, and each wavefront stages and
 // writes its own part of the output, so the stores of one step overlap the loads and MFMAs
 // of the next.  K is padded with zeros to a multiple of 32 inside LDS only.
+// PAIRS: output rows that start on 4 bytes and not on 16 (an even number of keys) leave as consecutive pairs (nt_epilogue_pairs).
+// Scores of 32 heads x 300 x 300, 16 x 254 x 254, 6 x 964 x 964: 8.9 / 7.3 / 11.1 us on gemm_nt_kernel with its stores of
+// sixteen values to each of four rows -> 6.9 / 5.6 / 10.3.  An odd number of keys stays there: single values in this kernel's order
+// gain up to some 400 keys (401: 7.2 -> 6.2) and lose beyond (1027: 13.2 -> 16.1).
 // ---------------------------------------------------------------------------
-template <int KP>
+template <int KP, bool PAIRS>
 __global__ __launch_bounds__(NT_THREADS, 2) void gemm_nt_shortk_kernel(GemmNtArgs g) {
     constexpr int BM = 128, BN = 64, WM = 64, WN = 32, TM = 4, TN = 2;
     constexpr int LDK = KP + 8;  // halfs per LDS row: an odd number of 16-byte slots, conflict-free fragment reads
@@ -1319,16 +1368,22 @@ __global__ __launch_bounds__(NT_THREADS, 2) void gemm_nt_shortk_kernel(GemmNtArg
                     acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb[b], fa[a], acc[a][b], 0, 0, 0);
         }
         __syncthreads(); // every wavefront is done with As before the next tile overwrites it
-        nt_epilogue<TM, TN, WM, WN>(g, acc, Es, s, it * BM, j0, wi, wj, wave, lane);
+        if constexpr (PAIRS) nt_epilogue_pairs<TM, TN, WM, WN>(g, acc, Es, s, it * BM, j0, wi, wj, wave, lane);
+        else nt_epilogue<TM, TN, WM, WN>(g, acc, Es, s, it * BM, j0, wi, wj, wave, lane);
     }
 }
 
 // g.tiles_i carries the number of workgroups that share a strip.
 template <int KP> static hipError_t launch_nt_shortk(const GemmNtArgs &g, int64_t stacks, hipStream_t st) {
     const size_t lds = (size_t)(64 + 128) * (KP + 8) * 2 + (size_t)4 * 32 * (64 + 8) * 2;
-    if (const hipError_t e = ensure_lds_limit<&gemm_nt_shortk_kernel<KP>>(); e != hipSuccess) return e;
     dim3 grid((unsigned)((g.N + 63) / 64 * g.tiles_i), (unsigned)stacks);
-    hipLaunchKernelGGL((gemm_nt_shortk_kernel<KP>), grid, dim3(NT_THREADS), lds, st, g);
+    if (g.vec_epilogue) {
+        if (const hipError_t e = ensure_lds_limit<&gemm_nt_shortk_kernel<KP, false>>(); e != hipSuccess) return e;
+        hipLaunchKernelGGL((gemm_nt_shortk_kernel<KP, false>), grid, dim3(NT_THREADS), lds, st, g);
+    } else {
+        if (const hipError_t e = ensure_lds_limit<&gemm_nt_shortk_kernel<KP, true>>(); e != hipSuccess) return e;
+        hipLaunchKernelGGL((gemm_nt_shortk_kernel<KP, true>), grid, dim3(NT_THREADS), lds, st, g);
+    }
     return hipGetLastError();
 }
 
@@ -1510,8 +1565,9 @@ hipError_t launch_gemm_nt(const Problem &p0, const void *A, const void *B, const
     g.vec_epilogue = p.o_is == 1 && p.o_js % 8 == 0 && p.o_bs % 8 == 0 && ((uintptr_t)out & 15u) == 0;
     g.ksplit = 1, g.k_len = p.K, g.partial = nullptr;
     const bool kfull = p.K % NT_BK == 0;
-    if (!q8 && p.K <= 128 && g.vec_epilogue && !g_gemm_nt_no_direct && (p.N + 63) / 64 <= 0x7fffffff) {
-        // resident-strip kernel; vec_epilogue means the output's i axis is contiguous.  Strips are
+    const bool pairs = p.o_is == 1 && p.o_js % 2 == 0 && p.o_bs % 2 == 0 && ((uintptr_t)out & 3u) == 0;
+    if (!q8 && p.K <= 128 && (g.vec_epilogue || pairs) && !g_gemm_nt_no_direct && (p.N + 63) / 64 <= 0x7fffffff) {
+        // resident-strip kernel, the output's i axis contiguous.  Strips are
         // split over several workgroups until the grid has a few workgroups per compute unit.
         const int64_t strips = (p.N + 63) / 64 * p.stacks, atiles = (p.M + 127) / 128;
         int parts = 1;
