@@ -22,7 +22,7 @@ RT_F32, RT_F16, RT_Q8_0F, RT_Q8_0H, RT_Q4_K = 0, 1, 2, 3, 4
 RT_KERNEL_NONE, RT_KERNEL_GEMV_Q8, RT_KERNEL_GEMV_Q4K, RT_KERNEL_GEMV_FLOAT = 0, 1, 2, 3
 RT_KERNEL_GEMM_F16, RT_KERNEL_GEMM_F32 = 4, 5
 
-_Shape = ctypes.c_int64 * RT_MAX_RANK
+_Shape = Shape = ctypes.c_int64 * RT_MAX_RANK
 
 
 class MatmulDesc(ctypes.Structure):
@@ -174,15 +174,12 @@ def make_desc(lhs_dt, lhs_shape, rhs_dt, rhs_shape, trans_lhs=False, trans_rhs=F
         raise ValueError("rank above RT_MAX_RANK")
     d.lhs_dt, d.rhs_dt = int(lhs_dt), int(rhs_dt)
     d.lhs_rank, d.rhs_rank = len(lhs_shape), len(rhs_shape)
-    for i, v in enumerate(lhs_shape):
-        d.lhs_shape[i] = int(v)
-    for i, v in enumerate(rhs_shape):
-        d.rhs_shape[i] = int(v)
+    d.lhs_shape[: len(lhs_shape)] = [int(v) for v in lhs_shape]
+    d.rhs_shape[: len(rhs_shape)] = [int(v) for v in rhs_shape]
     d.trans_lhs, d.trans_rhs, d.trans_out = int(trans_lhs), int(trans_rhs), int(trans_out)
     if bias_shape is not None:
         if len(bias_shape) > RT_MAX_RANK:
             raise ValueError("rank above RT_MAX_RANK")
         d.has_bias, d.bias_dt, d.bias_rank = 1, int(bias_dt), len(bias_shape)
-        for i, v in enumerate(bias_shape):
-            d.bias_shape[i] = int(v)
+        d.bias_shape[: len(bias_shape)] = [int(v) for v in bias_shape]
     return d

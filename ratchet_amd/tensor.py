@@ -18,6 +18,7 @@ from __future__ import annotations
 
 import ctypes
 import enum
+import math
 import os
 from typing import Optional, Sequence
 
@@ -44,6 +45,9 @@ class DType(enum.IntEnum):
         return {DType.F32: np.float32, DType.F16: np.float16}[self]
 
 
+_DTYPES = {int(d): d for d in DType}
+
+
 class OperationError(RuntimeError):
     """An Err(...) of the reference (anyhow / OperationError / TensorError)."""
 
@@ -68,6 +72,13 @@ class Device:
 
     def __init__(self, kind: str, ordinal: int = 0):
         self.kind, self.ordinal, self._ctx = kind, ordinal, None
+        self._torch_device = None
+
+    def torch_device(self):
+        """The torch.device of a GPU device (its name is parsed once, not per allocation)."""
+        if self._torch_device is None:
+            self._torch_device = _torch().device(f"cuda:{self.ordinal}")
+        return self._torch_device
 
     @staticmethod
     def request_device(req: DeviceRequest, ordinal: int = 0) -> "Device":
@@ -110,8 +121,8 @@ def _torch():
     return torch
 
 
-def _stream_ptr() -> ctypes.c_void_p:
-    return ctypes.c_void_p(_torch().cuda.current_stream().cuda_stream)
+def _stream_ptr() -> int:
+    return _torch().cuda.current_stream().cuda_stream
 
 
 def _check(st: int, device: Optional[Device] = None, panic: bool = False):
@@ -149,13 +160,12 @@ class Matmul:
         return tuple(shape[i] for i in range(rank.value))
 
     def compute_view(self):
-        shape = (ctypes.c_int64 * _ffi.RT_MAX_RANK)()
-        rank, dt = ctypes.c_int32(), ctypes.c_int32()
-        _check(_ffi.lib().rt_matmul_infer(ctypes.byref(self.desc), shape, ctypes.byref(rank), ctypes.byref(dt)))
-        return tuple(shape[i] for i in range(rank.value)), DType(dt.value)
+        shape, rank, dt = _ffi.Shape(), ctypes.c_int32(), ctypes.c_int32()
+        _check(_ffi.lib().rt_matmul_infer(self.desc, shape, rank, dt))
+        return tuple(shape[: rank.value]), _DTYPES[dt.value]
 
     def check_invariants(self):
-        st = _ffi.lib().rt_matmul_validate(ctypes.byref(self.desc))
+        st = _ffi.lib().rt_matmul_validate(self.desc)
         # a rank-1 operand passes graph construction in the reference and only
         # panics in GEMMSpec::new at compile time; resolve() reports it
         if st == _ffi.RT_ERR_INVALID_SHAPE and (len(self.lhs.shape) < 2 or len(self.rhs.shape) < 2):
@@ -253,7 +263,7 @@ class Attention:
             raise OperationError(_ffi.RT_ERR_INVALID_SHAPE, f"attention: kv_len {self.kv_len} of a cache of {cap}")
         if mask is not None and tuple(mask.shape[-2:]) != (Lq, self.kv_len):
             raise OperationError(_ffi.RT_ERR_INVALID_SHAPE, f"attention: mask {mask.shape} for [{Lq}, {self.kv_len}] scores")
-        if mask is not None and int(np.prod(mask.shape[:-2], dtype=np.int64)) != 1:
+        if mask is not None and math.prod(mask.shape[:-2]) != 1:
             # the kernel applies ONE [q_len, kv_len] mask to every batch and head (rt_attention_desc has a row stride only)
             raise OperationError(_ffi.RT_ERR_UNSUPPORTED, f"attention: a mask per batch or head ({mask.shape}) is not supported")
         d = _ffi.AttentionDesc()
@@ -262,7 +272,7 @@ class Attention:
         d.k_strides[:] = [H * cap * D, cap * D, D]
         d.v_strides[:] = [H * cap * D, cap * D, D]
         d.o_strides[:] = [Lq * H * D, D, H * D] if merge_heads else [H * Lq * D, Lq * D, D]
-        d.scale = float(1.0 / np.sqrt(D)) if scale is None else float(scale)
+        d.scale = 1.0 / math.sqrt(D) if scale is None else float(scale)
         d.causal = int(self.causal)
         d.mask_dtype = int(mask.dt) if mask is not None else int(DType.F32)
         d.mask_row_stride = self.kv_len
@@ -275,7 +285,7 @@ class Attention:
                 raise InvariantError(_ffi.RT_ERR_DTYPE_MISMATCH, "attention: q, k, v share a dtype")
         if self.mask is not None and self.mask.dt not in (DType.F32, DType.F16):
             raise InvariantError(_ffi.RT_ERR_DTYPE_MISMATCH, "attention: the mask is F32 or F16")
-        st = _ffi.lib().rt_attention_validate(ctypes.byref(self.desc))
+        st = _ffi.lib().rt_attention_validate(self.desc)
         _check(st, panic=st in (_ffi.RT_ERR_DTYPE_MISMATCH, _ffi.RT_ERR_INVALID_SHAPE))
 
     def srcs(self):
@@ -326,12 +336,36 @@ SPLIT_K = True
 POISON_OUTPUTS = False
 
 
+_strides3 = ctypes.c_int64 * 3
+
+
+def _write_key_and_value(k: "Tensor", v: "Tensor", stream: int):
+    """Both cache writes of an attention in one launch, where its keys and values are the two in-place writes of one step that
+    nobody has run yet; anything else is left to run by itself."""
+    a, b = k.op, v.op
+    if k.storage is not None or v.storage is not None or type(a) is not Cache or type(b) is not Cache or a.fresh or b.fresh:
+        return
+    if (a.cache.storage is None or b.cache.storage is None or a.cache.storage is b.cache.storage or k.dt != v.dt or k.shape != v.shape
+            or (a.offset, a.len, a.src_strides) != (b.offset, b.len, b.src_strides) or k.device is not v.device or k.device.kind != "gpu"):
+        return
+    for src in (a.source, b.source):
+        if src.storage is None:
+            src._execute(stream)
+        if src.device.kind != "gpu":
+            return
+    B, H, cap, D = a.cache.shape
+    st = _ffi.lib().rt_cache_write_kv_enqueue(k.device.ctx, int(k.dt), a.cache._ptr(), a.source._ptr(), b.cache._ptr(), b.source._ptr(),
+                                              _strides3(*a.src_strides), B, H, cap, a.offset, a.len, D, stream)
+    _check(st, k.device)
+    k.storage, v.storage = a.cache.storage, b.cache.storage
+
+
 class Tensor:
     """Lazy tensor: either resolved storage, or an operator node awaiting resolve()."""
 
     def __init__(self, shape: Sequence[int], dt: DType, device: Device, storage=None, op: Optional[Matmul] = None):
-        self.shape = tuple(int(s) for s in shape)
-        self.dt, self.device, self.storage, self.op = DType(dt), device, storage, op
+        self.shape = tuple(map(int, shape))
+        self.dt, self.device, self.storage, self.op = dt if type(dt) is DType else DType(dt), device, storage, op
         self.consumers = 0   # operator nodes built on this tensor
         if op is not None:
             for src in op.srcs():
@@ -389,7 +423,13 @@ class Tensor:
         return Tensor(self.shape, self.dt, Device.CPU, raw[:nbytes].view(self.dt.numpy()).reshape(self.shape).copy())
 
     def numel(self) -> int:
-        return int(np.prod(self.shape, dtype=np.int64))
+        return math.prod(self.shape)
+
+    def _ptr(self) -> int:
+        """data_ptr() as a number, which is what a call converts fastest."""
+        if self.storage is None or self.device.kind != "gpu":
+            raise OperationError(_ffi.RT_ERR_INVALID_ARG, "not a resolved GPU tensor")
+        return self.storage.data_ptr()
 
     def data_ptr(self) -> ctypes.c_void_p:
         if not (self.resolved() and self.device.is_gpu()):
@@ -474,77 +514,76 @@ class Tensor:
         dev = self.device
         if not dev.is_gpu():
             raise OperationError(_ffi.RT_ERR_NO_DEVICE, "resolve() needs a GPU tensor (try_gpu)")
-        self._execute()
-        _check(_ffi.lib().rt_sync(dev.ctx, _stream_ptr()), dev)
+        stream = _stream_ptr()
+        self._execute(stream)
+        _check(_ffi.lib().rt_sync(dev.ctx, stream), dev)
         return self
 
-    def _execute(self):
-        if self.resolved():
+    def _empty(self, nbytes: int):
+        return _torch().empty(nbytes, dtype=_torch().uint8, device=self.device.torch_device())
+
+    def _execute(self, stream: int):
+        """Enqueues every unresolved node below this one, then this one, on `stream` (asked of torch once per resolve: the ten
+        operators of an attention block and its MLP would otherwise spend 28 us on asking)."""
+        if self.storage is not None:
             return
-        op, dev, torch = self.op, self.device, _torch()
+        op, dev, L = self.op, self.device, _ffi.lib()
         act = _ffi.RT_ACT_NONE
+        kind = type(op)
         # an activation behind a product nobody else reads runs in that product's epilogue; a product with a second
         # consumer is computed once, rounded, and the activation reads it (as the reference's two operators do)
-        if (isinstance(op, Unary) and FUSE_ACTIVATIONS and isinstance(op.input.op, Matmul) and not op.input.resolved()
+        if (kind is Unary and FUSE_ACTIVATIONS and type(op.input.op) is Matmul and op.input.storage is None
                 and op.input.consumers <= 1):
             act, op = op.act, op.input.op
+            kind = Matmul
+        if kind is Attention:
+            _write_key_and_value(op.k, op.v, stream)
         for src in op.srcs():
-            src._execute()
-            if not src.device.is_gpu():
+            if src.storage is None:
+                src._execute(stream)
+            if src.device.kind != "gpu":
                 raise OperationError(_ffi.RT_ERR_NO_DEVICE, "operand is not on the GPU")
-        if isinstance(op, Softmax):
+        if kind is Softmax:
             # the kernel works in place (softmax.rs:47-49); the source tensor keeps its own storage
             out = op.input.storage.clone()
-            st = _ffi.lib().rt_softmax_enqueue(dev.ctx, int(self.dt), ctypes.c_void_p(out.data_ptr()), len(self.shape),
-                                               op.shape_arr, op.dim, _stream_ptr())
-            _check(st, dev)
+            _check(L.rt_softmax_enqueue(dev.ctx, int(self.dt), out.data_ptr(), len(self.shape), op.shape_arr, op.dim, stream), dev)
             self.storage = out
             return
-        esz = 4 if self.dt == DType.F32 else 2
-        out = torch.empty(max(self.numel() * esz, 16), dtype=torch.uint8, device=f"cuda:{dev.ordinal}")
+        if kind is Cache and not op.fresh:
+            B, H, cap, D = op.cache.shape
+            _check(L.rt_cache_write_enqueue(dev.ctx, int(self.dt), op.cache._ptr(), op.source._ptr(), _strides3(*op.src_strides), None, B, H, cap,
+                                            op.offset, op.len, D, stream), dev)
+            self.storage = op.cache.storage
+            return
+        out = self._empty(max(self.numel() * (4 if self.dt == DType.F32 else 2), 16))
         if POISON_OUTPUTS:
             out.fill_(0xFF)
-        if isinstance(op, Cache):
-            B, H, cap, D = op.cache.shape
-            strides = (ctypes.c_int64 * 3)(*op.src_strides)
-            dst = ctypes.c_void_p(out.data_ptr()) if op.fresh else None
-            st = _ffi.lib().rt_cache_write_enqueue(dev.ctx, int(self.dt), op.cache.data_ptr(), op.source.data_ptr(), strides,
-                                                   dst, B, H, cap, op.offset, op.len, D, _stream_ptr())
-            _check(st, dev)
-            self.storage = out if op.fresh else op.cache.storage
-            return
-        if isinstance(op, Attention):
+        ptr = out.data_ptr()
+        if kind is Matmul:
             need = ctypes.c_uint64()
-            _check(_ffi.lib().rt_attention_workspace_bytes(ctypes.byref(op.desc), ctypes.byref(need)), dev)
-            ws = torch.empty(need.value, dtype=torch.uint8, device=f"cuda:{dev.ordinal}") if need.value and op.use_workspace else None
-            st = _ffi.lib().rt_attention_enqueue(
-                dev.ctx, ctypes.byref(op.desc), op.q.data_ptr(), op.k.data_ptr(), op.v.data_ptr(),
-                op.mask.data_ptr() if op.mask is not None else None, ctypes.c_void_p(out.data_ptr()),
-                ctypes.c_void_p(ws.data_ptr()) if ws is not None else None, need.value if ws is not None else 0, _stream_ptr())
-            _check(st, dev)
-            self.storage = out
-            return
-        if isinstance(op, Unary):
-            st = _ffi.lib().rt_unary_enqueue(dev.ctx, op.act, int(self.dt), op.input.data_ptr(),
-                                             ctypes.c_void_p(out.data_ptr()), self.numel(), _stream_ptr())
-            _check(st, dev)
-            self.storage = out
-            return
-        if isinstance(op, Cast):
-            st = _ffi.lib().rt_cast_enqueue(dev.ctx, int(op.input.dt), int(op.dst_dt), op.input.data_ptr(),
-                                            ctypes.c_void_p(out.data_ptr()), self.numel(), _stream_ptr())
-            _check(st, dev)
-            self.storage = out
-            return
-        op.compute_spec()  # GEMMSpec::new asserts (rank >= 2, stacks)
-        need = ctypes.c_uint64()
-        _check(_ffi.lib().rt_matmul_workspace_bytes(dev.ctx, ctypes.byref(op.desc), ctypes.byref(need)), dev)
-        ws = torch.empty(need.value, dtype=torch.uint8, device=f"cuda:{dev.ordinal}") if need.value and SPLIT_K else None
-        st = _ffi.lib().rt_matmul_enqueue_ws(
-            dev.ctx, ctypes.byref(op.desc), op.lhs.data_ptr(), op.rhs.data_ptr(),
-            op.bias.data_ptr() if op.bias is not None else None, ctypes.c_void_p(out.data_ptr()), act,
-            ctypes.c_void_p(ws.data_ptr()) if ws is not None else None, need.value if ws is not None else 0, _stream_ptr())
-        _check(st, dev)
+            st = L.rt_matmul_workspace_bytes(dev.ctx, op.desc, need)
+            ws = None
+            if st == _ffi.RT_OK:
+                ws = self._empty(need.value) if need.value and SPLIT_K else None
+                st = L.rt_matmul_enqueue_ws(dev.ctx, op.desc, op.lhs._ptr(), op.rhs._ptr(), op.bias._ptr() if op.bias is not None else None, ptr, act,
+                                            ws.data_ptr() if ws is not None else None, need.value if ws is not None else 0, stream)
+            if st != _ffi.RT_OK:
+                op.compute_spec()  # GEMMSpec::new's asserts (rank >= 2, stacks) are panics; the enqueue reports them as errors
+                _check(st, dev)
+        elif kind is Attention:
+            need = ctypes.c_uint64()
+            _check(L.rt_attention_workspace_bytes(op.desc, need), dev)
+            ws = self._empty(need.value) if need.value and op.use_workspace else None
+            _check(L.rt_attention_enqueue(dev.ctx, op.desc, op.q._ptr(), op.k._ptr(), op.v._ptr(), op.mask._ptr() if op.mask is not None else None, ptr,
+                                          ws.data_ptr() if ws is not None else None, need.value if ws is not None else 0, stream), dev)
+        elif kind is Cache:
+            B, H, cap, D = op.cache.shape
+            _check(L.rt_cache_write_enqueue(dev.ctx, int(self.dt), op.cache._ptr(), op.source._ptr(), _strides3(*op.src_strides), ptr, B, H, cap,
+                                            op.offset, op.len, D, stream), dev)
+        elif kind is Unary:
+            _check(L.rt_unary_enqueue(dev.ctx, op.act, int(self.dt), op.input._ptr(), ptr, self.numel(), stream), dev)
+        else:
+            _check(L.rt_cast_enqueue(dev.ctx, int(op.input.dt), int(op.dst_dt), op.input._ptr(), ptr, self.numel(), stream), dev)
         self.storage = out
 
     # -- inspection ---------------------------------------------------------
