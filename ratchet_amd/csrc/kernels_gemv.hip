@@ -291,10 +291,11 @@ hipError_t launch_gemv_chunked(const Problem &p, const void *A, const void *B, c
     const bool q8 = p.a_dt == RT_Q8_0H, q4 = p.a_dt == RT_Q4_K;
     if ((!q8 && !q4) || p.act_dt != RT_F16 || g_gemv_disable_mfma) return hipErrorNotSupported;
     if (p.N <= 16 || p.N > 32) return hipErrorNotSupported;
-    // Q8_0H weights with enough rows that their 64 x 64 tiles give half of the compute units a workgroup are faster on
-    // the tiled kernel (10240 x 2560: 15.7 / 16.2 us at 17 / 32 vectors); with fewer rows (2560 x 2560: 40 tiles) the
-    // streaming launches stay ahead
-    if (q8 && p.K % 256 == 0 && p.stacks == 1 && (p.M + 63) / 64 >= dev.num_cus / 2) return hipErrorNotSupported;
+    // Q8_0H weights with enough rows that their 64 x 64 tiles give a quarter of the compute units a workgroup are faster on
+    // the kernels that read them once (17 / 32 vectors, here against there: 10240 x 2560 18 / 20 and 15.7 / 16.2 us, 7680 x 2560
+    // 12.1 / 13.1 and 9.1 / 9.5, 5120 x 4096 13.5 / 16.4 and 10.2 / 10.6, 4096 x 1024 7.3 / 6.9 and 4.5); with fewer rows the
+    // streaming launches stay ahead (2560 x 2560 7.5 / 8.3 and 9.7 / 10.1)
+    if (q8 && p.K % 256 == 0 && p.stacks == 1 && (p.M + 63) / 64 >= dev.num_cus / 4) return hipErrorNotSupported;
     for (int64_t j0 = 0; j0 < p.N; j0 += 16) {
         Problem c = p;
         c.N = p.N - j0 < 16 ? p.N - j0 : 16;
@@ -322,6 +323,12 @@ hipError_t launch_gemv(const Problem &p, const void *A, const void *B, const voi
         e = launch_gemv_q8h_mfma(p, A, B, bias, out, stream, dev);
         if (e != hipErrorNotSupported) return e;
     }
+    // 5..8 vectors against Q8_0H rows that none of these take (K no multiple of 256), enough of them that 64-row tiles give half of the
+    // compute units a workgroup: the tiled kernel (11392 x 352 at 5 / 8 vectors 11.3 / 17.2 us here, 6.2 / 6.0 there; 9088 x 2272
+    // 15.8 / 24.6 and 15.2 / 14.6; with fewer rows 3840 x 1440 6.8 / 11.6 and 10.5)
+    if (p.kernel == RT_KERNEL_GEMV_Q8 && p.a_dt == RT_Q8_0H && p.N >= 5 && p.stacks == 1 && p.K % 32 == 0 && (p.M + 63) / 64 >= dev.num_cus / 2 &&
+        p.b_ks == 1 && aligned16(A) && aligned16(B) && (p.b_js * 2) % 16 == 0)
+        return hipErrorNotSupported;
     if (p.kernel == RT_KERNEL_GEMV_Q4K) {
         // one vector: the row-streaming kernel; then the matrix-core kernel
         hipError_t e = launch_gemv_q4k_rowdot(p, A, B, bias, out, stream, dev);
@@ -334,9 +341,10 @@ hipError_t launch_gemv(const Problem &p, const void *A, const void *B, const voi
         if (e != hipErrorNotSupported) return e;
         // 5..8 vectors against an f16 weight with enough rows that 64-row tiles give half of the compute units a
         // workgroup: the weight-streaming GEMM, or the tiled kernel's 64 x 64 tiles (10240 x 2560, weights from HBM:
-        // 12.7 / 16 us against 19 / 24 / 26 us at 5 / 7 / 8 vectors here); the conditions are the ones under which
+        // 12.7 / 16 us against 19 / 24 / 26 us at 5 / 7 / 8 vectors here), from 6 vectors on where K ends in half a 64 (8192 x 2016: 10.5 us
+        // against 9.9 / 15.0 at 5 / 8 vectors; 16384 x 544: 6.0 against 10.7 / 15.6); the conditions are the ones under which
         // the tiled kernel takes the product
-        if (p.a_dt == RT_F16 && p.act_dt == RT_F16 && p.N >= 5 && p.stacks == 1 && p.K > 256 && p.K % 64 == 0 &&
+        if (p.a_dt == RT_F16 && p.act_dt == RT_F16 && p.N >= (p.K % 64 == 0 ? 5 : 6) && p.stacks == 1 && p.K > 256 && p.K % 32 == 0 &&
             (p.M + 63) / 64 >= dev.num_cus / 2 && p.a_ks == 1 && p.b_ks == 1 && aligned16(A) && aligned16(B) &&
             (p.a_rs * 2) % 16 == 0 && (p.b_js * 2) % 16 == 0 && !(p.o_js == 1 && p.o_is != 1))
             // (a row-major output would make the tiled kernel exchange the operands, and with the weight as its

@@ -67,6 +67,13 @@ def test_k_of_whole_units(device, dt, m, n, k):
     check(device, dt, m, n, k)
 
 
+@pytest.mark.parametrize("m,n,k", [  # the smallest numbers of activation rows that leave the streaming kernels, on both sides of the line
+    (8192, 5, 288), (8100, 5, 288), (8129, 8, 544), (8128, 8, 544), (9000, 4, 288), (16400, 7, 352), (4097, 17, 512), (4032, 17, 512), (5120, 32, 1024)])
+@pytest.mark.parametrize("dt", [DType.Q8_0H, DType.F16])
+def test_few_activation_rows(device, dt, m, n, k):
+    check(device, dt, m, n, k)
+
+
 @pytest.mark.parametrize("m,n,k", [(333, 70, 288), (1001, 300, 800), (2600, 130, 4000)])
 @pytest.mark.parametrize("dt", [DType.Q8_0H, DType.F16])
 def test_other_axis_contiguous(device, dt, m, n, k):
