@@ -386,7 +386,7 @@ rt_status rt_matmul_workspace_bytes(rt_ctx *ctx, const rt_matmul_desc *desc, uin
     rt_status st = rt::make_spec(*desc, spec, p, &why);
     if (st != RT_OK) return fail(ctx, st, why);
     // only the tiled kernels share a problem among workgroups; the streaming kernels take M <= 16
-    if (p.kernel == RT_KERNEL_GEMM_F16) *bytes = rt::gemm_nt_workspace_bytes(p, ctx->dev);
+    if (p.kernel == RT_KERNEL_GEMM_F16) *bytes = p.a_dt == RT_Q4_K ? rt::gemm_q4k_workspace_bytes(p, ctx->dev) : rt::gemm_nt_workspace_bytes(p, ctx->dev);
     if (p.kernel == RT_KERNEL_GEMM_F32) *bytes = rt::gemm_limb_workspace_bytes(p, ctx->dev);
     return RT_OK;
     RT_GUARD_END(ctx)

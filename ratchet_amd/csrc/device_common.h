@@ -177,6 +177,8 @@ hipError_t launch_gemm_stream(const Problem &p, const void *A, const void *B, co
 uint64_t gemm_nt_workspace_bytes(const Problem &p, const DeviceInfo &dev);
 hipError_t launch_gemm_nt(const Problem &p, const void *A, const void *B, const void *bias, void *out,
                           hipStream_t stream, const DeviceInfo &dev);
+uint64_t gemm_q4k_workspace_bytes(const Problem &p, const DeviceInfo &dev);
+hipError_t launch_splitk_sums(const Problem &p, const void *bias, void *out, float *partial, int ks, hipStream_t st);
 hipError_t launch_gemm_nn_smalln(const Problem &p, const void *A, const void *B, const void *bias, void *out,
                                  hipStream_t stream, const DeviceInfo &dev);
 hipError_t launch_unary(int act, int dtype, const void *src, void *dst, uint64_t numel, hipStream_t stream);

@@ -1245,6 +1245,17 @@ static hipError_t launch_splitk_reduce(const GemmNtArgs &g, int64_t stacks, hipS
     return hipGetLastError();
 }
 
+// The second pass for another file's kernel that left f32 sums of `ks` shares of problem p in `partial` [stack][share][N][M].
+hipError_t launch_splitk_sums(const Problem &p, const void *bias, void *out, float *partial, int ks, hipStream_t st) {
+    GemmNtArgs g{};
+    g.bias = (const half_t *)bias, g.out = (half_t *)out, g.partial = partial, g.ksplit = ks;
+    g.M = p.M, g.N = p.N;
+    g.o_bs = p.o_bs, g.o_is = p.o_is, g.o_js = p.o_js;
+    g.has_bias = p.has_bias, g.bias_on_rows = p.bias_on_rows, g.act = p.act;
+    g.vec_epilogue = p.o_is == 1 && p.o_js % 8 == 0 && p.o_bs % 8 == 0 && ((uintptr_t)out & 15u) == 0;
+    return launch_splitk_reduce(g, p.stacks, st);
+}
+
 template <int BM, int BN, int LW>
 static hipError_t launch_nt_q8w(const GemmNtArgs &g, int64_t stacks, hipStream_t st) {
     const size_t lds = (size_t)4 * (BM + BN) * NT_LDK * 2;

@@ -60,6 +60,11 @@ struct GemmQ4kArgs {
     int64_t o_bs, o_is, o_js;
     int tiles_j, remap, vec_out;
     int has_bias, bias_on_rows, act;
+    // K shared: blockIdx.z owns super-blocks [z * sb_len, (z + 1) * sb_len) and writes its f32 sums to partial [stack][share][N][M]; a
+    // second kernel adds them up, then bias, activation, rounding
+    int ksplit;
+    int64_t sb_len;
+    float *partial;
 };
 
 constexpr int QR_BN = 64; // activation rows per workgroup; weight rows: 16 per MFMA tile x TA tiles x MW multiplying wavefronts
@@ -95,10 +100,11 @@ __global__ __launch_bounds__(64 * (MW + LW), 2) void gemm_q4k_kernel(GemmQ4kArgs
     // (a division runs on the vector units: its result back into a scalar register, where it costs the main loop none of its own)
     const uint32_t ti = __builtin_amdgcn_readfirstlane(b / (uint32_t)g.tiles_j), tj = b - ti * (uint32_t)g.tiles_j;
     const int64_t i0 = (int64_t)ti * BM, j0 = (int64_t)tj * QR_BN;
-    const uint8_t *blocks = g.blocks + (g.a_stack == 1 ? 0 : s) * g.M * g.nsb * 144;
-    const half_t *X = g.X + (g.b_stack == 1 ? 0 : s) * g.b_bs;
-    const int64_t last = g.nsb - 1;
-    const bool vec_out = g.vec_out && i0 + BM <= g.M; // a whole tile of weight rows, stored 16 bytes at a time
+    const int64_t sb0 = (int64_t)blockIdx.z * g.sb_len, nsb = min(g.sb_len, g.nsb - sb0); // this workgroup's share of K: > 0 (launcher)
+    const uint8_t *blocks = g.blocks + ((g.a_stack == 1 ? 0 : s) * g.M * g.nsb + sb0) * 144;
+    const half_t *X = g.X + (g.b_stack == 1 ? 0 : s) * g.b_bs + sb0 * 256;
+    const int64_t last = nsb - 1;
+    const bool vec_out = g.vec_out && g.ksplit == 1 && i0 + BM <= g.M; // a whole tile of weight rows, stored 16 bytes at a time
 
     if (LW > 0 && wave >= MW) {
         // ---- loading wavefront lw: LDS-DMA instruction i of a stage (i = lw, lw + 4, ...; 33 in all) fills the 1 KB
@@ -339,12 +345,12 @@ __global__ __launch_bounds__(64 * (MW + LW), 2) void gemm_q4k_kernel(GemmQ4kArgs
     // two super-blocks per trip, one straight run of instructions (a branch inside it makes the compiler wait
     // for every load in flight)
     int64_t sb = 0;
-    for (; sb + 1 < g.nsb; sb += 2) {
+    for (; sb + 1 < nsb; sb += 2) {
         step(std::integral_constant<int, 0>{}, sb, r0, r1);
         step(std::integral_constant<int, 1>{}, sb + 1, r1, r0);
     }
     uint2_t hl[TB];
-    if (sb < g.nsb) {
+    if (sb < nsb) {
         step(std::integral_constant<int, 0>{}, sb, r0, r1);
         tile_ready();
         read_sums(0, hl);
@@ -356,6 +362,21 @@ __global__ __launch_bounds__(64 * (MW + LW), 2) void gemm_q4k_kernel(GemmQ4kArgs
     }
 
     // acc[a][bq][r]: weight row i0 + 32 wave + 16 a + fr, activation row j0 + 16 ((bq + wave) % 4) + 4 fg + r
+    if (g.ksplit > 1) {
+        float *pt = g.partial + (s * g.ksplit + blockIdx.z) * g.N * g.M;
+#pragma unroll
+        for (int a = 0; a < TA; a++) {
+            const int64_t i = i0 + wave * (16 * TA) + 16 * a + fr;
+#pragma unroll
+            for (int bq = 0; bq < TB; bq++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int64_t j = j0 + 16 * ((bq + wave) & 3) + 4 * fg + r;
+                    if (i < g.M && j < g.N) pt[j * g.M + i] = acc[a][bq][r];
+                }
+        }
+        return;
+    }
     half_t *out = g.out + s * g.o_bs;
     if (vec_out) {
         // Output contiguous along the weight rows: the tile goes through LDS (the activation stages are free: every
@@ -412,12 +433,50 @@ __global__ __launch_bounds__(64 * (MW + LW), 2) void gemm_q4k_kernel(GemmQ4kArgs
 RT_TUNABLE(g_gemm_q4k_cfg, 0); // 14 / 24: always one / two weight tiles per wavefront (for comparisons)
 RT_TUNABLE(g_gemm_q4k_disable, 0); // non-zero keeps Q4_K prefill on the generic kernel (for comparisons)
 
+// Weight tiles per wavefront and workgroups that share K, by an estimate in microseconds: 5.5 + step * super-blocks of a share, 0.95 a
+// step with one weight tile, 1.6 with two, and the second kernel's time.  A wavefront's super-blocks are a chain, so with few tiles a long K
+// took as long as with many; shared (M x K at activation rows, K whole and shared, us): 2560 x 10240 at 64 38.4 and 16.4, 3072 x 8192
+// at 32 31.6 and 15.4, at 100 31.6 and 21.0, 3584 x 9472 at 148 38.1 and 30, 1024 x 4096 at 128 17.6 and 11.7, 2560 x 2560 at 40
+// 12.3 and 10.2.  The margin of 0.3: 430 x 1280 at 228 took 10.1 whole and 10.9 in 5 shares, 828 x 1280 at 70 10.2 and 8.8.
+// Without a workspace (and with more tiles of 128 rows than compute units) K stays whole.
+struct Q4kChoice {
+    int ta = 2, ks = 1;
+};
+static bool gemm_q4k_takes(const Problem &p) {
+    return p.a_dt == RT_Q4_K && p.act_dt == RT_F16 && p.K % 256 == 0 && p.K >= 256 && p.b_ks == 1 && p.M >= 64 && p.N >= 17 && p.stacks <= 65535;
+}
+static Q4kChoice q4k_choose(const Problem &p, const DeviceInfo &dev, bool may_split) {
+    // Four multiplying wavefronts of 32 weight rows x 64 activation rows each; when the grid of 16-row wavefronts
+    // (64 weight rows per workgroup) still fits the compute units in one round, those: half the work per wavefront
+    // (8192 x 3072 at 64 / 128 rows: 15.7 / 16.8 us against 22.6 / 23.6; 3072 x 8192 at 256 rows: 35 against 52 us).
+    const int64_t tiles_j = (p.N + QR_BN - 1) / QR_BN, nsb = p.K / 256;
+    Q4kChoice best;
+    best.ta = ((p.M + 63) / 64) * tiles_j <= dev.num_cus ? 1 : 2;
+    if (!may_split || ((p.M + 127) / 128) * tiles_j * p.stacks > dev.num_cus) return best;
+    float least = 5.2f + (best.ta == 1 ? 0.95f : 1.6f) * nsb;
+    for (int ta = 1; ta <= 2; ta++) {
+        const int64_t n = ((p.M + 64 * ta - 1) / (64 * ta)) * tiles_j * p.stacks;
+        for (int ks = 2; ks <= 16 && n * ks <= dev.num_cus; ks++) {
+            const int64_t share = (nsb + ks - 1) / ks;
+            if ((ks - 1) * share >= nsb) continue;
+            const float us = 5.5f + (ta == 1 ? 0.95f : 1.6f) * share + 2.6f + 0.1f * ks + (float)(p.stacks * ks * p.M * p.N) * (4.f / 4.5e6f);
+            if (us < least) least = us, best.ta = ta, best.ks = ks;
+        }
+    }
+    return best;
+}
+// bytes of workspace with which launch_gemm_q4k shares this problem's K (0: it does not)
+uint64_t gemm_q4k_workspace_bytes(const Problem &p, const DeviceInfo &dev) {
+    if (!gemm_q4k_takes(p)) return 0;
+    const int ks = q4k_choose(p, dev, true).ks;
+    return ks > 1 ? (uint64_t)p.stacks * ks * p.M * p.N * sizeof(float) : 0;
+}
+
 // Q4_K weights x K-contiguous f16 activations, more rows than one streaming launch takes.
 // hipErrorNotSupported: another kernel must take the problem.
 hipError_t launch_gemm_q4k(const Problem &p, const void *A, const void *B, const void *bias, void *out, hipStream_t stream,
                            const DeviceInfo &dev) {
-    if (g_gemm_q4k_disable || p.a_dt != RT_Q4_K || p.act_dt != RT_F16) return hipErrorNotSupported;
-    if (p.K % 256 != 0 || p.K < 256 || p.b_ks != 1 || p.M < 64 || p.N < 17 || p.stacks > 65535) return hipErrorNotSupported;
+    if (g_gemm_q4k_disable || !gemm_q4k_takes(p)) return hipErrorNotSupported;
     if (((uintptr_t)A & 15u) || ((uintptr_t)B & 15u) || (p.b_js * 2) % 16 || (p.b_bs * 2) % 16) return hipErrorNotSupported;
     // 32-bit offsets within a stack, in bytes
     if (p.M * (p.K / 256) * 144 >= (int64_t(1) << 32) || p.N * p.b_js >= (int64_t(1) << 31)) return hipErrorNotSupported;
@@ -431,22 +490,22 @@ hipError_t launch_gemm_q4k(const Problem &p, const void *A, const void *B, const
     const int64_t tiles_j = (p.N + QR_BN - 1) / QR_BN;
     g.tiles_j = (int)tiles_j;
     g.vec_out = p.o_is == 1 && p.o_js % 8 == 0 && p.o_bs % 8 == 0 && ((uintptr_t)out & 15u) == 0;
+    Q4kChoice c = q4k_choose(p, dev, p.workspace && !((uintptr_t)p.workspace & 15u));
+    if (c.ks > 1 && p.workspace_bytes < (uint64_t)p.stacks * c.ks * p.M * p.N * sizeof(float)) c = q4k_choose(p, dev, false);
+    g.ksplit = c.ks, g.sb_len = (g.nsb + c.ks - 1) / c.ks, g.partial = (float *)p.workspace;
+    if (g_gemm_q4k_cfg) c.ta = g_gemm_q4k_cfg == 14 ? 1 : 2;
     auto go = [&](auto kernel, int bm, int lw) -> hipError_t {
         const int64_t tiles_i = (p.M + bm - 1) / bm;
         if (tiles_i * tiles_j > 0x7fffffff) return hipErrorNotSupported;
         g.remap = (tiles_i * tiles_j) % 8 == 0;
         if (const hipError_t e = ensure_lds_limit<decltype(kernel)::value>(); e != hipSuccess) return e;
-        hipLaunchKernelGGL(decltype(kernel)::value, dim3((unsigned)(tiles_i * tiles_j), (unsigned)p.stacks), dim3(64 * (4 + lw)), QR_LDS, stream, g);
-        return hipGetLastError();
+        hipLaunchKernelGGL(decltype(kernel)::value, dim3((unsigned)(tiles_i * tiles_j), (unsigned)p.stacks, (unsigned)c.ks), dim3(64 * (4 + lw)), QR_LDS, stream, g);
+        if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+        return c.ks > 1 ? launch_splitk_sums(p, bias, out, g.partial, c.ks, stream) : hipSuccess;
     };
-    // Four multiplying wavefronts of 32 weight rows x 64 activation rows each; when the grid of 16-row wavefronts
-    // (64 weight rows per workgroup) still fits the compute units in one round, those: half the work per wavefront
-    // (8192 x 3072 at 64 / 128 rows: 15.7 / 16.8 us against 22.6 / 23.6; 3072 x 8192 at 256 rows: 35 against 52 us).
-    const int64_t wgs_small = ((p.M + 63) / 64) * tiles_j, wgs = ((p.M + 127) / 128) * tiles_j * p.stacks;
-    const bool small = g_gemm_q4k_cfg == 14 || (g_gemm_q4k_cfg == 0 && wgs_small <= dev.num_cus);
-    if (small) return go(std::integral_constant<void (*)(GemmQ4kArgs), &gemm_q4k_kernel<1, 4, 4>>{}, 64, 4);
+    if (c.ta == 1) return go(std::integral_constant<void (*)(GemmQ4kArgs), &gemm_q4k_kernel<1, 4, 4>>{}, 64, 4);
     // more than one workgroup per compute unit: no loading wavefronts (see the file comment)
-    if (wgs > dev.num_cus) return go(std::integral_constant<void (*)(GemmQ4kArgs), &gemm_q4k_kernel<2, 4, 0>>{}, 128, 0);
+    if (((p.M + 127) / 128) * tiles_j * p.stacks > dev.num_cus) return go(std::integral_constant<void (*)(GemmQ4kArgs), &gemm_q4k_kernel<2, 4, 0>>{}, 128, 0);
     return go(std::integral_constant<void (*)(GemmQ4kArgs), &gemm_q4k_kernel<2, 4, 4>>{}, 128, 4);
 }
 
