@@ -64,8 +64,9 @@ struct GemmNtArgs {
 // Which output tile a workgroup takes.  Workgroup ids go round the 8 XCDs, each with an L2 of its own.
 // g.xi > 0: the grid of tiles is cut into xi x (8 / xi) equal blocks, one per XCD, and a block is walked in panels
 // of g.pj columns, so that the 32 workgroups an XCD runs at a time share the fewest operand rows
-// (nt_set_tiles chooses).  Otherwise XCD x takes the contiguous range x * ntiles / 8 .. of the tiles in row-major
-// order when that comes out even, and the plain order when not.  In 32 bits and with the block's sides from the host: every
+// (nt_set_tiles chooses).  Otherwise XCD x takes the x-th of eight contiguous ranges of the tiles in row-major order, the first
+// ntiles % 8 of them one longer (taken as they come, neighbours of a tile row would read its operands into eight L2s: f16, 300 rows x
+// 2560 x 10240 in 60 tiles of 128 x 128 and 4 shares 39.6 -> 35.3 us, 1300 rows x 8192 x 4096 in 572 of 160 x 128 133.5 -> 101.5).  In 32 bits and with the block's sides from the host: every
 // workgroup waits for this before its first load, and six 64-bit divisions were 0.3 us a launch (a 512-row prompt through
 // a layer with Q8_0H weights, four products: 178.8 -> 176.6 us).
 __device__ __forceinline__ void nt_tile_of(const GemmNtArgs &g, int64_t wg, int64_t &ti, int64_t &tj) {
@@ -78,7 +79,7 @@ __device__ __forceinline__ void nt_tile_of(const GemmNtArgs &g, int64_t wg, int6
         ti = (x >> g.xj_log2) * g.rows + qi, tj = (x & ((1u << g.xj_log2) - 1)) * g.cols + p * g.pj + (q - qi * w);
         return;
     }
-    const uint32_t ntiles = (uint32_t)g.tiles_i * (uint32_t)g.tiles_j, n = ntiles % 8 == 0 ? (id & 7) * (ntiles >> 3) + (id >> 3) : id;
+    const uint32_t ntiles = (uint32_t)g.tiles_i * (uint32_t)g.tiles_j, x = id & 7, n = x * (ntiles >> 3) + min(x, ntiles & 7) + (id >> 3);
     ti = n / (uint32_t)g.tiles_j, tj = n - (uint32_t)ti * (uint32_t)g.tiles_j;
 }
 
@@ -475,7 +476,7 @@ __global__ __launch_bounds__(NT_THREADS, (BM * BN <= 128 * 64 ? 3 : 1)) void gem
 // them, barrier (every read has returned, tile t + 1 is visible), the second step's MFMAs with
 // the reads of tile t + 1's first-step fragments between them.
 // ---------------------------------------------------------------------------
-template <int BM, int BN, int STAGES, int LW>
+template <int BM, int BN, int STAGES, int LW, bool TAIL>
 __global__ __launch_bounds__(NT_THREADS + 64 * LW) void gemm_nt_dl_kernel(GemmNtArgs g) {
     constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 16, TN = WN / 16;
     constexpr int CH = (BM + BN) / 8;  // 8-row chunks of one K tile: the A rows, then the B rows
@@ -488,7 +489,7 @@ __global__ __launch_bounds__(NT_THREADS + 64 * LW) void gemm_nt_dl_kernel(GemmNt
     half_t *ring = (half_t *)smem; // [STAGES][BM + BN][64]
 
     const int t = threadIdx.x, lane = t & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6); if (wave < 4) __builtin_amdgcn_s_setprio(3);
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
 
     int64_t ti, tj;
     nt_tile_of(g, blockIdx.x, ti, tj); // XCD-aware tile order (see the file comment)
@@ -504,16 +505,17 @@ __global__ __launch_bounds__(NT_THREADS + 64 * LW) void gemm_nt_dl_kernel(GemmNt
         // hold K-vector (l % 8) ^ ((row >> 1) & 7); BM is a multiple of 16, so the swizzle of a B
         // row is the same counted from the top of the stage as from the top of the B tile
         const int lw = wave - 4;
+        static_assert(LW % 2 == 0, "one K-vector per lane for all chunks");
+        const int kv = 8 * ((lane & 7) ^ ((lw * 4 + (lane >> 4)) & 7)); // (lane % 8) ^ (row / 2 % 8)
         const half_t *gp[LCH];
 #pragma unroll
         for (int c = 0; c < LCH; c++) {
             const int row = (lw + c * LW) * 8 + (lane >> 3);
-            gp[c] = row < BM ? (const half_t *)g.A + a_el + min(i0 + row, g.M - 1) * g.a_rs : g.B + b_el + min(j0 + (row - BM), g.N - 1) * g.b_js;
+            gp[c] = (row < BM ? (const half_t *)g.A + a_el + min(i0 + row, g.M - 1) * g.a_rs : g.B + b_el + min(j0 + (row - BM), g.N - 1) * g.b_js) + (TAIL ? 0 : kv);
         }
-        static_assert(LW % 2 == 0, "one K-vector per lane for all chunks");
-        const int kv = 8 * ((lane & 7) ^ ((lw * 4 + (lane >> 4)) & 7)); // (lane % 8) ^ (row / 2 % 8)
         auto issue_tile = [&](int stage, int tile) {
-            const int k = min(min(tile, nk - 1) * NT_BK + kv, kn - 8); // past the last tile that one again, past the end of K its last vector: never used
+            const int kt = min(tile, nk - 1) * NT_BK; // past the last tile that one again
+            const int k = TAIL ? min(kt + kv, kn - 8) : kt; // past the end of K its last vector: never used
             half_t *st = ring + stage * STAGE_HALFS;
             if (RT_NT_ABLATION & 1) return; // timing only: no tile loads
 #pragma unroll
@@ -597,7 +599,7 @@ __global__ __launch_bounds__(NT_THREADS + 64 * LW) void gemm_nt_dl_kernel(GemmNt
             }
         }
         meet(); // tile kt + 1 visible
-        if (kt + 1 == nk && kn % NT_BK) break; // K ends with the first half of this tile
+        if (TAIL && kt + 1 == nk && kn % NT_BK) break; // K ends with the first half of this tile
 #pragma unroll
         for (int m = 0; m < TM * TN; m++) {
             if (!(RT_NT_ABLATION & 2)) acc[m / TN][m % TN] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f1.fb[m % TN], f1.fa[m / TN], acc[m / TN][m % TN], 0, 0, 0);
@@ -650,7 +652,7 @@ __global__ __launch_bounds__(64 * WI * WJ) void gemm_nt_wide_kernel(GemmNtArgs g
 
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int t = threadIdx.x, lane = t & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6); if (wave < 4) __builtin_amdgcn_s_setprio(3);
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     int64_t ti, tj;
     nt_tile_of(g, blockIdx.x, ti, tj); // XCD-aware tile order (see the file comment)
     const int64_t i0 = ti * BM, j0 = tj * BN;
@@ -1398,14 +1400,19 @@ template <int KP> static hipError_t launch_nt_shortk(const GemmNtArgs &g, int64_
     return hipGetLastError();
 }
 
-template <int BM, int BN, int STAGES, int LW>
-static hipError_t launch_nt_dl(const GemmNtArgs &g, int64_t stacks, hipStream_t st) {
+template <int BM, int BN, int STAGES, int LW, bool TAIL>
+static hipError_t launch_nt_dl_as(const GemmNtArgs &g, int64_t stacks, hipStream_t st) {
     const size_t lds = (size_t)STAGES * (BM + BN) * NT_LDK * 2;
-    if (const hipError_t e = ensure_lds_limit<&gemm_nt_dl_kernel<BM, BN, STAGES, LW>>(); e != hipSuccess) return e;
+    if (const hipError_t e = ensure_lds_limit<&gemm_nt_dl_kernel<BM, BN, STAGES, LW, TAIL>>(); e != hipSuccess) return e;
     dim3 grid((unsigned)((int64_t)g.tiles_i * g.tiles_j), (unsigned)stacks, (unsigned)g.ksplit);
-    hipLaunchKernelGGL((gemm_nt_dl_kernel<BM, BN, STAGES, LW>), grid, dim3(NT_THREADS + 64 * LW), lds, st, g);
+    hipLaunchKernelGGL((gemm_nt_dl_kernel<BM, BN, STAGES, LW, TAIL>), grid, dim3(NT_THREADS + 64 * LW), lds, st, g);
     if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     return g.ksplit > 1 ? launch_splitk_reduce(g, stacks, st) : hipSuccess;
+}
+
+template <int BM, int BN, int STAGES, int LW>
+static hipError_t launch_nt_dl(const GemmNtArgs &g, int64_t stacks, hipStream_t st) {
+    return g.K % NT_BK ? launch_nt_dl_as<BM, BN, STAGES, LW, true>(g, stacks, st) : launch_nt_dl_as<BM, BN, STAGES, LW, false>(g, stacks, st);
 }
 
 static hipError_t launch_nt_wide(const GemmNtArgs &g, int64_t stacks, hipStream_t st) {
@@ -1612,10 +1619,8 @@ hipError_t launch_gemm_nt(const Problem &p0, const void *A, const void *B, const
         // A round of 320 x 256 tiles takes 12 + 0.030 K us on all compute units, one of 160 x 128 tiles 6.4 + 0.0080 K: four small
         // rounds are always longer (10240 x 2560 weights, 2048 activation rows: 108.5 us against 89.7), two never.  Three are
         // longer for a short K (1500 rows, K = 1024: 43.9 against 39.3), the same at K = 2560 and shorter beyond (1000 rows
-        // x 11008 x 4096: 107.0 against 118.9; two wide rounds against six small ones alike) -- unless the small tiles do not deal out
-        // evenly to the XCDs, whose L2s then share little (1300 rows x 8192 x 4096, 572 tiles: 133.5 against 114.2).
-        const bool even = tiles % 8 == 0;
-        const bool longer = 5 * rounds_wide < 2 * rounds && (3 * rounds_wide < rounds || !even || p.K <= 2048);
+        // x 11008 x 4096: 107.0 against 118.9; 1300 rows x 8192 x 4096: 101.5 against 102.6; two wide rounds against six small ones alike).
+        const bool longer = 5 * rounds_wide < 2 * rounds && (3 * rounds_wide < rounds || p.K <= 2048);
         if ((g_gemm_nt_wide == 2 || longer) && nt_set_tiles(g, 320, 256, 2)) return launch_nt_wide(g, p.stacks, stream);
     }
     if (!nt_set_tiles(g, c.bm, c.bn, q8 ? 1 : 2)) return hipErrorNotSupported;
