@@ -341,12 +341,16 @@ _strides3 = ctypes.c_int64 * 3
 
 def _write_key_and_value(k: "Tensor", v: "Tensor", stream: int):
     """Both cache writes of an attention in one launch, where its keys and values are the two in-place writes of one step that
-    nobody has run yet; anything else is left to run by itself."""
+    nobody has run yet and the values' source reads nothing that the keys' write changes; anything else is left to run by itself."""
     a, b = k.op, v.op
     if k.storage is not None or v.storage is not None or type(a) is not Cache or type(b) is not Cache or a.fresh or b.fresh:
         return
     if (a.cache.storage is None or b.cache.storage is None or a.cache.storage is b.cache.storage or k.dt != v.dt or k.shape != v.shape
             or (a.offset, a.len, a.src_strides) != (b.offset, b.len, b.src_strides) or k.device is not v.device or k.device.kind != "gpu"):
+        return
+    # the order of the operators stays what it is without this: the values' source runs behind the keys' write, unless all it
+    # reads is there already and is not that cache
+    if b.source.storage is None and any(s.storage is None or s.storage is a.cache.storage for s in b.source.op.srcs()):
         return
     for src in (a.source, b.source):
         if src.storage is None:
@@ -537,6 +541,8 @@ class Tensor:
             act, op = op.act, op.input.op
             kind = Matmul
         if kind is Attention:
+            if op.q.storage is None:
+                op.q._execute(stream)   # first, as in srcs(): it may read the caches as they were
             _write_key_and_value(op.k, op.v, stream)
         for src in op.srcs():
             if src.storage is None:

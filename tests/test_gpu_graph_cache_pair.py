@@ -61,3 +61,26 @@ def test_cache_writes_of_an_attention(device, monkeypatch, arrangement):
     assert torch.equal(got, want.transpose(1, 2).reshape(1, new, H * D))
     if arrangement != "fresh":
         assert torch.equal(values(KC), kd) and torch.equal(values(VC), vd)
+
+
+@pytest.mark.parametrize("reader", ["queries", "values"])
+def test_what_reads_the_caches_between_the_writes(device, reader):
+    """Queries from an attention over the same caches run before the writes, and values made of the key cache behind the keys' write."""
+    H, D, n = 2, 64, 16
+    gen = torch.Generator("cuda:0").manual_seed(5)
+    q, k1, v1, k2, v2, old = (torch.randn((1, H, n, D), generator=gen, device="cuda:0").half() for _ in range(6))
+    KC, VC = tensor(device, old), tensor(device, old)
+
+    def attend(first, lazy):
+        step = (lambda t: t) if lazy else (lambda t: t.resolve())
+        q2, keys, vals = tensor(device, q), tensor(device, k2), tensor(device, v2)
+        if reader == "queries":
+            q2 = step(first.attention(step(KC.cache_write(tensor(device, k1), 0)), step(VC.cache_write(tensor(device, v1), 0))))
+        written = step(KC.cache_write(keys, 0))
+        if reader == "values":
+            vals = step(KC.gelu())
+        return values(q2.attention(written, step(VC.cache_write(vals, 0))).resolve()).clone()
+
+    want = attend(tensor(device, q), lazy=False)
+    values(KC).copy_(old), values(VC).copy_(old)
+    assert torch.equal(attend(tensor(device, q), lazy=True), want)
