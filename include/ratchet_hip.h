@@ -341,12 +341,14 @@ RT_API rt_status rt_matmul_enqueue_ws(rt_ctx *ctx, const rt_matmul_desc *desc, c
  * tight serving loops, harnesses that forbid hipMalloc): the shares' partial sums go to a static
  * buffer of RT_STATIC_SCRATCH_BYTES that the library holds on each GPU it runs on, from
  * rt_ctx_create until the process ends.  Neither this call nor anything it launches allocates or
- * frees.  Products with f16 activations only: their results are those of rt_matmul_enqueue_ws with a
- * workspace of rt_matmul_workspace_bytes, bit for bit (the same kernels run).  A split that would need
- * more than the buffer holds is RT_ERR_UNSUPPORTED (on a device of up to 256 compute units none does);
- * a product that is not split, and every product with f32 activations, runs as rt_matmul_enqueue_fused
- * and touches no scratch.  All other calls on one GPU share the one buffer: those that can overlap there
- * (different streams, different contexts or threads) race; order them.
+ * frees.  For f16 activations against f16 or Q8_0H weights, K a multiple of 256, at least 2048, with
+ * equal shares of at least 1024, and output tiles of 160 x 128 for at most half of the compute units:
+ * their results are those of rt_matmul_enqueue_ws with a workspace of rt_matmul_workspace_bytes, bit
+ * for bit (the same kernels run).  A split that would need more than the buffer holds is
+ * RT_ERR_UNSUPPORTED (on a device of up to 256 compute units none does); every other product, and one
+ * that is not split, runs as rt_matmul_enqueue_fused and touches no scratch.  The calls that do share
+ * the one buffer of a GPU: those that can overlap there (different streams, different contexts or
+ * threads) race; order them.
  * No counterpart in the reference, whose operators never own scratch memory. */
 #define RT_STATIC_SCRATCH_BYTES (20u << 20)
 RT_API rt_status rt_matmul_enqueue_static(rt_ctx *ctx, const rt_matmul_desc *desc, const void *lhs, const void *rhs,

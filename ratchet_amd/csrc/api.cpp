@@ -437,9 +437,13 @@ rt_status rt_matmul_enqueue_static(rt_ctx *ctx, const rt_matmul_desc *desc, cons
     uint64_t need = 0;
     const rt_status st = rt_matmul_workspace_bytes(ctx, desc, &need);
     if (st != RT_OK) return st;
-    // Not split, or f32 activations: no scratch is touched.  f32 products never used the buffer, and a program may have them in
-    // flight on several streams at once.
-    if (need == 0 || (desc->lhs_dt != RT_F16 && desc->rhs_dt != RT_F16))
+    // Not split, or not one of the products the buffer is for (f32 activations and Q4_K weights are not): no scratch is touched, and a
+    // program may have them in flight on several streams at once.
+    rt_gemm_spec spec;
+    rt::Problem p;
+    std::string why;
+    if (need > 0 && rt::make_spec(*desc, spec, p, &why) != RT_OK) return fail(ctx, RT_ERR_INVALID_SHAPE, why);
+    if (need == 0 || (desc->lhs_dt != RT_F16 && desc->rhs_dt != RT_F16) || !rt::gemm_nt_static_split(p, ctx->dev))
         return rt_matmul_enqueue_ws(ctx, desc, lhs, rhs, bias, out, activation, nullptr, 0, stream);
     if (need > kStaticScratchBytes)
         return fail(ctx, RT_ERR_UNSUPPORTED,

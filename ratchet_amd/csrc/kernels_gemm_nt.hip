@@ -1549,6 +1549,20 @@ uint64_t gemm_nt_workspace_bytes(const Problem &p0, const DeviceInfo &dev) {
     return ks > 1 ? (uint64_t)p.stacks * ks * p.M * p.N * sizeof(float) : 0;
 }
 
+// Whether rt_matmul_enqueue_static may share this product's K, on the one buffer that all its calls on a GPU have in common.  A program
+// may have products in flight on several streams there that never touched it, so the products are those that it has always been for:
+// K whole units of 256, at most half a compute unit per 160 x 128 tile, and equal shares of at least 1024.
+bool gemm_nt_static_split(const Problem &p0, const DeviceInfo &dev) {
+    Problem p = p0;
+    nt_orient(p);
+    if ((p.a_dt != RT_F16 && p.a_dt != RT_Q8_0H) || p.K % 256 != 0) return false;
+    const int64_t tiles = ((p.M + 159) / 160) * ((p.N + 127) / 128) * p.stacks, units = p.K / 256;
+    if (tiles <= 0 || tiles * 2 > dev.num_cus) return false;
+    for (int ks = 2; ks <= 8 && tiles * ks <= dev.num_cus; ks++)
+        if (units % ks == 0 && units / ks >= 4) return true;
+    return false;
+}
+
 hipError_t launch_gemm_nt(const Problem &p0, const void *A, const void *B, const void *bias, void *out,
                           hipStream_t stream, const DeviceInfo &dev) {
     if (g_gemm_nt_disable) return hipErrorNotSupported;

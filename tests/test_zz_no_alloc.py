@@ -164,3 +164,36 @@ def test_products_with_f32_activations_never_touch_the_static_scratch(device, or
             run(L.rt_matmul_enqueue_static, x, out, stream)
     torch.cuda.synchronize()
     assert all(torch.equal(a, b) for a, b in zip(one, both))
+
+
+@pytest.mark.parametrize("wt,N,M,K", [("q4_k", 2560, 64, 10240), ("q8_0h", 3488, 118, 2592), ("f16", 4000, 23, 10656)])
+def test_products_outside_the_static_scratch(device, oracle, wt, N, M, K):
+    """Products that rt_matmul_enqueue_ws shares and that the static buffer is not for: in one pass, on two streams at once."""
+    rng = np.random.default_rng(6)
+    w = (rng.standard_normal((N, K)) * 0.05).astype(np.float32)
+    if wt == "q4_k":
+        blocks = rng.integers(0, 256, (N * K // 256, 144), dtype=np.uint8)
+        blocks[:, :4] = (rng.uniform(0.5, 2, (len(blocks), 2)) / 1024).astype(np.float16).view(np.uint8)
+        dw, dt = _dev(blocks), _ffi.RT_Q4_K
+    else:
+        dw, dt = (_dev(w.astype(np.float16)), _ffi.RT_F16) if wt == "f16" else (_dev(oracle.make_q8_0h(w)), _ffi.RT_Q8_0H)
+    xs = [_dev(rng.standard_normal((1, M, K)).astype(np.float16)) for _ in range(2)]
+    desc = _ffi.make_desc(dt, (N, K), _ffi.RT_F16, (1, M, K), False, True, True)
+    L, need = _ffi.lib(), ctypes.c_uint64()
+    assert L.rt_matmul_workspace_bytes(device.ctx, ctypes.byref(desc), ctypes.byref(need)) == _ffi.RT_OK and need.value > 0
+    streams = [torch.cuda.Stream() for _ in xs]
+
+    def run(fn, x, out, stream):
+        assert fn(device.ctx, ctypes.byref(desc), dw.data_ptr(), x.data_ptr(), None, ctypes.c_void_p(out.data_ptr()), _ffi.RT_ACT_NONE,
+                  ctypes.c_void_p(stream.cuda_stream)) == _ffi.RT_OK
+
+    one, both = ([torch.full((M * N,), float("nan"), dtype=torch.float16, device="cuda") for _ in xs] for _ in range(2))
+    torch.cuda.synchronize()
+    for x, out in zip(xs, one):
+        run(L.rt_matmul_enqueue_fused, x, out, streams[0])
+    torch.cuda.synchronize()
+    for _ in range(5):
+        for x, out, stream in zip(xs, both, streams):
+            run(L.rt_matmul_enqueue_static, x, out, stream)
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(one, both))
