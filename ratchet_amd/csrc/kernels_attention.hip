@@ -1013,6 +1013,8 @@ template <int MK, int THREADS> __global__ __launch_bounds__(THREADS) void attent
         for (int i = 0; i < AO_L; i++) {
             const float p = __builtin_amdgcn_exp2f(sc[i] - m_use);
             l += p;
+            // past the last key zeros: the last key again would make NaN of an infinite value, 0 * inf
+            if (key0 - grp + GROUPS * (i + 1) > g.kv_len && key0 + GROUPS * i >= g.kv_len) vr[i] = zero4;
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const uint32_t va = vr[i][e];
