@@ -339,24 +339,36 @@ POISON_OUTPUTS = False
 _strides3 = ctypes.c_int64 * 3
 
 
+def _overlap(x: "Tensor", y: "Tensor") -> bool:
+    """Whether two resolved GPU tensors share memory, by address: two tensors may wrap one allocation."""
+    a, b = x._ptr(), y._ptr()
+    return a < b + y.storage.nbytes and b < a + x.storage.nbytes
+
+
 def _write_key_and_value(k: "Tensor", v: "Tensor", stream: int):
     """Both cache writes of an attention in one launch, where its keys and values are the two in-place writes of one step that
-    nobody has run yet and the values' source reads nothing that the keys' write changes; anything else is left to run by itself."""
+    nobody has run yet; anything else is left to run by itself.  One by one they are: the keys' source, the keys' write, the values'
+    source, the values' write.  The launch runs both sources first and has no order between the two writes, so it is taken only where
+    the values' source neither reads what the keys' write changes nor writes a cache, and no write touches what the other reads or writes."""
     a, b = k.op, v.op
     if k.storage is not None or v.storage is not None or type(a) is not Cache or type(b) is not Cache or a.fresh or b.fresh:
         return
-    if (a.cache.storage is None or b.cache.storage is None or a.cache.storage is b.cache.storage or k.dt != v.dt or k.shape != v.shape
+    if (a.cache.storage is None or b.cache.storage is None or k.dt != v.dt or k.shape != v.shape
             or (a.offset, a.len, a.src_strides) != (b.offset, b.len, b.src_strides) or k.device is not v.device or k.device.kind != "gpu"):
         return
-    # the order of the operators stays what it is without this: the values' source runs behind the keys' write, unless all it
-    # reads is there already and is not that cache
-    if b.source.storage is None and any(s.storage is None or s.storage is a.cache.storage for s in b.source.op.srcs()):
+    if a.source.device.kind != "gpu" or b.source.device.kind != "gpu" or _overlap(a.cache, b.cache):
         return
-    for src in (a.source, b.source):
-        if src.storage is None:
-            src._execute(stream)
-        if src.device.kind != "gpu":
-            return
+    if b.source.storage is None and (type(b.source.op) is Cache or any(s.storage is None or s.device.kind != "gpu" or _overlap(s, a.cache)
+                                                                       for s in b.source.op.srcs())):
+        return
+    if a.source.storage is None:
+        a.source._execute(stream)
+    if v.storage is not None or _overlap(a.source, b.cache):   # (the keys' source may have read the new values)
+        return
+    if b.source.storage is None:
+        b.source._execute(stream)
+    if _overlap(b.source, a.cache):
+        return
     B, H, cap, D = a.cache.shape
     st = _ffi.lib().rt_cache_write_kv_enqueue(k.device.ctx, int(k.dt), a.cache._ptr(), a.source._ptr(), b.cache._ptr(), b.source._ptr(),
                                               _strides3(*a.src_strides), B, H, cap, a.offset, a.len, D, stream)

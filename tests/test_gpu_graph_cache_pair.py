@@ -84,3 +84,31 @@ def test_what_reads_the_caches_between_the_writes(device, reader):
     want = attend(tensor(device, q), lazy=False)
     values(KC).copy_(old), values(VC).copy_(old)
     assert torch.equal(attend(tensor(device, q), lazy=True), want)
+
+
+@pytest.mark.parametrize("reader", ["values are the key cache", "keys are the value cache", "keys are a write into the value cache", "values are a write into the keys",
+                                    "one memory for both"])
+def test_writes_whose_order_matters(device, reader):
+    """One cache is the other's source, or both are one memory in two tensors: as one write after the other leaves it."""
+    H, D, n = 4, 64, 256
+    gen = torch.Generator("cuda:0").manual_seed(9)
+    q, k, v, x, kc, vc = (torch.randn((1, H, n, D), generator=gen, device="cuda:0").half() for _ in range(6))
+
+    def attend(lazy):
+        step = (lambda t: t) if lazy else (lambda t: t.resolve())
+        memory = kc.clone()
+        KC, VC = tensor(device, memory), tensor(device, memory if reader == "one memory for both" else vc.clone())
+        keys, vals = tensor(device, k.clone()), tensor(device, v)
+        if reader == "values are the key cache":
+            vals = KC
+        if reader == "keys are the value cache":
+            keys = VC
+        if reader == "keys are a write into the value cache":
+            keys = step(VC.cache_write(tensor(device, x), 0))
+        written = step(KC.cache_write(keys, 0))
+        if reader == "values are a write into the keys":
+            vals = step(keys.cache_write(tensor(device, x), 0))
+        out = tensor(device, q).attention(written, step(VC.cache_write(vals, 0))).resolve()
+        return [values(t).clone() for t in (out, KC, VC)]
+
+    assert all(torch.equal(a, b) for a, b in zip(attend(lazy=True), attend(lazy=False)))
