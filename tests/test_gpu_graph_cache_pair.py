@@ -68,8 +68,8 @@ def test_what_reads_the_caches_between_the_writes(device, reader):
     """Queries from an attention over the same caches run before the writes, and values made of the key cache behind the keys' write."""
     H, D, n = 2, 64, 16
     gen = torch.Generator("cuda:0").manual_seed(5)
-    q, k1, v1, k2, v2, old = (torch.randn((1, H, n, D), generator=gen, device="cuda:0").half() for _ in range(6))
-    KC, VC = tensor(device, old), tensor(device, old)
+    q, k1, v1, k2, v2, k0, v0 = (torch.randn((1, H, n, D), generator=gen, device="cuda:0").half() for _ in range(7))
+    KC, VC = tensor(device, k0.clone()), tensor(device, v0.clone())
 
     def attend(first, lazy):
         step = (lambda t: t) if lazy else (lambda t: t.resolve())
@@ -82,7 +82,7 @@ def test_what_reads_the_caches_between_the_writes(device, reader):
         return values(q2.attention(written, step(VC.cache_write(vals, 0))).resolve()).clone()
 
     want = attend(tensor(device, q), lazy=False)
-    values(KC).copy_(old), values(VC).copy_(old)
+    values(KC).copy_(k0), values(VC).copy_(v0)
     assert torch.equal(attend(tensor(device, q), lazy=True), want)
 
 
