@@ -869,6 +869,20 @@ __device__ __forceinline__ float ad_row_sum(float v) {
     return v;
 }
 
+// Loads with a bound: past `bytes` the hardware returns zeros.  Rows of values past the last key are read so, at no instruction more than
+// the clamp of the others; the last key again, at probability zero, would make NaN of an infinite value (0 * inf).  (32 heads x 80, one row, the
+// values of loads past the end against a test per key behind them: 128 / 300 / 448 keys 3.23 / 5.10 / 5.09 -> 3.08 / 4.85 / 4.85 us; 1331 / 2048 in two
+// launches, which had no test, 6.82 / 7.15 -> 6.82 / 6.94, with an f16 mask 8.07 / 8.45 -> 6.97 / 7.29.)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t ad_bounded(const void *p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, 0x00027000); // raw, 32-bit data
+}
+// bytes from a head's values to the end of its last key's row (the launcher keeps them within 2^32)
+__device__ __forceinline__ uint32_t ad_value_bytes(const AttnArgs &g) { return 2u * ((uint32_t)(g.kv_len - 1) * (uint32_t)g.v_rs + (uint32_t)g.D); }
+__device__ __forceinline__ uint4_t ad_value(__amdgpu_buffer_rsrc_t v, const AttnArgs &g, int key, int segc) {
+    constexpr int NT = 2; // cache policy: non-temporal
+    return __builtin_bit_cast(uint4_t, __builtin_amdgcn_raw_buffer_load_b128(v, (int)(2u * ((uint32_t)min(key, g.kv_len) * (uint32_t)g.v_rs + 8u * (uint32_t)segc)), 0, NT));
+}
+
 // the mask value of a key in base-2 units (one query row: the mask's first)
 template <int MK> __device__ __forceinline__ float ad_mask(const void *mask, uint32_t key) {
     if constexpr (MK == 0) return 0.f;
@@ -887,7 +901,7 @@ template <int MK> __global__ __launch_bounds__(AD_THREADS) void attention_decode
     const int split = blockIdx.x, bh = blockIdx.y, b = bh / g.heads, h = bh - b * g.heads;
     const half_t *Q = g.Q + b * g.q_bs + h * g.q_hs;
     const half_t *K = g.K + b * g.k_bs + h * g.k_hs;
-    const half_t *V = g.V + b * g.v_bs + h * g.v_hs;
+    const auto V = ad_bounded(g.V + b * g.v_bs + h * g.v_hs, ad_value_bytes(g));
     const uint4_t zero4 = {0u, 0u, 0u, 0u};
     const int key0 = split * AD_KEYS + slot;
 
@@ -898,10 +912,7 @@ template <int MK> __global__ __launch_bounds__(AD_THREADS) void attention_decode
         kr[i] = __builtin_nontemporal_load((const uint4_t *)(K + (kc * (uint32_t)g.k_rs + 8u * segc)));
     }
 #pragma unroll
-    for (int i = 0; i < AD_L; i++) {
-        const uint32_t kc = (uint32_t)min(key0 + 16 * i, g.kv_len - 1);
-        vr[i] = __builtin_nontemporal_load((const uint4_t *)(V + (kc * (uint32_t)g.v_rs + 8u * segc)));
-    }
+    for (int i = 0; i < AD_L; i++) vr[i] = ad_value(V, g, key0 + 16 * i, segc);
     float mk[AD_L];
 #pragma unroll
     for (int i = 0; i < AD_L; i++) mk[i] = ad_mask<MK>(g.mask, (uint32_t)min(key0 + 16 * i, g.kv_len - 1));
@@ -972,7 +983,7 @@ template <int MK, int THREADS> __global__ __launch_bounds__(THREADS) void attent
     const int ns = g.D >> 3, segc = min(seg, ns - 1); // idle lanes repeat the last live lane's addresses and contribute zeros
     const int bh = blockIdx.x, b = bh / g.heads, h = bh - b * g.heads;
     const half_t *K = g.K + b * g.k_bs + h * g.k_hs;
-    const half_t *V = g.V + b * g.v_bs + h * g.v_hs;
+    const auto V = ad_bounded(g.V + b * g.v_bs + h * g.v_hs, ad_value_bytes(g));
     const uint4_t zero4 = {0u, 0u, 0u, 0u};
     uint4_t qv = *(const uint4_t *)(g.Q + b * g.q_bs + h * g.q_hs + 8 * segc);
     uint4_t kr[AO_L], vr[AO_L];
@@ -987,7 +998,8 @@ template <int MK, int THREADS> __global__ __launch_bounds__(THREADS) void attent
     if (seg >= ns) qv = zero4;
     float m = -INFINITY, l = 0.f, acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     for (int key0 = grp; key0 - grp < g.kv_len; key0 += KEYS) {
-        load(vr, V, (uint32_t)g.v_rs, key0);
+#pragma unroll
+        for (int i = 0; i < AO_L; i++) vr[i] = ad_value(V, g, key0 + GROUPS * i, segc);
         float sc[AO_L], m_new = m;
 #pragma unroll
         for (int i = 0; i < AO_L; i++) {
@@ -1013,8 +1025,6 @@ template <int MK, int THREADS> __global__ __launch_bounds__(THREADS) void attent
         for (int i = 0; i < AO_L; i++) {
             const float p = __builtin_amdgcn_exp2f(sc[i] - m_use);
             l += p;
-            // past the last key zeros: the last key again would make NaN of an infinite value, 0 * inf
-            if (key0 - grp + GROUPS * (i + 1) > g.kv_len && key0 + GROUPS * i >= g.kv_len) vr[i] = zero4;
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const uint32_t va = vr[i][e];
@@ -1057,7 +1067,8 @@ template <int MK, int THREADS> __global__ __launch_bounds__(THREADS) void attent
 // One workgroup per head: thread d combines dimension d of the head's splits.
 __global__ __launch_bounds__(128) void attention_decode_merge_kernel(AttnArgs g) {
     const int bh = blockIdx.x, b = bh / g.heads, h = bh - b * g.heads, d = threadIdx.x;
-    const float *base = g.partial + (size_t)bh * g.splits * AD_PSTRIDE;
+    const auto base = ad_bounded(g.partial + (size_t)bh * g.splits * AD_PSTRIDE, (uint32_t)g.splits * AD_PSTRIDE * 4u);
+    auto at = [&](int split, int i) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(base, (split * AD_PSTRIDE + i) * 4, 0, 0)); };
     // (maximum, sum, output) over the splits, sixteen splits' values requested at a time: the partial results come
     // from other XCDs' workgroups, so every round of loads is a trip to memory, and a cache of 2048 keys is one round.
     // Within a round the sixteen weights are independent of each other (one maximum first, then sixteen
@@ -1068,8 +1079,8 @@ __global__ __launch_bounds__(128) void attention_decode_merge_kernel(AttnArgs g)
         float ms[16], ls[16], os[16];
 #pragma unroll
         for (int u = 0; u < 16; u++) {
-            const float *ps = base + (size_t)min(s0 + u, g.splits - 1) * AD_PSTRIDE; // past the last split: re-read it, weight 0 below
-            ms[u] = s0 + u < g.splits ? ps[0] : -INFINITY, ls[u] = ps[1], os[u] = ps[4 + dc];
+            const float mu = at(s0 + u, 0); // past the last split zeros: with weight 0
+            ms[u] = s0 + u < g.splits ? mu : -INFINITY, ls[u] = at(s0 + u, 1), os[u] = at(s0 + u, 4 + dc);
         }
         float m_new = m;
 #pragma unroll
@@ -1208,7 +1219,8 @@ hipError_t launch_attention(const rt_attention_desc &d, const void *q, const voi
         return hipErrorNotSupported;
     // one query row: a stream over the keys and values, in one launch or, against a long cache and with the workspace for
     // it, split over workgroups
-    if (d.q_len == 1 && d.kv_len > 0 && d.head_dim % 8 == 0 && d.head_dim <= 128) {
+    // (its bounded loads count bytes in 32 bits up to one row of 128 past the last key)
+    if (d.q_len == 1 && d.kv_len > 0 && d.head_dim % 8 == 0 && d.head_dim <= 128 && (int64_t)d.kv_len * g.v_rs + 128 < (int64_t(1) << 31)) {
         const int mk = !mask ? 0 : g.mask_f32 ? 1 : 2, ds = attention_decode_splits(d);
         const bool can_split = ds > 0 && ds <= 65535 && workspace && !((uintptr_t)workspace & 15u) && workspace_bytes >= attention_decode_workspace_bytes(d);
         if (d.kv_len <= kDecodeOneKeys) {

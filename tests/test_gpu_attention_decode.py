@@ -74,14 +74,16 @@ def test_merge_of_split_launches(device, heads, head_dim, rows, keys):
     check(device, heads, head_dim, rows, keys, causal=True, probability=2.0**-11)
 
 
-@pytest.mark.parametrize("keys", [1, 64, 100, 200, 256, 300, 448])
-def test_infinite_value_at_the_last_key(device, keys):
-    """What the one-launch kernel reads in place of keys past the last one leaves no NaN: an infinite value stays infinite."""
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("keys", [1, 64, 100, 200, 256, 300, 448, 449, 512, 576, 700])
+def test_infinite_value_at_the_last_key(device, keys, masked):
+    """What the kernels read in place of keys past the last one leaves no NaN: an infinite value stays infinite."""
     gen = torch.Generator("cuda:0").manual_seed(keys)
     q = torch.randn((1, 2, 1, 64), generator=gen, device="cuda:0").half()
     k, v = (torch.randn((1, 2, keys, 64), generator=gen, device="cuda:0").half() for _ in range(2))
     v[:, :, -1, 3], v[:, :, -1, 60] = float("inf"), float("-inf")
-    got = tensor(device, q).attention(tensor(device, k), tensor(device, v), None).resolve().storage.view(torch.float16)[:128].view(2, 64)
+    mask = tensor(device, torch.zeros((1, keys), device="cuda:0")) if masked else None
+    got = tensor(device, q).attention(tensor(device, k), tensor(device, v), mask).resolve().storage.view(torch.float16)[:128].view(2, 64)
     assert (got[:, 3] == float("inf")).all() and (got[:, 60] == float("-inf")).all()
     finite = torch.ones(64, dtype=torch.bool, device="cuda:0")
     finite[3] = finite[60] = False
