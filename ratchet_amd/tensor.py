@@ -272,7 +272,7 @@ class Attention:
         d.k_strides[:] = [H * cap * D, cap * D, D]
         d.v_strides[:] = [H * cap * D, cap * D, D]
         d.o_strides[:] = [Lq * H * D, D, H * D] if merge_heads else [H * Lq * D, Lq * D, D]
-        d.scale = 1.0 / math.sqrt(D) if scale is None else float(scale)
+        d.scale = (1.0 / math.sqrt(D) if D > 0 else 1.0) if scale is None else float(scale)   # (no head_dim: refused as a shape)
         d.causal = int(self.causal)
         d.mask_dtype = int(mask.dt) if mask is not None else int(DType.F32)
         d.mask_row_stride = self.kv_len

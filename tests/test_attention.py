@@ -124,6 +124,13 @@ def test_guards_without_a_device():
         Tensor.from_data(np.zeros((1, 2, 4, 16), np.float32)).attention(q, q)
 
 
+def test_no_head_dim_is_an_invalid_shape():
+    q = Tensor.from_data(np.zeros((1, 2, 4, 0), np.float16))
+    with pytest.raises(InvariantError) as error:
+        q.attention(q, q)
+    assert error.value.status == _ffi.RT_ERR_INVALID_SHAPE
+
+
 # ---------------------------------------------------------------------------
 # GPU
 # ---------------------------------------------------------------------------
