@@ -1099,10 +1099,16 @@ __global__ __launch_bounds__(128) void attention_decode_merge_kernel(AttnArgs g)
     if (d < g.D) g.O[b * g.o_bs + h * g.o_hs + d] = (half_t)(o / l); // no visible key anywhere: 0 / 0 = NaN, as in the single pass
 }
 
-// Keys up to which a decode step runs in one launch.  32 heads x 80, one launch against two (up to 255 keys, against the tiled
-// kernel): 64 keys 3.6 and 4.3 us, 128 3.6 / 4.8, 255 4.0 / 7.9, 300 5.1 / 5.6, 400 5.7 / 5.9, 512 6.0 / 5.8 (16 heads x 128: 6.6 / 5.6).  A mask
-// tensor, which the two-launch kernel did not take before, adds 0.1 to 0.4 us (300 keys: 11.8 -> 5.7).
+// Whether a decode step runs in one launch though it may run in two.  A workgroup pulls a whole head's keys and values through one
+// compute unit, so the line is at what they are (keys x head_dim), unless the heads fill the device.  us, one launch and two: 32 heads x 80,
+// 257 / 384 / 448 keys 4.84 / 4.85 / 4.86 and 5.23 / 5.23 / 5.18; 16 x 128 at 257 / 384 / 416 5.08 / 4.80 / 5.49 and 5.33 / 5.23 / 5.21; 32 x 128 at
+// 290 / 384 / 448 5.22 / 5.66 / 6.45 and 5.26 / 5.31 / 5.59; 40 x 96 at 352 / 416 5.49 / 5.81 and 5.38 / 5.48; 256 x 128 at 257 / 448 8.49 / 10.50
+// and 8.83 / 12.11.  512 keys: 6.0 and 5.8 at 32 x 80.  Against the tiled kernel, which took fewer than 256 keys: 32 x 80 at 64 / 128 / 255 keys 3.1 /
+// 3.1 / 3.6 and 4.3 / 4.8 / 7.9.  A mask tensor adds 0.1 to 0.4 us to either.
 constexpr int kDecodeOneKeys = 448;
+static bool attention_decode_one(const rt_attention_desc &d) {
+    return d.kv_len <= 256 || (d.kv_len <= kDecodeOneKeys && (d.kv_len * d.head_dim <= 36 * 1024 || (int64_t)d.batch * d.heads >= 256));
+}
 template <int MK> static void launch_decode_one(const AttnArgs &g, unsigned stacks, hipStream_t st) {
     if (g.kv_len <= 128) hipLaunchKernelGGL((attention_decode_one_kernel<MK, 256>), dim3(stacks), dim3(256), 0, st, g);
     else if (g.kv_len <= 256) hipLaunchKernelGGL((attention_decode_one_kernel<MK, 512>), dim3(stacks), dim3(512), 0, st, g);
@@ -1218,12 +1224,12 @@ hipError_t launch_attention(const rt_attention_desc &d, const void *q, const voi
     if ((int64_t)d.kv_len * g.k_rs >= (int64_t(1) << 31) || (int64_t)d.kv_len * g.v_rs >= (int64_t(1) << 31))
         return hipErrorNotSupported;
     // one query row: a stream over the keys and values, in one launch or, against a long cache and with the workspace for
-    // it, split over workgroups
+    // it, split over workgroups (without one, a single launch up to as many keys as it takes)
     // (its bounded loads count bytes in 32 bits up to one row of 128 past the last key)
     if (d.q_len == 1 && d.kv_len > 0 && d.head_dim % 8 == 0 && d.head_dim <= 128 && (int64_t)d.kv_len * g.v_rs + 128 < (int64_t(1) << 31)) {
         const int mk = !mask ? 0 : g.mask_f32 ? 1 : 2, ds = attention_decode_splits(d);
         const bool can_split = ds > 0 && ds <= 65535 && workspace && !((uintptr_t)workspace & 15u) && workspace_bytes >= attention_decode_workspace_bytes(d);
-        if (d.kv_len <= kDecodeOneKeys) {
+        if (attention_decode_one(d) || (!can_split && d.kv_len <= kDecodeOneKeys)) {
             if (mk == 0) launch_decode_one<0>(g, (unsigned)stacks, stream);
             else if (mk == 1) launch_decode_one<1>(g, (unsigned)stacks, stream);
             else launch_decode_one<2>(g, (unsigned)stacks, stream);
