@@ -971,12 +971,10 @@ template <int MK> __global__ __launch_bounds__(AD_THREADS) void attention_decode
 
 // The same in one launch, for caches that one workgroup per head streams faster than two launches follow each other: a
 // thread count for up to 128, 256 and 512 keys, all of which are requested at once.  A group of 16 lanes keeps the maximum, sum and
-// output of its own keys, so no wavefront waits for another before the end; there the groups meet in LDS.  (Rounds of 512 keys
-// are right for any number of them, and slower than two launches: 32 heads x 80, 700 / 1024 / 2048 keys 7.4 / 8.0 / 15.1 us for
-// 6.0 / 5.8 / 7.0.)
+// output of its own keys, so no wavefront waits for another before the end; there the groups meet in LDS.
 constexpr int AO_L = 8;
-template <int MK, int THREADS> __global__ __launch_bounds__(THREADS) void attention_decode_one_kernel(AttnArgs g) {
-    constexpr int GROUPS = THREADS / 16, KEYS = GROUPS * AO_L, PARTS = THREADS / 128; // PARTS of GROUPS / PARTS = 8 groups each
+template <int MK, int THREADS> __global__ __launch_bounds__(THREADS) void attention_decode_one_kernel(AttnArgs g) { // kv_len <= THREADS / 2
+    constexpr int GROUPS = THREADS / 16, PARTS = THREADS / 128; // PARTS of GROUPS / PARTS = 8 groups each
     __shared__ float sm[GROUPS], sl[GROUPS];
     __shared__ __attribute__((aligned(16))) float so[GROUPS][16][8]; // [group][seg][8 dimensions]; afterwards [PARTS][128] partial sums
     const int t = threadIdx.x, seg = t & 15, grp = t >> 4;
@@ -984,56 +982,43 @@ template <int MK, int THREADS> __global__ __launch_bounds__(THREADS) void attent
     const int bh = blockIdx.x, b = bh / g.heads, h = bh - b * g.heads;
     const half_t *K = g.K + b * g.k_bs + h * g.k_hs;
     const auto V = ad_bounded(g.V + b * g.v_bs + h * g.v_hs, ad_value_bytes(g));
-    const uint4_t zero4 = {0u, 0u, 0u, 0u};
     uint4_t qv = *(const uint4_t *)(g.Q + b * g.q_bs + h * g.q_hs + 8 * segc);
     uint4_t kr[AO_L], vr[AO_L];
-    auto load = [&](uint4_t (&r)[AO_L], const half_t *p, uint32_t rs, int key0) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < AO_L; i++) {
-            const uint32_t kc = (uint32_t)min(key0 + GROUPS * i, g.kv_len - 1); // past the last key: a valid one, masked below
-            r[i] = __builtin_nontemporal_load((const uint4_t *)(p + (kc * rs + 8u * segc)));
+    for (int i = 0; i < AO_L; i++) {
+        const uint32_t kc = (uint32_t)min(grp + GROUPS * i, g.kv_len - 1); // past the last key: a valid one, masked below
+        kr[i] = __builtin_nontemporal_load((const uint4_t *)(K + (kc * (uint32_t)g.k_rs + 8u * segc)));
+    }
+#pragma unroll
+    for (int i = 0; i < AO_L; i++) vr[i] = ad_value(V, g, grp + GROUPS * i, segc);
+    if (seg >= ns) qv = uint4_t{0u, 0u, 0u, 0u};
+    float sc[AO_L], m = -INFINITY, l = 0.f, acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < AO_L; i++) {
+        const int key = grp + GROUPS * i;
+        float p = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const uint32_t qa = qv[e], ka = kr[i][e];
+            p = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, qa), __builtin_bit_cast(half2_t, ka), p, false);
         }
-    };
-    load(kr, K, (uint32_t)g.k_rs, grp);
-    if (seg >= ns) qv = zero4;
-    float m = -INFINITY, l = 0.f, acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int key0 = grp; key0 - grp < g.kv_len; key0 += KEYS) {
+        p = ad_row_sum(p) * g.scale_log2e;
+        if (MK) p += ad_mask<MK>(g.mask, (uint32_t)min(key, g.kv_len - 1));
+        sc[i] = key < g.kv_len ? p : -INFINITY;
+        m = fmaxf(m, sc[i]);
+    }
+    const float m_use = m == -INFINITY ? 0.f : m; // no visible key here: every weight is exp2(-inf) = 0
 #pragma unroll
-        for (int i = 0; i < AO_L; i++) vr[i] = ad_value(V, g, key0 + GROUPS * i, segc);
-        float sc[AO_L], m_new = m;
+    for (int i = 0; i < AO_L; i++) {
+        const float p = __builtin_amdgcn_exp2f(sc[i] - m_use);
+        l += p;
 #pragma unroll
-        for (int i = 0; i < AO_L; i++) {
-            const int key = key0 + GROUPS * i;
-            float p = 0.f;
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const uint32_t qa = qv[e], ka = kr[i][e];
-                p = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, qa), __builtin_bit_cast(half2_t, ka), p, false);
-            }
-            p = ad_row_sum(p) * g.scale_log2e;
-            if (MK) p += ad_mask<MK>(g.mask, (uint32_t)min(key, g.kv_len - 1));
-            sc[i] = key < g.kv_len ? p : -INFINITY;
-            m_new = fmaxf(m_new, sc[i]);
+        for (int e = 0; e < 4; e++) {
+            const uint32_t va = vr[i][e];
+            const half2_t v2 = __builtin_bit_cast(half2_t, va);
+            acc[2 * e] = fmaf(p, (float)v2[0], acc[2 * e]);
+            acc[2 * e + 1] = fmaf(p, (float)v2[1], acc[2 * e + 1]);
         }
-        if (key0 - grp + KEYS < g.kv_len) load(kr, K, (uint32_t)g.k_rs, key0 + KEYS);
-        const float m_use = m_new == -INFINITY ? 0.f : m_new; // no visible key yet: every weight is exp2(-inf) = 0
-        const float a = __builtin_amdgcn_exp2f(m - m_use);
-        l *= a;
-#pragma unroll
-        for (int e = 0; e < 8; e++) acc[e] *= a;
-#pragma unroll
-        for (int i = 0; i < AO_L; i++) {
-            const float p = __builtin_amdgcn_exp2f(sc[i] - m_use);
-            l += p;
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const uint32_t va = vr[i][e];
-                const half2_t v2 = __builtin_bit_cast(half2_t, va);
-                acc[2 * e] = fmaf(p, (float)v2[0], acc[2 * e]);
-                acc[2 * e + 1] = fmaf(p, (float)v2[1], acc[2 * e + 1]);
-            }
-        }
-        m = m_new;
     }
     if (seg == 0) sm[grp] = m, sl[grp] = l;
     *(float4_t *)&so[grp][seg][0] = float4_t{acc[0], acc[1], acc[2], acc[3]};
@@ -1103,7 +1088,7 @@ __global__ __launch_bounds__(128) void attention_decode_merge_kernel(AttnArgs g)
 // compute unit, so the line is at what they are (keys x head_dim), unless the heads fill the device.  us, one launch and two: 32 heads x 80,
 // 257 / 384 / 448 keys 4.84 / 4.85 / 4.86 and 5.23 / 5.23 / 5.18; 16 x 128 at 257 / 384 / 416 5.08 / 4.80 / 5.49 and 5.33 / 5.23 / 5.21; 32 x 128 at
 // 290 / 384 / 448 5.22 / 5.66 / 6.45 and 5.26 / 5.31 / 5.59; 40 x 96 at 352 / 416 5.49 / 5.81 and 5.38 / 5.48; 256 x 128 at 257 / 448 8.49 / 10.50
-// and 8.83 / 12.11.  512 keys: 6.0 and 5.8 at 32 x 80.  Against the tiled kernel, which took fewer than 256 keys: 32 x 80 at 64 / 128 / 255 keys 3.1 /
+// and 8.83 / 12.11.  512 keys: 6.0 and 5.8 at 32 x 80; in rounds of 512, 700 / 1024 / 2048 keys: 7.4 / 8.0 / 15.1 and 6.0 / 5.8 / 7.0.  Against the tiled kernel, which took fewer than 256 keys: 32 x 80 at 64 / 128 / 255 keys 3.1 /
 // 3.1 / 3.6 and 4.3 / 4.8 / 7.9.  A mask tensor adds 0.1 to 0.4 us to either.
 constexpr int kDecodeOneKeys = 448;
 static bool attention_decode_one(const rt_attention_desc &d) {
