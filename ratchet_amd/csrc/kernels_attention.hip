@@ -1175,12 +1175,16 @@ int attention_splits(const rt_attention_desc &d) {
     return s < 2 ? 1 : s;
 }
 
-// bytes of workspace a split launch of this problem needs (0: it runs in one pass)
-uint64_t attention_workspace_bytes(const rt_attention_desc &d) {
+// bytes of workspace a split launch of the tiled kernel needs for this problem (0: it runs in one pass)
+static uint64_t attention_tiled_workspace_bytes(const rt_attention_desc &d) {
     const int s = attention_splits(d);
     const uint64_t qb = (uint64_t)((d.q_len + AT_BQ - 1) / AT_BQ);
-    const uint64_t tiled = s <= 1 ? 0 : qb * (uint64_t)d.batch * d.heads * s * AT_BQ * (4 + attention_dp(d.head_dim)) * sizeof(float);
-    return std::max(tiled, attention_decode_workspace_bytes(d)); // whichever of the two split paths the launch takes
+    return s <= 1 ? 0 : qb * (uint64_t)d.batch * d.heads * s * AT_BQ * (4 + attention_dp(d.head_dim)) * sizeof(float);
+}
+// bytes of workspace with which a launch of this problem shares its keys: one query row takes the tiled kernel with it only beyond the
+// splits that the other's grid has
+uint64_t attention_workspace_bytes(const rt_attention_desc &d) {
+    return d.q_len == 1 && attention_decode_splits(d) <= 65535 ? attention_decode_workspace_bytes(d) : attention_tiled_workspace_bytes(d);
 }
 
 // f16 tensors, head_dim a multiple of 8 up to 128, rows 16-byte aligned.  `workspace` may be null
@@ -1201,7 +1205,7 @@ hipError_t launch_attention(const rt_attention_desc &d, const void *q, const voi
     g.splits = 1, g.partial = nullptr;
     // (Below eight key blocks one pass is faster still -- 8 heads x 400 x 400 x 80 8.8 us, three splits 10.0 -- and rounds more: 2.66e-4
     // against 2.58e-4 from the exact result, because each split rounds its probabilities against a maximum of its own.)
-    if (const uint64_t need = attention_workspace_bytes(d); need > 0 && workspace && workspace_bytes >= need && !((uintptr_t)workspace & 15u))
+    if (const uint64_t need = attention_tiled_workspace_bytes(d); need > 0 && workspace && workspace_bytes >= need && !((uintptr_t)workspace & 15u))
         g.splits = attention_splits(d), g.partial = (float *)workspace;
     const int64_t stacks = (int64_t)d.batch * d.heads;
     if (stacks > 65535) return hipErrorNotSupported;

@@ -124,6 +124,19 @@ def test_guards_without_a_device():
         Tensor.from_data(np.zeros((1, 2, 4, 16), np.float32)).attention(q, q)
 
 
+@pytest.mark.parametrize("rows,keys,floats", [
+    (1, 200, 0), (1, 255, 0),                        # one launch, no workspace
+    (1, 300, 3 * 132), (1, 2048, 16 * 132),          # what the streaming kernel's workgroups leave: nothing for the tiled kernel's 64 rows
+    (2, 200, 2 * 64 * (4 + 96)), (1, 128 * 65536, 16 * 64 * (4 + 96))])
+def test_workspace_is_that_of_the_kernel_that_runs(rows, keys, floats):
+    d, need = _ffi.AttentionDesc(), ctypes.c_uint64()
+    d.dtype, d.batch, d.heads, d.q_len, d.kv_len, d.head_dim, d.scale = _ffi.RT_F16, 1, 3, rows, keys, 80, 0.1
+    for s in (d.q_strides, d.k_strides, d.v_strides, d.o_strides):
+        s[:] = [0, 80, 240]
+    assert _ffi.lib().rt_attention_workspace_bytes(ctypes.byref(d), ctypes.byref(need)) == _ffi.RT_OK
+    assert need.value == 3 * 4 * floats
+
+
 def test_no_head_dim_is_an_invalid_shape():
     q = Tensor.from_data(np.zeros((1, 2, 4, 0), np.float16))
     with pytest.raises(InvariantError) as error:
