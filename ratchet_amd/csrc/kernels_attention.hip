@@ -869,7 +869,7 @@ __device__ __forceinline__ float ad_row_sum(float v) {
     return v;
 }
 
-// Loads with a bound: past `bytes` the hardware returns zeros.  Rows of values past the last key are read so, at no instruction more than
+// Loads with a bound: past `bytes` the hardware returns zeros.  Rows of values past the last key are read so, at one instruction more than
 // the clamp of the others; the last key again, at probability zero, would make NaN of an infinite value (0 * inf).  (32 heads x 80, one row, the
 // values of loads past the end against a test per key behind them: 128 / 300 / 448 keys 3.23 / 5.10 / 5.09 -> 3.08 / 4.85 / 4.85 us; 1331 / 2048 in two
 // launches, which had no test, 6.82 / 7.15 -> 6.82 / 6.94, with an f16 mask 8.07 / 8.45 -> 6.97 / 7.29.)
@@ -878,9 +878,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t ad_bounded(const void *p, uint
 }
 // bytes from a head's values to the end of its last key's row (the launcher keeps them within 2^32)
 __device__ __forceinline__ uint32_t ad_value_bytes(const AttnArgs &g) { return 2u * ((uint32_t)(g.kv_len - 1) * (uint32_t)g.v_rs + (uint32_t)g.D); }
+// A key past the last one is asked for at that end and not at its own row, which lies inside where rows share memory (v_rs < D, 0 for one
+// row of values for all keys).
 __device__ __forceinline__ uint4_t ad_value(__amdgpu_buffer_rsrc_t v, const AttnArgs &g, int key, int segc) {
     constexpr int NT = 2; // cache policy: non-temporal
-    return __builtin_bit_cast(uint4_t, __builtin_amdgcn_raw_buffer_load_b128(v, (int)(2u * ((uint32_t)min(key, g.kv_len) * (uint32_t)g.v_rs + 8u * (uint32_t)segc)), 0, NT));
+    const uint32_t at = key < g.kv_len ? 2u * ((uint32_t)key * (uint32_t)g.v_rs + 8u * (uint32_t)segc) : ad_value_bytes(g);
+    return __builtin_bit_cast(uint4_t, __builtin_amdgcn_raw_buffer_load_b128(v, (int)at, 0, NT));
 }
 
 // the mask value of a key in base-2 units (one query row: the mask's first)

@@ -88,3 +88,21 @@ def test_infinite_value_at_the_last_key(device, keys, masked):
     finite = torch.ones(64, dtype=torch.bool, device="cuda:0")
     finite[3] = finite[60] = False
     assert got[:, finite].isfinite().all()
+
+
+@pytest.mark.parametrize("stride", [0, 8])
+@pytest.mark.parametrize("keys", [100, 300, 700])
+def test_infinite_value_where_rows_share_memory(device, keys, stride):
+    """Rows of values that begin less than a row apart: a row past the last key would lie inside the values, and leaves no NaN either."""
+    gen = torch.Generator("cuda:0").manual_seed(keys)
+    q, k, v = (torch.randn(s, generator=gen, device="cuda:0").half() for s in ((1, 2, 1, 64), (1, 2, keys, 64), (1, 2, keys, 64)))
+    last = (keys - 1) * stride + 63
+    v.view(2, -1)[:, last] = float("inf")
+    node = tensor(device, q).attention(tensor(device, k), tensor(device, v), None)
+    node.op.desc.v_strides[2] = stride
+    got = node.resolve().storage.view(torch.float16)[:128].view(2, 64)
+    rows = v.as_strided((2, keys, 64), (keys * 64, stride, 1)).double()
+    p = torch.softmax((k[0].double() @ q[0].double().transpose(1, 2).contiguous()).transpose(1, 2) / 8, -1)
+    assert (got[:, 63] == float("inf")).all()
+    want, mag = ((p[:, 0, :, None] * r).sum(1) for r in (rows[..., :63], rows[..., :63].abs()))
+    assert ((got[:, :63].double() - want).abs() <= 2.0**-11 * want.abs() + (2.0**-20 + 2.0**-19) * mag + 2.0**-25).all()
