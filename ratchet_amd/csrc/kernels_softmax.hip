@@ -140,7 +140,12 @@ template <typename T> static hipError_t launch_softmax_t(void *x, int64_t rows, 
     if (rows == 0 || n == 0) return hipSuccess;
     const bool whole = n % EV == 0 && ((uintptr_t)x & 15u) == 0;
     const int64_t nvec = whole ? n / EV : (n + 2 * EV - 2) / EV; // vectors a row touches at the most
-    if (nvec <= 64 * 8 && (whole || n >= 128)) {
+    // Rows that do not begin on 16 bytes: a wavefront per row pays its edges where rows are few, and the workgroup per row of the other kernel
+    // then has them all in flight at once.  us, f32 there and here: 512 x 333 3.75 / 4.34, 1024 x 333 4.10 / 4.44, 1024 x 1001 5.95 / 5.72, 1800 x 333
+    // 4.81 / 4.95, 2200 x 133 / 333 4.24 / 4.12 and 5.71 / 5.35; f16: 512 x 133 3.24 / 4.02, 768 x 701 4.56 / 5.03, 1024 x 133 / 333 / 1001 3.41 / 4.07,
+    // 4.22 / 4.13 and 5.68 / 5.05, 2200 x 203 4.59 / 4.78, 3000 x 133 4.84 / 4.81.
+    const bool many = n >= 128 && rows >= (n >= (EV == 8 ? 320 : 1000) ? 1024 : EV == 8 ? 3000 : 2048);
+    if (nvec <= 64 * 8 && (whole || many)) {
         const int64_t blocks = (rows + 3) / 4;
         if (blocks > 0x7fffffff) return hipErrorInvalidValue;
         auto rows_of = [&](auto VPL) {

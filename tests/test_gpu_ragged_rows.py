@@ -33,6 +33,12 @@ def test_probabilities_times_values(device, heads, rows, keys, head_dim):
     close(got, p.double() @ v.double(), p.double().abs() @ v.double().abs(), keys)
 
 
+@pytest.mark.parametrize("heads,rows,keys,head_dim", [(2, 65, k, n) for k, n in ((31, 48), (33, 48), (63, 56), (65, 96), (127, 104), (129, 128))] +
+                         [(32, 577, k, n) for k, n in ((95, 56), (97, 96), (159, 48), (161, 40), (159, 104), (161, 128))])
+def test_probabilities_times_values_on_both_sides_of_the_rule(device, heads, rows, keys, head_dim):
+    test_probabilities_times_values(device, heads, rows, keys, head_dim)
+
+
 @pytest.mark.parametrize("head_dim", [8, 40, 64, 96, 128, 200])
 @pytest.mark.parametrize("heads,rows,keys", [(3, 64, 161), (2, 65, 162), (5, 130, 167), (1, 200, 254), (6, 300, 301), (2, 964, 964), (2, 1027, 333)])
 def test_scores(device, heads, rows, keys, head_dim):
@@ -56,12 +62,22 @@ def test_linear_outputs_of_any_width(device, rows, n, k):
 @pytest.mark.parametrize("dt,n", [("f32", 1), ("f32", 3), ("f32", 5), ("f32", 250), ("f32", 255), ("f32", 257), ("f32", 874), ("f32", 1025), ("f32", 2045), ("f32", 2049),
                                   ("f16", 1), ("f16", 7), ("f16", 9), ("f16", 254), ("f16", 505), ("f16", 513), ("f16", 964), ("f16", 1027), ("f16", 2049), ("f16", 4082), ("f16", 4091)])
 def test_softmax_rows_that_start_anywhere(device, dt, n):
+    softmax_rows(device, dt, 203, n)
+
+
+@pytest.mark.parametrize("dt,n", [("f32", 129), ("f32", 250), ("f32", 257), ("f32", 1025), ("f32", 2045), ("f16", 129), ("f16", 254), ("f16", 505), ("f16", 1027), ("f16", 2049), ("f16", 4082)])
+@pytest.mark.parametrize("rows", [1025, 3001])  # many of them: a wavefront a row (fewer: a workgroup)
+def test_many_softmax_rows_that_start_anywhere(device, dt, rows, n):
+    softmax_rows(device, dt, rows, n)
+
+
+def softmax_rows(device, dt, rows, n):
     t, d = (torch.float32, DType.F32) if dt == "f32" else (torch.float16, DType.F16)
-    x = (torch.randn((203, n), generator=torch.Generator("cuda:0").manual_seed(n), device="cuda:0") * 3).to(t)
+    x = (torch.randn((rows, n), generator=torch.Generator("cuda:0").manual_seed(n), device="cuda:0") * 3).to(t)
     x[4], x[5, n - 1], x[6, 0] = -float("inf"), float("nan"), float("inf")  # none of it reaches a neighbour's row
     e = torch.exp(x.double() - x.double().amax(-1, keepdim=True))
     want = e / e.sum(-1, keepdim=True)
-    got = Tensor((203, n), d, device, x.clone().view(torch.uint8).reshape(-1)).softmax(1).resolve().storage.view(t)[: x.numel()].view(x.shape).double()
+    got = Tensor((rows, n), d, device, x.clone().view(torch.uint8).reshape(-1)).softmax(1).resolve().storage.view(t)[: x.numel()].view(x.shape).double()
     assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.isnan(want[4:7]).all()
     size = (x.double() - x.double().amax(-1, keepdim=True)).abs().clamp(max=200)
     rel = 2.0**-24 * (size + 4 + 2 + 32 + 6 + 1) + (2.0**-11 if dt == "f16" else 0)
