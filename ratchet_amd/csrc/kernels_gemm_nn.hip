@@ -282,7 +282,7 @@ RT_TUNABLE(g_gemm_nn_disable, 0);
 
 // hipErrorNotSupported: the problem does not fit; the generic tiled GEMM runs instead.
 hipError_t launch_gemm_nn_smalln(const Problem &p, const void *A, const void *B, const void *bias, void *out,
-                                 hipStream_t stream, const DeviceInfo &) {
+                                 hipStream_t stream, const DeviceInfo &dev) {
     if (g_gemm_nn_disable) return hipErrorNotSupported;
     if (p.a_dt != RT_F16 || p.act_dt != RT_F16) return hipErrorNotSupported;
     if (p.a_ks != 1 || p.b_js != 1 || p.o_js != 1) return hipErrorNotSupported;
@@ -290,6 +290,13 @@ hipError_t launch_gemm_nn_smalln(const Problem &p, const void *A, const void *B,
     if (p.stacks > 65535 || (p.M + NNT_BM - 1) / NNT_BM * p.stacks > 0x7fffffff) return hipErrorNotSupported;
     if (((uintptr_t)A & 15u) || ((uintptr_t)B & 15u) || ((uintptr_t)out & 15u)) return hipErrorNotSupported;
     if (p.b_ks % 8 || p.b_bs % 8 || p.o_is % 8 || p.o_bs % 8) return hipErrorNotSupported;
+    // Rows of A that start anywhere (MODE 2) pay for their edges per workgroup: a short K stays on the generic kernel, a longer one where the
+    // workgroups are more than the compute units.  us, there and here: 16 x [315 x K] . [K x 40] at K = 25 / 33 4.72 / 5.21 and 5.5 / 5.2, x 80 at K = 57 /
+    // 77 / 111 5.51 / 6.13, 6.19 / 6.26 and 6.92 / 6.28, x 128 at K = 91 / 133 / 201 6.18 / 6.96, 7.56 / 7.66 and 9.5 / 8.2; 32 x [925 x K] . [K x 40] at K =
+    // 133 / 201 8.15 / 8.92 and 9.80 / 9.39, x 80 at K = 91 / 111 9.70 / 11.13 and 11.57 / 11.24, x 128 at K = 133 / 201 12.98 / 14.18 and 16.09 / 14.96.
+    const bool rounds = (p.M + NNT_BM - 1) / NNT_BM * p.stacks > dev.num_cus;
+    const int64_t least_k = rounds ? (p.N > 48 && p.N <= 96 ? 97 : 161) : p.N <= 48 ? 33 : p.N <= 96 ? 65 : 129;
+    if ((p.K % 8 || p.a_rs % 8 || p.a_bs % 8) && p.K < least_k) return hipErrorNotSupported;
     GemmNnArgs g{};
     g.A = (const half_t *)A, g.B = (const half_t *)B, g.bias = (const half_t *)bias, g.out = (half_t *)out;
     g.M = p.M, g.N = p.N, g.K = p.K;
