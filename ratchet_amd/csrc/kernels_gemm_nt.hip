@@ -36,6 +36,7 @@
 namespace rt {
 
 typedef uint32_t uint4_d __attribute__((ext_vector_type(4), aligned(4)));
+typedef float float4_d __attribute__((ext_vector_type(4), aligned(4)));
 
 struct GemmNtArgs {
     const void *A;       // f16 [.., M, K] or Q8_0H codes
@@ -1214,17 +1215,14 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(GemmNtArgs g) {
     for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += (int64_t)gridDim.x * blockDim.x) {
         const int64_t j = idx / mq, i = (idx - j * mq) << 2;
         const int n = (int)min<int64_t>(4, g.M - i);
-        float v[4] = {0.f, 0.f, 0.f, 0.f};
-        const float *src = pt + j * g.M + i;
-        if ((g.M & 3) == 0) {
-            for (int sp = 0; sp < g.ksplit; sp++) {
-                const float4_t t = *(const float4_t *)(src + sp * sstride);
-                v[0] += t[0], v[1] += t[1], v[2] += t[2], v[3] += t[3];
-            }
-        } else {
-            for (int sp = 0; sp < g.ksplit; sp++)
-                for (int e = 0; e < n; e++) v[e] += src[sp * sstride + e];
-        }
+        // a row's last values end a group of four that begins in front of theirs: whole loads, at any multiple of four bytes
+        // (value by value Q4_K 62 rows x 1059 x 7680 in 15 shares took 20.2 us for both kernels, 12.7 so; 323 x 1149 x 3072 in four 18.1 and 16.0)
+        const int back = 4 - n;
+        const float *src = pt + j * g.M + i - back;
+        float4_t sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+        for (int sp = 0; sp < g.ksplit; sp++) sum += *(const float4_d *)(src + sp * sstride);
+        const float v[4] = {back & 2 ? (back & 1 ? sum[3] : sum[2]) : back ? sum[1] : sum[0], back & 2 ? sum[3] : back ? sum[2] : sum[1], back ? sum[3] : sum[2], sum[3]};
         half_t r[4];
         for (int e = 0; e < 4; e++) {
             float t = v[e];

@@ -59,6 +59,12 @@ def test_k_of_whole_blocks(device, dt, m, n, k):
     check(device, dt, m, n, k)
 
 
+@pytest.mark.parametrize("m", [161, 162, 163, 164])
+@pytest.mark.parametrize("dt", [DType.Q8_0H, DType.F16])
+def test_sums_of_shares_of_any_row_length(device, dt, m):
+    check(device, dt, m, 9, 4128)
+
+
 @pytest.mark.parametrize("m,n,k", [
     (300, 300, 1024), (1024, 64, 4096), (200, 9, 8192), (2560, 512, 2304), (9000, 200, 512), (7681, 511, 512), (2560, 520, 10240), (10240, 512, 768),
 ])
