@@ -1488,8 +1488,10 @@ RT_TUNABLE(g_gemm_nt_disable, 0);
 
 // The tiles of the kernels that load global -> LDS and how K is shared among workgroups: the cheapest by an estimate in microseconds,
 //   3 + rounds * (fixed - 3 + step * (1 + crowd * busy) * tiles of 64 k in a share) + the second kernel's time,
-// busy the share of the compute units that has a workgroup.  The constants are a fit to every tile and split of 14 f16 and 18
-// Q8_0H products on the device (worst case 7 % above the best choice, most within 1 %).  The largest tile alone, cut along K where
+// busy the share of the compute units that has a workgroup.  The constants are a fit to the tiles and splits of 166 f16 and 176 Q8_0H
+// products on the device (200 to 12000 x 9 to 1500, K from 96 to 14336), each with the weights in the caches and from HBM: the choice is 0.4 and 0.2 %
+// above the best one on average, 16 and 7 % at worst.  (Fitted to few products with the weights in the caches, 128 x 128 tiles of f16 came out ahead of
+// 96 x 128 ones that are faster either way: 9901 x 253 x 3840 45.7 and 41.3 us, 2229 x 943 x 3840 37.5 and 31.4.)  The largest tile alone, cut along K where
 // it left half of the compute units idle, was the rule before: [512 x 2560] . [2560 x 2560]^T Q8_0H 30.2 -> 17.7 us (64 x 128 tiles,
 // K whole), [512 x 2560] . [7680 x 2560]^T 43 -> 34.7 (128 x 128), 128 rows x 2560 x 2560 25.1 -> 12.7 (64 x 64, K in three),
 // 1000 x 4096 x 4096 65.6 -> 52.8; f16 30 -> 15.9 of the first kind, [700 x 1280] . [5120 x 1280]^T 17.3 -> 14.9.
@@ -1498,9 +1500,9 @@ struct NtTile {
     float fixed, step;
 };
 constexpr int kNtTiles = 5;
-constexpr NtTile kTilesF16[kNtTiles] = {{160, 128, 8.6f, 0.333f}, {128, 128, 8.1f, 0.27f}, {96, 128, 7.2f, 0.285f}, {64, 128, 6.6f, 0.182f}, {64, 64, 6.0f, 0.13f}};
-constexpr NtTile kTilesQ8w[kNtTiles] = {{160, 128, 8.6f, 0.70f}, {128, 128, 8.0f, 0.51f}, {96, 128, 7.5f, 0.42f}, {64, 128, 6.7f, 0.26f}, {64, 64, 6.2f, 0.17f}};
-constexpr NtTile kTilesQ8r[kNtTiles] = {{160, 128, 8.2f, 0.70f}, {128, 128, 8.8f, 0.48f}, {96, 128, 7.7f, 0.42f}, {64, 128, 7.2f, 0.295f}, {64, 64, 6.7f, 0.21f}};
+constexpr NtTile kTilesF16[kNtTiles] = {{160, 128, 8.6f, 0.415f}, {128, 128, 8.6f, 0.32f}, {96, 128, 7.2f, 0.285f}, {64, 128, 7.2f, 0.195f}, {64, 64, 4.5f, 0.137f}};
+constexpr NtTile kTilesQ8w[kNtTiles] = {{160, 128, 8.6f, 0.69f}, {128, 128, 7.6f, 0.47f}, {96, 128, 7.5f, 0.417f}, {64, 128, 7.2f, 0.255f}, {64, 64, 5.7f, 0.185f}};
+constexpr NtTile kTilesQ8r[kNtTiles] = {{160, 128, 8.2f, 0.70f}, {128, 128, 9.2f, 0.43f}, {96, 128, 7.7f, 0.427f}, {64, 128, 7.3f, 0.295f}, {64, 64, 6.7f, 0.222f}};
 struct NtChoice {
     int bm = 160, bn = 128;
     int ks = 1;        // workgroups that share one tile's K
@@ -1511,7 +1513,7 @@ static bool nt_q8_whole(const Problem &p) { return p.K % 256 == 0 && p.a_bs % 51
 static NtChoice nt_choose(const Problem &p, const DeviceInfo &dev, bool may_split) {
     const bool q8 = p.a_dt == RT_Q8_0H;
     const NtTile *tiles = !q8 ? kTilesF16 : nt_q8_whole(p) ? kTilesQ8w : kTilesQ8r;
-    const float crowd = q8 ? 0.23f : 0.37f;
+    const float crowd = q8 ? 0.23f : 0.37f, pass = q8 ? 1.7f : 2.4f;
     const int64_t nk = (p.K + NT_BK - 1) / NT_BK;
     NtChoice best;
     best.k_len = p.K;
@@ -1522,14 +1524,15 @@ static NtChoice nt_choose(const Problem &p, const DeviceInfo &dev, bool may_spli
         if (t.bm < 128 && n > dev.num_cus) continue; // narrow tiles only where they all run at once
         for (int ks = 1; ks <= (may_split ? 16 : 1); ks++) {
             if (ks > 1 && n * ks > dev.num_cus) break; // the partial sums stay within 256 of the largest tiles on 256 compute units
-            // where K is whole units of 256 (which gemm_nt_q8w_kernel's shares are too) equal shares, of whole 512s or of at least 1024; else
-            // shares of at least 512, the last one shorter
-            const int64_t share = (nk + ks - 1) / ks;
-            const bool equal = p.K % (512 * ks) == 0 || (p.K % (256 * ks) == 0 && p.K / ks >= 1024);
-            if (ks > 1 && (p.K % 256 == 0 ? !equal : share < 8 || (ks - 1) * share >= nk)) continue;
+            // Where K is whole units of 256 so are the shares (gemm_nt_q8w_kernel's have to be): equal ones of whole 512s, or of at least 1024 with a
+            // shorter last one; else shares of at least 512, the last one shorter.  (Equal ones alone left a K of 17 or 43 units whole, and 56 of
+            // them on 70 tiles in two: 4480 rows Q8_0H at 32, K = 4352 / 11008 / 14336 22.7 / 51 / 39.5 us and in three shares 14.3 / 26.1 / 30.6.)
+            const int64_t unit = p.K % 256 == 0 ? 4 : 1, share = ((nk + ks - 1) / ks + unit - 1) / unit * unit;
+            const int64_t least_share = p.K % 256 == 0 && p.K % (512 * ks) != 0 ? 16 : 8;
+            if (ks > 1 && (share < least_share || (ks - 1) * share >= nk)) continue;
             const int64_t rounds = (n * ks + dev.num_cus - 1) / dev.num_cus;
             const float busy = std::min(1.f, (float)(n * ks) / dev.num_cus);
-            const float second = ks == 1 ? 0.f : 1.9f + 0.1f * ks + (float)(p.stacks * ks * p.M * p.N) * (4.f / 4.5e6f);
+            const float second = ks == 1 ? 0.f : pass + 0.1f * ks + (float)(p.stacks * ks * p.M * p.N) * (4.f / 4.5e6f);
             const float us = 3.f + rounds * (t.fixed - 3.f + t.step * (1.f + crowd * busy) * share) + second;
             if (us < least) least = us, best.bm = t.bm, best.bn = t.bn, best.ks = ks, best.k_len = ks == 1 ? p.K : share * NT_BK;
         }

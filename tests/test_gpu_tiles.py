@@ -59,6 +59,12 @@ def test_k_of_whole_blocks(device, dt, m, n, k):
     check(device, dt, m, n, k)
 
 
+@pytest.mark.parametrize("m,n,k", [(4480, 32, 4352), (4400, 40, 11008), (161, 9, 2816), (1027, 65, 4352), (2051, 33, 5888)])  # whole 256s, the last share shorter
+@pytest.mark.parametrize("dt", [DType.Q8_0H, DType.F16])
+def test_unequal_shares(device, dt, m, n, k):
+    check(device, dt, m, n, k)
+
+
 @pytest.mark.parametrize("m", [161, 162, 163, 164])
 @pytest.mark.parametrize("dt", [DType.Q8_0H, DType.F16])
 def test_sums_of_shares_of_any_row_length(device, dt, m):
