@@ -1565,6 +1565,12 @@ uint64_t gemm_nt_workspace_bytes(const Problem &p0, const DeviceInfo &dev) {
     return ks > 1 ? (uint64_t)p.stacks * ks * p.M * p.N * sizeof(float) : 0;
 }
 
+// whether launch_gemm_nt shares this problem's K with the workspace it was given
+bool gemm_nt_will_share(const Problem &p, const DeviceInfo &dev) {
+    const uint64_t need = p.workspace && !((uintptr_t)p.workspace & 15u) ? gemm_nt_workspace_bytes(p, dev) : 0;
+    return need > 0 && p.workspace_bytes >= need;
+}
+
 // Whether rt_matmul_enqueue_static may share this product's K, on the one buffer that all its calls on a GPU have in common.  A program
 // may have products in flight on several streams there that never touched it, so the products are those that it has always been for:
 // K whole units of 256, at most half a compute unit per 160 x 128 tile, and equal shares of at least 1024.

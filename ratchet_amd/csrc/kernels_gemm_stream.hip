@@ -388,6 +388,18 @@ template <int TA, bool Q8> static hipError_t gs_tb(int tb, const GemmStreamArgs 
     return hipErrorNotSupported;
 }
 
+// weight rows of a workgroup: every compute unit gets one workgroup with its share of the rows, up to 48; more rows: whole rounds of such shares
+static int gs_rows(int64_t M, const DeviceInfo &dev) {
+    const int64_t rounds = (M + 48 * (int64_t)dev.num_cus - 1) / (48 * (int64_t)dev.num_cus);
+    const int64_t per = (M + rounds * dev.num_cus - 1) / (rounds * dev.num_cus);
+    return (int)((per + 7) / 8 * 8);
+}
+// a weight with so few rows that a quarter of the compute units would stay idle is the tiled kernels' (they cut K)
+bool gemm_stream_fills(int64_t M, const DeviceInfo &dev) {
+    const int64_t rows_wg = gs_rows(M, dev);
+    return (M + rows_wg - 1) / rows_wg * 4 >= (int64_t)dev.num_cus * 3;
+}
+
 // f16 or Q8_0H weights (rows of K), K-contiguous f16 activations, one stack.
 // Measured at 10240 x 2560 with the weights from HBM (this kernel / the tiled one, us): f16 weights 16 rows 12.5 / 16.1,
 // 32: 14.4 / 17.7, 48: 16.1 / 19.3, 64: 17.3 / 20.5, 96: 20.4 / 25.2, 112: 22.0 / 26.5, 128: 22.2 / 27.2; Q8_0H 16: 11.9 /
@@ -401,14 +413,9 @@ hipError_t launch_gemm_stream(const Problem &p, const void *A, const void *B, co
     if (p.stacks != 1 || p.N < 1 || p.N > max_n || p.N > (q8 ? 96 : 128) || p.K % 256 != 0 || p.K < 256 || p.b_ks != 1) return hipErrorNotSupported;
     if (f16 && (p.a_ks != 1 || p.a_rs != p.K)) return hipErrorNotSupported;
     if (((uintptr_t)A & 15u) || ((uintptr_t)B & 15u) || (p.b_js * 2) % 16) return hipErrorNotSupported;
-    // every compute unit gets one workgroup with its share of the rows, up to 48; more rows: whole rounds of such shares
-    const int64_t rounds = (p.M + 48 * (int64_t)dev.num_cus - 1) / (48 * (int64_t)dev.num_cus);
-    const int64_t per = (p.M + rounds * dev.num_cus - 1) / (rounds * dev.num_cus);
-    const int rows_wg = (int)((per + 7) / 8 * 8);
-    const int ta = (rows_wg + 15) / 16;
+    const int rows_wg = gs_rows(p.M, dev), ta = (rows_wg + 15) / 16;
     const int64_t nwg = (p.M + rows_wg - 1) / rows_wg;
-    // a weight with so few rows that a quarter of the compute units would stay idle is the tiled kernels' (they cut K)
-    if (nwg * 4 < (int64_t)dev.num_cus * 3 || ta > 3) return hipErrorNotSupported;
+    if (!gemm_stream_fills(p.M, dev) || ta > 3) return hipErrorNotSupported;
     // a share's offsets are 32-bit: 48 rows of K, 128 activation rows of b_js
     if ((int64_t)rows_wg * p.K * 2 >= (int64_t(1) << 31) || p.N * p.b_js * 2 >= (int64_t(1) << 31)) return hipErrorNotSupported;
     GemmStreamArgs g{};

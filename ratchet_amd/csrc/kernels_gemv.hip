@@ -291,11 +291,14 @@ hipError_t launch_gemv_chunked(const Problem &p, const void *A, const void *B, c
     const bool q8 = p.a_dt == RT_Q8_0H, q4 = p.a_dt == RT_Q4_K;
     if ((!q8 && !q4) || p.act_dt != RT_F16 || g_gemv_disable_mfma) return hipErrorNotSupported;
     if (p.N <= 16 || p.N > 32) return hipErrorNotSupported;
-    // Q8_0H weights with enough rows that their 64 x 64 tiles give a quarter of the compute units a workgroup are faster on
-    // the kernels that read them once (17 / 32 vectors, here against there: 10240 x 2560 18 / 20 and 15.7 / 16.2 us, 7680 x 2560
-    // 12.1 / 13.1 and 9.1 / 9.5, 5120 x 4096 13.5 / 16.4 and 10.2 / 10.6, 4096 x 1024 7.3 / 6.9 and 4.5); with fewer rows the
-    // streaming launches stay ahead (2560 x 2560 7.5 / 8.3 and 9.7 / 10.1)
-    if (q8 && p.K % 256 == 0 && p.stacks == 1 && (p.M + 63) / 64 >= dev.num_cus / 4) return hipErrorNotSupported;
+    // Q8_0H weights that a kernel reads once are faster there: where their 64 x 64 tiles give half of the compute units a workgroup; and from a
+    // quarter on (with fewer the streaming launches stay ahead: 2560 x 2560 at 17 / 32 vectors 7.5 / 8.3 us here, 9.7 / 10.1 there) where
+    // launch_gemm_stream takes them (7680 x 2560 12.1 / 13.1 and 9.1 / 9.5, 5120 x 4096 13.5 / 16.4 and 10.2 / 10.6, 4096 x 1024 7.3 / 6.9 and 4.5), where the tiles
+    // share K (4352 x 4096 16.7 / 19.9 and 14.7 / 15.0) or where a K above 4096 makes these launches slow (4352 x 4352 22.1 / 27.3 and, K whole, 22.7
+    // / 22.7).  Between them they stay: 4352 x 1024 7.5 / 8.1 and 8.1 / 8.1, x 4096 without a workspace 16.8 / 19.9 and 21.4 / 21.4.
+    if (const int64_t tiles = (p.M + 63) / 64; q8 && p.K % 256 == 0 && p.stacks == 1 && tiles >= dev.num_cus / 4 &&
+        (tiles >= dev.num_cus / 2 || p.K > 4096 || gemm_stream_fills(p.M, dev) || gemm_nt_will_share(p, dev)))
+        return hipErrorNotSupported;
     for (int64_t j0 = 0; j0 < p.N; j0 += 16) {
         Problem c = p;
         c.N = p.N - j0 < 16 ? p.N - j0 : 16;

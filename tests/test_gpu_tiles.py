@@ -65,6 +65,12 @@ def test_unequal_shares(device, dt, m, n, k):
     check(device, dt, m, n, k)
 
 
+@pytest.mark.parametrize("m", [4096, 4097, 4584, 4600])  # weight rows that fill the streaming kernel's grid, and the ones between that do not
+@pytest.mark.parametrize("n,k", [(17, 1024), (32, 4096), (24, 4352)])
+def test_few_rows_between_the_kernels(device, m, n, k):
+    check(device, DType.Q8_0H, m, n, k)
+
+
 @pytest.mark.parametrize("m", [161, 162, 163, 164])
 @pytest.mark.parametrize("dt", [DType.Q8_0H, DType.F16])
 def test_sums_of_shares_of_any_row_length(device, dt, m):
