@@ -465,9 +465,12 @@ static Q4kChoice q4k_choose(const Problem &p, const DeviceInfo &dev, bool may_sp
     }
     return best;
 }
-// bytes of workspace with which launch_gemm_q4k shares this problem's K (0: it does not)
+// bytes of workspace with which launch_gemm_q4k shares this problem's K (0: it does not, or launch_gemv_chunked takes the problem first)
 uint64_t gemm_q4k_workspace_bytes(const Problem &p, const DeviceInfo &dev) {
     if (!gemm_q4k_takes(p)) return 0;
+    Problem chunk = p;
+    chunk.N = 16;
+    if (p.N <= 32 && gemv_q4k_mfma_fits(chunk, dev)) return 0;
     const int ks = q4k_choose(p, dev, true).ks;
     return ks > 1 ? (uint64_t)p.stacks * ks * p.M * p.N * sizeof(float) : 0;
 }

@@ -299,13 +299,38 @@ RT_TUNABLE(g_gemv_q4k_disable_mfma, 0);
 // Tunable: 1 or 2 forces that many 16-row groups per workgroup (0 = by residency, see the launcher).
 RT_TUNABLE(g_gemv_q4k_mfma_rg, 0);
 
+struct Q4kShape {
+    int sbw, nwaves, rg = 1, rows_wg = 16;
+    size_t lds;
+};
+static Q4kShape q4k_shape(const Problem &p, const DeviceInfo &dev) {
+    Q4kShape c;
+    const int nsb = (int)(p.K / 256);
+    c.sbw = nsb > 16 ? 2 : 1;                                 // K above 4096: two super-blocks per wavefront
+    c.nwaves = nsb < 4 ? 4 : (nsb + c.sbw - 1) / c.sbw;       // the final sum uses 256 threads
+    // Rows per workgroup: 16, unless the activations' LDS (9..16 vectors) leaves one workgroup per compute unit and
+    // the 16-row workgroups would run in rounds; then every compute unit gets one workgroup with its share of the
+    // rows, up to 32 (8192 rows, 16 vectors: 512 workgroups in two rounds 9.3 us -> 256 in one 7.7 us).
+    const size_t lds_x = (size_t)c.nwaves * p.N * (256 + kQ4kXPad + 16) * 2;
+    if (p.N > 8 && p.stacks == 1 && 2 * (lds_x + (size_t)c.nwaves * 1024) > 160 * 1024 && (p.M + 15) / 16 > dev.num_cus) {
+        const int64_t per = ((p.M + dev.num_cus - 1) / dev.num_cus + 7) & ~(int64_t)7;
+        if (per <= 32) c.rows_wg = (int)per, c.rg = (c.rows_wg + 15) / 16;
+    }
+    if (g_gemv_q4k_mfma_rg > 0 && p.N > 8) c.rg = g_gemv_q4k_mfma_rg, c.rows_wg = 16 * c.rg;
+    c.lds = lds_x + (size_t)c.nwaves * c.rg * 1024;
+    return c;
+}
+// whether launch_gemv_q4k_mfma takes a Q4_K product of this size (K whole super-blocks), whatever its strides
+bool gemv_q4k_mfma_fits(const Problem &p, const DeviceInfo &dev) {
+    return p.N >= 1 && p.N <= 16 && p.K >= 256 && p.K <= (p.N <= 8 ? 8192 : 4096) && q4k_shape(p, dev).lds <= 160 * 1024;
+}
+
 // Q4_K weights, f16 activations, 1..16 vectors, K a multiple of 256 and at most 4096 (8192 with up to 8 vectors).
 // hipErrorNotSupported means another kernel must run.
 hipError_t launch_gemv_q4k_mfma(const Problem &p, const void *A, const void *B, const void *bias, void *out,
                                 hipStream_t stream, const DeviceInfo &dev) {
     if (g_gemv_q4k_disable_mfma) return hipErrorNotSupported;
-    if (p.a_dt != RT_Q4_K || p.act_dt != RT_F16 || p.N < 1 || p.N > 16 || p.K % 256 != 0 || p.K < 256 || p.K > (p.N <= 8 ? 8192 : 4096))
-        return hipErrorNotSupported;
+    if (p.a_dt != RT_Q4_K || p.act_dt != RT_F16 || p.K % 256 != 0 || !gemv_q4k_mfma_fits(p, dev)) return hipErrorNotSupported;
     if (p.stacks > 65535 || p.b_ks != 1) return hipErrorNotSupported;
     const int64_t bjs = p.N == 1 ? 0 : p.b_js;
     if (((uintptr_t)A & 15u) || ((uintptr_t)B & 15u) || (bjs * 2) % 16 || (p.b_bs * 2) % 16) return hipErrorNotSupported;
@@ -317,21 +342,8 @@ hipError_t launch_gemv_q4k_mfma(const Problem &p, const void *A, const void *B, 
     g.o_bs = p.o_bs, g.o_is = p.o_is, g.o_js = p.o_js;
     g.has_bias = p.has_bias, g.bias_on_rows = p.bias_on_rows, g.act = p.act;
     if (p.has_bias && ((uintptr_t)bias & 1u)) return hipErrorNotSupported;
-    const int sbw = g.nsb > 16 ? 2 : 1;       // K above 4096: two super-blocks per wavefront
-    const int nwaves = g.nsb < 4 ? 4 : (g.nsb + sbw - 1) / sbw; // the final sum uses 256 threads
-    // Rows per workgroup: 16, unless the activations' LDS (9..16 vectors) leaves one workgroup per compute unit and
-    // the 16-row workgroups would run in rounds; then every compute unit gets one workgroup with its share of the
-    // rows, up to 32 (8192 rows, 16 vectors: 512 workgroups in two rounds 9.3 us -> 256 in one 7.7 us).
-    const size_t lds_x = (size_t)nwaves * g.NC * (256 + kQ4kXPad + 16) * 2;
-    int rg = 1, rows_wg = 16;
-    if (g.NC > 8 && p.stacks == 1 && 2 * (lds_x + (size_t)nwaves * 1024) > 160 * 1024 && (p.M + 15) / 16 > dev.num_cus) {
-        const int64_t per = ((p.M + dev.num_cus - 1) / dev.num_cus + 7) & ~(int64_t)7;
-        if (per <= 32) rows_wg = (int)per, rg = (rows_wg + 15) / 16;
-    }
-    if (g_gemv_q4k_mfma_rg > 0 && g.NC > 8) rg = g_gemv_q4k_mfma_rg, rows_wg = 16 * rg;
+    const auto [sbw, nwaves, rg, rows_wg, lds] = q4k_shape(p, dev);
     g.rows_wg = rows_wg;
-    const size_t lds = lds_x + (size_t)nwaves * rg * 1024;
-    if (lds > 160 * 1024) return hipErrorNotSupported;
     const int64_t groups = (p.M + rows_wg - 1) / rows_wg;
     if (groups > 0x7fffffff) return hipErrorNotSupported;
     dim3 grid((unsigned)groups, (unsigned)p.stacks);

@@ -40,3 +40,16 @@ def test_shares(device, oracle, monkeypatch, stack, m, k, n, split):
             mag = xd.abs().view(n, -1, 256).sum(-1) @ (945 * sb[i, ..., 0] + 63 * sb[i, ..., 1]).T + 2
             err = (got[i] - want).abs()
             assert (err <= 2.0**-11 * want.abs() + 2.0**-24 * (k / 256 * 2 + 14 + 16) * mag + 2.0**-25).all(), float((err / mag).max())
+
+
+@pytest.mark.parametrize("m,n,k,shared", [(2560, 32, 4096, False), (2560, 17, 2560, False), (2560, 33, 4096, True), (2560, 32, 4352, True),
+                                          (5000, 32, 2560, False), (5000, 17, 4096, True)])
+def test_workspace_only_where_the_shares_run(device, m, n, k, shared):
+    """Up to 32 activation rows run on the streaming kernel, which shares nothing, as far as its LDS goes."""
+    import ctypes
+
+    from ratchet_amd import _ffi
+    need = ctypes.c_uint64()
+    d = _ffi.make_desc(_ffi.RT_Q4_K, (m, k), _ffi.RT_F16, (1, n, k), False, True, True)
+    assert _ffi.lib().rt_matmul_workspace_bytes(device.ctx, ctypes.byref(d), ctypes.byref(need)) == _ffi.RT_OK
+    assert (need.value > 0) == shared
