@@ -1524,12 +1524,14 @@ static NtChoice nt_choose(const Problem &p, const DeviceInfo &dev, bool may_spli
         if (t.bm < 128 && n > dev.num_cus) continue; // narrow tiles only where they all run at once
         for (int ks = 1; ks <= (may_split ? 16 : 1); ks++) {
             if (ks > 1 && n * ks > dev.num_cus) break; // the partial sums stay within 256 of the largest tiles on 256 compute units
-            // Where K is whole units of 256 so are the shares (gemm_nt_q8w_kernel's have to be): equal ones of whole 512s, or of at least 1024 with a
-            // shorter last one; else shares of at least 512, the last one shorter.  (Equal ones alone left a K of 17 or 43 units whole, and 56 of
-            // them on 70 tiles in two: 4480 rows Q8_0H at 32, K = 4352 / 11008 / 14336 22.7 / 51 / 39.5 us and in three shares 14.3 / 26.1 / 30.6.)
-            const int64_t unit = p.K % 256 == 0 ? 4 : 1, share = ((nk + ks - 1) / ks + unit - 1) / unit * unit;
-            const int64_t least_share = p.K % 256 == 0 && p.K % (512 * ks) != 0 ? 16 : 8;
-            if (ks > 1 && (share < least_share || (ks - 1) * share >= nk)) continue;
+            // Where K is whole units of 256 so are the shares (gemm_nt_q8w_kernel's have to be): equal ones of whole 512s or of at least 1024, and from
+            // K = 2560 on of at least 1024 with a shorter last one (below, the smaller of two shares is hardly worth the second kernel).  Else
+            // shares of at least 512, the last one shorter.  (Equal ones alone left a K of 17 or 43 units whole, and 56 of them on 70 tiles in two:
+            // 4480 rows Q8_0H at 32, K = 4352 / 11008 / 14336 22.7 / 51 / 39.5 us and in three shares 15.3 / 26.4 / 31.2.)
+            const bool whole = p.K % 256 == 0;
+            const int64_t unit = whole ? 4 : 1, share = ((nk + ks - 1) / ks + unit - 1) / unit * unit;
+            if (ks > 1 && (share < (whole && p.K % (512 * ks) != 0 ? 16 : 8) || (ks - 1) * share >= nk)) continue;
+            if (ks > 1 && whole && p.K < 2560 && p.K % (256 * ks) != 0) continue;
             const int64_t rounds = (n * ks + dev.num_cus - 1) / dev.num_cus;
             const float busy = std::min(1.f, (float)(n * ks) / dev.num_cus);
             const float second = ks == 1 ? 0.f : pass + 0.1f * ks + (float)(p.stacks * ks * p.M * p.N) * (4.f / 4.5e6f);
