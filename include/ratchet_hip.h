@@ -341,8 +341,9 @@ RT_API rt_status rt_matmul_enqueue_ws(rt_ctx *ctx, const rt_matmul_desc *desc, c
  * tight serving loops, harnesses that forbid hipMalloc): the shares' partial sums go to a static
  * buffer of RT_STATIC_SCRATCH_BYTES that the library holds on each GPU it runs on, from
  * rt_ctx_create until the process ends.  Neither this call nor anything it launches allocates or
- * frees.  For f16 activations against f16 or Q8_0H weights, K a multiple of 256, at least 2048, with
- * equal shares of at least 1024, and output tiles of 160 x 128 for at most half of the compute units:
+ * frees.  For f16 activations against f16 or Q8_0H weights, K a multiple of 256 of at least 2048 that
+ * equal shares of at least 1024 could cut, and output tiles of 160 x 128 for at most half of the compute
+ * units (which tiles and shares run, down to 512 of K, is the library's choice, as with a workspace):
  * their results are those of rt_matmul_enqueue_ws with a workspace of rt_matmul_workspace_bytes, bit
  * for bit (the same kernels run).  A split that would need more than the buffer holds is
  * RT_ERR_UNSUPPORTED (on a device of up to 256 compute units none does); every other product, and one
@@ -435,10 +436,10 @@ RT_API rt_status rt_attention_validate(const rt_attention_desc *desc);
  * queries and many keys -- a decode step against a long cache -- where one workgroup per head would
  * leave most compute units idle.  The workspace holds partial (maximum, sum, output) triples in f32
  * between the two kernels of such a launch; its contents before and after are irrelevant.  One query
- * row (with or without a mask tensor) runs a streaming kernel of its own: in one launch up to 256 keys
- * (below 256 no workspace is asked for), and up to 448 where the heads are narrow or many or there is
- * no workspace; beyond that with the workspace in two launches (128 keys per workgroup), and without
- * one on the tiled kernel. */
+ * row (with or without a mask tensor) runs a streaming kernel of its own: in one launch up to 256 keys,
+ * and up to 448 where the heads are narrow or many or there is no workspace (one is asked for from 256
+ * keys on, also where the one launch will not use it); beyond that with the workspace in two launches
+ * (128 keys per workgroup), and without one on the tiled kernel. */
 RT_API rt_status rt_attention_workspace_bytes(const rt_attention_desc *desc, uint64_t *bytes);
 /* `workspace` may be NULL (or smaller than rt_attention_workspace_bytes): the launch then runs in one
  * pass.  Launches that share a workspace must not overlap. */

@@ -1103,7 +1103,8 @@ template <int MK> static void launch_decode_one(const AttnArgs &g, unsigned stac
     else hipLaunchKernelGGL((attention_decode_one_kernel<MK, 1024>), dim3(stacks), dim3(1024), 0, st, g);
 }
 // splits of the two-launch decode kernel for this problem, or 0 when it does not apply: one query row (the causal rule
-// then hides nothing), a cache long enough to be worth two kernels
+// then hides nothing), a cache long enough to be worth two kernels.  (Up to 448 keys one launch may run all the same; callers have
+// always been asked for the workspace from 256 keys on, 68 KB at 32 heads.)
 static int attention_decode_splits(const rt_attention_desc &d) {
     if (d.q_len != 1 || d.kv_len < 256 || d.head_dim % 8 != 0 || d.head_dim > 128) return 0;
     return (d.kv_len + AD_KEYS - 1) / AD_KEYS;

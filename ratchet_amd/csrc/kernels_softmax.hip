@@ -9,7 +9,8 @@
 // read whole (the neighbour's values, which may be changing, are dropped; at the tensor's ends it is read value by value) and its own values
 // are written one by one: 6 x 964 x 964 in f16 15.2 us on the
 // kernel below, which re-reads a row (from L2) for each of its three passes, -> 8.1; 8 x 874 x 874 in f32 17.2 -> 11.3.  It keeps the rows too
-// long for registers and those of fewer than 128 values, for which it has more wavefronts (6 x 62 x 62 in f16: 2.9 and 3.8).
+// long for registers and, where they are few (launch_softmax_t) or have fewer than 128 values, those for which it has more wavefronts
+// (6 x 62 x 62 in f16: 2.9 and 3.8).
 //
 // Role in the reference: ops/softmax.rs:52-183 (one 128-thread workgroup per row, reductions
 // through workgroup memory, arithmetic in the tensor's own type).  Differences, both tighter:
