@@ -176,7 +176,8 @@ hipError_t launch_gemm_stream(const Problem &p, const void *A, const void *B, co
                               const DeviceInfo &dev);
 uint64_t gemm_nt_workspace_bytes(const Problem &p, const DeviceInfo &dev);
 bool gemm_nt_static_split(const Problem &p, const DeviceInfo &dev);
-bool gemm_nt_will_share(const Problem &p, const DeviceInfo &dev);
+bool gemv_chunks_unless_shared(const Problem &p, const DeviceInfo &dev);
+hipError_t gemv_chunks(const Problem &p, const void *A, const void *B, const void *bias, void *out, hipStream_t stream, const DeviceInfo &dev);
 bool gemv_q4k_mfma_fits(const Problem &p, const DeviceInfo &dev);
 bool gemm_stream_fills(int64_t M, const DeviceInfo &dev);
 hipError_t launch_gemm_nt(const Problem &p, const void *A, const void *B, const void *bias, void *out,

@@ -1567,12 +1567,6 @@ uint64_t gemm_nt_workspace_bytes(const Problem &p0, const DeviceInfo &dev) {
     return ks > 1 ? (uint64_t)p.stacks * ks * p.M * p.N * sizeof(float) : 0;
 }
 
-// whether launch_gemm_nt shares this problem's K with the workspace it was given
-bool gemm_nt_will_share(const Problem &p, const DeviceInfo &dev) {
-    const uint64_t need = p.workspace && !((uintptr_t)p.workspace & 15u) ? gemm_nt_workspace_bytes(p, dev) : 0;
-    return need > 0 && p.workspace_bytes >= need;
-}
-
 // Whether rt_matmul_enqueue_static may share this product's K, on the one buffer that all its calls on a GPU have in common.  A program
 // may have products in flight on several streams there that never touched it, so the products are those that it has always been for:
 // K whole units of 256, at most half a compute unit per 160 x 128 tile, and equal shares of at least 1024.
@@ -1650,6 +1644,8 @@ hipError_t launch_gemm_nt(const Problem &p0, const void *A, const void *B, const
     }
     NtChoice c = nt_choose(p, dev, p.K > 256 && p.workspace && !((uintptr_t)p.workspace & 15u));
     if (c.ks > 1 && p.workspace_bytes < (uint64_t)p.stacks * c.ks * p.M * p.N * sizeof(float)) c = nt_choose(p, dev, false);
+    if (c.ks == 1 && gemv_chunks_unless_shared(p, dev)) // 17 to 32 rows of Q8_0H: faster in streaming launches
+        if (const hipError_t e = gemv_chunks(p, A, B, bias, out, stream, dev); e != hipErrorNotSupported) return e;
     if (c.ks > 1) g.ksplit = c.ks, g.k_len = c.k_len, g.partial = (float *)p.workspace;
     if (!q8 && kfull && c.ks == 1 && g_gemm_nt_wide != 1 && p.a_rs >= 0 && p.b_js >= 0 && 2 * 320 * std::max(p.a_rs, p.b_js) < (int64_t(1) << 32)) {
         const int64_t tiles = ((p.M + 159) / 160) * ((p.N + 127) / 128), wide = ((p.M + 319) / 320) * ((p.N + 255) / 256) * p.stacks;

@@ -278,27 +278,15 @@ template <int NC> static void launch_float(int act_dt, bool vec, dim3 grid, hipS
 // Tunable: non-zero keeps Q8_0H weights on the VALU kernel (for comparisons).
 RT_TUNABLE(g_gemv_disable_mfma, 0);
 
-// Returns hipErrorNotSupported when the operands do not meet the alignment the
-// streaming kernels assume; the caller then takes the tiled GEMM, which has no
-// such requirement.
 // A few more activation vectors than one streaming launch takes: one launch per 16 of them.  Each
 // launch streams the weights again (after the first mostly from the Infinity Cache), which still beats
 // the tiled kernels while the MFMA work is small: measured at 8192 x 3072 Q4_K, 17 / 32 vectors take
 // 12 / 14 us (48: 21) against 15 us tiled: the tiled kernels take over from 33.  (10240 x 2560 Q8_0H:
 // 18 / 20 us, 48 / 64 vectors 29 / 38.)
-hipError_t launch_gemv_chunked(const Problem &p, const void *A, const void *B, const void *bias, void *out,
-                               hipStream_t stream, const DeviceInfo &dev) {
+hipError_t gemv_chunks(const Problem &p, const void *A, const void *B, const void *bias, void *out, hipStream_t stream, const DeviceInfo &dev) {
     const bool q8 = p.a_dt == RT_Q8_0H, q4 = p.a_dt == RT_Q4_K;
     if ((!q8 && !q4) || p.act_dt != RT_F16 || g_gemv_disable_mfma) return hipErrorNotSupported;
     if (p.N <= 16 || p.N > 32) return hipErrorNotSupported;
-    // Q8_0H weights that a kernel reads once are faster there: where their 64 x 64 tiles give half of the compute units a workgroup; and from a
-    // quarter on (with fewer the streaming launches stay ahead: 2560 x 2560 at 17 / 32 vectors 7.5 / 8.3 us here, 9.7 / 10.1 there) where
-    // launch_gemm_stream takes them (7680 x 2560 12.1 / 13.1 and 9.1 / 9.5, 5120 x 4096 13.5 / 16.4 and 10.2 / 10.6, 4096 x 1024 7.3 / 6.9 and 4.5), where the tiles
-    // share K (4352 x 4096 16.7 / 19.9 and 14.7 / 15.0) or where a K above 4096 makes these launches slow (4352 x 4352 22.1 / 27.3 and, K whole, 22.7
-    // / 22.7).  Between them they stay: 4352 x 1024 7.5 / 8.1 and 8.1 / 8.1, x 4096 without a workspace 16.8 / 19.9 and 21.4 / 21.4.
-    if (const int64_t tiles = (p.M + 63) / 64; q8 && p.K % 256 == 0 && p.stacks == 1 && tiles >= dev.num_cus / 4 &&
-        (tiles >= dev.num_cus / 2 || p.K > 4096 || gemm_stream_fills(p.M, dev) || gemm_nt_will_share(p, dev)))
-        return hipErrorNotSupported;
     for (int64_t j0 = 0; j0 < p.N; j0 += 16) {
         Problem c = p;
         c.N = p.N - j0 < 16 ? p.N - j0 : 16;
@@ -314,6 +302,30 @@ hipError_t launch_gemv_chunked(const Problem &p, const void *A, const void *B, c
     return hipSuccess;
 }
 
+// Q8_0H weights that a kernel reads once are faster there: where their 64 x 64 tiles give half of the compute units a workgroup; and from a
+// quarter on (with fewer the streaming launches stay ahead: 2560 x 2560 at 17 / 32 vectors 7.5 / 8.3 us here, 9.7 / 10.1 there) where
+// launch_gemm_stream takes them (7680 x 2560 12.1 / 13.1 and 9.1 / 9.5, 5120 x 4096 13.5 / 16.4 and 10.2 / 10.6, 4096 x 1024 7.3 / 6.9 and 4.5), where the tiles
+// share K (4352 x 4096 16.7 / 19.9 and 14.7 / 15.0) or where a K above 4096 makes these launches slow (4352 x 4352 22.1 / 27.3 and, K whole, 22.7
+// / 22.7).  Between them they stay: 4352 x 1024 7.5 / 8.1 and 8.1 / 8.1, x 4096 without a workspace 16.7 / 19.9 and 21.4 / 21.4.  Those whose
+// tiles could share K are left to launch_gemm_nt, which knows whether they do and calls gemv_chunks where not: what the families
+// decline does not depend on the workspace, so that a plan, which asks first the one that ran last, runs what a call without a plan does.
+static bool q8h_between(const Problem &p, const DeviceInfo &dev) {
+    const int64_t tiles = (p.M + 63) / 64;
+    return p.a_dt == RT_Q8_0H && p.K % 256 == 0 && p.K <= 4096 && p.stacks == 1 && tiles >= dev.num_cus / 4 && tiles < dev.num_cus / 2 && !gemm_stream_fills(p.M, dev);
+}
+bool gemv_chunks_unless_shared(const Problem &p, const DeviceInfo &dev) {
+    return q8h_between(p, dev) && p.N > 16 && p.N <= 32 && gemm_nt_workspace_bytes(p, dev) > 0;
+}
+hipError_t launch_gemv_chunked(const Problem &p, const void *A, const void *B, const void *bias, void *out, hipStream_t stream, const DeviceInfo &dev) {
+    if (p.a_dt == RT_Q8_0H && p.K % 256 == 0 && p.stacks == 1 && (p.M + 63) / 64 >= dev.num_cus / 4 &&
+        (!q8h_between(p, dev) || gemv_chunks_unless_shared(p, dev)))
+        return hipErrorNotSupported;
+    return gemv_chunks(p, A, B, bias, out, stream, dev);
+}
+
+// Returns hipErrorNotSupported when the operands do not meet the alignment the
+// streaming kernels assume; the caller then takes the tiled GEMM, which has no
+// such requirement.
 hipError_t launch_gemv(const Problem &p, const void *A, const void *B, const void *bias, void *out,
                        hipStream_t stream, const DeviceInfo &dev) {
     if (p.kernel == RT_KERNEL_GEMV_Q8 && p.a_dt == RT_Q8_0H && !g_gemv_disable_mfma) {

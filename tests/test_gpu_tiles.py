@@ -71,6 +71,32 @@ def test_few_rows_between_the_kernels(device, m, n, k):
     check(device, DType.Q8_0H, m, n, k)
 
 
+@pytest.mark.parametrize("m,n,k", [(4352, 17, 4096), (4352, 32, 1024), (4352, 24, 4352), (4096, 20, 4096)])
+def test_a_plan_gives_the_same_bits_whatever_workspace_came_before(device, m, n, k):
+    """A plan offers its product first to the family that took it last; with and without a workspace it runs what a call without a plan does."""
+    import ctypes
+
+    from ratchet_amd import _ffi
+    L, gen = _ffi.lib(), torch.Generator("cuda:0").manual_seed(m + n)
+    w, _ = weights(device, gen, DType.Q8_0H, (), m, k)
+    x = torch.randn((n, k), generator=gen, device="cuda:0").half()
+    desc = _ffi.make_desc(_ffi.RT_Q8_0H, (m, k), _ffi.RT_F16, (1, n, k), False, True, True)
+    need, plan = ctypes.c_uint64(), ctypes.c_void_p()
+    assert L.rt_matmul_workspace_bytes(device.ctx, ctypes.byref(desc), ctypes.byref(need)) == _ffi.RT_OK
+    ws = torch.empty(max(need.value, 16), dtype=torch.uint8, device="cuda:0")
+    assert L.rt_matmul_plan_create(device.ctx, ctypes.byref(desc), _ffi.RT_ACT_NONE, ctypes.byref(plan)) == _ffi.RT_OK
+    stream, ptrs = torch.cuda.current_stream().cuda_stream, (w.storage.data_ptr(), x.data_ptr(), None)
+    try:
+        for size in (need.value, 0, 0, need.value, need.value, 0):
+            a, b = (torch.full((n, m), float("nan"), dtype=torch.float16, device="cuda:0") for _ in range(2))
+            args = (ws.data_ptr() if size else None, size, stream)
+            assert L.rt_matmul_plan_enqueue(plan, *ptrs, a.data_ptr(), *args) == _ffi.RT_OK
+            assert L.rt_matmul_enqueue_ws(device.ctx, ctypes.byref(desc), *ptrs, b.data_ptr(), _ffi.RT_ACT_NONE, *args) == _ffi.RT_OK
+            assert torch.equal(a, b), size
+    finally:
+        L.rt_matmul_plan_destroy(plan)
+
+
 @pytest.mark.parametrize("m", [161, 162, 163, 164])
 @pytest.mark.parametrize("dt", [DType.Q8_0H, DType.F16])
 def test_sums_of_shares_of_any_row_length(device, dt, m):
