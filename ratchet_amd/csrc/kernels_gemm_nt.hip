@@ -1644,7 +1644,7 @@ hipError_t launch_gemm_nt(const Problem &p0, const void *A, const void *B, const
     }
     NtChoice c = nt_choose(p, dev, p.K > 256 && p.workspace && !((uintptr_t)p.workspace & 15u));
     if (c.ks > 1 && p.workspace_bytes < (uint64_t)p.stacks * c.ks * p.M * p.N * sizeof(float)) c = nt_choose(p, dev, false);
-    if (c.ks == 1 && gemv_chunks_unless_shared(p, dev)) // 17 to 32 rows of Q8_0H: faster in streaming launches
+    if (!RT_NT_ABLATION && c.ks == 1 && gemv_chunks_unless_shared(p, dev)) // 17 to 32 rows of Q8_0H: faster in streaming launches (the timing-only builds have this file alone)
         if (const hipError_t e = gemv_chunks(p, A, B, bias, out, stream, dev); e != hipErrorNotSupported) return e;
     if (c.ks > 1) g.ksplit = c.ks, g.k_len = c.k_len, g.partial = (float *)p.workspace;
     if (!q8 && kfull && c.ks == 1 && g_gemm_nt_wide != 1 && p.a_rs >= 0 && p.b_js >= 0 && 2 * 320 * std::max(p.a_rs, p.b_js) < (int64_t(1) << 32)) {

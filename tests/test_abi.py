@@ -23,6 +23,14 @@ def test_header_symbols_are_exported():
     assert sorted(_ffi.SIGNATURES) == syms  # the Python binding covers the same set
 
 
+def test_both_libraries_resolve_every_symbol():
+    """The measurement probes hold the tiled GEMM's file on its own: what it calls elsewhere would be missing there."""
+    _ffi.lib()
+    from ratchet_amd import build
+    for path in (_ffi.LIB_PATH, build.PROBES_LIB):
+        ctypes.CDLL(path, mode=os.RTLD_NOW)
+
+
 def test_rust_crate_declares_every_symbol():
     """crates/ratchet-hip-sys/src/lib.rs (source only: no rustc in the image) declares every symbol the header
     exports, with as many arguments, and nothing the header does not have."""

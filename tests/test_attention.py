@@ -334,7 +334,7 @@ def test_equals_the_three_operator_sequence(device, oracle):
 @gpu
 def test_one_query_against_a_long_cache_streams_the_keys(device, oracle):
     """A decode step (one query row, at least 256 cached keys, no mask tensor, a workspace) takes the streaming
-    kernel: every head dimension it serves (idle lanes past head_dim / 8), key counts off the 128-key workgroups
+    kernels, in one launch or, with more or wider keys, two: every head dimension it serves (idle lanes past head_dim / 8), key counts off the 128-key workgroups
     and off the 16-key loads, the cache read in place with rows past kv_len poisoned, heads merged on the way
     out, a dominant key in the last workgroup's share, and the causal flag, which hides nothing from one query."""
     rng = np.random.default_rng(21)
@@ -354,7 +354,7 @@ def test_one_query_against_a_long_cache_streams_the_keys(device, oracle):
         assert not np.isnan(got).any(), (B, H, kv_len, D)
         assert_close(got, want, ("decode", B, H, kv_len, D))
         single = Q.attention(K, V, kv_len=kv_len)
-        single.op.use_workspace = False                        # the tiled kernel, one pass
+        single.op.use_workspace = False                        # the tiled kernel, one pass (up to 448 keys the streaming one launch)
         np.testing.assert_allclose(got.astype(np.float32), single.resolve().to(Device.CPU).storage.astype(np.float32),
                                    rtol=4e-3, atol=1e-3, err_msg=str((B, H, kv_len, D)))
         merged = Q.attention(K, V, kv_len=kv_len, merge_heads=True).resolve().to(Device.CPU).storage
