@@ -339,10 +339,10 @@ POISON_OUTPUTS = False
 _strides3 = ctypes.c_int64 * 3
 
 
-def _overlap(x: "Tensor", y: "Tensor") -> bool:
-    """Whether two resolved GPU tensors share memory, by address: two tensors may wrap one allocation."""
-    a, b = x._ptr(), y._ptr()
-    return a < b + y.storage.nbytes and b < a + x.storage.nbytes
+def _touches(storage, lo: int, hi: int) -> bool:
+    """Whether a GPU tensor's storage has bytes in [lo, hi): by address, since two tensors may wrap one allocation."""
+    p = storage.data_ptr()
+    return p < hi and lo < p + storage.nbytes
 
 
 def _write_key_and_value(k: "Tensor", v: "Tensor", stream: int):
@@ -356,21 +356,27 @@ def _write_key_and_value(k: "Tensor", v: "Tensor", stream: int):
     if (a.cache.storage is None or b.cache.storage is None or k.dt != v.dt or k.shape != v.shape
             or (a.offset, a.len, a.src_strides) != (b.offset, b.len, b.src_strides) or k.device is not v.device or k.device.kind != "gpu"):
         return
-    if a.source.device.kind != "gpu" or b.source.device.kind != "gpu" or _overlap(a.cache, b.cache):
+    keys, vals, ks, vs = a.cache.storage, b.cache.storage, a.source, b.source
+    kc, vc = keys.data_ptr(), vals.data_ptr()
+    kc_end, vc_end = kc + keys.nbytes, vc + vals.nbytes
+    if ks.device.kind != "gpu" or vs.device.kind != "gpu" or (kc < vc_end and vc < kc_end):
         return
-    if b.source.storage is None and (type(b.source.op) is Cache or any(s.storage is None or s.device.kind != "gpu" or _overlap(s, a.cache)
-                                                                       for s in b.source.op.srcs())):
+    if vs.storage is None:
+        if type(vs.op) is Cache:
+            return
+        for s in vs.op.srcs():
+            if s.storage is None or s.device.kind != "gpu" or _touches(s.storage, kc, kc_end):
+                return
+    if ks.storage is None:
+        ks._execute(stream)
+    if v.storage is not None or _touches(ks.storage, vc, vc_end):   # (the keys' source may have read the new values)
         return
-    if a.source.storage is None:
-        a.source._execute(stream)
-    if v.storage is not None or _overlap(a.source, b.cache):   # (the keys' source may have read the new values)
-        return
-    if b.source.storage is None:
-        b.source._execute(stream)
-    if _overlap(b.source, a.cache):
+    if vs.storage is None:
+        vs._execute(stream)
+    if _touches(vs.storage, kc, kc_end):
         return
     B, H, cap, D = a.cache.shape
-    st = _ffi.lib().rt_cache_write_kv_enqueue(k.device.ctx, int(k.dt), a.cache._ptr(), a.source._ptr(), b.cache._ptr(), b.source._ptr(),
+    st = _ffi.lib().rt_cache_write_kv_enqueue(k.device.ctx, int(k.dt), kc, ks.storage.data_ptr(), vc, vs.storage.data_ptr(),
                                               _strides3(*a.src_strides), B, H, cap, a.offset, a.len, D, stream)
     _check(st, k.device)
     k.storage, v.storage = a.cache.storage, b.cache.storage
