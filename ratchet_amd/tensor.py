@@ -542,7 +542,8 @@ class Tensor:
         return self
 
     def _empty(self, nbytes: int):
-        return _torch().empty(nbytes, dtype=_torch().uint8, device=self.device.torch_device())
+        torch = _torch()
+        return torch.empty(nbytes, dtype=torch.uint8, device=self.device.torch_device())
 
     def _execute(self, stream: int):
         """Enqueues every unresolved node below this one, then this one, on `stream` (asked of torch once per resolve: the ten
