@@ -104,7 +104,7 @@ __global__ __launch_bounds__(64 * (MW + LW), 2) void gemm_q4k_kernel(GemmQ4kArgs
     const uint8_t *blocks = g.blocks + ((g.a_stack == 1 ? 0 : s) * g.M * g.nsb + sb0) * 144;
     const half_t *X = g.X + (g.b_stack == 1 ? 0 : s) * g.b_bs + sb0 * 256;
     const int64_t last = nsb - 1;
-    const bool vec_out = g.vec_out && g.ksplit == 1 && i0 + BM <= g.M; // a whole tile of weight rows, stored 16 bytes at a time
+    const bool vec_out = g.vec_out && g.ksplit == 1; // stored 16 bytes at a time
 
     if (LW > 0 && wave >= MW) {
         // ---- loading wavefront lw: LDS-DMA instruction i of a stage (i = lw, lw + 4, ...; 33 in all) fills the 1 KB
@@ -377,6 +377,31 @@ __global__ __launch_bounds__(64 * (MW + LW), 2) void gemm_q4k_kernel(GemmQ4kArgs
         }
         return;
     }
+    // The bias before any store, since a load behind one is waited for by itself, and tiles past the last weight row through LDS too: with
+    // both in the stores of an edge tile, whose outputs went one by one, the launch took 4 us longer wherever M % 128 was not 0
+    // (M x K at activation rows, before and now, us: 1760 x 256 at 1683 12.9 and 8.6, 4288 x 256 at 206 9.2 and 5.4, 10848 x 2816 at 95 24.8 and
+    // 20.7, 4192 x 768 at 318 12.9 and 8.4; 8192 x 3072 at 1000 75.0 and 75.2).
+    if (g.has_bias) {
+        if (g.bias_on_rows) {
+#pragma unroll
+            for (int a = 0; a < TA; a++) {
+                const float bi = (float)(g.bias + i0)[min(wave * (16 * TA) + 16 * a + fr, (int)min<int64_t>(BM, g.M - i0) - 1)];
+#pragma unroll
+                for (int bq = 0; bq < TB; bq++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) acc[a][bq][r] += bi;
+            }
+        } else {
+#pragma unroll
+            for (int bq = 0; bq < TB; bq++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const float bj = (float)(g.bias + j0)[min(16 * ((bq + wave) & 3) + 4 * fg + r, (int)min<int64_t>(QR_BN, g.N - j0) - 1)];
+#pragma unroll
+                    for (int a = 0; a < TA; a++) acc[a][bq][r] += bj;
+                }
+        }
+    }
     half_t *out = g.out + s * g.o_bs;
     if (vec_out) {
         // Output contiguous along the weight rows: the tile goes through LDS (the activation stages are free: every
@@ -387,26 +412,19 @@ __global__ __launch_bounds__(64 * (MW + LW), 2) void gemm_q4k_kernel(GemmQ4kArgs
         static_assert((size_t)QR_BN * OLD * 2 <= (size_t)QR_XST * QR_XSB, "the staged output tile fits the activation stages");
         rt_with_act(g.act, [&](auto has_act) {
 #pragma unroll
-            for (int a = 0; a < TA; a++) {
-                const int il = wave * (16 * TA) + 16 * a + fr;
-                const float bi = (g.has_bias && g.bias_on_rows) ? (float)g.bias[i0 + il] : 0.f;
+            for (int a = 0; a < TA; a++)
 #pragma unroll
                 for (int bq = 0; bq < TB; bq++)
 #pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        const int jl = 16 * ((bq + wave) & 3) + 4 * fg + r;
-                        float v = acc[a][bq][r] + bi;
-                        if (g.has_bias && !g.bias_on_rows) v += (float)g.bias[min(j0 + jl, g.N - 1)];
-                        Os[jl * OLD + il] = (half_t)rt_act_k<decltype(has_act)::value>(v);
-                    }
-            }
+                    for (int r = 0; r < 4; r++)
+                        Os[(16 * ((bq + wave) & 3) + 4 * fg + r) * OLD + wave * (16 * TA) + 16 * a + fr] = (half_t)rt_act_k<decltype(has_act)::value>(acc[a][bq][r]);
         });
         tile_ready();
 #pragma unroll
         for (int k = 0; k < 2 * TA; k++) {
             constexpr int CPR = BM / 8; // 16-byte pieces per row
             const int idx = t + 64 * MW * k, row = idx / CPR, c = idx % CPR;
-            if (j0 + row < g.N) *(uint4_t *)(out + (j0 + row) * g.o_js + i0 + 8 * c) = *(const uint4_t *)(Os + row * OLD + 8 * c);
+            if (j0 + row < g.N && i0 + 8 * c < g.M) *(uint4_t *)(out + (j0 + row) * g.o_js + i0 + 8 * c) = *(const uint4_t *)(Os + row * OLD + 8 * c);
         }
         return;
     }
@@ -420,11 +438,7 @@ __global__ __launch_bounds__(64 * (MW + LW), 2) void gemm_q4k_kernel(GemmQ4kArgs
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
                     const int64_t j = j0 + 16 * ((bq + wave) & 3) + 4 * fg + r;
-                    if (j >= g.N) continue;
-                    float v = acc[a][bq][r];
-                    if (g.has_bias) v += (float)g.bias[g.bias_on_rows ? i : j];
-                    v = rt_act_k<decltype(has_act)::value>(v);
-                    out[i * g.o_is + j * g.o_js] = (half_t)v;
+                    if (j < g.N) out[i * g.o_is + j * g.o_js] = (half_t)rt_act_k<decltype(has_act)::value>(acc[a][bq][r]);
                 }
         }
     });
@@ -492,7 +506,7 @@ hipError_t launch_gemm_q4k(const Problem &p, const void *A, const void *B, const
     g.has_bias = p.has_bias, g.bias_on_rows = p.bias_on_rows, g.act = p.act;
     const int64_t tiles_j = (p.N + QR_BN - 1) / QR_BN;
     g.tiles_j = (int)tiles_j;
-    g.vec_out = p.o_is == 1 && p.o_js % 8 == 0 && p.o_bs % 8 == 0 && ((uintptr_t)out & 15u) == 0;
+    g.vec_out = p.o_is == 1 && p.M % 8 == 0 && p.o_js % 8 == 0 && p.o_bs % 8 == 0 && ((uintptr_t)out & 15u) == 0;
     Q4kChoice c = q4k_choose(p, dev, p.workspace && !((uintptr_t)p.workspace & 15u));
     if (c.ks > 1 && p.workspace_bytes < (uint64_t)p.stacks * c.ks * p.M * p.N * sizeof(float)) c = q4k_choose(p, dev, false);
     g.ksplit = c.ks, g.sb_len = (g.nsb + c.ks - 1) / c.ks, g.partial = (float *)p.workspace;
