@@ -46,6 +46,8 @@
 // W.gemm(x, b, false, true, true) (crates/ratchet-nn/src/linear.rs:17-24).
 #include "device_common.h"
 
+#include <algorithm>
+
 namespace rt {
 
 struct GemmQ4kArgs {
@@ -444,17 +446,353 @@ __global__ __launch_bounds__(64 * (MW + LW), 2) void gemm_q4k_kernel(GemmQ4kArgs
     });
 }
 
+// ---------------------------------------------------------------------------
+// The same for many activation rows: 256 weight rows x 128 activation rows per workgroup, one workgroup per compute unit, eight
+// wavefronts of 64 x 64 outputs on 32 x 32 x 16 MFMAs.
+//
+// Everything comes by LDS-DMA, the raw blocks too: a load that gives every lane 16 bytes of a row of its own is 64 lines to the
+// compute unit's memory pipeline, and those loads were what the kernel above spends a third of its time on here; as runs of 144
+// consecutive bytes they are a fifth of that.  Half the tile's activations per weight byte and half the fragment reads per MFMA are the
+// larger tile's.  Measured, the kernel above and this: 8192 x 3072 against 1000 / 2048 activation rows 75.2 / 160 -> 60.2 / 122 us (0.84 PFLOP/s; with
+// the MFMAs alone it is 41, and 36 without any of them).  What bounds it: MFMAs and what stands between them share a SIMD's issue (a step of a super-block
+// is 4.4 us of which the MFMAs are 2.7 at the clock the chip then runs at), the LDS-DMA takes 0.5 of it, the sums of x 0.3.
+//
+// Lane half h = lane / 32 owns the 64 bytes h of a super-block's qs (sub-blocks 4 h .. + 3).  A super-block is two halves of eight
+// steps: half H is chunk 2 h + H of 32 bytes, four steps of eight low nibbles and four of high ones.  A pair of nibbles stays where
+// v_perm puts it, as the f16 subnormals q * 2^-24 (16 q * 2^-24), and one packed multiplication with sc * 2^10 (2^6) makes it
+// sc * q * 2^-14 exactly; the 2^14 goes into d.
+//
+// A SIMD overlaps the vector instructions of one wavefront with the MFMAs of the other, and a wavefront's own with the MFMA before them:
+// so the decoding of the step after, the header of the super-block after, the folds and the sums of x stand between the MFMAs, a few
+// behind each.  Two stages of activations (a half super-block each), two of blocks; the barrier of a half stands
+// before its last step, whose operands are in registers by then, so that the first reads of the next half run under that step.
+// What is loaded there has a half's time to land.
+//
+// Sums of x: of the four wavefronts that share 64 activation rows, number w sums fragment w % 2 over the low (w < 2) or high nibbles'
+// K; it takes its fragments and nibbles in an order that makes those its first ones, so that the code is the same for all.
+// ---------------------------------------------------------------------------
+constexpr int QW_BM = 256, QW_BN = 128;
+constexpr int QW_ROWB = 17 * 16;          // bytes per staged activation row: 16 K-vectors and one of padding
+constexpr int QW_XB = QW_BN * QW_ROWB;    // bytes per stage of activations = 34 LDS-DMA instructions
+constexpr int QW_WB = QW_BM * 144;        // of blocks = 36 instructions; rows 144 bytes apart start 4 banks apart
+constexpr int QW_SXB = QW_BN * 2 * 16;    // of the sums of x of a super-block: [row][lane half], f16 high parts of four, then low parts
+constexpr size_t QW_LDS = 2 * (size_t)(QW_XB + QW_WB + QW_SXB) ;
+
+__global__ __launch_bounds__(512, 2) void gemm_q4k_wide_kernel(GemmQ4kArgs g) {
+    constexpr int TA = 2, TB = 2;
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    uint8_t *Xs = smem, *Ws = smem + 2 * QW_XB, *Sx = smem + 2 * (QW_XB + QW_WB);
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int fr = lane & 31, fh = lane >> 5;
+    const int wi = wave >> 1, wj = wave & 1, wc = wi >> 1, wb = wi & 1;
+    const int64_t s = blockIdx.y;
+    uint32_t blk = blockIdx.x;
+    if (g.remap) blk = (blk & 7) * (gridDim.x >> 3) + (blk >> 3); // as above
+    const uint32_t ti = __builtin_amdgcn_readfirstlane(blk / (uint32_t)g.tiles_j), tj = blk - ti * (uint32_t)g.tiles_j;
+    const int64_t i0 = (int64_t)ti * QW_BM, j0 = (int64_t)tj * QW_BN;
+    const int64_t sb0 = (int64_t)blockIdx.z * g.sb_len, nsb = min(g.sb_len, g.nsb - sb0), last = nsb - 1; // this workgroup's share of K: > 0 (launcher)
+    const uint8_t *blocks = g.blocks + ((g.a_stack == 1 ? 0 : s) * g.M * g.nsb + sb0) * 144;
+    const half_t *X = g.X + (g.b_stack == 1 ? 0 : s) * g.b_bs + sb0 * 256;
+
+    // LDS-DMA instruction i of a stage (wavefront i % 8) fills slots 64 i .. + 63 of 16 bytes.  Rows past the end repeat the last one.
+    constexpr int ND = 5;
+    const int ix = min(wave + 32, 33), iw5 = min(wave + 32, 35); // the fifth of a wavefront that has four repeats the stage's last
+    const uint32_t x4 = 1024u * (uint32_t)(ix - wave), w4 = 1024u * (uint32_t)(iw5 - wave);
+    uint32_t xoff[ND], woff[ND];
+#pragma unroll
+    for (int n = 0; n < ND; n++) {
+        const uint32_t px = 64u * (uint32_t)min(wave + 8 * n, 33) + (uint32_t)lane, xr = px / 17u, xv = min(px - 17u * xr, 15u);
+        const uint32_t pw = 64u * (uint32_t)min(wave + 8 * n, 35) + (uint32_t)lane, wr = pw / 9u, wv = pw - 9u * wr;
+        xoff[n] = 2u * ((uint32_t)min(j0 + (int64_t)xr, g.N - 1) * (uint32_t)g.b_js + 128u * (xv >> 3) + 8u * (xv & 7u));
+        woff[n] = (uint32_t)min(i0 + (int64_t)wr, g.M - 1) * (uint32_t)g.nsb * 144u + 16u * wv; // < 2^32: launcher
+    }
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)smem + 1024u * (uint32_t)wave;
+    // as asm: see issue_x above
+    auto dma = [&](uint32_t dst, uint32_t off, const void *base) __attribute__((always_inline)) {
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds0 + dst), "v"(off), "s"(base) : "m0", "memory");
+    };
+    auto issue_x = [&](int half, int64_t sb) __attribute__((always_inline)) { // into stage `half`
+        const half_t *xk = X + min(sb, last) * 256 + 64 * half; // past the end: the last one again, never used
+#pragma unroll
+        for (int n = 0; n < 4; n++) dma((uint32_t)(half * QW_XB + 8192 * n), xoff[n], xk);
+        dma((uint32_t)(half * QW_XB) + x4, xoff[4], xk);
+    };
+    auto issue_w = [&](uint32_t stage, int64_t sb) __attribute__((always_inline)) { // stage in bytes
+        const uint8_t *bsb = blocks + min(sb, last) * 144;
+#pragma unroll
+        for (int n = 0; n < 4; n++) dma(2 * QW_XB + stage + 8192u * n, woff[n], bsb);
+        dma(2 * QW_XB + stage + w4, woff[4], bsb);
+    };
+    // This wavefront's loads have landed, its LDS stores are done and its reads have returned; past the barrier so have everyone's.
+    auto meet = [&]() __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    struct Scl {
+        half2_t s[2]; // per half: of the sub-block taken first, second; sc * 2^10 for low nibbles, sc * 2^6 for high ones
+    };
+    struct Fin {
+        float d, dmin; // d * 2^14
+        uint32_t mn[2];
+    };
+    const uint32_t upper = fh ? ~0u : 0u; // sub-blocks 4..7: the scales and mins split over two bytes
+    const uint32_t order[2] = {wc ? 0x04000401u : 0x04010400u, wc ? 0x04020403u : 0x04030402u}; // v_perm's bytes of the two scales
+    const half2_t k1024 = {(half_t)1024.0f, (half_t)1024.0f}, kup = {(half_t)(wc ? 64.0f : 1024.0f), (half_t)(wc ? 1024.0f : 64.0f)};
+    const uint32_t mask[2] = {wc ? 0xF0F0F0F0u : 0x0F0F0F0Fu, wc ? 0x0F0F0F0Fu : 0xF0F0F0F0u};
+    auto header = [&](const uint4_t &h, Scl &sc, Fin &f) __attribute__((always_inline)) {
+        const uint32_t S0 = h[1], S1 = h[2], S2 = h[3];
+        const uint32_t sc47 = (S2 & 0x0F0F0F0Fu) | ((S0 >> 2) & 0x30303030u), mn47 = ((S2 >> 4) & 0x0F0F0F0Fu) | ((S1 >> 2) & 0x30303030u);
+        const uint32_t scw = (sc47 & upper) | (S0 & 0x3F3F3F3Fu & ~upper);
+        const uint32_t mnw = (mn47 & upper) | (S1 & 0x3F3F3F3Fu & ~upper);
+        sc.s[0] = (__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, scw, order[0])) - k1024) * kup;
+        sc.s[1] = (__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, scw, order[1])) - k1024) * kup;
+        f.mn[0] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, mnw, 0x04010400u)) - k1024);
+        f.mn[1] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, mnw, 0x04030402u)) - k1024);
+        const half2_t dm = __builtin_bit_cast(half2_t, h[0]);
+        f.d = (float)dm[0] * 16384.0f, f.dmin = (float)dm[1];
+    };
+    const float16_t zero = {};
+    float16_t acc[TA][TB], P[TA][TB];
+#pragma unroll
+    for (int a = 0; a < TA; a++)
+#pragma unroll
+        for (int b = 0; b < TB; b++) acc[a][b] = zero, P[a][b] = zero;
+    Scl sc[TA];
+    Fin now[TA], fin[TA]; // of the super-block at hand, of the one before
+    uint4_t hdr[TA], pc[TA][2], wf[2][TA]; // raw header; the half's two pieces; weight fragments of two steps
+    half8_t xf[2][TB], sf[TB];
+#pragma unroll
+    for (int a = 0; a < TA; a++) fin[a] = Fin{0.f, 0.f, {0u, 0u}};
+    // half `hf` of the weight fragment of step T of half H: four of its 8 values sc * q * 2^-14 of this lane's row
+    auto wpart = [&](auto Hc, auto Tc, int a, int hf, uint4_t &w) __attribute__((always_inline)) {
+        constexpr int H = decltype(Hc)::value, T = decltype(Tc)::value;
+        const uint32_t v = pc[a][(T & 3) >> 1][2 * (T & 1) + hf] & mask[T >> 2];
+        const half_t sv = sc[a].s[H][T >> 2];
+        const half2_t s2 = {sv, sv};
+        w[2 * hf] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0u, v, 0x04010400u)) * s2);
+        w[2 * hf + 1] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0u, v, 0x04030402u)) * s2);
+    };
+    uint32_t wat = (uint32_t)(144 * (64 * wi + fr)); // this lane's row of blocks in the current stage
+    auto read_piece = [&](int half, int p) __attribute__((always_inline)) {
+#pragma unroll
+        for (int a = 0; a < TA; a++) pc[a][p] = *(const uint4_t *)(Ws + wat + 64 * fh + (16 + 32 * half + 16 * p + 32 * 144 * a));
+    };
+    auto read_header = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int a = 0; a < TA; a++) hdr[a] = *(const uint4_t *)(Ws + wat + 32 * 144 * a);
+    };
+    uint32_t xat[TB][2], slane[TB]; // this lane's row of the activation fragments, the one it sums first: at the sub-block taken first, second; of their sums
+#pragma unroll
+    for (int b = 0; b < TB; b++) {
+        const int row = 64 * wj + 32 * (b ^ wb) + fr;
+        xat[b][0] = (uint32_t)(QW_ROWB * row + 128 * fh + 64 * wc), xat[b][1] = xat[b][0] + (wc ? -64 : 64), slane[b] = (uint32_t)(32 * row + 16 * fh);
+    }
+    auto xread = [&](int half, int T) __attribute__((always_inline)) {
+#pragma unroll
+        for (int b = 0; b < TB; b++) xf[T & 1][b] = __builtin_bit_cast(half8_t, *(const uint4_t *)(Xs + xat[b][T >> 2] + (half * QW_XB + 16 * (T & 3))));
+    };
+    auto read_sums = [&](uint32_t q) __attribute__((always_inline)) { // of parity q, in bytes of Sx
+#pragma unroll
+        for (int b = 0; b < TB; b++) sf[b] = __builtin_bit_cast(half8_t, *(const uint4_t *)(Sx + q + slane[b]));
+    };
+    const half2_t ones = {(half_t)1.0f, (half_t)1.0f};
+    // What is left of the super-block before, tile by tile: its sums times d, and its min term
+    auto fold = [&](int a, int b) __attribute__((always_inline)) {
+        const half8_t mf = __builtin_bit_cast(half8_t, uint4_t{fin[a].mn[0], fin[a].mn[1], fin[a].mn[0], fin[a].mn[1]});
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[a][b][r] = fmaf(fin[a].d, P[a][b][r], acc[a][b][r]);
+        P[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sf[b], mf, zero, 0, 0, 0);
+    };
+    auto fold_min = [&](int a, int b) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[a][b][r] = fmaf(-fin[a].dmin, P[a][b][r], acc[a][b][r]);
+    };
+    uint32_t wcur = 0, par = 0; // bytes: stage of this super-block's blocks, parity of its sums
+    // Half H of a super-block.
+    auto run_half = [&](auto Hc, int64_t sb) __attribute__((always_inline)) {
+        constexpr int H = decltype(Hc)::value;
+        float S = 0.f;
+        auto sum_x = [&](int T, int c) __attribute__((always_inline)) {
+            S = __builtin_amdgcn_fdot2(half2_t{xf[T & 1][0][2 * c], xf[T & 1][0][2 * c + 1]}, ones, S, false);
+        };
+        auto step = [&](auto Tc) __attribute__((always_inline)) {
+            constexpr int T = decltype(Tc)::value;
+            if constexpr (T < 7) xread(H, T + 1);
+            if constexpr (T == 5) { // the registers' last values have been decoded
+                if (H == 1) wat += QW_WB - 2 * wcur, read_header();
+                read_piece(H ^ 1, 0);
+            }
+            if constexpr (T == 7) {
+                meet();
+                xread(H ^ 1, 0);
+                read_piece(H ^ 1, 1);
+                if (H == 1) read_sums(par);
+                issue_x(H, sb + 1);
+                if (H == 1) issue_w(wcur, sb + 2);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int m = 0; m < TA * TB; m++) {
+                const int a = m / TB, b = m % TB;
+                if (H == 0 && T == 0) fold_min(a, b);
+                P[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[T & 1][b], __builtin_bit_cast(half8_t, wf[T & 1][a]), H == 0 && T == 0 ? zero : P[a][b], 0, 0, 0);
+                if constexpr (H == 1 && T == 7) {
+                    if (b == 0) header(hdr[a], sc[a], now[a]);
+                }
+                wpart(std::integral_constant<int, T == 7 ? H ^ 1 : H>{}, std::integral_constant<int, (T + 1) % 8>{}, a, b, wf[(T + 1) & 1][a]);
+                if (T < 4) sum_x(T, m);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if constexpr (T == 4) { // high part: the sum truncated to f16; low part: the exact remainder, rounded
+                const half2_t h = __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_pkrtz(S, 0.f));
+                *(half_t *)(Sx + par + slane[0] + 4 * H + 2 * wc) = h[0];
+                *(half_t *)(Sx + par + slane[0] + 8 + 4 * H + 2 * wc) = __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_pkrtz(S - (float)h[0], 0.f))[0];
+            }
+        };
+        step(std::integral_constant<int, 0>{});
+        if constexpr (H == 0)
+#pragma unroll
+            for (int a = 0; a < TA; a++) fin[a] = now[a];
+        step(std::integral_constant<int, 1>{});
+        step(std::integral_constant<int, 2>{});
+        step(std::integral_constant<int, 3>{});
+        step(std::integral_constant<int, 4>{});
+        step(std::integral_constant<int, 5>{});
+        step(std::integral_constant<int, 6>{});
+        step(std::integral_constant<int, 7>{});
+    };
+    static_assert(TB == 2 && TA * TB == 4, "a step's MFMAs: half a weight fragment and a quarter of the sum of x behind each");
+
+    issue_x(0, 0);
+    issue_w(0, 0);
+    issue_x(1, 0);
+    issue_w(QW_WB, 1);
+    asm volatile("s_waitcnt vmcnt(10)\n\ts_barrier" ::: "memory"); // the first two have landed
+    read_header();
+    read_piece(0, 0);
+    read_piece(0, 1);
+    xread(0, 0);
+#pragma unroll
+    for (int a = 0; a < TA; a++) {
+        header(hdr[a], sc[a], now[a]);
+#pragma unroll
+        for (int hf = 0; hf < 2; hf++) wpart(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, a, hf, wf[0][a]);
+    }
+#pragma unroll
+    for (int b = 0; b < TB; b++) sf[b] = half8_t{}; // nothing before the first super-block
+    for (int64_t sb = 0; sb < nsb; sb++) {
+#pragma unroll
+        for (int m = 0; m < TA * TB; m++) {
+            fold(m / TB, m % TB);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        run_half(std::integral_constant<int, 0>{}, sb);
+        run_half(std::integral_constant<int, 1>{}, sb);
+        wcur = QW_WB - wcur, par ^= QW_SXB;
+    }
+#pragma unroll
+    for (int m = 0; m < TA * TB; m++) fold(m / TB, m % TB);
+#pragma unroll
+    for (int m = 0; m < TA * TB; m++) fold_min(m / TB, m % TB);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // nothing lands once the output goes through LDS
+
+    // acc[a][b][r]: weight row i0 + 64 wi + 32 a + fr, activation row j0 + 64 wj + 32 (b ^ wb) + 8 (r / 4) + 4 fh + r % 4
+    const int iw = 64 * wi + fr;
+    if (g.ksplit > 1) {
+        float *pt = g.partial + (s * g.ksplit + blockIdx.z) * g.N * g.M;
+#pragma unroll
+        for (int a = 0; a < TA; a++) {
+            const int64_t i = i0 + iw + 32 * a;
+#pragma unroll
+            for (int b = 0; b < TB; b++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int64_t j = j0 + 64 * wj + 32 * (b ^ wb) + 8 * (r >> 2) + 4 * fh + (r & 3);
+                    if (i < g.M && j < g.N) pt[j * g.M + i] = acc[a][b][r];
+                }
+        }
+        return;
+    }
+    // the bias before any store: behind one, every load would be waited for by itself
+    if (g.has_bias) {
+        if (g.bias_on_rows) {
+#pragma unroll
+            for (int a = 0; a < TA; a++) {
+                const float bi = (float)(g.bias + i0)[min(iw + 32 * a, (int)min<int64_t>(QW_BM, g.M - i0) - 1)];
+#pragma unroll
+                for (int b = 0; b < TB; b++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) acc[a][b][r] += bi;
+            }
+        } else {
+#pragma unroll
+            for (int b = 0; b < TB; b++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const float bj = (float)(g.bias + j0)[min(64 * wj + 32 * (b ^ wb) + 8 * (r >> 2) + 4 * fh + (r & 3), (int)min<int64_t>(QW_BN, g.N - j0) - 1)];
+#pragma unroll
+                    for (int a = 0; a < TA; a++) acc[a][b][r] += bj;
+                }
+        }
+    }
+    half_t *out = g.out + s * g.o_bs;
+    if (g.vec_out) { // through LDS, as above
+        constexpr int OLD = QW_BM + 8, CPR = QW_BM / 8;
+        half_t *Os = (half_t *)smem;
+        static_assert((size_t)QW_BN * OLD * 2 <= QW_LDS, "the staged output tile fits");
+        __syncthreads(); // every wavefront's LDS-DMA has landed
+        rt_with_act(g.act, [&](auto has_act) {
+#pragma unroll
+            for (int a = 0; a < TA; a++)
+#pragma unroll
+                for (int b = 0; b < TB; b++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++)
+                        Os[(64 * wj + 32 * (b ^ wb) + 8 * (r >> 2) + 4 * fh + (r & 3)) * OLD + iw + 32 * a] = (half_t)rt_act_k<decltype(has_act)::value>(acc[a][b][r]);
+        });
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < QW_BN * CPR / 512; k++) {
+            const int idx = t + 512 * k, row = idx / CPR, c = idx % CPR;
+            if (j0 + row < g.N && i0 + 8 * c < g.M) *(uint4_t *)(out + (j0 + row) * g.o_js + i0 + 8 * c) = *(const uint4_t *)(Os + row * OLD + 8 * c);
+        }
+        return;
+    }
+    rt_with_act(g.act, [&](auto has_act) {
+#pragma unroll
+        for (int a = 0; a < TA; a++) {
+            const int64_t i = i0 + iw + 32 * a;
+            if (i >= g.M) continue;
+#pragma unroll
+            for (int b = 0; b < TB; b++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int64_t j = j0 + 64 * wj + 32 * (b ^ wb) + 8 * (r >> 2) + 4 * fh + (r & 3);
+                    if (j < g.N) out[i * g.o_is + j * g.o_js] = (half_t)rt_act_k<decltype(has_act)::value>(acc[a][b][r]);
+                }
+        }
+    });
+}
+
 RT_TUNABLE(g_gemm_q4k_cfg, 0); // 14 / 24: always one / two weight tiles per wavefront (for comparisons)
 RT_TUNABLE(g_gemm_q4k_disable, 0); // non-zero keeps Q4_K prefill on the generic kernel (for comparisons)
 
-// Weight tiles per wavefront and workgroups that share K, by an estimate in microseconds: 5.5 + step * super-blocks of a share, 0.95 a
-// step with one weight tile, 1.6 with two, and the second kernel's time.  A wavefront's super-blocks are a chain, so with few tiles a long K
+// Kernel and workgroups that share K, by an estimate in microseconds.  Of the first kernel: 5.5 + step * super-blocks of a share, 0.95 a
+// step with one weight tile per wavefront, 1.6 with two, and the second kernel's time; more tiles of 128 rows than compute units run as
+// many rounds, from four on they level out.  A wavefront's super-blocks are a chain, so with few tiles a long K
 // took as long as with many; shared (M x K at activation rows, K whole and shared, us): 2560 x 10240 at 64 38.4 and 16.4, 3072 x 8192
 // at 32 31.6 and 15.4, at 100 31.6 and 21.0, 3584 x 9472 at 148 38.1 and 30, 1024 x 4096 at 128 17.6 and 11.7, 2560 x 2560 at 40
 // 12.3 and 10.2.  The margin of 0.3: 430 x 1280 at 228 took 10.1 whole and 10.9 in 5 shares, 828 x 1280 at 70 10.2 and 8.8.
-// Without a workspace (and with more tiles of 128 rows than compute units) K stays whole.
+// Without a workspace (and, of the first kernel, with more tiles of 128 rows than compute units) K stays whole.
+// Of the 256 x 128 tiles: 7 + step * super-blocks of a workgroup, 3.4 a step while half the compute units rest, 4.5 (the clock falls) from 70 %
+// of them on.  They are taken where that is less, by 3 % for what the estimate does not know (first kernel and this, us): 8192 x 3072 at
+// 1000 75.2 and 60.2, 3072 x 8192 at 1000 91.6 and, in two shares, 75.3, 2560 x 10240 at 512 60.3 and, in six, 46.4, 6720 x 1024 at 939 31.2 and 24.2, 12864 x 7936 at
+// 211 88.9 and 79.3; left to the first kernel: 13312 x 3840 at 569 (260 tiles) 94 and 128, 5376 x 1696 at 276 20 and 26, 4544 x 1536 at 775 23.6 and 29.4.
 struct Q4kChoice {
-    int ta = 2, ks = 1;
+    int ta = 2, ks = 1; // 16-row tiles per wavefront: 1, 2; 4: gemm_q4k_wide_kernel
 };
 static bool gemm_q4k_takes(const Problem &p) {
     return p.a_dt == RT_Q4_K && p.act_dt == RT_F16 && p.K % 256 == 0 && p.K >= 256 && p.b_ks == 1 && p.M >= 64 && p.N >= 17 && p.stacks <= 65535;
@@ -463,19 +801,33 @@ static Q4kChoice q4k_choose(const Problem &p, const DeviceInfo &dev, bool may_sp
     // Four multiplying wavefronts of 32 weight rows x 64 activation rows each; when the grid of 16-row wavefronts
     // (64 weight rows per workgroup) still fits the compute units in one round, those: half the work per wavefront
     // (8192 x 3072 at 64 / 128 rows: 15.7 / 16.8 us against 22.6 / 23.6; 3072 x 8192 at 256 rows: 35 against 52 us).
-    const int64_t tiles_j = (p.N + QR_BN - 1) / QR_BN, nsb = p.K / 256;
+    const int64_t tiles_j = (p.N + QR_BN - 1) / QR_BN, nsb = p.K / 256, cus = dev.num_cus;
+    const int64_t wgs = ((p.M + 127) / 128) * tiles_j * p.stacks;
+    auto sums = [&](int ks) { return 2.6f + 0.1f * ks + (float)(p.stacks * ks * p.M * p.N) * (4.f / 4.5e6f); }; // the second kernel
     Q4kChoice best;
-    best.ta = ((p.M + 63) / 64) * tiles_j <= dev.num_cus ? 1 : 2;
-    if (!may_split || ((p.M + 127) / 128) * tiles_j * p.stacks > dev.num_cus) return best;
+    best.ta = ((p.M + 63) / 64) * tiles_j <= cus ? 1 : 2;
     float least = 5.2f + (best.ta == 1 ? 0.95f : 1.6f) * nsb;
-    for (int ta = 1; ta <= 2; ta++) {
-        const int64_t n = ((p.M + 64 * ta - 1) / (64 * ta)) * tiles_j * p.stacks;
-        for (int ks = 2; ks <= 16 && n * ks <= dev.num_cus; ks++) {
-            const int64_t share = (nsb + ks - 1) / ks;
-            if ((ks - 1) * share >= nsb) continue;
-            const float us = 5.5f + (ta == 1 ? 0.95f : 1.6f) * share + 2.6f + 0.1f * ks + (float)(p.stacks * ks * p.M * p.N) * (4.f / 4.5e6f);
-            if (us < least) least = us, best.ta = ta, best.ks = ks;
+    if (wgs > cus) {
+        least = 5.2f + 1.6f * (float)nsb * (wgs <= 4 * cus ? (float)((wgs + cus - 1) / cus) : (float)wgs / (float)cus + 0.5f);
+    } else if (may_split) {
+        for (int ta = 1; ta <= 2; ta++) {
+            const int64_t n = ((p.M + 64 * ta - 1) / (64 * ta)) * tiles_j * p.stacks;
+            for (int ks = 2; ks <= 16 && n * ks <= cus; ks++) {
+                const int64_t share = (nsb + ks - 1) / ks;
+                if ((ks - 1) * share >= nsb) continue;
+                const float us = 5.5f + (ta == 1 ? 0.95f : 1.6f) * share + sums(ks);
+                if (us < least) least = us, best.ta = ta, best.ks = ks;
+            }
         }
+    }
+    // the 256 x 128 tiles
+    const int64_t n = ((p.M + QW_BM - 1) / QW_BM) * ((p.N + QW_BN - 1) / QW_BN) * p.stacks;
+    for (int ks = 1; ks <= (may_split ? 16 : 1) && (ks == 1 || n * ks <= cus); ks++) {
+        const int64_t share = (nsb + ks - 1) / ks;
+        if ((ks - 1) * share >= nsb) continue;
+        const float step = 3.4f + 1.1f * std::min(1.f, std::max(0.f, 5.f * (float)(n * ks) / (float)cus - 2.5f));
+        const float us = 7.f + step * (float)((n * ks + cus - 1) / cus * share) + (ks > 1 ? sums(ks) : 0.f);
+        if (1.03f * us < least) least = 1.03f * us, best.ta = 4, best.ks = ks;
     }
     return best;
 }
@@ -505,25 +857,26 @@ hipError_t launch_gemm_q4k(const Problem &p, const void *A, const void *B, const
     g.o_bs = p.o_bs, g.o_is = p.o_is, g.o_js = p.o_js;
     g.has_bias = p.has_bias, g.bias_on_rows = p.bias_on_rows, g.act = p.act;
     const int64_t tiles_j = (p.N + QR_BN - 1) / QR_BN;
-    g.tiles_j = (int)tiles_j;
     g.vec_out = p.o_is == 1 && p.M % 8 == 0 && p.o_js % 8 == 0 && p.o_bs % 8 == 0 && ((uintptr_t)out & 15u) == 0;
     Q4kChoice c = q4k_choose(p, dev, p.workspace && !((uintptr_t)p.workspace & 15u));
     if (c.ks > 1 && p.workspace_bytes < (uint64_t)p.stacks * c.ks * p.M * p.N * sizeof(float)) c = q4k_choose(p, dev, false);
     g.ksplit = c.ks, g.sb_len = (g.nsb + c.ks - 1) / c.ks, g.partial = (float *)p.workspace;
     if (g_gemm_q4k_cfg) c.ta = g_gemm_q4k_cfg == 14 ? 1 : 2;
-    auto go = [&](auto kernel, int bm, int lw) -> hipError_t {
-        const int64_t tiles_i = (p.M + bm - 1) / bm;
+    auto go = [&](auto kernel, int bm, int bn, int waves, size_t lds) -> hipError_t {
+        const int64_t tiles_i = (p.M + bm - 1) / bm, tiles_j = (p.N + bn - 1) / bn;
+        g.tiles_j = (int)tiles_j;
         if (tiles_i * tiles_j > 0x7fffffff) return hipErrorNotSupported;
         g.remap = (tiles_i * tiles_j) % 8 == 0;
         if (const hipError_t e = ensure_lds_limit<decltype(kernel)::value>(); e != hipSuccess) return e;
-        hipLaunchKernelGGL(decltype(kernel)::value, dim3((unsigned)(tiles_i * tiles_j), (unsigned)p.stacks, (unsigned)c.ks), dim3(64 * (4 + lw)), QR_LDS, stream, g);
+        hipLaunchKernelGGL(decltype(kernel)::value, dim3((unsigned)(tiles_i * tiles_j), (unsigned)p.stacks, (unsigned)c.ks), dim3(64 * waves), lds, stream, g);
         if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
         return c.ks > 1 ? launch_splitk_sums(p, bias, out, g.partial, c.ks, stream) : hipSuccess;
     };
-    if (c.ta == 1) return go(std::integral_constant<void (*)(GemmQ4kArgs), &gemm_q4k_kernel<1, 4, 4>>{}, 64, 4);
+    if (c.ta == 4) return go(std::integral_constant<void (*)(GemmQ4kArgs), &gemm_q4k_wide_kernel>{}, QW_BM, QW_BN, 8, QW_LDS);
+    if (c.ta == 1) return go(std::integral_constant<void (*)(GemmQ4kArgs), &gemm_q4k_kernel<1, 4, 4>>{}, 64, QR_BN, 8, QR_LDS);
     // more than one workgroup per compute unit: no loading wavefronts (see the file comment)
-    if (((p.M + 127) / 128) * tiles_j * p.stacks > dev.num_cus) return go(std::integral_constant<void (*)(GemmQ4kArgs), &gemm_q4k_kernel<2, 4, 0>>{}, 128, 0);
-    return go(std::integral_constant<void (*)(GemmQ4kArgs), &gemm_q4k_kernel<2, 4, 4>>{}, 128, 4);
+    if (((p.M + 127) / 128) * tiles_j * p.stacks > dev.num_cus) return go(std::integral_constant<void (*)(GemmQ4kArgs), &gemm_q4k_kernel<2, 4, 0>>{}, 128, QR_BN, 4, QR_LDS);
+    return go(std::integral_constant<void (*)(GemmQ4kArgs), &gemm_q4k_kernel<2, 4, 4>>{}, 128, QR_BN, 8, QR_LDS);
 }
 
 } // namespace rt
