@@ -109,8 +109,8 @@ template <int O0, int O1> __device__ __forceinline__ void at_tr_read2(uint64_t &
     asm volatile("ds_read_b64_tr_b16 %0, %2 offset:%3\n\tds_read_b64_tr_b16 %1, %2 offset:%4" : "=&v"(v0), "=&v"(v1) : "v"(a0), "n"(O0), "n"(O1) : "memory");
 }
 
-// DP: head_dim padded to a multiple of 32.  MK: 0 no mask tensor; 1 an additive mask tensor, read from memory where it is
-// used; 2 the same, its [64 queries x 64 keys] block travelling through the ring with the keys and values (see below).  DC: head_dim itself when the
+// DP: head_dim padded to a multiple of 32.  MK: 0 no mask tensor; 1, 2 an additive mask tensor (f32, f16), a block ahead through registers; 3 the same,
+// its [64 queries x 64 keys] block travelling through the ring with the keys and values (see below).  DC: head_dim itself when the
 // kernel is built for one (64, 80, 96, 128), else 0 and head_dim is the argument's: with a constant row length the
 // fragment addresses inside a stage differ by constants, which the LDS instructions carry as immediate offsets, so
 // a block costs three address additions instead of eighteen.
@@ -122,15 +122,17 @@ template <int O0, int O1> __device__ __forceinline__ void at_tr_read2(uint64_t &
 // block twice as long, do the same work in the same number of instructions per wavefront and half as many steps.
 // It needs the registers of a wavefront to stay within 128 and three stages of 128 keys within the LDS
 // (head_dim up to 96).
-// The mask tensor.  Read where it is used (eight loads per lane in the middle of a step, which the compiler has to
-// await with every load into LDS still in flight: the ring drains on every step, 25.7 us at 32 x 512 x 512 x 80 where
-// the causal flag takes 10.0) it is the slow path, yet a tensor is what the reference's callers pass
-// (phi3/attn.rs:148-151).  With rows of whole 16-byte vectors (MK == 2) the block's 64 x 64 mask values are two more
+// The mask tensor.  Read where it is used (eight loads per lane in the middle of a step, which had to be
+// awaited with every load into LDS still in flight: the ring drained on every step, 25.7 us at 32 x 512 x 512 x 80 where
+// the causal flag takes 10.0) it would be the slow path, yet a tensor is what the reference's callers pass
+// (phi3/attn.rs:148-151).  With rows of whole 16-byte vectors (MK == 3) the block's 64 x 64 mask values are two more
 // LDS-DMA instructions per wavefront and block, counted with the others, stored behind the values in the stage with
-// the row's 16-byte chunks XOR-swizzled like the keys', and read back as two vectors per lane.
+// the row's 16-byte chunks XOR-swizzled like the keys', and read back as two vectors per lane (13.0 us).  Rows that start anywhere
+// (any odd number of keys), and sixteen wavefronts, have a lane's two vectors of four requested a block ahead (13.9 there;
+// 8 heads x 1261 x 1261 x 128 in f16 69.7 -> 42.0, 32 x 517 x 517 x 40 32.3 -> 24.6, 16 x 700 x 700 x 96 28.4 -> 20.5).
 template <int DP, int MK, int DC, int NKQ>
 __global__ __launch_bounds__(256 * NKQ) void attention_kernel(AttnArgs g) {
-    constexpr bool MASK = MK != 0, MST = MK == 2;
+    constexpr bool MASK = MK != 0, MST = MK == 3;
     static_assert(NKQ == 2 || (NKQ == 4 && DP <= 96 && !MST), "eight wavefronts, or sixteen for head_dim up to 96 (not with a staged mask)");
     constexpr int BK = 32 * NKQ, WAVES = 4 * NKQ; // keys of a block; wavefronts
     static_assert(DC == 0 || (DC % 8 == 0 && DC <= DP && DC > DP - 32), "a fixed head_dim belongs to its padded size");
@@ -268,7 +270,7 @@ __global__ __launch_bounds__(256 * NKQ) void attention_kernel(AttnArgs g) {
     // then everybody's have
     auto publish = [&](auto keep) {
         asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_waitcnt(at_waitcnt(decltype(keep)::value * (NI + NIM)));
+        __builtin_amdgcn_s_waitcnt(at_waitcnt(decltype(keep)::value * (NI + NIM))); // (MK 1, 2: a mask's loads are younger than what this waits for, or awaited with it)
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
@@ -289,15 +291,37 @@ __global__ __launch_bounds__(256 * NKQ) void attention_kernel(AttnArgs g) {
     if (g.splits > 1) kb_lo = (int)((uint32_t)(nkb_all * split) / (uint32_t)g.splits), kb_hi = (int)((uint32_t)(nkb_all * (split + 1)) / (uint32_t)g.splits);
     const int nkb = kb_hi - kb_lo;
     const int last = max(kb_hi - 1, 0);
+    // The mask values of this lane's scores, row 16 qt + fr, keys 32 kh + 16 b2 + 4 fg .. + 3 of a block: requested a block ahead.
+    using MT = std::conditional_t<MK == 1, float, half_t>;
+    typedef MT mask4_t __attribute__((ext_vector_type(4)));
+    typedef MT mask4_u __attribute__((ext_vector_type(4), aligned(sizeof(MT)))); // rows start anywhere
+    mask4_t mnext[2];
+    auto load_mask = [&](int kb) __attribute__((always_inline)) {
+        if constexpr (MASK && !MST) {
+            const MT *mrow = (const MT *)g.mask + (int64_t)min(qrow, g.q_len - 1) * g.mask_rs;
+            const int c = kb * BK + 32 * kh + 4 * fg;
+            if (kb * BK + BK <= g.kv_len) { // uniform
+#pragma unroll
+                for (int b2 = 0; b2 < 2; b2++) mnext[b2] = *(const mask4_u *)(mrow + c + 16 * b2);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; e++) mnext[e >> 2][e & 3] = mrow[min(c + 16 * (e >> 2) + (e & 3), g.kv_len - 1)];
+            }
+        }
+    };
     // prologue: the first STAGES - 1 blocks requested (an index past the end repeats the last block, so
     // that every step issues and awaits the same number of loads), the first one landed
     if (nkb > 0) {
+        load_mask(kb_lo);
 #pragma unroll
         for (int sidx = 0; sidx < STAGES - 1; sidx++) issue_loads_at(sidx, min(kb_lo + sidx, last));
     }
-    const half_t *mrow = nullptr;
-    if constexpr (MASK && !MST) mrow = (const half_t *)g.mask; // indexed below by its own element type
     if (nkb > 0) publish(std::integral_constant<int, STAGES - 2>{});
+    // awaited here: a first use inside the loop would put the wait for the query's loads, and with them for every LDS-DMA in
+    // flight, into every step (the kernels without a mask in registers wait by themselves, and later)
+    if constexpr (MASK && !MST)
+#pragma unroll
+        for (int kk = 0; kk < KK; kk++) asm volatile("" : "+v"(fq[kk]));
     // fragment addressing inside a stage (halfs).  Sixteen rows further down the swizzle repeats, so the second key
     // tile and the second half of the value rows are 16 dvec chunks away from the first.
     const int tile_halfs = 128 * dvec;
@@ -322,6 +346,8 @@ __global__ __launch_bounds__(256 * NKQ) void attention_kernel(AttnArgs g) {
         constexpr bool LEAN = decltype(lean_c)::value;
         const int kb = kb_lo + it;
         const int k0 = kb * BK;
+        mask4_t mcur[2] = {mnext[0], mnext[1]};
+        load_mask(min(kb + 1, last));
         // the stage the previous step used is free (everybody passed the barrier that ended it)
         issue_loads_at(it + STAGES - 1, min(kb + STAGES - 1, last));
         const half_t *st = ring + (it % STAGES) * stage_halfs;
@@ -415,13 +441,8 @@ __global__ __launch_bounds__(256 * NKQ) void attention_kernel(AttnArgs g) {
                 for (int r = 0; r < 4; r++) {
                     const int key = kw0 + 16 * b2 + 4 * fg + r;
                     float s = S[b2][r] * g.scale_log2e;
-                    if constexpr (MST) {
-                        s += mvals[b2][r] * kLog2e;
-                    } else if constexpr (MASK) {
-                        const int64_t mi = (int64_t)min(qrow, g.q_len - 1) * g.mask_rs + min(key, g.kv_len - 1);
-                        const float mv = g.mask_f32 ? ((const float *)mrow)[mi] : (float)mrow[mi];
-                        s += mv * kLog2e;
-                    }
+                    if constexpr (MST) s += mvals[b2][r] * kLog2e;
+                    else if constexpr (MASK) s += (float)mcur[b2][r] * kLog2e;
                     if (key >= g.kv_len || (g.causal && key > qrow + off)) s = -INFINITY;
                     S[b2][r] = s;
                     bmax = fmaxf(bmax, s);
@@ -553,7 +574,7 @@ __global__ __launch_bounds__(256 * NKQ) void attention_kernel(AttnArgs g) {
     }
 }
 
-// Many query rows, no mask tensor: a workgroup of four wavefronts owns 128 query rows of one head, a wavefront 32 of them
+// Many query rows: a workgroup of four wavefronts owns 128 query rows of one head, a wavefront 32 of them
 // (two MFMA tiles) against all 64 keys of every block.  What bounds the kernel above is instructions: its wavefronts
 // own 16 rows x 32 keys a step, and a step's key and value fragment reads, its cross-lane maxima, its
 // bookkeeping and its barrier are as many for 16 rows as for 32, for 32 keys as for 64.  Here a fragment read from LDS
@@ -561,15 +582,17 @@ __global__ __launch_bounds__(256 * NKQ) void attention_kernel(AttnArgs g) {
 // end.  Two workgroups share a compute unit (two stages of the ring at head_dim 128, three below), so that one's
 // softmax runs beside the other's MFMAs.  The LDS-DMA is issued from assembly: behind the builtin the compiler makes
 // every transposing read wait for all loads into LDS; no register is written by it, and publish() waits for it.
-// DC: head_dim (64, 80, 96 or 128).
+// DC: head_dim (64, 80, 96 or 128).  MK: no mask tensor, an f32 one, an f16 one; a lane's 32 mask values of a block are requested a block ahead, eight
+// vectors of four that may start anywhere, and awaited with the block's keys and values, so there the ring has two stages (us, the kernel above and
+// this: 40 heads x 1373 x 1375 x 128 f32 149 and 81, 32 x 1298 x 1298 x 96 f16 89 and 70, 32 x 2048 x 2048 x 96, rows of whole vectors, 152 and 93).
 constexpr int AL_BQ = 128, AL_BK = 64;
-constexpr int al_stages(int dc) { return dc > 96 ? 2 : 3; }
+constexpr int al_stages(int dc, int mk) { return mk || dc > 96 ? 2 : 3; }
 typedef __fp16 fp16x4_t __attribute__((ext_vector_type(4)));
 
-template <int DC>
+template <int DC, int MK>
 __global__ __launch_bounds__(256, 2) void attention_long_kernel(AttnArgs g) {
     constexpr int KK = (DC + 31) / 32, DT = (DC + 15) / 16, DV = DC / 8; // MFMA steps over head_dim, output tiles, 16-byte chunks per row
-    constexpr int STAGES = al_stages(DC);
+    constexpr int STAGES = al_stages(DC, MK);
     constexpr int BLK = AL_BK * DC;             // halfs of one packed block of keys (or values)
     constexpr int NI = (2 * DV + 3) / 4;        // load instructions per wavefront and block (64 chunks each: DV for the keys, DV for the values)
     constexpr bool SWZ = DC == 64 || DC == 128; // rows whose chunks are XOR-swizzled (at_chunk_pos)
@@ -676,6 +699,38 @@ __global__ __launch_bounds__(256, 2) void attention_long_kernel(AttnArgs g) {
 #pragma unroll
     for (int d = 0; d < VN; d++) voff[d] = BLK + 8 * at_chunk_pos(4 * fg + (fr >> 2), 2 * d + ((fr & 3) >> 1), DV) + 4 * (fr & 1);
 
+    // The mask values of this lane's scores, rows qw + 16 u + fr, keys 16 bt + 4 fg .. + 3 of a block: requested a block ahead, awaited with its keys
+    // and values, and kept in base-2 units.
+    using MT = std::conditional_t<MK == 1, float, half_t>;
+    typedef MT mask4_t __attribute__((ext_vector_type(4)));
+    typedef MT mask4_u __attribute__((ext_vector_type(4), aligned(sizeof(MT)))); // rows start anywhere
+    constexpr int MU = MK ? 2 : 1, MB = MK ? 4 : 1;
+    mask4_t mnext[MU][MB];
+    float4_t mk[MU][MB];
+    auto load_mask = [&](int kb) __attribute__((always_inline)) {
+        if constexpr (MK != 0) {
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const MT *mrow = (const MT *)g.mask + (int64_t)min(qw + 16 * u + fr, g.q_len - 1) * g.mask_rs;
+                const int c = kb * AL_BK + 4 * fg;
+                if (kb * AL_BK + AL_BK <= g.kv_len) { // uniform
+#pragma unroll
+                    for (int bt = 0; bt < 4; bt++) mnext[u][bt] = *(const mask4_u *)(mrow + c + 16 * bt);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 16; e++) mnext[u][e >> 2][e & 3] = mrow[min(c + 16 * (e >> 2) + (e & 3), g.kv_len - 1)];
+                }
+            }
+        }
+    };
+    auto take_mask = [&]() __attribute__((always_inline)) {
+        if constexpr (MK != 0) {
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) mk[u][e >> 2][e & 3] = (float)mnext[u][e >> 2][e & 3] * kLog2e;
+        }
+    };
     auto step = [&](int stage, int kb, auto lean_c) __attribute__((always_inline)) {
         constexpr bool LEAN = decltype(lean_c)::value;
         const half_t *st = ring + stage * 2 * BLK;
@@ -697,7 +752,7 @@ __global__ __launch_bounds__(256, 2) void attention_long_kernel(AttnArgs g) {
 #pragma unroll
         for (int u = 0; u < 2; u++) {
             float bmax = -INFINITY;
-            if constexpr (LEAN) { // scale > 0: the maximum of the raw scores, the scale folded into the exponent's argument
+            if constexpr (LEAN && MK == 0) { // scale > 0: the maximum of the raw scores, the scale folded into the exponent's argument
 #pragma unroll
                 for (int e = 0; e < 16; e++) bmax = fmaxf(bmax, S[u][e >> 2][e & 3]);
                 bmax *= g.scale_log2e;
@@ -705,8 +760,8 @@ __global__ __launch_bounds__(256, 2) void attention_long_kernel(AttnArgs g) {
 #pragma unroll
                 for (int e = 0; e < 16; e++) {
                     const int key = kb * AL_BK + 16 * (e >> 2) + 4 * fg + (e & 3);
-                    float s = S[u][e >> 2][e & 3] * g.scale_log2e;
-                    if (key >= g.kv_len || (g.causal && key > qw + 16 * u + fr + off)) s = -INFINITY;
+                    float s = MK ? fmaf(S[u][e >> 2][e & 3], g.scale_log2e, mk[u][e >> 2][e & 3]) : S[u][e >> 2][e & 3] * g.scale_log2e;
+                    if (!LEAN && (key >= g.kv_len || (g.causal && key > qw + 16 * u + fr + off))) s = -INFINITY;
                     S[u][e >> 2][e & 3] = s;
                     bmax = fmaxf(bmax, s);
                 }
@@ -722,7 +777,7 @@ __global__ __launch_bounds__(256, 2) void attention_long_kernel(AttnArgs g) {
             const float m_use = m_new == -INFINITY ? 0.f : m_new; // a row without a finite score yet: exp2(-inf - 0) = 0
             alpha[u] = __builtin_amdgcn_exp2f(m_run[u] - m_use);
             m_run[u] = m_new;
-            const float sc = LEAN ? g.scale_log2e : 1.f;
+            const float sc = LEAN && MK == 0 ? g.scale_log2e : 1.f;
             float psum = 0.f;
 #pragma unroll
             for (int e = 0; e < 16; e += 2) {
@@ -755,7 +810,7 @@ __global__ __launch_bounds__(256, 2) void attention_long_kernel(AttnArgs g) {
     };
     // blocks that cross neither the end of the keys nor this wavefront's diagonal need no test per element
     int n_lean = 0;
-    if (g.scale_log2e > 0.f) {
+    if (MK || g.scale_log2e > 0.f) {
         n_lean = g.kv_len / AL_BK;
         if (g.causal) n_lean = min(n_lean, qw + off + 1 < 0 ? 0 : (qw + off + 1) / AL_BK);
         n_lean = min(n_lean, nkb_w);
@@ -763,13 +818,17 @@ __global__ __launch_bounds__(256, 2) void attention_long_kernel(AttnArgs g) {
     if (nkb > 0) {
 #pragma unroll
         for (int sidx = 0; sidx < STAGES - 1; sidx++) issue_loads(sidx, min(sidx, last));
+        load_mask(0);
         publish(std::integral_constant<int, STAGES - 2>{});
+        take_mask();
         int cur = 0, fill = STAGES - 1, kb = 0;
         // three loops, so that each keeps the accumulators in registers of its own
         auto turn = [&](auto body) __attribute__((always_inline)) {
             issue_loads(fill, min(kb + STAGES - 1, last)); // past the end: the last block again, into a stage nobody reads
+            load_mask(min(kb + 1, last));
             body();
             publish(std::integral_constant<int, STAGES - 2>{});
+            take_mask();
             cur = cur + 1 == STAGES ? 0 : cur + 1, fill = fill + 1 == STAGES ? 0 : fill + 1;
         };
         for (; kb < n_lean; kb++) turn([&]() { step(cur, kb, std::true_type{}); });
@@ -791,11 +850,15 @@ __global__ __launch_bounds__(256, 2) void attention_long_kernel(AttnArgs g) {
     }
 }
 
-template <int DC> static hipError_t launch_attention_long(const AttnArgs &g, int stacks, hipStream_t st) {
-    if (const hipError_t e = ensure_lds_limit<&attention_long_kernel<DC>>(); e != hipSuccess) return e;
-    hipLaunchKernelGGL((attention_long_kernel<DC>), dim3((unsigned)((g.q_len + AL_BQ - 1) / AL_BQ), (unsigned)stacks), dim3(256),
-                       (size_t)al_stages(DC) * 2 * AL_BK * DC * sizeof(half_t), st, g);
+template <int DC, int MK> static hipError_t launch_attention_long_k(const AttnArgs &g, int stacks, hipStream_t st) {
+    if (const hipError_t e = ensure_lds_limit<&attention_long_kernel<DC, MK>>(); e != hipSuccess) return e;
+    hipLaunchKernelGGL((attention_long_kernel<DC, MK>), dim3((unsigned)((g.q_len + AL_BQ - 1) / AL_BQ), (unsigned)stacks), dim3(256),
+                       (size_t)al_stages(DC, MK) * 2 * AL_BK * DC * sizeof(half_t), st, g);
     return hipGetLastError();
+}
+template <int DC> static hipError_t launch_attention_long(const AttnArgs &g, int stacks, hipStream_t st) {
+    if (!g.mask) return launch_attention_long_k<DC, 0>(g, stacks, st);
+    return g.mask_f32 ? launch_attention_long_k<DC, 1>(g, stacks, st) : launch_attention_long_k<DC, 2>(g, stacks, st);
 }
 
 // Second pass of a split launch: per row, the partial (maximum, sum, output) triples of the splits are
@@ -1116,9 +1179,9 @@ static uint64_t attention_decode_workspace_bytes(const rt_attention_desc &d) {
 }
 
 template <int DP, int MK, int DC, int NKQ> static hipError_t launch_attention_k(const AttnArgs &g, int stacks, hipStream_t st) {
-    constexpr int STAGES = MK == 2 ? 3 : at_stages(DP, NKQ);
+    constexpr int STAGES = MK == 3 ? 3 : at_stages(DP, NKQ);
     // the ring of packed key + value (+ mask) blocks; the merge of the key parts reuses it
-    const size_t stage = (size_t)2 * (32 * NKQ) * g.D * sizeof(half_t) + (MK == 2 ? (size_t)AT_BQ * (32 * NKQ) * (g.mask_f32 ? 4 : 2) : 0);
+    const size_t stage = (size_t)2 * (32 * NKQ) * g.D * sizeof(half_t) + (MK == 3 ? (size_t)AT_BQ * (32 * NKQ) * (g.mask_f32 ? 4 : 2) : 0);
     const size_t ring = STAGES * stage;
     const size_t merge = (size_t)(NKQ - 1) * 4 * (2 + 4 * (DP / 16)) * 64 * sizeof(float);
     const size_t lds = ring > merge ? ring : merge;
@@ -1144,26 +1207,34 @@ template <int DP, int MK, int DC, int NKQ> static hipError_t launch_attention_k(
 // head_dim 80, eight / sixteen wavefronts: 512 keys 10.0 / 10.7 us, 1024: 15.1 / 15.1, 1536: 21.3 / 20.1, 4096: 43.6 / 41.6;
 // 6 heads x 1500 x 1500 x 64 (Whisper): 17.8 / 15.8; 32 x 2048 x 2048 x 96 causal: 78.3 / 71.8
 RT_TUNABLE(g_attention_wide_from, 1280);
-RT_TUNABLE(g_attention_mask_direct, 0); // non-zero: a mask tensor is always read from memory where it is used (for comparisons)
 
 template <int DP, int MK, int DC> static hipError_t launch_attention_dm(const AttnArgs &g, int stacks, hipStream_t st) {
-    if constexpr (DP <= 96 && MK != 2) {
+    if constexpr (DP <= 96 && MK != 3) {
         if (g.splits == 1 && g.kv_len >= g_attention_wide_from) return launch_attention_k<DP, MK, DC, 4>(g, stacks, st);
     }
     return launch_attention_k<DP, MK, DC, 2>(g, stacks, st);
 }
 
+// whether a mask tensor's rows are whole 16-byte vectors
+static bool attention_stages_mask(const AttnArgs &g) {
+    const int64_t mrb = g.mask_rs * (g.mask_f32 ? 4 : 2);
+    return ((uintptr_t)g.mask & 15u) == 0 && mrb % 16 == 0 && mrb >= 16 && mrb < (int64_t(1) << 31);
+}
+
 // the kernel built for this head_dim (Whisper 64, Phi-2 80, Phi-3 96, Llama-class 128), else the one that takes it as an argument
 template <int DP, int DC> static hipError_t launch_attention_dp(const AttnArgs &g, int stacks, hipStream_t st) {
-    // a mask tensor whose rows are whole 16-byte vectors travels through the ring; any other is read where it is used
-    const int64_t mrb = g.mask_rs * (g.mask_f32 ? 4 : 2);
-    const int mk = !g.mask ? 0 : ((((uintptr_t)g.mask & 15u) == 0 && mrb % 16 == 0 && mrb >= 16 && mrb < (int64_t(1) << 31) && !g_attention_mask_direct) ? 2 : 1);
-    if (g.D == DC) {
-        if (mk == 2) return launch_attention_dm<DP, 2, DC>(g, stacks, st);
-        return mk ? launch_attention_dm<DP, 1, DC>(g, stacks, st) : launch_attention_dm<DP, 0, DC>(g, stacks, st);
-    }
-    if (mk == 2) return launch_attention_dm<DP, 2, 0>(g, stacks, st);
-    return mk ? launch_attention_dm<DP, 1, 0>(g, stacks, st) : launch_attention_dm<DP, 0, 0>(g, stacks, st);
+    // a mask tensor whose rows are whole 16-byte vectors travels through the ring; any other, and with sixteen wavefronts, a block ahead through registers
+    const int mk = !g.mask ? 0 : attention_stages_mask(g) ? 3 : g.mask_f32 ? 1 : 2;
+    auto go = [&](auto dc) -> hipError_t {
+        constexpr int D0 = decltype(dc)::value;
+        switch (mk) {
+        case 0: return launch_attention_dm<DP, 0, D0>(g, stacks, st);
+        case 1: return launch_attention_dm<DP, 1, D0>(g, stacks, st);
+        case 2: return launch_attention_dm<DP, 2, D0>(g, stacks, st);
+        default: return launch_attention_dm<DP, 3, D0>(g, stacks, st);
+        }
+    };
+    return g.D == DC ? go(std::integral_constant<int, DC>{}) : go(std::integral_constant<int, 0>{});
 }
 
 static int attention_dp(int head_dim) { return head_dim <= 64 ? 64 : (head_dim <= 96 ? 96 : 128); }
@@ -1247,7 +1318,14 @@ hipError_t launch_attention(const rt_attention_desc &d, const void *q, const voi
     // below four blocks the error there is the smaller one (1.02 times as large here at 64 keys, 1.01 at 130, 1.00 at 256).
     // Up to 64 rows the kernel with 64 of them per workgroup: half of the long one's wavefronts would have none (512 heads x 16
     // rows x 2048 keys x head_dim 64: 44.9 and 55.4 us; 65 rows 74 and 53).
-    if (!mask && g.splits == 1 && d.q_len > AT_BQ && d.kv_len >= 4 * AL_BK && 8 * (((int64_t)d.q_len + AL_BQ - 1) / AL_BQ * stacks) >= 7 * (int64_t)g.resident) {
+    // With a mask tensor from five sixteenths on, since it costs the other kernel more, and, where that one stages the mask, with a little more
+    // than a workgroup's rows for half the compute units (us, that one and this: 160 workgroups, 32 x 513 x 2001 x 128, 105 and 84; 192, 16 x 1500 x
+    // 1500 x 64, 49 and 44; 96, 16 x 703 x 703 x 96, 20 and 28; staged, 32 x 632 x 632 x 96 29 and 27, 40 x 400 x 400 x 80 20.9 and 22.5, 16 x 1024 x
+    // 1024 x 96 22 and 32).
+    const int64_t wgs = ((int64_t)d.q_len + AL_BQ - 1) / AL_BQ * stacks;
+    const bool many = !mask ? 8 * wgs >= 7 * (int64_t)g.resident
+                            : 16 * wgs >= 5 * (int64_t)g.resident && (!attention_stages_mask(g) || 20 * stacks * d.q_len >= 11 * (int64_t)dev.num_cus * AL_BQ);
+    if (g.splits == 1 && d.q_len > AT_BQ && d.kv_len >= 4 * AL_BK && many) {
         switch (d.head_dim) {
         case 64: return launch_attention_long<64>(g, (int)stacks, stream);
         case 80: return launch_attention_long<80>(g, (int)stacks, stream);
