@@ -341,7 +341,7 @@ RT_API rt_status rt_matmul_enqueue_ws(rt_ctx *ctx, const rt_matmul_desc *desc, c
  * tight serving loops, harnesses that forbid hipMalloc): the shares' partial sums go to a static
  * buffer of RT_STATIC_SCRATCH_BYTES that the library holds on each GPU it runs on, from
  * rt_ctx_create until the process ends.  Neither this call nor anything it launches allocates or
- * frees.  For f16 activations against f16 or Q8_0H weights, K a multiple of 256 of at least 2048 that
+ * frees.  For f16 activations against f16 or (more than 16 rows of them) Q8_0H weights, K a multiple of 256 of at least 2048 that
  * equal shares of at least 1024 could cut, and output tiles of 160 x 128 for at most half of the compute
  * units (which tiles and shares run, down to 512 of K, is the library's choice, as with a workspace):
  * their results are those of rt_matmul_enqueue_ws with a workspace of rt_matmul_workspace_bytes, bit

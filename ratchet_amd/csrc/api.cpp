@@ -385,7 +385,9 @@ rt_status rt_matmul_workspace_bytes(rt_ctx *ctx, const rt_matmul_desc *desc, uin
     std::string why;
     rt_status st = rt::make_spec(*desc, spec, p, &why);
     if (st != RT_OK) return fail(ctx, st, why);
-    // only the tiled kernels share a problem among workgroups; the streaming kernels take M <= 16
+    // only the tiled kernels share a problem among workgroups; of up to 16 vectors they take those whose K is too long for the streaming kernels
+    if (p.kernel == RT_KERNEL_GEMV_Q4K && p.N >= 3) *bytes = rt::gemm_q4k_workspace_bytes(p, ctx->dev);
+    if (p.kernel == RT_KERNEL_GEMV_Q8 && rt::gemm_nt_q8h_few(p, ctx->dev)) *bytes = rt::gemm_nt_workspace_bytes(p, ctx->dev);
     if (p.kernel == RT_KERNEL_GEMM_F16) *bytes = p.a_dt == RT_Q4_K ? rt::gemm_q4k_workspace_bytes(p, ctx->dev) : rt::gemm_nt_workspace_bytes(p, ctx->dev);
     if (p.kernel == RT_KERNEL_GEMM_F32) *bytes = rt::gemm_limb_workspace_bytes(p, ctx->dev);
     return RT_OK;
@@ -437,13 +439,13 @@ rt_status rt_matmul_enqueue_static(rt_ctx *ctx, const rt_matmul_desc *desc, cons
     uint64_t need = 0;
     const rt_status st = rt_matmul_workspace_bytes(ctx, desc, &need);
     if (st != RT_OK) return st;
-    // Not split, or not one of the products the buffer is for (f32 activations and Q4_K weights are not): no scratch is touched, and a
-    // program may have them in flight on several streams at once.
+    // Not split, or not one of the products the buffer is for (f32 activations, Q4_K weights and up to 16 vectors against Q8_0H ones are not): no
+    // scratch is touched, and a program may have them in flight on several streams at once.
     rt_gemm_spec spec;
     rt::Problem p;
     std::string why;
     if (need > 0 && rt::make_spec(*desc, spec, p, &why) != RT_OK) return fail(ctx, RT_ERR_INVALID_SHAPE, why);
-    if (need == 0 || (desc->lhs_dt != RT_F16 && desc->rhs_dt != RT_F16) || !rt::gemm_nt_static_split(p, ctx->dev))
+    if (need == 0 || (desc->lhs_dt != RT_F16 && desc->rhs_dt != RT_F16) || p.kernel != RT_KERNEL_GEMM_F16 || !rt::gemm_nt_static_split(p, ctx->dev))
         return rt_matmul_enqueue_ws(ctx, desc, lhs, rhs, bias, out, activation, nullptr, 0, stream);
     if (need > kStaticScratchBytes)
         return fail(ctx, RT_ERR_UNSUPPORTED,

@@ -179,6 +179,10 @@ bool gemm_nt_static_split(const Problem &p, const DeviceInfo &dev);
 bool gemv_chunks_unless_shared(const Problem &p, const DeviceInfo &dev);
 hipError_t gemv_chunks(const Problem &p, const void *A, const void *B, const void *bias, void *out, hipStream_t stream, const DeviceInfo &dev);
 bool gemv_q4k_mfma_fits(const Problem &p, const DeviceInfo &dev);
+bool gemv_q8h_mfma_well(const Problem &p, const DeviceInfo &dev);
+bool gemm_q4k_few(const Problem &p, const DeviceInfo &dev);
+bool gemm_nt_q8h_few(const Problem &p, const DeviceInfo &dev);
+bool gemv_q8h_few_leave(const Problem &p, const DeviceInfo &dev);
 bool gemm_stream_fills(int64_t M, const DeviceInfo &dev);
 hipError_t launch_gemm_nt(const Problem &p, const void *A, const void *B, const void *bias, void *out,
                           hipStream_t stream, const DeviceInfo &dev);

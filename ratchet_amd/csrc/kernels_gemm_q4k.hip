@@ -795,7 +795,7 @@ struct Q4kChoice {
     int ta = 2, ks = 1; // 16-row tiles per wavefront: 1, 2; 4: gemm_q4k_wide_kernel
 };
 static bool gemm_q4k_takes(const Problem &p) {
-    return p.a_dt == RT_Q4_K && p.act_dt == RT_F16 && p.K % 256 == 0 && p.K >= 256 && p.b_ks == 1 && p.M >= 64 && p.N >= 17 && p.stacks <= 65535;
+    return p.a_dt == RT_Q4_K && p.act_dt == RT_F16 && p.K % 256 == 0 && p.K >= 256 && p.b_ks == 1 && p.M >= 64 && p.N >= 3 && p.stacks <= 65535;
 }
 static Q4kChoice q4k_choose(const Problem &p, const DeviceInfo &dev, bool may_split) {
     // Four multiplying wavefronts of 32 weight rows x 64 activation rows each; when the grid of 16-row wavefronts
@@ -835,17 +835,27 @@ static Q4kChoice q4k_choose(const Problem &p, const DeviceInfo &dev, bool may_sp
 uint64_t gemm_q4k_workspace_bytes(const Problem &p, const DeviceInfo &dev) {
     if (!gemm_q4k_takes(p)) return 0;
     Problem chunk = p;
-    chunk.N = 16;
+    chunk.N = std::min<int64_t>(p.N, 16);
     if (p.N <= 32 && gemv_q4k_mfma_fits(chunk, dev)) return 0;
     const int ks = q4k_choose(p, dev, true).ks;
     return ks > 1 ? (uint64_t)p.stacks * ks * p.M * p.N * sizeof(float) : 0;
+}
+// Whether 3 to 16 vectors are launch_gemm_q4k's: where the streaming matrix-core kernel's LDS ends (9 to 16 from K = 4352, 3 to 8 from 8448 on), up to
+// 8, which the streaming kernel without matrix cores takes, only with K shared.  us, M x K, that or the generic kernel, here, here with K whole: 2560 x 4352 at 9
+// / 16 vectors 71 / 72, 10.3, 18.3; x 10240 161 / 163, 13.5, 38; x 14336 224 / 227, 16, 52; 1280 x 8448 at 3 / 8 15.6 / 23.5, 10.4, 32; 2560 x 10240 at 3 / 5 / 8 18.1 / 23.7 / 33.9,
+// 14.0, 38.
+bool gemm_q4k_few(const Problem &p, const DeviceInfo &dev) {
+    if (!gemm_q4k_takes(p) || p.N > 16 || gemv_q4k_mfma_fits(p, dev)) return false;
+    if (p.N > 8) return true;
+    const uint64_t need = gemm_q4k_workspace_bytes(p, dev);
+    return need > 0 && p.workspace && !((uintptr_t)p.workspace & 15u) && p.workspace_bytes >= need;
 }
 
 // Q4_K weights x K-contiguous f16 activations, more rows than one streaming launch takes.
 // hipErrorNotSupported: another kernel must take the problem.
 hipError_t launch_gemm_q4k(const Problem &p, const void *A, const void *B, const void *bias, void *out, hipStream_t stream,
                            const DeviceInfo &dev) {
-    if (g_gemm_q4k_disable || !gemm_q4k_takes(p)) return hipErrorNotSupported;
+    if (g_gemm_q4k_disable || !gemm_q4k_takes(p) || (p.N <= 16 && !gemm_q4k_few(p, dev))) return hipErrorNotSupported;
     if (((uintptr_t)A & 15u) || ((uintptr_t)B & 15u) || (p.b_js * 2) % 16 || (p.b_bs * 2) % 16) return hipErrorNotSupported;
     // 32-bit offsets within a stack, in bytes
     if (p.M * (p.K / 256) * 144 >= (int64_t(1) << 32) || p.N * p.b_js >= (int64_t(1) << 31)) return hipErrorNotSupported;

@@ -323,11 +323,23 @@ hipError_t launch_gemv_chunked(const Problem &p, const void *A, const void *B, c
     return gemv_chunks(p, A, B, bias, out, stream, dev);
 }
 
+// Whether launch_gemv leaves 5..8 vectors against Q8_0H weights to the kernels behind it (see there); launch_gemm_nt takes those without a workspace only then
+bool gemv_q8h_few_leave(const Problem &p, const DeviceInfo &dev) {
+    if (p.K % 256 != 0 || gemv_q8h_mfma_well(p, dev)) return false;
+    if (p.stacks == 1 && gemm_stream_fills(p.M, dev)) return true;
+    return gemm_nt_q8h_few(p, dev) && p.workspace && !((uintptr_t)p.workspace & 15u) && p.workspace_bytes >= gemm_nt_workspace_bytes(p, dev);
+}
+
 // Returns hipErrorNotSupported when the operands do not meet the alignment the
 // streaming kernels assume; the caller then takes the tiled GEMM, which has no
 // such requirement.
 hipError_t launch_gemv(const Problem &p, const void *A, const void *B, const void *bias, void *out,
                        hipStream_t stream, const DeviceInfo &dev) {
+    // 5..8 vectors whose K is more than the matrix-core kernel does well or at all: one pass over the weight in launch_gemm_stream where it fills the device
+    // (5120 x 10240 at 5 / 8 vectors 36 / 43 us here, 23 / 24 there), the tiles where they share K (gemm_nt_q8h_few)
+    if (p.kernel == RT_KERNEL_GEMV_Q8 && p.a_dt == RT_Q8_0H && p.N >= 5 && p.b_ks == 1 && aligned16(A) && aligned16(B) && (p.b_js * 2) % 16 == 0 && (p.b_bs * 2) % 16 == 0 &&
+        gemv_q8h_few_leave(p, dev))
+        return hipErrorNotSupported;
     if (p.kernel == RT_KERNEL_GEMV_Q8 && p.a_dt == RT_Q8_0H && !g_gemv_disable_mfma) {
         // f16 activations, one or two vectors: the row-streaming kernel; three or four: the row-streaming kernel on
         // the 4x4x4 matrix instruction; then the matrix-core kernel; shapes all of them decline fall through
@@ -345,6 +357,7 @@ hipError_t launch_gemv(const Problem &p, const void *A, const void *B, const voi
         p.b_ks == 1 && aligned16(A) && aligned16(B) && (p.b_js * 2) % 16 == 0)
         return hipErrorNotSupported;
     if (p.kernel == RT_KERNEL_GEMV_Q4K) {
+        if (p.N >= 3 && aligned16(A) && aligned16(B) && (p.b_js * 2) % 16 == 0 && (p.b_bs * 2) % 16 == 0 && gemm_q4k_few(p, dev)) return hipErrorNotSupported;
         // one vector: the row-streaming kernel; then the matrix-core kernel
         hipError_t e = launch_gemv_q4k_rowdot(p, A, B, bias, out, stream, dev);
         if (e != hipErrorNotSupported) return e;
@@ -358,9 +371,10 @@ hipError_t launch_gemv(const Problem &p, const void *A, const void *B, const voi
         // workgroup: the weight-streaming GEMM, or the tiled kernel's 64 x 64 tiles (10240 x 2560, weights from HBM:
         // 12.7 / 16 us against 19 / 24 / 26 us at 5 / 7 / 8 vectors here), from 6 vectors on where K ends in half a 64 (8192 x 2016: 10.5 us
         // against 9.9 / 15.0 at 5 / 8 vectors; 16384 x 544: 6.0 against 10.7 / 15.6); the conditions are the ones under which
-        // the tiled kernel takes the product
+        // the tiled kernel takes the product.  With fewer rows, where launch_gemm_stream takes it (4096 x 2560 at 5 / 8 vectors 7.1 / 9.7 us here, 5.6
+        // there, 3200 x 512 4.4 / 5.5 and 4.0 / 3.6, 5536 x 10240 26.9 / 38.4 and 20.6 / 21.4)
         if (p.a_dt == RT_F16 && p.act_dt == RT_F16 && p.N >= (p.K % 64 == 0 ? 5 : 6) && p.stacks == 1 && p.K > 256 && p.K % 32 == 0 &&
-            (p.M + 63) / 64 >= dev.num_cus / 2 && p.a_ks == 1 && p.b_ks == 1 && aligned16(A) && aligned16(B) &&
+            ((p.M + 63) / 64 >= dev.num_cus / 2 || (gemm_stream_fills(p.M, dev) && p.K % 256 == 0 && p.a_rs == p.K)) && p.a_ks == 1 && p.b_ks == 1 && aligned16(A) && aligned16(B) &&
             (p.a_rs * 2) % 16 == 0 && (p.b_js * 2) % 16 == 0 && !(p.o_js == 1 && p.o_is != 1))
             // (a row-major output would make the tiled kernel exchange the operands, and with the weight as its
             // activation side it declines: such a product stays here)

@@ -336,14 +336,58 @@ static hipError_t launch_rg(int rg, dim3 grid, int nwaves, size_t lds, hipStream
     }
 }
 
+struct Q8hShape {
+    int upw, nwaves, rg, rows_wg; // units per wavefront, wavefronts, row groups and rows per workgroup
+    size_t lds;
+};
+static Q8hShape q8h_shape(const Problem &p, const DeviceInfo &dev) {
+    const int nunits = (int)(p.K / kUnitK), NC = (int)p.N;
+    // Units per wavefront: as few as keeps the workgroup within 16 wavefronts.
+    int upw = g_gemv_mfma_upw;
+    if (upw == 0) upw = nunits <= 16 ? 1 : (nunits <= 32 ? 2 : 4);
+    while (upw < 4 && (nunits + upw - 1) / upw > 16) upw *= 2;
+    int nwaves = (nunits + upw - 1) / upw;
+    if (nwaves < 4) nwaves = 4;                   // the final sum uses 256 threads
+    // Rows per workgroup.  16 (one MFMA row group) while all workgroups are resident at once: more groups per
+    // workgroup mean more loads per wavefront and a longer tail after the last one returns.  With many vectors the
+    // activations' LDS leaves room for two workgroups per compute unit, or one, and the grid then runs in rounds
+    // (10240 rows, 16 vectors: 640 workgroups, one per compute unit = 3 rounds, 13.2 us).  There every compute unit
+    // gets one workgroup with its share of the rows, ceil(rows / num_cus) rounded up to 8, in up to four row groups
+    // the last of which may be half empty (40 rows per workgroup: 10.5 us; 9 / 12 vectors 11.0 / 11.4 -> 10.3 / 10.4;
+    // two workgroups of 24 rows per compute unit measured slower than either, 12.3 us at 9 vectors).
+    int rg = g_gemv_mfma_rg, rows_wg = 0;
+    if (rg == 0) {
+        rg = 1;
+        const size_t lds_x = (size_t)nwaves * NC * (upw * kUnitK + kXPad) * 2;
+        auto fit = [&](int r) { // workgroups of r row groups that fit a compute unit
+            const int by_lds = (int)((160 * 1024) / (lds_x + (size_t)nwaves * r * 1024)), by_waves = 32 / nwaves;
+            return by_lds < by_waves ? by_lds : by_waves;
+        };
+        if (upw == 1 && p.stacks == 1 && (p.M + 15) / 16 > (int64_t)dev.num_cus * fit(1)) {
+            const int64_t per = ((p.M + dev.num_cus - 1) / dev.num_cus + 7) & ~(int64_t)7;
+            if (per <= 64 && fit((int)(per + 15) / 16) >= 1) rows_wg = (int)per, rg = (rows_wg + 15) / 16;
+        }
+    }
+    if (upw * rg > 4) rg = 4 / upw > 0 ? 4 / upw : 1; // at most 16 weight loads in flight per lane
+    if (rows_wg == 0 || rows_wg > 16 * rg) rows_wg = 16 * rg;
+    return {upw, nwaves, rg, rows_wg, (size_t)nwaves * NC * (upw * kUnitK + kXPad) * 2 + (size_t)nwaves * rg * 1024};
+}
+// whether launch_gemv_q8h_mfma takes a Q8_0H product of this size, whatever its strides
+static bool gemv_q8h_mfma_fits(const Problem &p, const DeviceInfo &dev) {
+    if (p.N < 1 || p.N > 16 || p.K % kUnitK != 0 || p.K < kUnitK || p.K > 16384) return false;
+    const Q8hShape c = q8h_shape(p, dev);
+    return c.nwaves <= 16 && c.lds <= 160 * 1024;
+}
+// and, with five vectors and more, where it is still the fastest: with four units of K per wavefront its loads are too few (2560 x 10240 at 5 / 7
+// vectors 19.6 / 20 us, 15 on tiles that share K; x 8192, two units, 6.5 and 13.6)
+bool gemv_q8h_mfma_well(const Problem &p, const DeviceInfo &dev) { return gemv_q8h_mfma_fits(p, dev) && (p.N < 5 || p.K <= 8192); }
+
 // Q8_0H weights, f16 activations, 1..16 vectors, K a multiple of 256.
 // hipErrorNotSupported means the shape or alignment does not fit this kernel
 // and another one must run.
 hipError_t launch_gemv_q8h_mfma(const Problem &p, const void *A, const void *B, const void *bias, void *out,
                                 hipStream_t stream, const DeviceInfo &dev) {
-    if (p.a_dt != RT_Q8_0H || p.act_dt != RT_F16 || p.N < 1 || p.N > 16 || p.K % kUnitK != 0 || p.K < kUnitK)
-        return hipErrorNotSupported;
-    if (p.stacks > 65535 || p.K > 16384) return hipErrorNotSupported;
+    if (p.a_dt != RT_Q8_0H || p.act_dt != RT_F16 || p.stacks > 65535 || !gemv_q8h_mfma_fits(p, dev)) return hipErrorNotSupported;
     const int64_t bjs = p.N == 1 ? 0 : p.b_js;
     if (((uintptr_t)A & 15u) || ((uintptr_t)B & 15u) || (bjs * 2) % 16 || (p.b_bs * 2) % 16) return hipErrorNotSupported;
     if (p.b_ks != 1) return hipErrorNotSupported;
@@ -360,38 +404,8 @@ hipError_t launch_gemv_q8h_mfma(const Problem &p, const void *A, const void *B, 
     g.o_bs = p.o_bs, g.o_is = p.o_is, g.o_js = p.o_js;
     g.has_bias = p.has_bias, g.bias_on_rows = p.bias_on_rows, g.act = p.act, g.lin = g_gemv_mfma_lin;
 
-    // Units per wavefront: as few as keeps the workgroup within 16 wavefronts.
-    int upw = g_gemv_mfma_upw;
-    if (upw == 0) upw = g.nunits <= 16 ? 1 : (g.nunits <= 32 ? 2 : 4);
-    while (upw < 4 && (g.nunits + upw - 1) / upw > 16) upw *= 2;
-    int nwaves = (g.nunits + upw - 1) / upw;
-    if (nwaves > 16) return hipErrorNotSupported; // K > 16384
-    if (nwaves < 4) nwaves = 4;                   // the final sum uses 256 threads
-    // Rows per workgroup.  16 (one MFMA row group) while all workgroups are resident at once: more groups per
-    // workgroup mean more loads per wavefront and a longer tail after the last one returns.  With many vectors the
-    // activations' LDS leaves room for two workgroups per compute unit, or one, and the grid then runs in rounds
-    // (10240 rows, 16 vectors: 640 workgroups, one per compute unit = 3 rounds, 13.2 us).  There every compute unit
-    // gets one workgroup with its share of the rows, ceil(rows / num_cus) rounded up to 8, in up to four row groups
-    // the last of which may be half empty (40 rows per workgroup: 10.5 us; 9 / 12 vectors 11.0 / 11.4 -> 10.3 / 10.4;
-    // two workgroups of 24 rows per compute unit measured slower than either, 12.3 us at 9 vectors).
-    int rg = g_gemv_mfma_rg, rows_wg = 0;
-    if (rg == 0) {
-        rg = 1;
-        const size_t lds_x = (size_t)nwaves * g.NC * (upw * kUnitK + kXPad) * 2;
-        auto fit = [&](int r) { // workgroups of r row groups that fit a compute unit
-            const int by_lds = (int)((160 * 1024) / (lds_x + (size_t)nwaves * r * 1024)), by_waves = 32 / nwaves;
-            return by_lds < by_waves ? by_lds : by_waves;
-        };
-        if (upw == 1 && p.stacks == 1 && (p.M + 15) / 16 > (int64_t)dev.num_cus * fit(1)) {
-            const int64_t per = ((p.M + dev.num_cus - 1) / dev.num_cus + 7) & ~(int64_t)7;
-            if (per <= 64 && fit((int)(per + 15) / 16) >= 1) rows_wg = (int)per, rg = (rows_wg + 15) / 16;
-        }
-    }
-    if (upw * rg > 4) rg = 4 / upw > 0 ? 4 / upw : 1; // at most 16 weight loads in flight per lane
-    if (rows_wg == 0 || rows_wg > 16 * rg) rows_wg = 16 * rg;
+    const auto [upw, nwaves, rg, rows_wg, lds] = q8h_shape(p, dev);
     g.rows_wg = rows_wg;
-    const size_t lds = (size_t)nwaves * g.NC * (upw * kUnitK + kXPad) * 2 + (size_t)nwaves * rg * 1024;
-    if (lds > 160 * 1024) return hipErrorNotSupported;
     const int64_t groups = (p.M + rows_wg - 1) / rows_wg;
     if (groups > 0x7fffffff) return hipErrorNotSupported;
     dim3 grid((unsigned)groups, (unsigned)p.stacks);
