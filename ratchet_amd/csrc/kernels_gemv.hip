@@ -46,36 +46,26 @@ __device__ __forceinline__ void gemv_store(const GemvArgs &g, int64_t s, int64_t
 }
 
 // Loads 16 consecutive activations starting at x[k0] as floats.
-template <typename AT> __device__ __forceinline__ void load_x16(const AT *x, float (&xf)[16]);
-template <> __device__ __forceinline__ void load_x16<half_t>(const half_t *x, float (&xf)[16]) {
+__device__ __forceinline__ void load_x16(const half_t *x, float (&xf)[16]) {
     half8_t a = *(const half8_t *)x, b = *(const half8_t *)(x + 8);
 #pragma unroll
     for (int i = 0; i < 8; i++) xf[i] = (float)a[i], xf[8 + i] = (float)b[i];
 }
-template <> __device__ __forceinline__ void load_x16<float>(const float *x, float (&xf)[16]) {
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-        float4_t a = *(const float4_t *)(x + 4 * v);
-#pragma unroll
-        for (int i = 0; i < 4; i++) xf[4 * v + i] = a[i];
-    }
-}
-
 // ---------------------------------------------------------------------------
-// Q8_0 weights.  Chunk = 16 int8 (half a block) + the block's scale.
+// Q8_0H weights x f16 activations (what the matrix-core kernels decline).  Chunk = 16 int8 (half a block) + the block's scale.
 // ---------------------------------------------------------------------------
-template <typename AT, int NC, int U>
+template <int NC, int U>
 __global__ __launch_bounds__(kGemvThreads) void gemv_q8_kernel(GemvArgs g) {
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
     const int64_t s = blockIdx.y;
     // an operand's stack is either the full stack or 1 (broadcast)
     const int64_t sa = g.a_stack == 1 ? 0 : s, sb = g.b_stack == 1 ? 0 : s;
     const int nchunks = (int)(g.K >> 4);
-    const AT *x = (const AT *)g.X + sb * g.b_bs;
+    const half_t *x = (const half_t *)g.X + sb * g.b_bs;
     for (int64_t row = (int64_t)blockIdx.x * kGemvWaves + wave; row < g.M; row += (int64_t)gridDim.x * kGemvWaves) {
         const int64_t rowel = (sa * g.M + row) * g.K;
         const uint8_t *q = g.A + rowel;
-        const AT *sc = (const AT *)g.scales + (rowel >> 5);
+        const half_t *sc = (const half_t *)g.scales + (rowel >> 5);
         float acc[NC];
 #pragma unroll
         for (int j = 0; j < NC; j++) acc[j] = 0.f;
@@ -99,7 +89,7 @@ __global__ __launch_bounds__(kGemvThreads) void gemv_q8_kernel(GemvArgs g) {
 #pragma unroll
                     for (int j = 0; j < NC; j++) {
                         float xf[16];
-                        load_x16<AT>(x + j * g.b_js + 16 * (int64_t)c, xf);
+                        load_x16(x + j * g.b_js + 16 * (int64_t)c, xf);
                         float part = 0.f;
 #pragma unroll
                         for (int i = 0; i < 16; i++) part += wf[i] * xf[i];
@@ -110,7 +100,96 @@ __global__ __launch_bounds__(kGemvThreads) void gemv_q8_kernel(GemvArgs g) {
         }
 #pragma unroll
         for (int j = 0; j < NC; j++) acc[j] = wave_sum(acc[j]);
-        gemv_store<AT, NC>(g, s, row, lane, acc);
+        gemv_store<half_t, NC>(g, s, row, lane, acc);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Q8_0F weights x f32 activations.  A workgroup of four wavefronts takes four weight rows, wavefront w every fourth step of 256 k from the w-th
+// on; a lane takes four codes of each row and the four activations of each vector beside them, so that both come in runs of consecutive bytes (with
+// sixteen codes to a lane, its 64 bytes of activations are a line of their own in each of four loads, and every row asks
+// for them again), and an activation is read once for four rows.  A block's scale is applied to the sum of four products.
+// us at 1 / 2 / 4 / 8 vectors, with a row per wavefront and sixteen codes to a lane, and here: 10240 x 2560 10.6 / 17.0 / 31 / 62 and 7.1 / 9.0 / 12.1 / 17.8;
+// 2560 x 10240 10.5 / 17.6 / 32 / 57 and 9.5 / 10.3 / 13.1 / 19.1; 5536 x 2080 6.8 / 11.0 / 18.0 / 33 and 5.2 / 5.9 / 7.9 / 10.4.  Bound by the weight's bytes (4.2 TB/s at one
+// vector), then by the vector instructions: 84 for a lane's four codes of four rows against eight vectors, and by the loads of the activations.
+// ---------------------------------------------------------------------------
+constexpr int kQ8fRows = 4;
+template <int NC, int U>
+__global__ __launch_bounds__(kGemvThreads) void gemv_q8f_kernel(GemvArgs g) {
+    constexpr int R = kQ8fRows;
+    __shared__ float red[kGemvWaves][R][NC];
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int64_t s = blockIdx.y, sa = g.a_stack == 1 ? 0 : s, sb = g.b_stack == 1 ? 0 : s; // an operand's stack is either the full stack or 1 (broadcast)
+    const float *x = (const float *)g.X + sb * g.b_bs;
+    const int64_t row0 = (int64_t)blockIdx.x * R;
+    const uint8_t *q[R];
+    const float *sc[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) { // rows past the end repeat the last one; never stored
+        const int64_t el = (sa * g.M + min(row0 + r, g.M - 1)) * g.K;
+        q[r] = g.A + el, sc[r] = (const float *)g.scales + (el >> 5);
+    }
+    float acc[R][NC];
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int j = 0; j < NC; j++) acc[r][j] = 0.f;
+    const int K = (int)g.K, last = K - 4;
+    for (int k0 = 256 * wave; k0 < K; k0 += 256 * kGemvWaves * U) {
+        uint32_t w[U][R];
+        float d[U][R];
+#pragma unroll
+        for (int u = 0; u < U; u++) { // past the end: the row's last codes, left out below
+            const uint32_t k = (uint32_t)min(k0 + 256 * kGemvWaves * u + 4 * lane, last);
+#pragma unroll
+            for (int r = 0; r < R; r++) w[u][r] = __builtin_nontemporal_load((const uint32_t *)(q[r] + k)), d[u][r] = sc[r][k >> 5];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int k = k0 + 256 * kGemvWaves * u + 4 * lane;
+            if (k < K) {
+                float wf[R][4];
+#pragma unroll
+                for (int r = 0; r < R; r++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) wf[r][e] = (float)(int8_t)(w[u][r] >> (8 * e));
+#pragma unroll
+                for (int j = 0; j < NC; j++) {
+                    const float4_t xv = *(const float4_t *)(x + j * g.b_js + k);
+#pragma unroll
+                    for (int r = 0; r < R; r++) {
+                        float p = wf[r][0] * xv[0];
+#pragma unroll
+                        for (int e = 1; e < 4; e++) p = fmaf(wf[r][e], xv[e], p);
+                        acc[r][j] = fmaf(d[u][r], p, acc[r][j]);
+                    }
+                }
+            }
+        }
+    }
+    // the lanes' sums: halves and quarters of the wavefront swap, so that a quarter is left with one row, whose sixteen lanes then add up
+    float v[NC];
+#pragma unroll
+    for (int j = 0; j < NC; j++) {
+        auto add = [](auto p) { return __builtin_bit_cast(float, (uint32_t)p[0]) + __builtin_bit_cast(float, (uint32_t)p[1]); };
+        const float a = add(__builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, acc[0][j]), __builtin_bit_cast(uint32_t, acc[2][j]), false, false)); // rows 0 and 2
+        const float b = add(__builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, acc[1][j]), __builtin_bit_cast(uint32_t, acc[3][j]), false, false)); // 1 and 3
+        v[j] = add(__builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false));                          // quarter l / 16: row l / 16
+        v[j] += wave_dpp<0x128>(v[j]); // row_ror:8, 4, 2, 1
+        v[j] += wave_dpp<0x124>(v[j]);
+        v[j] += wave_dpp<0x122>(v[j]);
+        v[j] += wave_dpp<0x121>(v[j]);
+        if ((lane & 15) == j) red[wave][lane >> 4][j] = v[j];
+    }
+    __syncthreads();
+    if (t < R * NC) {
+        const int r = t / NC, j = t - r * NC;
+        if (row0 + r < g.M) {
+            float o = (red[0][r][j] + red[1][r][j]) + (red[2][r][j] + red[3][r][j]);
+            if (g.has_bias) o += ((const float *)g.bias)[g.bias_on_rows ? row0 + r : (int64_t)j];
+            ((float *)g.out)[s * g.o_bs + (row0 + r) * g.o_is + j * g.o_js] = rt_act(o, g.act);
+        }
     }
 }
 
@@ -154,8 +233,8 @@ __global__ __launch_bounds__(kGemvThreads) void gemv_q4k_kernel(GemvArgs g) {
 #pragma unroll
                 for (int j = 0; j < NC; j++) {
                     float xl[16], xh[16];
-                    load_x16<half_t>(x + j * g.b_js + k_lo, xl);
-                    load_x16<half_t>(x + j * g.b_js + k_hi, xh);
+                    load_x16(x + j * g.b_js + k_lo, xl);
+                    load_x16(x + j * g.b_js + k_hi, xh);
                     float part = 0.f;
 #pragma unroll
                     for (int i = 0; i < 16; i++) {
@@ -243,11 +322,11 @@ __global__ __launch_bounds__(kGemvThreads) void gemv_float_kernel(GemvArgs g) {
 // ---------------------------------------------------------------------------
 static inline bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
 
-template <int NC> static void launch_q8(int act_dt, dim3 grid, hipStream_t st, const GemvArgs &g) {
-    if (act_dt == RT_F16)
-        hipLaunchKernelGGL((gemv_q8_kernel<half_t, NC, 4>), grid, dim3(kGemvThreads), 0, st, g);
-    else
-        hipLaunchKernelGGL((gemv_q8_kernel<float, NC, 4>), grid, dim3(kGemvThreads), 0, st, g);
+template <int NC> static void launch_q8f(dim3 grid, hipStream_t st, const GemvArgs &g) {
+    hipLaunchKernelGGL((gemv_q8f_kernel<NC, (NC <= 4 ? 4 : 2)>), grid, dim3(kGemvThreads), 0, st, g);
+}
+template <int NC> static void launch_q8(dim3 grid, hipStream_t st, const GemvArgs &g) {
+    hipLaunchKernelGGL((gemv_q8_kernel<NC, 4>), grid, dim3(kGemvThreads), 0, st, g);
 }
 template <int NC> static void launch_q4k(dim3 grid, hipStream_t st, const GemvArgs &g) {
     hipLaunchKernelGGL((gemv_q4k_kernel<NC>), grid, dim3(kGemvThreads), 0, st, g);
@@ -405,7 +484,14 @@ hipError_t launch_gemv(const Problem &p, const void *A, const void *B, const voi
         if (!x_ok || !aligned16(A) || p.K % 32 != 0) return hipErrorNotSupported;
         const uint64_t numel = (uint64_t)p.a_stack * p.M * p.K;
         g.scales = (const uint8_t *)A + rt_q8_0_scale_offset(numel);
-        RT_DISPATCH_NC(p.N, launch_q8<NC>(p.act_dt, grid, stream, g));
+        if (p.a_dt == RT_Q8_0F) {
+            const int64_t groups = (p.M + kQ8fRows - 1) / kQ8fRows;
+            if (groups > 0x7fffffff || p.K > 0x7fffffff - 8192) return hipErrorNotSupported; // (its steps count in 32 bits)
+            grid.x = (unsigned)groups;
+            RT_DISPATCH_NC(p.N, launch_q8f<NC>(grid, stream, g));
+        } else {
+            RT_DISPATCH_NC(p.N, launch_q8<NC>(grid, stream, g));
+        }
         break;
     }
     case RT_KERNEL_GEMV_Q4K: {

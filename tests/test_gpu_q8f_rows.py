@@ -1,0 +1,50 @@
+"""Q8_0F weights against 1 to 8 f32 vectors (gemv_q8f_kernel): weight rows that end inside a workgroup's four, K that ends inside a step of 256 and inside
+the four wavefronts' steps, stacks, both orders of the output, bias along either axis, infinities, against float64.
+
+The tolerance: a product is rounded once, four of them and their scale's make five roundings, a lane adds one sum per 1024 k, and ten additions
+join the lanes and wavefronts: 2^-24 of the magnitudes for each, and one for the bias."""
+import numpy as np
+import pytest
+import torch
+
+from ratchet_amd import DType, Tensor
+
+pytestmark = pytest.mark.gpu
+
+
+def make(m, k, rng, s=1):
+    codes = rng.integers(-128, 128, (s * m, k), dtype=np.int8)
+    d = rng.uniform(0.5, 2, (s * m, k // 32)).astype(np.float32) / 128
+    pad = lambda b: np.concatenate([b, np.zeros(-len(b) % 256, np.uint8)])
+    raw = np.concatenate([pad(codes.reshape(-1).view(np.uint8)), pad(d.reshape(-1).view(np.uint8))])
+    return raw, codes.astype(np.float64) * np.repeat(d.astype(np.float64), 32, axis=1)
+
+
+@pytest.mark.parametrize("n", range(1, 9))
+@pytest.mark.parametrize("stack,m,k", [((), 1, 32), ((), 3, 96), ((), 5, 256), ((), 1001, 288), ((), 66, 1024), ((), 7, 1056), ((), 130, 4128), ((3,), 9, 640)])
+def test_against_float64(device, stack, m, k, n):
+    rng = np.random.default_rng(m + k + n)
+    s = stack[0] if stack else 1
+    raw, w = make(m, k, rng, s)
+    w = w.reshape(s, m, k)
+    x, bias = rng.standard_normal((*stack, n, k)).astype(np.float32), rng.standard_normal(m).astype(np.float32)
+    W, X = Tensor.from_quantized(raw, DType.Q8_0F, (*stack, m, k), device), Tensor.from_data(x, None, device)
+    for to in (True, False):
+        b = bias if to else rng.standard_normal(n).astype(np.float32)
+        got = W.gemm(X, Tensor.from_data(b, None, device), False, True, to).resolve().storage.view(torch.float32)[: s * m * n].cpu().numpy().astype(np.float64)
+        got = got.reshape(s, n, m) if to else got.reshape(s, m, n).transpose(0, 2, 1)
+        for i in range(s):
+            xd = x.reshape(s, n, k)[i].astype(np.float64)
+            want = xd @ w[i].T + (b[None, :] if to else b[:, None])
+            mag = np.abs(xd) @ np.abs(w[i]).T
+            assert (np.abs(got[i] - want) <= 2.0**-24 * ((k / 1024 + 16) * mag + np.abs(want))).all(), (np.abs(got[i] - want) / mag).max() * 2**24
+
+
+def test_infinite_activation(device):
+    """Only the outputs of its vector are touched, also where it stands past another lane's end of the row."""
+    raw, w = make(10, 288, np.random.default_rng(1))
+    x = np.ones((3, 288), np.float32)
+    x[1, 287] = np.inf
+    out = Tensor.from_quantized(raw, DType.Q8_0F, (10, 288), device).gemm(Tensor.from_data(x, None, device), None, False, True, True).resolve()
+    out = out.storage.view(torch.float32)[:30].view(3, 10).cpu().numpy()
+    assert np.isfinite(out[[0, 2]]).all() and (out[1] == np.where(w[:, 287] == 0, np.nan, np.sign(w[:, 287]) * np.inf))[w[:, 287] != 0].all()
