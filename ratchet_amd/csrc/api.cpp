@@ -136,7 +136,7 @@ rt_status lower_matmul(rt_ctx *ctx, const rt_matmul_desc &desc, int32_t activati
 using Launcher = hipError_t (*)(const rt::Problem &, const void *, const void *, const void *, void *, hipStream_t,
                                 const rt::DeviceInfo &);
 constexpr Launcher kLaunchers[] = {rt::launch_gemv,          // streaming kernels
-                                   rt::launch_gemv_chunked,  // Q8_0H / Q4_K weights against a few vectors more than one streaming launch takes
+                                   rt::launch_gemv_chunked,  // quantized weights against a few vectors more than one streaming launch takes
                                    rt::launch_gemm_stream,   // f16 / Q8_0H weights against a few dozen activation rows: one pass over the weight
                                    rt::launch_gemm_nt,       // K-contiguous f16 / Q8_0H problems: the large-tile kernel
                                    rt::launch_gemm_nn_smalln, // f16 products with an untransposed narrow rhs (attention P.V)

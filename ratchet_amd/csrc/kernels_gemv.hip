@@ -11,6 +11,8 @@
 // ops/gemm.rs:342-492 which the reference uses for those shapes.
 #include "device_common.h"
 
+#include <algorithm>
+
 namespace rt {
 
 struct GemvArgs {
@@ -395,7 +397,27 @@ static bool q8h_between(const Problem &p, const DeviceInfo &dev) {
 bool gemv_chunks_unless_shared(const Problem &p, const DeviceInfo &dev) {
     return q8h_between(p, dev) && p.N > 16 && p.N <= 32 && gemm_nt_workspace_bytes(p, dev) > 0;
 }
+// 9 to 16 vectors against a small Q8_0F weight: two launches of the streaming kernel, each of which reads the weight at the rate of a launch of few
+// bytes, where the limb kernel splits K over a workspace and merges, or without one walks all of it (us at 9 / 16 vectors, the limb kernel with a
+// workspace, without, and two launches: 1001 x 4096 21.0 / 22.6, 69 and 8.9 / 11.0; 512 x 10240 21.0 / 22.1, 166 and 15.2 / 18.9; 4096 x 1280 12.9 / 13.1,
+// 25 and 9.6 / 10.9; 384 x 1536 12.5, 28 and 6.8 / 7.7).  Beyond 4096 rows or five million codes that kernel fills the device and reads the codes
+// once (4096 x 2560 15.4, here 12.6 / 17.1; 8192 x 640 13.5, here 11.3 / 14.7).  From K = 1024 on, since the sums are no less exact there (relative error
+// against float64 at K = 800 / 1280 / 2048 / 4096 here 9.4e-8 / 9.5e-8 / 9.6e-8 / 9.9e-8, there 9.2e-8 / 9.8e-8 / 1.08e-7 / 1.29e-7).
+static bool gemv_q8f_chunks(const Problem &p) {
+    return p.a_dt == RT_Q8_0F && p.act_dt == RT_F32 && p.N > kGemvMaxCols && p.N <= 2 * kGemvMaxCols && p.stacks == 1 && p.b_ks == 1 && p.K >= 1024 &&
+           p.M <= 4096 && p.M * p.K <= 5 << 20;
+}
 hipError_t launch_gemv_chunked(const Problem &p, const void *A, const void *B, const void *bias, void *out, hipStream_t stream, const DeviceInfo &dev) {
+    if (gemv_q8f_chunks(p)) {
+        for (int64_t j0 = 0; j0 < p.N; j0 += kGemvMaxCols) {
+            Problem c = p;
+            c.N = std::min<int64_t>(p.N - j0, kGemvMaxCols), c.kernel = RT_KERNEL_GEMV_Q8;
+            const float *bc = bias && !p.bias_on_rows ? (const float *)bias + j0 : (const float *)bias;
+            // what it declines (a misaligned operand) it declines on the first chunk
+            if (const hipError_t e = launch_gemv(c, A, (const float *)B + j0 * p.b_js, bc, (float *)out + j0 * p.o_js, stream, dev); e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
     if (p.a_dt == RT_Q8_0H && p.K % 256 == 0 && p.stacks == 1 && (p.M + 63) / 64 >= dev.num_cus / 4 &&
         (!q8h_between(p, dev) || gemv_chunks_unless_shared(p, dev)))
         return hipErrorNotSupported;

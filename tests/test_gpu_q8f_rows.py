@@ -2,7 +2,7 @@
 the four wavefronts' steps, stacks, both orders of the output, bias along either axis, infinities, against float64.
 
 The tolerance: a product is rounded once, four of them and their scale's make five roundings, a lane adds one sum per 1024 k, and ten additions
-join the lanes and wavefronts: 2^-24 of the magnitudes for each, and one for the bias."""
+join the lanes and wavefronts: 2^-24 of the magnitudes for each, and one for the bias.  The limb kernel adds a sum per MFMA of 32 k."""
 import numpy as np
 import pytest
 import torch
@@ -38,6 +38,26 @@ def test_against_float64(device, stack, m, k, n):
             want = xd @ w[i].T + (b[None, :] if to else b[:, None])
             mag = np.abs(xd) @ np.abs(w[i]).T
             assert (np.abs(got[i] - want) <= 2.0**-24 * ((k / 1024 + 16) * mag + np.abs(want))).all(), (np.abs(got[i] - want) / mag).max() * 2**24
+
+
+@pytest.mark.parametrize("n", (9, 15, 16, 17))
+@pytest.mark.parametrize("m,k", [(1, 1024), (4096, 1024), (4097, 1024), (33, 992), (1279, 4096), (1281, 4096), (130, 4128)])
+def test_two_launches(device, m, k, n):
+    """9 to 16 vectors go in two launches at K >= 1024, up to 4096 rows and 5 x 2^20 codes: on both sides of each of these, the vectors also 4 bytes past an
+    aligned address (the limb kernel takes those)."""
+    rng = np.random.default_rng(m + k + n)
+    raw, w = make(m, k, rng)
+    x, bm, bn = (rng.standard_normal(s).astype(np.float32) for s in ((n, k), m, n))
+    W = Tensor.from_quantized(raw, DType.Q8_0F, (m, k), device)
+    room = torch.zeros(4 * n * k + 16, dtype=torch.uint8, device="cuda:0")
+    room[4 : 4 + 4 * n * k] = torch.from_numpy(x.view(np.uint8).reshape(-1)).to("cuda:0")
+    xd = x.astype(np.float64)
+    mag = np.abs(xd) @ np.abs(w).T
+    for X in (Tensor.from_data(x, None, device), Tensor((n, k), DType.F32, device, room[4 : 4 + 4 * n * k])):
+        for to in (True, False):
+            got = W.gemm(X, Tensor.from_data(bm if to else bn, None, device), False, True, to).resolve().storage.view(torch.float32)[: m * n].cpu().numpy().astype(np.float64)
+            got, want = (got.reshape(n, m), xd @ w.T + bm[None, :]) if to else (got.reshape(m, n).T, xd @ w.T + bn[:, None])
+            assert (np.abs(got - want) <= 2.0**-24 * ((k / 32 + 16) * mag + np.abs(want))).all(), (np.abs(got - want) / mag).max() * 2**24
 
 
 def test_infinite_activation(device):
