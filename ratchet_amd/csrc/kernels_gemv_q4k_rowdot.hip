@@ -27,6 +27,8 @@
 // crates/ratchet-loader/src/k_quants.rs:94-103); role in the reference: ops/gemv.rs:333-558.
 #include "device_common.h"
 
+#include <algorithm>
+
 namespace rt {
 
 struct GemvQ4kRowdotArgs {
@@ -210,12 +212,12 @@ static hipError_t launch_q4k_rowdot_w(dim3 grid, size_t lds, hipStream_t st, con
 
 template <int STEPS>
 static hipError_t launch_q4k_rowdot_s(int waves, int rows, dim3 grid, size_t lds, hipStream_t st, const GemvQ4kRowdotArgs &g) {
+    if constexpr (STEPS < 4)
+        if (rows == 4) return waves == 4 ? launch_q4k_rowdot_w<STEPS, 4, 4>(grid, lds, st, g) : launch_q4k_rowdot_w<STEPS, 2, 4>(grid, lds, st, g);
     if (waves == 4) {
-        if (rows == 4) return launch_q4k_rowdot_w<STEPS, 4, 4>(grid, lds, st, g);
         if (rows == 2) return launch_q4k_rowdot_w<STEPS, 4, 2>(grid, lds, st, g);
         return launch_q4k_rowdot_w<STEPS, 4, 1>(grid, lds, st, g);
     }
-    if (rows == 4) return launch_q4k_rowdot_w<STEPS, 2, 4>(grid, lds, st, g);
     if (rows == 2) return launch_q4k_rowdot_w<STEPS, 2, 2>(grid, lds, st, g);
     return launch_q4k_rowdot_w<STEPS, 2, 1>(grid, lds, st, g);
 }
@@ -231,11 +233,19 @@ hipError_t launch_gemv_q4k_rowdot(const Problem &p, const void *A, const void *B
     const uint32_t nsb = (uint32_t)(p.K / 256), nvec = 9u * nsb;
     const int steps = (int)((nvec + 63) / 64);
     if (steps > 6) return hipErrorNotSupported;
-    // rows per wavefront and wavefronts per workgroup: the most that still give the grid three workgroups per compute unit
-    int waves = 4, rows = 4;
-    while (rows > 1 && (p.M + waves * rows - 1) / (waves * rows) * p.stacks < 3 * (int64_t)dev.num_cus) rows >>= 1;
-    if (rows == 1 && (p.M + waves - 1) / waves * p.stacks < 3 * (int64_t)dev.num_cus) waves = 2;
-    if (g_gemv_q4k_rowdot_rows > 0) rows = g_gemv_q4k_rowdot_rows;
+    // rows per wavefront and wavefronts per workgroup: the most that still give the grid three workgroups per compute unit.  From four steps per row on,
+    // no more than two rows: four rows' vectors leave registers for two wavefronts per SIMD (four and five steps) or one (six), and too few loads are in
+    // flight (us with four rows / two: 16384 x 8192 30.6 / 22.9, 16384 x 10240 37.3 / 27.2, 14336 x 7168 17.7 / 15.4, 16384 x 6144 17.1 / 16.1; three steps,
+    // 16384 x 5120, 12.5 / 12.4).  With five or six steps a compute unit holds three workgroups of one row or two of two: where the first would leave a
+    // part of the grid for a second turn and the second would not, two rows (us with one / two: 4096 x 8192 7.9 / 6.8, 3080 x 8192 7.3 / 6.8, 4096 x 10240
+    // 8.9 / 8.1; where both leave some, 5120 x 8192, 9.3 / 10.5).
+    const int64_t cus = dev.num_cus;
+    const auto groups_of = [&](int w, int r) { return (p.M + w * r - 1) / (w * r) * p.stacks; };
+    int waves = 4, rows = steps >= 4 ? 2 : 4;
+    while (rows > 1 && groups_of(waves, rows) < 3 * cus) rows >>= 1;
+    if (steps >= 5 && rows == 1 && groups_of(waves, 1) > 3 * cus && groups_of(waves, 2) <= 2 * cus) rows = 2;
+    if (rows == 1 && groups_of(waves, 1) < 3 * cus) waves = 2;
+    if (g_gemv_q4k_rowdot_rows > 0) rows = steps >= 4 ? std::min(g_gemv_q4k_rowdot_rows, 2) : g_gemv_q4k_rowdot_rows;
     if (g_gemv_q4k_rowdot_waves > 0) waves = g_gemv_q4k_rowdot_waves;
     const int64_t groups = (p.M + waves * rows - 1) / (waves * rows);
     if (groups > 0x7fffffff) return hipErrorNotSupported;
