@@ -1,6 +1,7 @@
 // Q4_K weights x f16 activations for many activation rows (prefill), the weights never touching LDS:
 // every multiplying wavefront decodes the raw blocks of its own 32 weight rows in registers, straight
-// into the MFMA operand, and only the activation tile goes through LDS.
+// into the MFMA operand, and only the activation tile goes through LDS.  Where its 256 x 128 tiles fill
+// the device a second kernel (gemm_q4k_wide_kernel, below) takes both through LDS, the blocks raw.
 //
 //   y[j, i] = sum_sb ( d_i,sb * sum_sub sum_{k in sub} x[j,k] (sc_i,sub q_i,k)  -  dmin_i,sb * sum_sub mn_i,sub S[j,sub] )
 //   S[j, sub] = sum_{k in sub} x[j, k]

@@ -4,7 +4,8 @@
 // from HBM into registers with 128-bit loads and dequantized in registers;
 // there is no LDS staging of weights.  One wavefront owns one row at a time
 // and its 64 lanes stride the row in 16-byte chunks, so every load
-// instruction of a wavefront covers 1 KiB of contiguous weights.
+// instruction of a wavefront covers 1 KiB of contiguous weights; Q8_0F
+// weights have a workgroup per four rows (gemv_q8f_kernel).
 //
 // Roles in the reference: ops/gemv.rs:156-574 (the workgroup and subgroup
 // GEMV generators) and, for 2..8 activation rows, the scalar QGEMM of

@@ -382,6 +382,15 @@ static bool gemv_q8h_mfma_fits(const Problem &p, const DeviceInfo &dev) {
 // vectors 19.6 / 20 us, 15 on tiles that share K; x 8192, two units, 6.5 and 13.6)
 bool gemv_q8h_mfma_well(const Problem &p, const DeviceInfo &dev) { return gemv_q8h_mfma_fits(p, dev) && (p.N < 5 || p.K <= 8192); }
 
+// Whether 5 to 16 vectors against Q8_0H weights are launch_gemm_nt's with K shared: where the streaming matrix-core kernel's LDS ends (9 to 16 from K = 5120
+// on) or its loads are few (from 8448 on) and the weights do not fill launch_gemm_stream, which needs no workspace.  us, M x K, before and here: 2560 x 5120 at 16 vectors 22.5 and 11.0, x 8192 at 9 / 16
+// 35.2 and 13.5, x 10240 at 5 / 8 / 16 19.6 / 24.4 / 42.9 and 15.2, 1280 x 14336 19.8 / 21.6 / 58 and 12.6.
+bool gemm_nt_q8h_few(const Problem &p, const DeviceInfo &dev) {
+    if (p.a_dt != RT_Q8_0H || p.act_dt != RT_F16 || p.N < 5 || p.N > 16 || p.K % 256 != 0 || p.b_ks != 1 || gemv_q8h_mfma_well(p, dev)) return false;
+    if (p.N <= 8 && p.M < 512) return false; // 200 x 14336 at 6 vectors 10.9 us there, 11.4 here
+    return !(p.stacks == 1 && gemm_stream_fills(p.M, dev)) && gemm_nt_workspace_bytes(p, dev) > 0;
+}
+
 // Q8_0H weights, f16 activations, 1..16 vectors, K a multiple of 256.
 // hipErrorNotSupported means the shape or alignment does not fit this kernel
 // and another one must run.
