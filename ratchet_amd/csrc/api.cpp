@@ -89,6 +89,11 @@ struct DeviceGuard {
     bool ok = false;
     explicit DeviceGuard(int ordinal) {
         if (hipGetDevice(&prev) != hipSuccess) prev = -1;
+        // the usual case: nothing to set, nothing to put back (the two hipSetDevice were 0.57 of 4.28 us per rt_matmul_enqueue_ws)
+        if ((ok = prev == ordinal)) {
+            prev = -1;
+            return;
+        }
         ok = hipSetDevice(ordinal) == hipSuccess;
     }
     ~DeviceGuard() {
