@@ -20,7 +20,7 @@
 // 8 values of sub-block 2 g (t < 4) or 2 g + 1 (t >= 4) of activation row lane % 16, so four dot
 // products against ones per step give S for exactly the (row, sub-block pair) that the min-term MFMA
 // wants from this lane.  Wavefront w sums the 16 activation rows of fragment w and shares them
-// through LDS (f16 high + low parts, exact to 2^-22); the min term of super-block sb is one MFMA per
+// through LDS (two f16 parts, q4k_sum_parts); the min term of super-block sb is one MFMA per
 // output tile, run under super-block sb + 1.
 //
 // A workgroup owns 128 weight rows x 64 activation rows: four multiplying wavefronts (32 weight rows
@@ -81,6 +81,21 @@ constexpr int QR_XSB = QR_BN * QR_ROWB; // bytes per stage = 33 LDS-DMA instruct
 constexpr int QR_XST = 2;
 constexpr size_t QR_LDS = (size_t)QR_XST * QR_XSB + 2 * QR_BN * 4 * 8;
 
+// Sums of x as MFMA operands.  32 f16 activations sum to up to 32 * 65504, so it is S / 32 that is held (dot products against 1 / 32, which are
+// exact; dmin takes the 32): h = S / 32 rounded to f16, and l = (S / 32 - h) * 2^11 rounded, against mn and mn * 2^-11, both exact.  Neither part
+// can overflow, and h + l * 2^-11 is S to 23 bits, one less than f32 (and S itself below 1 / 2).  Without the scales a sum beyond 2 * 65504 was cut
+// off there.  Relative error of the f32 sums against float64, 2560 x 10240 at 16 rows, before and now: activations N(0, 1) 2.77e-7 and 2.71e-7, their
+// absolute values 3.3e-6 and 2.6e-6, those times 4096 0.40 and 2.6e-6.
+constexpr float kQ4kSumDiv = 32.0f, kQ4kSumLow = 2048.0f;
+__device__ __forceinline__ uint2_t q4k_sum_parts(float s0, float s1) { // of two sums, divided by 32: (h, h), (l, l)
+    const half2_t h = {(half_t)s0, (half_t)s1};
+    const half2_t l = {(half_t)((s0 - (float)h[0]) * kQ4kSumLow), (half_t)((s1 - (float)h[1]) * kQ4kSumLow)};
+    return uint2_t{__builtin_bit_cast(uint32_t, h), __builtin_bit_cast(uint32_t, l)};
+}
+__device__ __forceinline__ uint32_t q4k_low_mins(uint32_t mn) { // what the low parts are multiplied with
+    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, mn) * half2_t{(half_t)(1 / kQ4kSumLow), (half_t)(1 / kQ4kSumLow)});
+}
+
 // TA: MFMA tiles of weight rows per wavefront; MW: multiplying wavefronts (4: each sums the activation fragment of its number);
 // LW: wavefronts that only issue the LDS-DMA (4, one per SIMD, or none: the multiplying ones issue it)
 template <int TA, int MW, int LW>
@@ -90,7 +105,7 @@ __global__ __launch_bounds__(64 * (MW + LW), 2) void gemm_q4k_kernel(GemmQ4kArgs
     static_assert(MW == 4, "wavefront w sums the x of activation fragment w: four fragments, four wavefronts");
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     uint8_t *Xs = smem;                             // [QR_XST][64 rows][33 slots of 16 bytes]: K-vector v of row r in slot v
-    uint2_t *Sx = (uint2_t *)(Xs + QR_XST * QR_XSB); // [2][64][4]: sums of x of super-block parity p, row, lane group: (high pair, low pair)
+    uint2_t *Sx = (uint2_t *)(Xs + QR_XST * QR_XSB); // [2][64][4]: sums of x of super-block parity p, row, lane group: q4k_sum_parts
 
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -176,7 +191,7 @@ __global__ __launch_bounds__(64 * (MW + LW), 2) void gemm_q4k_kernel(GemmQ4kArgs
         half2_t s_lo, n_lo, s_hi, n_hi;
     };
     struct Fin {
-        float d, dmin;
+        float d, dmin; // dmin * 32
         uint32_t mn;
     };
     const int sh = 16 * (fg & 1);
@@ -194,7 +209,7 @@ __global__ __launch_bounds__(64 * (MW + LW), 2) void gemm_q4k_kernel(GemmQ4kArgs
         sc.s_lo = half2_t{lo, lo}, sc.s_hi = half2_t{hi, hi};
         sc.n_lo = sc.s_lo * (half_t)-1024.0f, sc.n_hi = sc.s_hi * (half_t)-1024.0f;
         const half2_t dm = __builtin_bit_cast(half2_t, r.hdr[0]);
-        f.d = (float)dm[0], f.dmin = (float)dm[1], f.mn = __builtin_bit_cast(uint32_t, m2);
+        f.d = (float)dm[0], f.dmin = (float)dm[1] * kQ4kSumDiv, f.mn = __builtin_bit_cast(uint32_t, m2);
     };
     // weight fragment of step T: 8 values sc * q of this thread's row
     auto wfrag = [&](auto Tc, const Raw &r, const Scl &sc) {
@@ -259,7 +274,7 @@ __global__ __launch_bounds__(64 * (MW + LW), 2) void gemm_q4k_kernel(GemmQ4kArgs
     const uint32_t xlane = (uint32_t)(QR_ROWB * fr + 128 * fg);
     uint2_t *sx_mine = Sx + (16 * wave + fr) * 4 + fg;
     sx_mine[QR_BN * 4] = uint2_t{0u, 0u}; // parity 1 is read (against zero mins) under super-block 0
-    const half2_t ones = {(half_t)1.0f, (half_t)1.0f};
+    const half2_t part32 = {(half_t)(1 / kQ4kSumDiv), (half_t)(1 / kQ4kSumDiv)};
 
     // The min term of the super-block before (parity Q) and its fold into the accumulators.
     auto read_sums = [&](int Q, uint2_t (&hl)[TB]) {
@@ -273,7 +288,7 @@ __global__ __launch_bounds__(64 * (MW + LW), 2) void gemm_q4k_kernel(GemmQ4kArgs
             const half8_t sf = __builtin_bit_cast(half8_t, uint4_t{hl[bq][0], hl[bq][1], 0u, 0u});
 #pragma unroll
             for (int a = 0; a < TA; a++) {
-                const half8_t mf = __builtin_bit_cast(half8_t, uint4_t{fin[Q][a].mn, fin[Q][a].mn, 0u, 0u});
+                const half8_t mf = __builtin_bit_cast(half8_t, uint4_t{fin[Q][a].mn, q4k_low_mins(fin[Q][a].mn), 0u, 0u});
                 const float4_t T = __builtin_amdgcn_mfma_f32_16x16x32_f16(sf, mf, zero, 0, 0, 0);
 #pragma unroll
                 for (int r = 0; r < 4; r++) acc[a][bq][r] = fmaf(-fin[Q][a].dmin, T[r], fmaf(fin[Q][a].d, P[Q][a][bq][r], acc[a][bq][r]));
@@ -310,7 +325,9 @@ __global__ __launch_bounds__(64 * (MW + LW), 2) void gemm_q4k_kernel(GemmQ4kArgs
         // of their MFMAs, one read in front of every second MFMA, one right behind every MFMA (where a bare loop of
         // MFMAs, packed FMAs and fragment reads issues them for 2 ns instead of 10: bench.py --issue-calibration);
         // with two weight tiles per wavefront all were the same or up to 4 % slower, with one tile the last was
-        // 6 % faster.
+        // 6 % faster.  Below two places are pinned where there are loading wavefronts, with which the compiler otherwise spreads a
+        // super-block over more registers than there are (8192 x 3072 at 200 rows, two weight tiles, without / with 25.6 / 20.8 us, 6144 x 2048 at 240 19.0 /
+        // 15.3; one tile, 8192 x 3072 at 128 rows, 14.8 / 14.4).
         auto mfma_step = [&](auto Tc) {
             constexpr int T = decltype(Tc)::value;
             if constexpr (T < 7) xread(T + 1, xf[(T + 1) & 1]);
@@ -325,20 +342,19 @@ __global__ __launch_bounds__(64 * (MW + LW), 2) void gemm_q4k_kernel(GemmQ4kArgs
             const half8_t xs0 = xf[T & 1][0];
             float &S = T < 4 ? S0 : S1;
 #pragma unroll
-            for (int c = 0; c < 4; c++) S = __builtin_amdgcn_fdot2(half2_t{xs0[2 * c], xs0[2 * c + 1]}, ones, S, false);
+            for (int c = 0; c < 4; c++) S = __builtin_amdgcn_fdot2(half2_t{xs0[2 * c], xs0[2 * c + 1]}, part32, S, false);
         };
         mfma_step(std::integral_constant<int, 0>{});
         mfma_step(std::integral_constant<int, 1>{});
         mfma_step(std::integral_constant<int, 2>{});
         mfma_step(std::integral_constant<int, 3>{});
+        if (TA == 2 && LW > 0) __builtin_amdgcn_sched_barrier(0);
         mfma_step(std::integral_constant<int, 4>{});
         mfma_step(std::integral_constant<int, 5>{});
         mfma_step(std::integral_constant<int, 6>{});
         mfma_step(std::integral_constant<int, 7>{});
-        // high part: the sum truncated to f16 (any f16 near it will do); low part: the exact remainder, rounded
-        const half2_t h = __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_pkrtz(S0, S1));
-        const half2_t l = __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_pkrtz(S0 - (float)h[0], S1 - (float)h[1]));
-        sx_mine[PP * QR_BN * 4] = uint2_t{__builtin_bit_cast(uint32_t, h), __builtin_bit_cast(uint32_t, l)};
+        if (TA == 1) __builtin_amdgcn_sched_barrier(0);
+        sx_mine[PP * QR_BN * 4] = q4k_sum_parts(S0, S1);
         xcur = xcur == QR_XST - 1 ? 0 : xcur + 1;
     };
 

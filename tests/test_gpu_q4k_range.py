@@ -1,0 +1,45 @@
+"""Q4_K products over the range of f16 activations: 32 of one sign sum to up to 32 x 65504, which the kernels hold as f16 parts, and small ones to f16
+subnormals.  Against float64, at the sizes of each kernel that does so, with a workspace and without.
+
+The tolerance is that of the other Q4_K tests: f32 accumulators that round once per 16 or 32 k and share, sums of x that round once per addition and to
+23 bits as parts, all relative to what the two terms of a weight may reach before they cancel, and the f16 rounding of the output."""
+import numpy as np
+import pytest
+import torch
+
+from ratchet_amd import DType, Tensor
+
+pytestmark = pytest.mark.gpu
+
+FEW = [(70, 8448, 3), (1030, 8448, 8), (1000, 4352, 9), (640, 10240, 16)]  # K shared, and whole without a workspace
+PREFILL = [(3072, 512, 64), (8192, 512, 200), (8192, 768, 300)]  # one and two weight tiles per wavefront, with and without loading wavefronts
+
+
+def product(oracle, device, m, k, n, x, d_exp, seed):
+    """got, want and the magnitudes of the terms, for weights d * sc * q - dmin * mn of d about 2^d_exp and terms of one size."""
+    rng = np.random.default_rng(seed)
+    blocks = rng.integers(0, 256, (m * k // 256, 144), dtype=np.uint8)
+    blocks[:, :4] = (rng.uniform(0.5, 2, (len(blocks), 2)) * np.array([2.0**d_exp, 2.0 ** (d_exp + 3)])).astype(np.float16).view(np.uint8)
+    w = torch.from_numpy(np.asarray(oracle.q4k_dequantize(blocks.reshape(-1)), dtype=np.float64).reshape(m, k)).to("cuda:0")
+    sb = torch.from_numpy(blocks[:, :4].copy().view(np.float16).astype(np.float64).reshape(m, k // 256, 2)).to("cuda:0")
+    X = torch.from_numpy(x).to("cuda:0")
+    t = Tensor((n, k), DType.F16, device, X.view(torch.uint8).reshape(-1))
+    got = Tensor.from_quantized(blocks.reshape(-1), DType.Q4_K, (m, k), device).gemm(t, None, False, True, True).resolve()
+    got = got.storage.view(torch.float16)[: m * n].view(n, m).double()
+    mag = X.double().abs().view(n, -1, 256).sum(-1) @ (945 * sb[..., 0] + 63 * sb[..., 1]).T
+    return got, X.double() @ w.T, mag
+
+
+@pytest.mark.parametrize("split", [True, False])
+@pytest.mark.parametrize("size,d_exp", [(5000.0, -18), (65504.0, -22), (2.0**-14, -2)])
+@pytest.mark.parametrize("m,k,n", FEW + PREFILL)
+def test_one_sign_per_block(device, oracle, monkeypatch, m, k, n, size, d_exp, split):
+    import ratchet_amd.tensor as mirror
+    monkeypatch.setattr(mirror, "SPLIT_K", split)
+    rng = np.random.default_rng(m + k + n)
+    sign = np.repeat(rng.choice([-1.0, 1.0], (n, k // 32)), 32, axis=1)
+    x = (sign * rng.uniform(0.9, 1.0, (n, k)) * size).astype(np.float16)
+    got, want, mag = product(oracle, device, m, k, n, x, d_exp, m + k)
+    assert want.abs().max() < 60000  # (in f16)
+    err = (got - want).abs()
+    assert (err <= 2.0**-11 * want.abs() + 2.0**-24 * (k / 256 * 2 + 54) * mag + 2.0**-25).all(), float((err / mag).max())
