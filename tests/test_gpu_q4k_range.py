@@ -43,3 +43,38 @@ def test_one_sign_per_block(device, oracle, monkeypatch, m, k, n, size, d_exp, s
     assert want.abs().max() < 60000  # (in f16)
     err = (got - want).abs()
     assert (err <= 2.0**-11 * want.abs() + 2.0**-24 * (k / 256 * 2 + 54) * mag + 2.0**-25).all(), float((err / mag).max())
+
+
+@pytest.mark.parametrize("split", [True, False])
+@pytest.mark.parametrize("bias", [True, False])
+@pytest.mark.parametrize("stack,m,k,n", [((), 70, 8448, 3), ((), 2560, 10240, 5), ((), 1030, 8448, 8), ((2,), 130, 14336, 4)])
+def test_infinite_activation(device, oracle, monkeypatch, stack, m, k, n, bias, split):
+    """3 to 8 rows: a weight times an infinity is one, of its sign, with a workspace and without; the other rows' outputs are what they would be."""
+    import ratchet_amd.tensor as mirror
+    monkeypatch.setattr(mirror, "SPLIT_K", split)
+    rng = np.random.default_rng(m + k + n)
+    s = stack[0] if stack else 1
+    blocks = rng.integers(0, 256, (s * m * k // 256, 144), dtype=np.uint8)
+    blocks[:, :4] = (rng.uniform(0.5, 2, (len(blocks), 2)) / 1024).astype(np.float16).view(np.uint8)
+    w = torch.from_numpy(np.asarray(oracle.q4k_dequantize(blocks.reshape(-1)), dtype=np.float64).reshape(s, m, k)).to("cuda:0")
+    sb = torch.from_numpy(blocks[:, :4].copy().view(np.float16).astype(np.float64).reshape(s, m, k // 256, 2)).to("cuda:0")
+    x = rng.standard_normal((*stack, n, k)).astype(np.float16)
+    x.reshape(s, n, k)[0, 1, 777] = np.inf
+    x.reshape(s, n, k)[s - 1, n - 1, [0, k - 1]] = -np.inf, np.inf
+    X, b = torch.from_numpy(x).to("cuda:0"), torch.from_numpy(rng.standard_normal(m).astype(np.float16)).to("cuda:0")
+    t = lambda v: Tensor(tuple(v.shape), DType.F16, device, v.contiguous().view(torch.uint8).reshape(-1))
+    W = Tensor.from_quantized(blocks.reshape(-1), DType.Q4_K, (*stack, m, k), device)
+    for to in (True, False):
+        got = W.gemm(t(X), t(b) if bias and to else None, False, True, to).resolve().storage.view(torch.float16)[: s * m * n]
+        got = (got.view(s, n, m) if to else got.view(s, m, n).transpose(1, 2)).double()
+        for i in range(s):
+            xd = X.view(s, n, k)[i].double()
+            want = (xd[:, None, :] * w[i][None]).sum(-1) + (b.double() if bias and to else 0)
+            finite = xd.isfinite().all(1)
+            mag = xd.abs().view(n, -1, 256).sum(-1) @ (945 * sb[i, ..., 0] + 63 * sb[i, ..., 1]).T + 2
+            err = (got[i] - want).abs()
+            assert (err <= 2.0**-11 * want.abs() + 2.0**-24 * (k / 256 * 2 + 54) * mag + 2.0**-25)[finite].all()
+            special = ~finite
+            assert int(special.sum()) == len({(0, 1), (s - 1, n - 1)} & {(i, j) for j in range(n)})
+            assert torch.equal(got[i][special].isnan(), want[special].isnan())
+            assert torch.equal(got[i][special].nan_to_num(0.0), want[special].nan_to_num(0.0)) and not got[i][special].isfinite().any()
