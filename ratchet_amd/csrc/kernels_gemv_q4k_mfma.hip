@@ -10,7 +10,10 @@
 // integer below 1024 (exact in f16), so the eight sub-blocks of a super-block chain
 // through one accumulator and d is applied once, in f32; the second term is one more
 // MFMA whose K axis holds the eight sub-block sums of x split into f16 high and low
-// parts (exact to 2^-22) against the integer mins.  No weight is ever rounded.
+// parts against the integer mins.  No weight is ever rounded.  32 f16 activations sum to up
+// to 32 * 65504, so the parts hold S / 32 (dot products against 1 / 32, exact; dmin takes the 32):
+// h = S / 32 rounded and l = (S / 32 - h) * 2^11 rounded, the latter against mn * 2^-11; together 23
+// bits of S.  (Held without the scales a sum beyond 65504 was infinite there and the output NaN.)
 //
 // The block stream is read once, straight from HBM into registers: a lane issues three
 // 16-byte loads per super-block (the header and two pieces of qs) for row n = lane % 16;
@@ -43,13 +46,20 @@ constexpr int kQ4kXPad = 8;
 
 __device__ __forceinline__ int q4k_x_koff(int g) { return 16 * (g & 1) + 8 * (g >> 1); }
 
-// 4 bytes holding integers 0..255 -> two half2 holding the same integers (1024 + b, minus 1024).
+// 4 bytes holding integers 0..255 -> two half2 holding the same integers (1024 + b, minus 1024), or those times f, exactly for a power of two.
 __device__ __forceinline__ void q4k_bytes_to_half(uint32_t v, half2_t &lo, half2_t &hi) {
     const uint32_t a = __builtin_amdgcn_perm(0x64646464u, v, 0x04010400u);
     const uint32_t b = __builtin_amdgcn_perm(0x64646464u, v, 0x04030402u);
     const half2_t k = {(half_t)1024.0f, (half_t)1024.0f};
     lo = __builtin_bit_cast(half2_t, a) - k;
     hi = __builtin_bit_cast(half2_t, b) - k;
+}
+__device__ __forceinline__ void q4k_bytes_to_half(uint32_t v, half2_t &lo, half2_t &hi, half_t f) {
+    const uint32_t a = __builtin_amdgcn_perm(0x64646464u, v, 0x04010400u);
+    const uint32_t b = __builtin_amdgcn_perm(0x64646464u, v, 0x04030402u);
+    const half2_t f2 = {f, f}, k = f2 * (half_t)-1024.0f;
+    lo = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, a), f2, k);
+    hi = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, b), f2, k);
 }
 
 // 8 nibble-bytes (two dwords, each byte 0..15) -> 8 halfs holding sc * nibble, exactly:
@@ -172,10 +182,10 @@ __global__ __launch_bounds__(1024) void gemv_q4k_mfma_kernel(GemvQ4kArgs g) {
     for (int i = 0; i < XL; i++) {
         const int v = i * 64 + lane;
         const half8_t h = __builtin_bit_cast(half8_t, xv[i]);
-        const half2_t one2 = {(half_t)1, (half_t)1};
+        const half2_t part32 = {(half_t)0.03125f, (half_t)0.03125f};
         float sum = 0.f;
 #pragma unroll
-        for (int e = 0; e < 4; e++) sum = __builtin_amdgcn_fdot2(half2_t{h[2 * e], h[2 * e + 1]}, one2, sum, false);
+        for (int e = 0; e < 4; e++) sum = __builtin_amdgcn_fdot2(half2_t{h[2 * e], h[2 * e + 1]}, part32, sum, false);
         sum += wave_dpp<0xB1>(sum); // quad_perm [1,0,3,2]: four consecutive lanes hold the four vectors of a sub-block
         sum += wave_dpp<0x4E>(sum); // quad_perm [2,3,0,1]
         if (v < nvec) {
@@ -183,7 +193,7 @@ __global__ __launch_bounds__(1024) void gemv_q4k_mfma_kernel(GemvQ4kArgs g) {
             *(uint4_t *)(xs + j * XROW + 8 * kv) = xv[i];
             if ((kv & 3) == 0) {
                 const half_t hi = (half_t)sum;
-                const half_t lo = (half_t)(sum - (float)hi);
+                const half_t lo = (half_t)fmaf((float)hi, -2048.0f, sum * 2048.0f); // exact up to the last rounding
                 sxs[j * 16 + (kv >> 2)] = hi;
                 sxs[j * 16 + 8 + (kv >> 2)] = lo;
             }
@@ -191,6 +201,7 @@ __global__ __launch_bounds__(1024) void gemv_q4k_mfma_kernel(GemvQ4kArgs g) {
     }
     asm volatile("" ::: "memory"); // the reads below are by the same wavefront; DS operations complete in order
 
+    const half_t mf = (half_t)(grp == 0 ? 1.0f : grp == 1 ? 1.0f / 2048.0f : 0.0f); // the min term's factor: of the high parts, the low parts, unused K
     const int xj = min(n, NC - 1); // lanes beyond NC re-read a valid row; their outputs are dropped
     const half_t *xrow = xs + xj * XROW + q4k_x_koff(grp);
 #pragma unroll
@@ -198,7 +209,7 @@ __global__ __launch_bounds__(1024) void gemv_q4k_mfma_kernel(GemvQ4kArgs g) {
         const uint4_t hdr = hdr_[rg], qa = qa_[rg], qb = qb_[rg];
         // 4. unpack the 6-bit scales and mins (ggml get_scale_min_k4), four per dword
         const half2_t dm = __builtin_bit_cast(half2_t, hdr[0]);
-        const float d = live ? (float)dm[0] : 0.f, dmin = live ? (float)dm[1] : 0.f;
+        const float d = live ? (float)dm[0] : 0.f, dmin = live ? 32.0f * (float)dm[1] : 0.f;
         const uint32_t S0 = hdr[1], S1 = hdr[2], S2 = hdr[3];
         const uint32_t sc03 = S0 & 0x3F3F3F3Fu, mn03 = S1 & 0x3F3F3F3Fu;
         const uint32_t sc47 = (S2 & 0x0F0F0F0Fu) | ((S0 >> 2) & 0x30303030u);
@@ -206,8 +217,8 @@ __global__ __launch_bounds__(1024) void gemv_q4k_mfma_kernel(GemvQ4kArgs g) {
         half2_t sch[4], mnh[4];
         q4k_bytes_to_half(sc03, sch[0], sch[1]);
         q4k_bytes_to_half(sc47, sch[2], sch[3]);
-        q4k_bytes_to_half(mn03, mnh[0], mnh[1]);
-        q4k_bytes_to_half(mn47, mnh[2], mnh[3]);
+        q4k_bytes_to_half(mn03, mnh[0], mnh[1], mf);
+        q4k_bytes_to_half(mn47, mnh[2], mnh[3], mf);
         auto scale_of = [&](int j) -> half_t { return sch[j >> 1][j & 1]; };
 
         // 5. regroup so that every lane holds 8 nibbles of each of the 8 sub-blocks:
@@ -231,8 +242,7 @@ __global__ __launch_bounds__(1024) void gemv_q4k_mfma_kernel(GemvQ4kArgs g) {
             }
         }
         // 6. the min term: K slots 0..7 = high parts of the 8 sub-block sums, 8..15 = low parts, rest zero
-        half8_t bm = {mnh[0][0], mnh[0][1], mnh[1][0], mnh[1][1], mnh[2][0], mnh[2][1], mnh[3][0], mnh[3][1]};
-        if (grp >= 2) bm = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+        const half8_t bm = {mnh[0][0], mnh[0][1], mnh[1][0], mnh[1][1], mnh[2][0], mnh[2][1], mnh[3][0], mnh[3][1]};
         const half8_t am = __builtin_bit_cast(half8_t, *(const uint4_t *)(sxs + xj * 16 + 8 * (grp & 1)));
         const float4_t zero = {0.f, 0.f, 0.f, 0.f};
         const float4_t T = __builtin_amdgcn_mfma_f32_16x16x32_f16(am, bm, zero, 0, 0, 0);

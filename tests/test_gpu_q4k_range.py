@@ -13,6 +13,7 @@ pytestmark = pytest.mark.gpu
 
 FEW = [(70, 8448, 3), (1030, 8448, 8), (1000, 4352, 9), (640, 10240, 16)]  # K shared, and whole without a workspace
 PREFILL = [(3072, 512, 64), (8192, 512, 200), (8192, 768, 300)]  # one and two weight tiles per wavefront, with and without loading wavefronts
+STREAM = [(520, 1024, 1), (520, 4096, 2), (512, 8192, 4), (1030, 5120, 8), (512, 4096, 16), (8192, 512, 16), (1030, 768, 29)]  # gemv_q4k_mfma_kernel
 WIDE = [(8192, 768, 1000), (7937, 1280, 1001)]  # gemm_q4k_wide_kernel
 
 
@@ -33,7 +34,7 @@ def product(oracle, device, m, k, n, x, d_exp, seed):
 
 @pytest.mark.parametrize("split", [True, False])
 @pytest.mark.parametrize("size,d_exp", [(5000.0, -18), (65504.0, -22), (2.0**-14, -2)])
-@pytest.mark.parametrize("m,k,n", FEW + PREFILL + WIDE)
+@pytest.mark.parametrize("m,k,n", FEW + PREFILL + WIDE + STREAM)
 def test_one_sign_per_block(device, oracle, monkeypatch, m, k, n, size, d_exp, split):
     import ratchet_amd.tensor as mirror
     monkeypatch.setattr(mirror, "SPLIT_K", split)
