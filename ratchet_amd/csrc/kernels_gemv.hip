@@ -28,6 +28,7 @@ struct GemvArgs {
     int64_t b_bs, b_js;
     int64_t o_bs, o_is, o_js;
     int has_bias, bias_on_rows, act;
+    int64_t row_first; // gemv_q8f_kernel: this launch's first weight row
 };
 
 constexpr int kGemvThreads = 256;
@@ -125,7 +126,7 @@ __global__ __launch_bounds__(kGemvThreads) void gemv_q8f_kernel(GemvArgs g) {
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int64_t s = blockIdx.y, sa = g.a_stack == 1 ? 0 : s, sb = g.b_stack == 1 ? 0 : s; // an operand's stack is either the full stack or 1 (broadcast)
     const float *x = (const float *)g.X + sb * g.b_bs;
-    const int64_t row0 = (int64_t)blockIdx.x * R;
+    const int64_t row0 = g.row_first + (int64_t)blockIdx.x * R;
     const uint8_t *q[R];
     const float *sc[R];
 #pragma unroll
@@ -508,10 +509,15 @@ hipError_t launch_gemv(const Problem &p, const void *A, const void *B, const voi
         const uint64_t numel = (uint64_t)p.a_stack * p.M * p.K;
         g.scales = (const uint8_t *)A + rt_q8_0_scale_offset(numel);
         if (p.a_dt == RT_Q8_0F) {
-            const int64_t groups = (p.M + kQ8fRows - 1) / kQ8fRows;
-            if (groups > 0x7fffffff || p.K > 0x7fffffff - 8192) return hipErrorNotSupported; // (its steps count in 32 bits)
-            grid.x = (unsigned)groups;
-            RT_DISPATCH_NC(p.N, launch_q8f<NC>(grid, stream, g));
+            if (p.K > 0x7fffffff - 8192) return hipErrorNotSupported; // (its steps count in 32 bits)
+            // a launch's threads along an axis are fewer than 2^32: 67 million rows and more go in several
+            const int64_t groups = (p.M + kQ8fRows - 1) / kQ8fRows, most = 0xffffffffu / kGemvThreads;
+            for (int64_t first = 0; first < groups; first += most) {
+                grid.x = (unsigned)std::min(groups - first, most), g.row_first = first * kQ8fRows;
+                RT_DISPATCH_NC(p.N, launch_q8f<NC>(grid, stream, g));
+                if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+            }
+            return hipSuccess;
         } else {
             RT_DISPATCH_NC(p.N, launch_q8<NC>(grid, stream, g));
         }

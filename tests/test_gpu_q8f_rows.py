@@ -68,3 +68,22 @@ def test_infinite_activation(device):
     out = Tensor.from_quantized(raw, DType.Q8_0F, (10, 288), device).gemm(Tensor.from_data(x, None, device), None, False, True, True).resolve()
     out = out.storage.view(torch.float32)[:30].view(3, 10).cpu().numpy()
     assert np.isfinite(out[[0, 2]]).all() and (out[1] == np.where(w[:, 287] == 0, np.nan, np.sign(w[:, 287]) * np.inf))[w[:, 287] != 0].all()
+
+
+@pytest.mark.parametrize("n", (1, 2))
+def test_more_rows_than_one_launch(device, n):
+    """A launch's threads number less than 2^32, 2^24 - 1 workgroups of four rows: the rows beyond go in a second one.  On both sides of that, and at either end."""
+    m, k = 2**26 + 5, 32
+    gen = torch.Generator("cuda:0").manual_seed(n)
+    codes = torch.empty((m, k), dtype=torch.int8, device="cuda:0").random_(-127, 128, generator=gen)
+    d = torch.rand(m, generator=gen, device="cuda:0") / 64 + 2.0**-8
+    pad = lambda b: torch.nn.functional.pad(b.view(torch.uint8).reshape(-1), (0, -b.numel() * b.element_size() % 256))
+    x, bias = torch.randn((n, k), generator=gen, device="cuda:0"), torch.randn(m, generator=gen, device="cuda:0")
+    t = lambda v, shape, dt=DType.F32: Tensor(shape, dt, device, v.contiguous().view(torch.uint8).reshape(-1))
+    got = t(torch.cat([pad(codes), pad(d)]), (m, k), DType.Q8_0F).gemm(t(x, (n, k)), t(bias, (m,)), False, True, True).resolve().storage.view(torch.float32)[: m * n].view(n, m)
+    assert got.isfinite().all()
+    edge = 4 * (2**24 - 1)
+    for rows in (slice(0, 64), slice(edge - 64, edge + 64), slice(m - 64, m)):
+        w = codes[rows].double() * d[rows].double()[:, None]
+        want, mag = x.double() @ w.T + bias[rows].double(), x.double().abs() @ w.abs().T
+        assert ((got[:, rows] - want).abs() <= 2.0**-24 * (16 * mag + want.abs())).all()
