@@ -394,7 +394,7 @@ rt_status rt_matmul_workspace_bytes(rt_ctx *ctx, const rt_matmul_desc *desc, uin
     if (p.kernel == RT_KERNEL_GEMV_Q4K && p.N >= 3) *bytes = rt::gemm_q4k_workspace_bytes(p, ctx->dev);
     if (p.kernel == RT_KERNEL_GEMV_Q8 && rt::gemm_nt_q8h_few(p, ctx->dev)) *bytes = rt::gemm_nt_workspace_bytes(p, ctx->dev);
     if (p.kernel == RT_KERNEL_GEMM_F16) *bytes = p.a_dt == RT_Q4_K ? rt::gemm_q4k_workspace_bytes(p, ctx->dev) : rt::gemm_nt_workspace_bytes(p, ctx->dev);
-    if (p.kernel == RT_KERNEL_GEMM_F32) *bytes = rt::gemm_limb_workspace_bytes(p, ctx->dev);
+    if (p.kernel == RT_KERNEL_GEMM_F32 && !rt::gemv_q8f_chunks(p)) *bytes = rt::gemm_limb_workspace_bytes(p, ctx->dev);
     return RT_OK;
     RT_GUARD_END(ctx)
 }

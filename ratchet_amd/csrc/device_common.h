@@ -177,6 +177,7 @@ hipError_t launch_gemm_stream(const Problem &p, const void *A, const void *B, co
 uint64_t gemm_nt_workspace_bytes(const Problem &p, const DeviceInfo &dev);
 bool gemm_nt_static_split(const Problem &p, const DeviceInfo &dev);
 bool gemv_chunks_unless_shared(const Problem &p, const DeviceInfo &dev);
+bool gemv_q8f_chunks(const Problem &p);
 hipError_t gemv_chunks(const Problem &p, const void *A, const void *B, const void *bias, void *out, hipStream_t stream, const DeviceInfo &dev);
 bool gemv_q4k_mfma_fits(const Problem &p, const DeviceInfo &dev);
 bool gemv_q8h_mfma_well(const Problem &p, const DeviceInfo &dev);

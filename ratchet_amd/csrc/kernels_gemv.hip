@@ -118,6 +118,8 @@ __global__ __launch_bounds__(kGemvThreads) void gemv_q8_kernel(GemvArgs g) {
 // vector), then by the vector instructions: 84 for a lane's four codes of four rows against eight vectors, and by the loads of the activations.
 // ---------------------------------------------------------------------------
 constexpr int kQ8fRows = 4;
+constexpr int kQ8fLongK = 1024; // from here on the sums are no less exact than the limb kernel's (gemv_q8f_chunks)
+typedef float float4_u __attribute__((ext_vector_type(4), aligned(4))); // activations start at any f32: the loads take them as they are
 template <int NC, int U>
 __global__ __launch_bounds__(kGemvThreads) void gemv_q8f_kernel(GemvArgs g) {
     constexpr int R = kQ8fRows;
@@ -160,7 +162,7 @@ __global__ __launch_bounds__(kGemvThreads) void gemv_q8f_kernel(GemvArgs g) {
                     for (int e = 0; e < 4; e++) wf[r][e] = (float)(int8_t)(w[u][r] >> (8 * e));
 #pragma unroll
                 for (int j = 0; j < NC; j++) {
-                    const float4_t xv = *(const float4_t *)(x + j * g.b_js + k);
+                    const float4_t xv = *(const float4_u *)(x + j * g.b_js + k);
 #pragma unroll
                     for (int r = 0; r < R; r++) {
                         float p = wf[r][0] * xv[0];
@@ -405,8 +407,8 @@ bool gemv_chunks_unless_shared(const Problem &p, const DeviceInfo &dev) {
 // 25 and 9.6 / 10.9; 384 x 1536 12.5, 28 and 6.8 / 7.7).  Beyond 4096 rows or five million codes that kernel fills the device and reads the codes
 // once (4096 x 2560 15.4, here 12.6 / 17.1; 8192 x 640 13.5, here 11.3 / 14.7).  From K = 1024 on, since the sums are no less exact there (relative error
 // against float64 at K = 800 / 1280 / 2048 / 4096 here 9.4e-8 / 9.5e-8 / 9.6e-8 / 9.9e-8, there 9.2e-8 / 9.8e-8 / 1.08e-7 / 1.29e-7).
-static bool gemv_q8f_chunks(const Problem &p) {
-    return p.a_dt == RT_Q8_0F && p.act_dt == RT_F32 && p.N > kGemvMaxCols && p.N <= 2 * kGemvMaxCols && p.stacks == 1 && p.b_ks == 1 && p.K >= 1024 &&
+bool gemv_q8f_chunks(const Problem &p) {
+    return p.a_dt == RT_Q8_0F && p.act_dt == RT_F32 && p.N > kGemvMaxCols && p.N <= 2 * kGemvMaxCols && p.stacks == 1 && p.b_ks == 1 && p.K >= kQ8fLongK &&
            p.M <= 4096 && p.M * p.K <= 5 << 20;
 }
 hipError_t launch_gemv_chunked(const Problem &p, const void *A, const void *B, const void *bias, void *out, hipStream_t stream, const DeviceInfo &dev) {
@@ -415,7 +417,7 @@ hipError_t launch_gemv_chunked(const Problem &p, const void *A, const void *B, c
             Problem c = p;
             c.N = std::min<int64_t>(p.N - j0, kGemvMaxCols), c.kernel = RT_KERNEL_GEMV_Q8;
             const float *bc = bias && !p.bias_on_rows ? (const float *)bias + j0 : (const float *)bias;
-            // what it declines (a misaligned operand) it declines on the first chunk
+            // what it declines (a weight off 16 bytes) it declines on the first chunk
             if (const hipError_t e = launch_gemv(c, A, (const float *)B + j0 * p.b_js, bc, (float *)out + j0 * p.o_js, stream, dev); e != hipSuccess) return e;
         }
         return hipSuccess;
@@ -505,7 +507,10 @@ hipError_t launch_gemv(const Problem &p, const void *A, const void *B, const voi
 
     switch (p.kernel) {
     case RT_KERNEL_GEMV_Q8: {
-        if (!x_ok || !aligned16(A) || p.K % 32 != 0) return hipErrorNotSupported;
+        // gemv_q8f_kernel's loads take vectors at any f32: from K = 1024 on, as gemv_q8f_chunks, which asks for no workspace whatever the pointer (us, the
+        // limb kernel and this: 10240 x 2560 at 1 / 8 vectors 44.6 and 7.6 / 17.9, 1001 x 4096 at 12, with a workspace there, 21.1 and 9.0)
+        const bool any_f32 = p.a_dt == RT_Q8_0F && p.K >= kQ8fLongK && ((uintptr_t)B & 3u) == 0;
+        if (!(x_ok || any_f32) || !aligned16(A) || p.K % 32 != 0) return hipErrorNotSupported;
         const uint64_t numel = (uint64_t)p.a_stack * p.M * p.K;
         g.scales = (const uint8_t *)A + rt_q8_0_scale_offset(numel);
         if (p.a_dt == RT_Q8_0F) {

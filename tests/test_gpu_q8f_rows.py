@@ -3,11 +3,13 @@ the four wavefronts' steps, stacks, both orders of the output, bias along either
 
 The tolerance: a product is rounded once, four of them and their scale's make five roundings, a lane adds one sum per 1024 k, and ten additions
 join the lanes and wavefronts: 2^-24 of the magnitudes for each, and one for the bias.  The limb kernel adds a sum per MFMA of 32 k."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
-from ratchet_amd import DType, Tensor
+from ratchet_amd import DType, Tensor, _ffi
 
 pytestmark = pytest.mark.gpu
 
@@ -44,7 +46,7 @@ def test_against_float64(device, stack, m, k, n):
 @pytest.mark.parametrize("m,k", [(1, 1024), (4096, 1024), (4097, 1024), (33, 992), (1279, 4096), (1281, 4096), (130, 4128)])
 def test_two_launches(device, m, k, n):
     """9 to 16 vectors go in two launches at K >= 1024, up to 4096 rows and 5 x 2^20 codes: on both sides of each of these, the vectors also 4 bytes past an
-    aligned address (the limb kernel takes those)."""
+    aligned address."""
     rng = np.random.default_rng(m + k + n)
     raw, w = make(m, k, rng)
     x, bm, bn = (rng.standard_normal(s).astype(np.float32) for s in ((n, k), m, n))
@@ -87,3 +89,27 @@ def test_more_rows_than_one_launch(device, n):
         w = codes[rows].double() * d[rows].double()[:, None]
         want, mag = x.double() @ w.T + bias[rows].double(), x.double().abs() @ w.abs().T
         assert ((got[:, rows] - want).abs() <= 2.0**-24 * (16 * mag + want.abs())).all()
+
+
+@pytest.mark.parametrize("n", (1, 2, 5, 8, 9, 16))
+def test_vectors_at_any_address(device, n):
+    """One kernel whatever 4-byte address the vectors start at, for which no workspace is asked: the same bits as on an aligned one."""
+    m, k = 1003, 1056
+    rng = np.random.default_rng(n)
+    raw, _ = make(m, k, rng)
+    x = torch.from_numpy(rng.standard_normal((n, k)).astype(np.float32)).to("cuda:0")
+    W = Tensor.from_quantized(raw, DType.Q8_0F, (m, k), device)
+    outs = []
+    for at in (0, 4, 8, 12, 20):
+        room = torch.zeros(4 * n * k + 32, dtype=torch.uint8, device="cuda:0")
+        room[at : at + 4 * n * k] = x.view(torch.uint8).reshape(-1)
+        out = W.gemm(Tensor((n, k), DType.F32, device, room[at : at + 4 * n * k]), None, False, True, True).resolve()
+        outs.append(out.storage.view(torch.float32)[: m * n].clone())
+    assert outs[0].isfinite().all() and all(torch.equal(outs[0], o) for o in outs[1:])
+
+
+@pytest.mark.parametrize("m,k,n,asks", [(1001, 4096, 8, False), (1001, 4096, 9, False), (1001, 4096, 16, False), (1001, 4096, 17, True), (1001, 992, 16, True), (4097, 1024, 16, True)])
+def test_workspace_only_where_it_is_used(device, m, k, n, asks):
+    d, need = _ffi.make_desc(DType.Q8_0F, (m, k), DType.F32, (n, k), False, True, True), ctypes.c_uint64()
+    assert _ffi.lib().rt_matmul_workspace_bytes(device.ctx, ctypes.byref(d), ctypes.byref(need)) == _ffi.RT_OK
+    assert (need.value > 0) == asks
