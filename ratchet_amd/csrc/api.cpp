@@ -148,7 +148,7 @@ constexpr Launcher kLaunchers[] = {rt::launch_gemv,          // streaming kernel
                                    rt::launch_gemm_f32_small, // f32 products too small to split into limbs
                                    rt::launch_gemm_limb,     // f32 activations against f32 operands or Q8_0F weights: bf16 matrix cores, exact limbs
                                    rt::launch_gemm_f32,      // f32 products whose operands each have a contiguous axis
-                                   rt::launch_gemm_q4k,      // Q4_K weights against many activation rows
+                                   rt::launch_gemm_q4k,      // Q4_K weights against many activation rows, and against few where K is too long for the streaming kernels
                                    rt::launch_gemm};         // anything
 constexpr int kNumLaunchers = (int)(sizeof(kLaunchers) / sizeof(kLaunchers[0])), kFirstTiled = 2;
 

@@ -33,10 +33,10 @@
 // 3072 x 8192 at 1000 rows 99.8 -> 91.9).  A staged row is 32 K-vectors
 // and one of padding: the 16 rows of a fragment read start 4 banks apart and a read address is a
 // base + 16 * step, an immediate.  One barrier per super-block.  The output tile leaves through LDS
-// as 16-byte stores when the output is contiguous along the weight rows.
+// as 16-byte stores when the output is contiguous along the weight rows.  Also few rows against a K too long for the streaming kernels (gemm_q4k_few).
 //
 // What bounds it (measured by leaving parts out): the parts add up.  A wavefront's MFMAs (8 issue
-// cycles each when vector instructions follow), its 335 vector instructions per super-block and the
+// cycles each when vector instructions follow), its 339 vector instructions per super-block and the
 // LDS pipe time of the compute unit's fragment reads (128 KB per super-block at 128 B/clk) each
 // cost their full time whatever the order of instructions.  Two multiplying wavefronts per SIMD were
 // measured: with 16 x 64 outputs each they double the fragment reads (27.7 against 26.7 us), with
@@ -906,7 +906,7 @@ bool gemm_q4k_few(const Problem &p, const DeviceInfo &dev) {
     return need > 0 && p.workspace && !((uintptr_t)p.workspace & 15u) && p.workspace_bytes >= need;
 }
 
-// Q4_K weights x K-contiguous f16 activations, more rows than one streaming launch takes.
+// Q4_K weights x K-contiguous f16 activations: more rows than one streaming launch takes, and gemm_q4k_few.
 // hipErrorNotSupported: another kernel must take the problem.
 hipError_t launch_gemm_q4k(const Problem &p, const void *A, const void *B, const void *bias, void *out, hipStream_t stream,
                            const DeviceInfo &dev) {
