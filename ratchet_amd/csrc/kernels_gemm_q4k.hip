@@ -897,8 +897,8 @@ uint64_t gemm_q4k_workspace_bytes(const Problem &p, const DeviceInfo &dev) {
 }
 // Whether 3 to 16 vectors are launch_gemm_q4k's: where the streaming matrix-core kernel's LDS ends (9 to 16 from K = 4352, 3 to 8 from 8448 on), up to
 // 8, which the streaming kernel without matrix cores takes, only with K shared.  us, M x K, that or the generic kernel, here, here with K whole: 2560 x 4352 at 9
-// / 16 vectors 71 / 72, 10.3, 18.3; x 10240 161 / 163, 13.5, 38; x 14336 224 / 227, 16, 52; 1280 x 8448 at 3 / 8 15.6 / 23.5, 10.4, 32; 2560 x 10240 at 3 / 5 / 8 18.1 / 23.7 / 33.9,
-// 14.0, 38.
+// / 16 vectors 71 / 72, 10.3, 18.3; x 10240 161 / 163, 13.5, 38; x 14336 224 / 227, 16, 52; 1280 x 8448 at 3 / 8 15.6 / 23.0, 9.7, 32; 2560 x 10240 at 3 / 5 / 8 16.8 / 21.9 / 32.2,
+// 12.5, 38.
 bool gemm_q4k_few(const Problem &p, const DeviceInfo &dev) {
     if (!gemm_q4k_takes(p) || p.N > 16 || gemv_q4k_mfma_fits(p, dev)) return false;
     if (p.N > 8) return true;
